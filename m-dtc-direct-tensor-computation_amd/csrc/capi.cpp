@@ -606,11 +606,11 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
                 else DTC_TRY(batch_add_domain(sb, b->mesh, d, mod, b->escale[i], R * g, s));
             }
         }
-        DTC_TRY(batch_finalize(sb, precision));
         // the multigrid preconditioner of the mixed solve: the geometric V-cycle over
         // the voxel lattice (HEX08 micro), or for HEX20 micro elements a p-multigrid
         // whose coarse space is the HEX08 twin of the same voxels and domain groups
         sb.precond = (precision == DTC_FP32_REFINE && b->o.precond == DTC_PC_MG) ? DTC_PC_MG : DTC_PC_JACOBI;
+        DTC_TRY(batch_finalize(sb, precision));
         sb.mg_degree = b->o.mg_degree > 0 ? b->o.mg_degree : 2;
         sb.p08 = nullptr;
         if (sb.micro20 && sb.precond == DTC_PC_MG) {
@@ -620,6 +620,7 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
             tw.a = b->a0;
             tw.micro20 = false;
             tw.timing = false;
+            tw.precond = sb.precond;
             DTC_TRY(batch_begin(tw, gd.data(), (int64_t)gd.size()));
             for (int i : list) {
                 const dtc_domain_desc& d = b->d[i];
@@ -668,13 +669,10 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
     if (!concurrent) {
         for (int k = 0; k < NS; ++k) DTC_TRY(solve_sub(k, false));
     } else {
-        // multigrid hierarchies and launch-shape tuning one sub-batch after another
-        // (the tuning launches are timed: none may overlap another sub-batch's work),
-        // then concurrent solves, conc at a time (one host thread per sub-batch, each
+        // multigrid hierarchies one sub-batch after another, then concurrent solves, conc at a time (one host thread per sub-batch, each
         // on its stream); the error message of a failed solve is carried back to this thread
         for (int k = 0; k < NS; ++k) {
             DTC_TRY(prep_sub(k));
-            DTC_TRY(batch_autotune(b->subs[k]->sb));
             DTC_HIP(hipStreamSynchronize(b->subs[k]->sb.stream));
         }
         std::vector<int> rc(NS, DTC_OK);

@@ -77,8 +77,7 @@ struct DevMem {
 // ---------------------------------------------------------------- constants
 constexpr int R24 = 24;          // load cases of the HEX08 macro element
 constexpr int BX = 8, BY = 4, BZ = 4;   // owned nodes of one solver brick
-constexpr int HX = BX + 2, HY = BY + 2, HZ = BZ + 2;   // halo node tile
-constexpr int EX = BX + 1, EY = BY + 1, EZ = BZ + 1;   // element tile
+constexpr int EX = BX + 1, EY = BY + 1, EZ = BZ + 1;   // elements that touch a brick's nodes
 
 // HEX08 local node offsets in gen_quadmesh order (f-src/mod_gen_quadmesh.f90:298-306)
 __host__ __device__ constexpr int h08_off(int l, int d) {
@@ -128,6 +127,7 @@ struct DomInfo {
     int lc_base;              // first macro load case of this group of 24
     int bnx, bny, bnz;        // brick grid
     int brick_begin, brick_end;
+    int cl_begin, cl_end;     // HEX08: matvec clusters (ClusterInfo)
     int64_t lat_off;          // offset into the lattice map
     int64_t vox_off;          // offset into the voxel modulus array
     int64_t node_begin, node_end;
@@ -140,7 +140,18 @@ struct BrickInfo {
     int dom;
     int x0, y0, z0;           // first owned lattice node
     int node_begin, node_end; // owned solver nodes (contiguous)
-    int e_off, e_cnt;         // solid elements of the element tile in the brick element tables
+};
+
+// A HEX08 matvec work unit: a run of consecutive solver nodes (of one or more bricks)
+// with every element that touches one of them.  At most CL_CAP nodes, CL_CAP64 in the
+// batches solved in FP64: the cap bounds the accumulators that a workgroup of k_ebe
+// keeps in LDS (288 or 576 bytes a node).
+constexpr int CL_CAP = 128, CL_CAP64 = 64;
+struct ClusterInfo {
+    int dom;
+    int node_begin, node_end;
+    int brick_begin, brick_end;   // bricks that hold the nodes
+    int e_off, e_cnt;             // elements in the cluster element tables
 };
 
 // New Chebyshev-Jacobi direction of one unknown, c1 d + c2 D^-1 (b - t) with t = (K x)
@@ -149,10 +160,6 @@ struct BrickInfo {
 __device__ __forceinline__ float cheb_dir(float c1, float d, float c2, float di, float b, float t) {
     return c1 * d + c2 * di * (b - t);
 }
-
-// brick halo table entries: solver node | BC_BIT for a Dirichlet node, -1 = no node
-constexpr int BC_BIT = 1 << 30;
-constexpr int NODE_MASK = BC_BIT - 1;
 
 // 45 coefficients of the HEX08 element stiffness in the signed Walsh basis
 // (E = 1); see walsh_blocks() in solver.hip.

@@ -12,13 +12,13 @@
 //    Khat is block diagonal (3x3, 2x2, 1x1 blocks, 45 coefficients), so one
 //    element product costs two 8-point Hadamard butterflies per direction
 //    plus 45 multiplies instead of a dense 24x24 product.
-//  * Tiling: the lattice of kept nodes is cut into bricks of 8x4x4 owned
-//    nodes.  A workgroup stages the halo (10x6x6 nodes) of its brick in LDS,
-//    computes every element touching an owned node (9x5x5 voxels) and
-//    accumulates into LDS in 8 parity classes (elements of one class share
-//    no node), then writes its owned nodes once.  No atomics, deterministic.
+//  * Tiling: the lattice of kept nodes is cut into bricks of 8x4x4 nodes, taken
+//    along a Z-curve, and runs of them into clusters of at most 128 nodes.  A
+//    workgroup computes every element that touches a node of its cluster,
+//    adds their outputs up in LDS in a fixed order and writes its nodes once
+//    (ebe.hpp).  No atomics, deterministic.
 //  * Vectors: node-major [node][3][24], nodes numbered brick by brick so a
-//    brick's owned nodes are contiguous.  All 24 load cases advance in
+//    cluster's nodes are contiguous.  All 24 load cases advance in
 //    lockstep with their own alpha/beta; a converged load case freezes.
 //  * Reductions: per-brick partial sums in FP64, then one workgroup per
 //    domain sums them in brick order (deterministic).
@@ -30,10 +30,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
-#include <map>
-#include <mutex>
-#include <tuple>
 #include <type_traits>
 
 #include "bc.hpp"
@@ -46,8 +42,8 @@ namespace {
 constexpr int R = R24;
 constexpr int NT_UPD = 192;    // multiple of 24: a thread keeps one load case
 
-// IN_JS (FP32 Chebyshev step only): x = cin D^-1 v, the first smoothing step from
-// x = 0 formed while staging v, so that it is never stored as a vector
+// IN_U: x with the Dirichlet values; IN_JS (FP32 Chebyshev step only): x = cin D^-1 v, the
+// first smoothing step from x = 0 formed while reading v, so that it is never stored
 enum InMode { IN_V = 0, IN_U = 1, IN_JS = 2 };
 enum OutMode { OUT_MASKED_DOT = 0, OUT_RESID = 1, OUT_PLAIN = 2, OUT_MASKED = 3, OUT_CHEB = 4, OUT_BRES = 5 };
 
@@ -110,8 +106,8 @@ __device__ inline void fht_inv_tail(T v[8]) {
 }
 
 // y = Kw w on the (mode, direction) groups; w, y indexed [mode][dir]
-template <typename T>
-__device__ inline void walsh_apply(const WK<T>& k, const T w[8][3], T y[8][3]) {
+template <typename K, typename T>
+__device__ inline void walsh_apply(const WK<K>& k, const T w[8][3], T y[8][3]) {
 #define M3(o, i0, d0, i1, d1, i2, d2)                                                         \
     {                                                                                         \
         T a0 = w[i0][d0], a1 = w[i1][d1], a2 = w[i2][d2];                                     \
@@ -141,71 +137,12 @@ __device__ inline void walsh_apply(const WK<T>& k, const T w[8][3], T y[8][3]) {
 #undef M2
 }
 
-// ---------------------------------------------------------------- wave sums
-// DPP lane move of an FP64 value (two 32-bit moves); lanes whose source lies
-// outside their 16-lane row receive 0.
-template <int CTRL>
-__device__ inline double dpp_f64(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-// RC partial sums per lane (RC = 4 or 2) -> per 16-lane row, the row sum of each
-// of the RC values, in fixed order: log2(RC) halving exchanges between lane pairs
-// (each lane keeps half of the values and adds its partner's copies), then
-// row_shr by RC, 2 RC, .. 8 accumulates each residue class of the row into its
-// last lanes.  Returns true on the RC lanes 16-RC..15 of each row, which then
-// hold the sum of value `*lc` in `*v`.
-template <int RC>
-__device__ inline bool row_sums(const double (&a)[RC], int lane, double* v, int* lc) {
-    const bool b0 = lane & 1, b1 = lane & 2;
-    double k;
-    int l;
-    if constexpr (RC == 4) {
-        double k0 = b0 ? a[2] : a[0], k1 = b0 ? a[3] : a[1];
-        const double s0 = b0 ? a[0] : a[2], s1 = b0 ? a[1] : a[3];
-        k0 += dpp_f64<0xB1>(s0);   // quad_perm [1,0,3,2]
-        k1 += dpp_f64<0xB1>(s1);
-        k = b1 ? k1 : k0;
-        const double s = b1 ? k0 : k1;
-        k += dpp_f64<0x4E>(s);     // quad_perm [2,3,0,1]
-        l = 2 * (int)b0 + (int)b1;
-        k += dpp_f64<0x114>(k);    // row_shr:4
-        k += dpp_f64<0x118>(k);    // row_shr:8
-    } else {
-        static_assert(RC == 2, "two or four load cases per chunk");
-        k = b0 ? a[1] : a[0];
-        k += dpp_f64<0xB1>(b0 ? a[0] : a[1]);
-        l = (int)b0;
-        k += dpp_f64<0x112>(k);    // row_shr:2
-        k += dpp_f64<0x114>(k);
-        k += dpp_f64<0x118>(k);
-    }
-    *v = k;
-    *lc = l;
-    return (lane & 15) >= 16 - RC;
-}
-
 // ---------------------------------------------------------------- matvec
-// Load cases are processed in chunks of RC: one (node, direction) segment of a
-// chunk is one 16-byte vector V (float4 / double2).
+// RC load cases of one (node, direction) are one 16-byte vector V (float4 / double2)
 template <typename T> struct MvCfg;
 template <> struct MvCfg<float> { static constexpr int RC = 4; using V = float4; };
 template <> struct MvCfg<double> { static constexpr int RC = 2; using V = double2; };
-constexpr int MV_NT = 512;
-constexpr int MV_NT_SP = 256;     // sparse-brick variant
-constexpr int MV_SLOTS = 384;     // (owned node, element corner) pairs of a sparse brick, at most
-constexpr int NH = HX * HY * HZ, NET = EX * EY * EZ, NO = BX * BY * BZ;
-constexpr int OB_BIAS = 1 + BX + BX * BY;   // owned-layout base of tile element (0,0,0) is -OB_BIAS
-
-// offsets of element corner b (bit 0 x, bit 1 y, bit 2 z) in the halo and owned node layouts
-__host__ __device__ constexpr int hcorner(int b) { return (b & 1) + HX * ((b >> 1) & 1) + HX * HY * (b >> 2); }
-__host__ __device__ constexpr int ocorner(int b) { return (b & 1) + BX * ((b >> 1) & 1) + BX * BY * (b >> 2); }
-// halo index of owned node o
-__host__ __device__ constexpr int ohalo(int o) {
-    return (o % BX + 1) + HX * ((o / BX) % BY + 1) + HX * HY * (o / (BX * BY) + 1);
-}
+constexpr int NET = EX * EY * EZ, NO = BX * BY * BZ;   // elements that touch a brick, its nodes
 
 __device__ inline float vcomp(const float4& v, int w) { return w == 0 ? v.x : w == 1 ? v.y : w == 2 ? v.z : v.w; }
 __device__ inline double vcomp(const double2& v, int w) { return w == 0 ? v.x : v.y; }
@@ -216,543 +153,19 @@ __device__ inline double2 vneg(const double2& v) { return make_double2(-v.x, -v.
 __device__ inline void vadd(float4& a, const float4& b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
 __device__ inline void vadd(double2& a, const double2& b) { a.x += b.x; a.y += b.y; }
 
-struct MvArgs {
-    const BrickInfo* bricks;
-    const int* blist;           // bricks of this launch (blist[boff + blockIdx.x]), or null: brick = blockIdx.x
-    int boff;
-    const DomInfo* doms;
-    const int* halo;            // [brick][NH]
-    const unsigned char* nmask; // [brick][NO]: solid tile elements around each owned node
-    const int* einfo;           // tile elements, packed
-    const void* eE;             // tile element moduli (T)
-    const int* done;            // may be null
-    double* partial;            // [brick][24]
-    // OUT_CHEB / OUT_BRES only
-    const void* bvec;           // right-hand side b
-    const void* dinv;           // Jacobi scaling
-    void* dvec;                 // Chebyshev direction
-    float c1, c2;               // Chebyshev coefficients of this step
-    int cflags;                 // CH_* : where the previous direction comes from, whether d is stored
-    float cin = 0.f;            // IN_JS: the zero-start step's coefficient
-};
 // OUT_CHEB direction handling: the previous direction d is read from dvec
 // (CH_READ_D), or equals the current iterate (CH_D_FROM_X: the step after a
 // zero-start step, where x_1 = d_0), or is absent (c1 = 0); the new direction
 // is stored only when a later step reads it (CH_WRITE_D).
 constexpr int CH_READ_D = 1, CH_D_FROM_X = 2, CH_WRITE_D = 4;
 
-// y = K x for every brick of the batch.  One workgroup per (brick, chunk
-// range): blockIdx.y splits the NCH chunks into gridDim.y equal ranges, so that
-// small grids (coarse multigrid levels, single domains) still fill the chip.
-// Chunk loop over the load cases:
-//   stage   the halo of x (10x6x6 nodes) goes to LDS (16-byte loads, issued
-//           one chunk ahead into registers);
-//   product every solid element of the 9x5x5 tile is one task per load case
-//           (Walsh-basis product); the output of corner b lands in the corner
-//           buffer b at the owned node it belongs to.  A (corner, node) slot
-//           has exactly one element, so plain stores suffice: no atomics, no
-//           colouring barriers;
-//   gather  each owned (node, direction) sums its corner buffers in corner
-//           order (deterministic) and is written once.
-// OUT_MASKED_DOT zeroes Dirichlet rows and writes per-brick sums of x.y;
 // the zero-start smoothing step fused into the next step (DTC_CHEB_FUSE=0: stored by k_cheb)
 inline bool cheb_fuse() {
     const char* e = std::getenv("DTC_CHEB_FUSE");
     return !(e && e[0] == '0');
 }
 
-// whole-segment output stores of the FP32 matvec (DTC_MV_DEFER=0: per-chunk stores)
-inline bool mv_defer() {
-    const char* e = std::getenv("DTC_MV_DEFER");
-    return !(e && e[0] == '0');
-}
-
-// OUT_RESID writes -y on free rows and sums y.y; OUT_PLAIN writes y;
-// OUT_MASKED zeroes Dirichlet rows; OUT_BRES writes b - y on free rows and 0 on
-// Dirichlet rows; OUT_CHEB applies one Chebyshev-Jacobi step to the owned nodes,
-//   d = c1 d + c2 D^-1 (b - y),  yout = x + d   (yout must not alias x),
-// and, when partial is set, writes per-brick sums of b . yout.
-// launch bounds: at least 4 waves per SIMD (2 workgroups of 8 waves per CU), which
-// caps the kernel at 128 VGPRs
-// IO32 (T = double, IN_V only): 1 = x and y are FP32 vectors, 2 = x is an FP32
-// vector and y an FP64 one; the arithmetic is FP64
-// SPARSE: the variant for bricks with at most MV_SLOTS (owned node, element corner)
-// pairs: 256 threads, and the corner outputs go to compact slots (the pairs of
-// each owned node, in corner order, after those of the nodes before it) instead
-// of 8 full corner buffers, so that four workgroups fit one CU.  The sums are
-// those of the dense form without its zero terms: the results are identical.
-// PART (OUT_CHEB): per-brick sums of b . x are written (A.partial set).
-template <typename T, int IN, int OUT, int IO32 = 0, bool SPARSE = false, bool PART = false, bool DEFER_Y = true>
-__global__ __launch_bounds__(SPARSE ? MV_NT_SP : MV_NT, 4) void k_matvec(MvArgs A, WK<T> wk, const T* __restrict__ xin,
-                                                                      T* __restrict__ yout) {
-    constexpr int RC = MvCfg<T>::RC, SX = 3 * RC, NCH = R / RC;
-    using V = typename MvCfg<T>::V;
-    constexpr int NT = SPARSE ? MV_NT_SP : MV_NT;
-    constexpr int NLD = (NH * 3 + NT - 1) / NT;
-    constexpr int NW = NT / 64;
-    constexpr bool SUMS = OUT == OUT_MASKED_DOT || OUT == OUT_RESID || (OUT == OUT_CHEB && PART);
-    constexpr int NSLOT = SPARSE ? MV_SLOTS * 3 : (OB_BIAS + 8 * NO) * 3 + 64 + 2;
-    __shared__ int s_node[NH];
-    __shared__ int s_info[NET];
-    __shared__ T s_E[NET];
-    __shared__ unsigned char s_nm[NO];
-    __shared__ double s_wred[SUMS ? NCH : 1][NW * 4][RC];   // per chunk, wave row and load case
-    __shared__ V s_x[NH * 3];
-    // corner buffers (the bias keeps element bases non-negative), then a trash
-    // area for the outputs of corners outside the owned nodes (lane l writes
-    // vectors l .. l + 2; the contents are never read)
-    __shared__ V s_c[NSLOT];
-    __shared__ short s_hn[NH];                   // halo positions that hold a node, compact
-    __shared__ unsigned char s_ol[NO];           // owned position of the brick's k-th solver node
-    __shared__ int s_wcnt[((NH + NT - 1) / NT) * NW];
-    __shared__ short s_sb[SPARSE ? NO : 1];      // SPARSE: first slot of each owned position
-    static_assert(!IO32 || (sizeof(T) == 8 && IN == IN_V), "FP32 vectors with FP64 arithmetic");
-    static_assert(IN != IN_JS || (sizeof(T) == 4 && OUT == OUT_CHEB && !SPARSE), "zero-start input: FP32 Chebyshev");
-
-    const int bid = A.blist ? A.blist[A.boff + blockIdx.x] : (int)blockIdx.x;
-    const int tid = threadIdx.x;
-    const int* __restrict__ halo = A.halo + (int64_t)bid * NH;
-    // Set-up loads in as few dependent steps as possible: the halo row and the node
-    // masks need only the brick index and are issued before the brick record
-    // arrives; the element list needs the record and is issued before the done
-    // flag is tested (a finished domain's brick wastes these loads)
-    constexpr int NHP = (NH + NT - 1) / NT;
-    int hq[NHP];
-#pragma unroll
-    for (int kk = 0; kk < NHP; ++kk) {
-        const int h = tid + kk * NT;
-        hq[kk] = h < NH ? halo[h] : -1;
-    }
-    const unsigned char nmv = tid < NO ? A.nmask[(int64_t)bid * NO + tid] : (unsigned char)0;
-    // the brick record's fields are all loaded here, in one round trip (the compiler
-    // otherwise loads each field where it is first used, one round trip each)
-    BrickInfo B = A.bricks[bid];
-    asm volatile("" : "+s"(B.dom), "+s"(B.x0), "+s"(B.y0), "+s"(B.z0), "+s"(B.node_begin), "+s"(B.node_end),
-                 "+s"(B.e_off), "+s"(B.e_cnt));
-    static_assert(NET <= (SPARSE ? MV_NT_SP : MV_NT), "one tile element per thread");
-    int eiv = 0;
-    T eEv = T(0);
-    if (tid < B.e_cnt) {
-        eiv = A.einfo[B.e_off + tid];
-        eEv = static_cast<const T*>(A.eE)[B.e_off + tid];
-    }
-    if (A.done && A.done[B.dom]) return;
-    const V* xv = reinterpret_cast<const V*>(xin);
-    V* yv = reinterpret_cast<V*>(yout);
-    const int c0 = (int)blockIdx.y * NCH / (int)gridDim.y, c1 = ((int)blockIdx.y + 1) * NCH / (int)gridDim.y;
-
-    // Only halo positions and owned positions that hold a node carry work: on
-    // sparse (trabecular) domains a brick holds about a third of its 128
-    // positions.  s_ol = owned position of solver node node_begin + k (owned
-    // nodes are numbered in position order).  Staging, measured per precision:
-    //  * FP32 (EARLY_X false): compact list s_hn of halo positions with a node
-    //    (wave ballots, prefix over the waves); x loads issued after the barrier
-    //    for the existing (node, direction) items only;
-    //  * FP64 (EARLY_X true): x loads for every halo slot issued first, straight
-    //    from the brick table, before any barrier.
-    constexpr bool EARLY_X = sizeof(T) == 8;
-    const int n_own = B.node_end - B.node_begin;
-    int nh = NH;
-    int pf_off[NLD], pf_xi[NLD];   // 16-byte offset in x and destination in s_x of this thread's items
-    V reg[NLD];                    // x segments of the next chunk to stage, loaded one chunk ahead
-    T pf_sc[IN == IN_JS ? NLD : 1]; // IN_JS: cin times the item's Jacobi scaling
-    auto prefetch = [&](int chunk) {
-#pragma unroll
-        for (int k = 0; k < NLD; ++k) {
-            V v;
-            vzero(v);
-            if (pf_off[k] >= 0) {
-                if constexpr (IO32) {
-                    const float2 f = reinterpret_cast<const float2*>(xin)[pf_off[k] + chunk];
-                    v = make_double2((double)f.x, (double)f.y);
-                } else {
-                    v = xv[pf_off[k] + chunk];
-                }
-            }
-            reg[k] = v;
-        }
-    };
-    if constexpr (EARLY_X) {
-#pragma unroll
-        for (int k = 0; k < NLD; ++k) {
-            const int i = tid + k * NT;
-            int o = -1;
-            if (IN == IN_V && i < NH * 3) {
-                const int q = halo[i / 3];
-                if (q >= 0) o = ((q & NODE_MASK) * 3 + i % 3) * NCH;
-            }
-            pf_off[k] = o;
-            pf_xi[k] = i;
-        }
-        if (IN != IN_U) prefetch(c0);
-    }
-    {
-        // halo positions h = tid + k NT (one pass with 512 threads, two with 256)
-        bool exk[NHP];
-#pragma unroll
-        for (int kk = 0; kk < NHP; ++kk) {
-            const int h = tid + kk * NT;
-            const int q = hq[kk];
-            if (h < NH) s_node[h] = q;
-            const bool ex = q >= 0;
-            exk[kk] = ex;
-            const int hx = h % HX, hy = (h / HX) % HY, hz = h / (HX * HY);
-            if (ex && hx >= 1 && hx <= BX && hy >= 1 && hy <= BY && hz >= 1 && hz <= BZ)
-                s_ol[(q & NODE_MASK) - B.node_begin] = (unsigned char)((hx - 1) + BX * ((hy - 1) + BY * (hz - 1)));
-        }
-        if (tid < NO) s_nm[tid] = nmv;
-        if constexpr (!EARLY_X) {
-            // compact list of the halo positions that hold a node, in position order
-            const int lane = tid & 63, wv = tid >> 6;
-            unsigned long long bal[NHP];
-#pragma unroll
-            for (int kk = 0; kk < NHP; ++kk) {
-                bal[kk] = __ballot(exk[kk]);
-                if (lane == 0) s_wcnt[kk * NW + wv] = __popcll(bal[kk]);
-            }
-            __syncthreads();
-            nh = 0;
-#pragma unroll
-            for (int kk = 0; kk < NHP; ++kk) {
-                int base = nh;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const int c = s_wcnt[kk * NW + w];
-                    if (w < wv) base += c;
-                    nh += c;
-                }
-                if (exk[kk]) s_hn[base + __popcll(bal[kk] & ((1ull << lane) - 1))] = (short)(tid + kk * NT);
-            }
-        }
-    }
-    const int ne = B.e_cnt;
-    if (tid < ne) {
-        s_info[tid] = eiv;
-        s_E[tid] = eEv;
-    }
-    __syncthreads();
-    if constexpr (SPARSE) {
-        // slot bases: exclusive prefix of the element counts of the owned positions
-        // (wave 0, two positions per lane); visible after the barrier below
-        if (tid < 64) {
-            const int c0 = __popc((unsigned)s_nm[2 * tid]), c1 = __popc((unsigned)s_nm[2 * tid + 1]);
-            int v = c0 + c1;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int u = __shfl_up(v, o);
-                if (tid >= o) v += u;
-            }
-            const int ex = v - c0 - c1;
-            s_sb[2 * tid] = (short)ex;
-            s_sb[2 * tid + 1] = (short)(ex + c0);
-        }
-    }
-
-    if constexpr (!EARLY_X) {
-#pragma unroll
-        for (int k = 0; k < NLD; ++k) {
-            const int i = tid + k * NT;
-            int o = -1, xi = 0;
-            if (i < 3 * nh) {
-                const int h = s_hn[i / 3], d = i % 3;
-                o = ((s_node[h] & NODE_MASK) * 3 + d) * NCH;
-                xi = h * 3 + d;
-            }
-            pf_off[k] = o;
-            pf_xi[k] = xi;
-            if constexpr (IN == IN_JS)   // the product order of k_cheb's zero start: (c2 dinv) v
-                pf_sc[k] = o >= 0 ? (T)A.cin * reinterpret_cast<const T*>(A.dinv)[o / NCH] : T(0);
-        }
-        if (IN != IN_U) prefetch(c0);
-    }
-
-    // s_x <- x of `chunk` (IN_V: from the prefetch registers; IN_U: x + BC values)
-    auto stage = [&](int chunk) {
-        if constexpr (IN == IN_JS) {
-#pragma unroll
-            for (int k = 0; k < NLD; ++k)
-                if (pf_off[k] >= 0) {
-                    V v = reg[k];
-                    T* vp = reinterpret_cast<T*>(&v);
-#pragma unroll
-                    for (int w = 0; w < RC; ++w) vp[w] = pf_sc[k] * vp[w];
-                    s_x[pf_xi[k]] = v;
-                }
-        } else if (IN == IN_V) {
-#pragma unroll
-            for (int k = 0; k < NLD; ++k)
-                if (pf_off[k] >= 0) s_x[pf_xi[k]] = reg[k];
-        } else {
-            const DomInfo D = A.doms[B.dom];
-            T* sx = reinterpret_cast<T*>(s_x);
-            for (int i = tid; i < nh * SX; i += NT) {
-                const int h = EARLY_X ? i / SX : (int)s_hn[i / SX], rem = i % SX, d = rem / RC, r = rem % RC;
-                const int lc = chunk * RC + r;
-                const int q = s_node[h];
-                T v = T(0);
-                if (q >= 0) {
-                    if (q & BC_BIT) {
-                        const int hx = h % HX, hy = (h / HX) % HY, hz = h / (HX * HY);
-                        double c[3], N[20];
-                        node_coord(D, B.x0 - 1 + hx, B.y0 - 1 + hy, B.z0 - 1 + hz, c);
-                        macro_shape(D.macro_order, c, D.min_c, D.max_c, N);
-                        v = (T)bc_value_m(D.macro_order, N, d, D.lc_base + lc);
-                    } else if (xin) {
-                        v = xin[((int64_t)(q & NODE_MASK) * 3 + d) * R + lc];
-                    }
-                }
-                sx[h * SX + rem] = v;
-            }
-        }
-    };
-
-    // chunk-invariant gather items of this thread: (owned solver node, direction)
-    // i = tid + j * NT < 3 n_own
-    constexpr int NG = (NO * 3 + NT - 1) / NT;
-    int g_off[NG], g_xi[NG];
-    unsigned g_m[NG];
-    T e_di[NG];   // OUT_CHEB: Jacobi scaling of the item
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-        const int i = tid + j * NT;
-        int off = -1, xi = 0;
-        unsigned m = 0;
-        if (i < 3 * n_own) {
-            const int o = s_ol[i / 3], d = i % 3, h = ohalo(o);
-            const int q = s_node[h];
-            off = ((q & NODE_MASK) * 3 + d) * NCH;
-            xi = h * 3 + d;
-            m = (unsigned)s_nm[o] | ((q & BC_BIT) ? 256u : 0u) | ((unsigned)o << 9) | ((unsigned)d << 16);
-        }
-        g_off[j] = off;
-        g_xi[j] = xi;
-        g_m[j] = m;
-        e_di[j] = T(0);
-        if (OUT == OUT_CHEB && off >= 0 && !(m & 256u)) e_di[j] = reinterpret_cast<const T*>(A.dinv)[off / NCH];
-    }
-
-    // corner slots that no element writes (element absent) are zero for the whole
-    // launch, so the gather adds all 8 corner buffers without tests
-    if constexpr (!SPARSE)
-        for (int i = tid; i < n_own * 24; i += NT) {
-            const int o = s_ol[i / 24], b = (i / 3) % 8, d = i % 3;
-            if (!((s_nm[o] >> b) & 1)) vzero(s_c[(OB_BIAS + b * NO + o) * 3 + d]);
-        }
-    stage(c0);
-    if (IN != IN_U && c0 + 1 < c1) prefetch(c0 + 1);
-    __syncthreads();
-
-    // FP32 dense Chebyshev step (one gather item per thread): the outputs of all
-    // chunks stay in registers and each item's 24 load cases are stored together
-    // after the last chunk, so every 96-byte node segment is written whole
-    // (per-chunk 16-byte stores left partly written lines to be written back more
-    // than once: 1.05 GB of writes per launch on the bench batch, 0.54 GB with
-    // whole segments, 5 % faster; the Q = K P step measured 5 % slower with it).
-    // The host launcher picks DEFER_Y = false with DTC_MV_DEFER=0 (A/B measurements).
-    constexpr bool DEFER = DEFER_Y && OUT == OUT_CHEB && !SPARSE && IO32 == 0 && sizeof(T) == 4 && NG == 1;
-    V ybuf[DEFER ? NCH : 1];
-#pragma unroll
-    for (int k = 0; k < (DEFER ? NCH : 1); ++k) vzero(ybuf[k]);
-
-    // Per chunk: element products -> barrier -> stage the next chunk and issue
-    // the loads of the one after -> gather -> barrier.  The next chunk is staged
-    // before the gather, so the wait for its x loads (and for any earlier
-    // stores) sits behind a whole element phase instead of right behind the
-    // gather's stores.
-    for (int chunk = c0; chunk < c1; ++chunk) {
-        // gather operands of this chunk: b and d (OUT_BRES / OUT_CHEB) from memory,
-        // x from LDS before the next chunk overwrites it
-        V e_b[NG], e_d[NG], e_x[NG];
-#pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            vzero(e_b[j]);
-            vzero(e_d[j]);
-            vzero(e_x[j]);
-            if (g_off[j] >= 0) {
-                const int vi = g_off[j] + chunk;
-                if (OUT == OUT_BRES || OUT == OUT_CHEB) e_b[j] = reinterpret_cast<const V*>(A.bvec)[vi];
-                if (OUT == OUT_CHEB && (A.cflags & CH_READ_D)) e_d[j] = reinterpret_cast<const V*>(A.dvec)[vi];
-                if (OUT == OUT_MASKED_DOT || OUT == OUT_CHEB) e_x[j] = s_x[g_xi[j]];
-            }
-        }
-
-        // ---- element products: task t = (tile element t / RC, load case t % RC)
-        {
-            const T* sx = reinterpret_cast<const T*>(s_x);
-            T* sc = reinterpret_cast<T*>(s_c);
-            const int ntask = ne * RC;
-#pragma unroll 1
-            for (int t = tid; t < ntask; t += NT) {
-                const int r = t % RC, k = t / RC;
-                const int info = s_info[k];
-                const T E = s_E[k];
-                const unsigned mask = (unsigned)info >> 24;
-                const T* xb = sx + (info & 511) * SX + r;
-                T* cb = sc + ((info >> 9) & 255) * SX + r;
-                T w[8][3], y[8][3];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    T v[8];
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) v[b] = xb[hcorner(b) * SX + d * RC];
-                    fht_fwd(v);
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) w[b][d] = v[b];
-                }
-                walsh_apply(wk, w, y);
-                T o[3][8];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    // mode 0 (rigid translation) carries no force: the first
-                    // inverse butterfly of the pair (0, 1) reduces to (-y1, y1)
-                    const T y1 = y[1][d] * E;
-                    o[d][0] = -y1;
-                    o[d][1] = y1;
-#pragma unroll
-                    for (int b = 2; b < 8; b += 2) {
-                        const T a = y[b][d] * E, c = y[b + 1][d] * E;
-                        o[d][b] = a - c;
-                        o[d][b + 1] = a + c;
-                    }
-                    fht_inv_tail(o[d]);
-                }
-                if constexpr (SPARSE) {
-                    // owned corners only: slot of node ob = first slot + rank of corner b among its elements
-                    const int ob0 = ((info >> 9) & 255) - OB_BIAS;
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) {
-                        if (!(mask & (1u << b))) continue;
-                        const int ob = ob0 + ocorner(b);
-                        const int slot = s_sb[ob] + __popc((unsigned)s_nm[ob] & ((1u << b) - 1u));
-                        T* dst = sc + slot * SX + r;
-#pragma unroll
-                        for (int d = 0; d < 3; ++d) dst[d * RC] = o[d][b];
-                    }
-                } else {
-                    // corners outside the owned nodes write to this lane's trash slot
-                    T* trash = sc + ((OB_BIAS + 8 * NO) * 3 + (tid & 63)) * RC;
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) {
-                        T* dst = (mask & (1u << b)) ? cb + (b * NO + ocorner(b)) * SX : trash;
-#pragma unroll
-                        for (int d = 0; d < 3; ++d) dst[d * RC] = o[d][b];
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        if (chunk + 1 < c1) {
-            stage(chunk + 1);
-            if (IN != IN_U && chunk + 2 < c1) prefetch(chunk + 2);
-        }
-
-        // ---- gather: thread per owned (node, direction), all RC load cases in one vector
-        double acc[RC];
-#pragma unroll
-        for (int w = 0; w < RC; ++w) acc[w] = 0.0;
-#pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            if (g_off[j] < 0) continue;
-            const unsigned m = g_m[j];
-            const int od = (int)(m >> 9);          // o | d << 7
-            const int o = od & 127, d = od >> 7;
-            V y;
-            vzero(y);
-            if constexpr (SPARSE) {
-                const int sb = s_sb[o], cnt = __popc((unsigned)s_nm[o]);
-#pragma unroll
-                for (int b = 0; b < 8; ++b)
-                    if (b < cnt) vadd(y, s_c[(sb + b) * 3 + d]);
-            } else {
-#pragma unroll
-                for (int b = 0; b < 8; ++b) vadd(y, s_c[(OB_BIAS + b * NO + o) * 3 + d]);
-            }
-            const bool bc = (m & 256u) != 0;
-            const int vi = g_off[j] + chunk;
-            if (OUT == OUT_MASKED_DOT) {
-                if (bc) vzero(y);
-#pragma unroll
-                for (int w = 0; w < RC; ++w) acc[w] += (double)vcomp(e_x[j], w) * (double)vcomp(y, w);
-            } else if (OUT == OUT_RESID) {
-                if (bc) vzero(y); else y = vneg(y);
-#pragma unroll
-                for (int w = 0; w < RC; ++w) acc[w] += (double)vcomp(y, w) * (double)vcomp(y, w);
-            } else if (OUT == OUT_MASKED) {
-                if (bc) vzero(y);
-            } else if (OUT == OUT_BRES || OUT == OUT_CHEB) {
-                const V bv = e_b[j];
-                if (OUT == OUT_BRES) {
-                    if (bc) vzero(y);
-                    else {
-                        V t = bv;
-                        vadd(t, vneg(y));
-                        y = t;
-                    }
-                } else {
-                    V* dp = reinterpret_cast<V*>(A.dvec) + vi;
-                    V dn, xn;
-                    vzero(dn);
-                    vzero(xn);
-                    if (!bc) {
-                        const T di = e_di[j];
-                        const V xv = e_x[j];
-                        const V dv = (A.cflags & CH_D_FROM_X) ? xv : e_d[j];
-                        T* dnp = reinterpret_cast<T*>(&dn);
-                        T* xnp = reinterpret_cast<T*>(&xn);
-#pragma unroll
-                        for (int w = 0; w < RC; ++w) {
-                            const T r = vcomp(bv, w) - vcomp(y, w);
-                            dnp[w] = (T)A.c1 * vcomp(dv, w) + (T)A.c2 * di * r;
-                            xnp[w] = vcomp(xv, w) + dnp[w];
-                        }
-                    }
-                    if (A.cflags & CH_WRITE_D) *dp = dn;
-                    y = xn;
-                    if (PART)
-#pragma unroll
-                        for (int w = 0; w < RC; ++w) acc[w] += (double)vcomp(bv, w) * (double)vcomp(y, w);
-                }
-            }
-            if constexpr (IO32 == 1) {
-                reinterpret_cast<float2*>(yout)[vi] = make_float2((float)y.x, (float)y.y);
-            } else if constexpr (DEFER) {
-#pragma unroll
-                for (int k = 0; k < NCH; ++k)
-                    if (k == chunk - c0) ybuf[k] = y;
-            } else {
-                yv[vi] = y;
-            }
-        }
-        if constexpr (SUMS) {
-            // every lane holds the RC load cases of the chunk: fixed-order row sums
-            // (waves past the last gather item hold zeros)
-            const int lane = tid & 63, row = (tid >> 6) * 4 + (lane >> 4);
-            double v = 0.0;
-            int lc = lane & (RC - 1);
-            bool out = (lane & 15) >= 16 - RC;
-            if ((tid & ~63) < 3 * n_own) out = row_sums<RC>(acc, lane, &v, &lc);
-            if (out) s_wred[chunk][row][lc] = v;
-        }
-        __syncthreads();
-    }
-    if constexpr (DEFER) {
-        if (g_off[0] >= 0) {
-#pragma unroll
-            for (int k = 0; k < NCH; ++k)
-                if (c0 + k < c1) yv[g_off[0] + c0 + k] = ybuf[k];
-        }
-    }
-    if (SUMS && tid < R &&
-        tid / RC >= c0 && tid / RC < c1) {
-        const int ch = tid / RC, r = tid % RC;
-        double s = 0.0;
-#pragma unroll
-        for (int w = 0; w < NW * 4; ++w) s += s_wred[ch][w][r];
-        A.partial[(int64_t)bid * R + tid] = s;
-    }
-}
-
-#include "matvec_mf.hpp"
+#include "ebe.hpp"
 
 // ---------------------------------------------------------------- vector kernels
 // per brick, thread t keeps load case t % 24
@@ -895,14 +308,15 @@ __global__ __launch_bounds__(RED_NT) void k_red_init(const DomInfo* __restrict__
 }
 
 __global__ __launch_bounds__(RED_NT) void k_red_alpha(const DomInfo* __restrict__ doms, const int* __restrict__ done,
-                                                      const double* __restrict__ ppq, int* __restrict__ active,
-                                                      const double* __restrict__ rz, double* __restrict__ alpha) {
+                                                      const double* __restrict__ ppq, int clus,
+                                                      int* __restrict__ active, const double* __restrict__ rz,
+                                                      double* __restrict__ alpha) {
     __shared__ double s_out[4 * R];
     const int d = blockIdx.x, tid = threadIdx.x;
     if (done[d]) return;
     const DomInfo D = doms[d];
     double pq[R];
-    dom_sum24(ppq, D.brick_begin, D.brick_end, s_out, pq);
+    dom_sum24(ppq, clus ? D.cl_begin : D.brick_begin, clus ? D.cl_end : D.brick_end, s_out, pq);
     if (tid < R) {
         const int lc = tid;
         int a = active[d * R + lc];
@@ -1036,111 +450,15 @@ constexpr double ORTH_DROP = 1e-10;   // of P^T P
 
 // Gram partial sums over the rows of one slice of a domain's nodes:
 //   g[0] = A^T B, g[1] = A^T C (NGR = 2; zero for NGR = 1), FP64 sums of the
-// products of FP32 (or FP64) operands.  Lane (i, j) of a wave keeps rows 3i..3i+2 x columns 3j..3j+2; the
-// four waves take every fourth vector row.  The loads of the next GU rows of a
-// wave are issued before the products of the current ones (a slice is a long
-// sequential walk per wave); the waves' sums are added in wave order.
-template <int NGR, typename TA = float, typename TB = float, int GU = 4>
-__global__ __launch_bounds__(GR_NT) void k_gram(const int4* __restrict__ slices, const int* __restrict__ done,
-                                               const TA* __restrict__ A, const TB* __restrict__ B,
-                                               const TB* __restrict__ C, double* __restrict__ gpart) {
-    __shared__ double s_g[NGR * RR];
-    const int4 sl = slices[blockIdx.x];   // domain, first node, end node
-    if (done[sl.x]) return;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int ci = 3 * (lane >> 3), cj = 3 * (lane & 7);
-    double g[NGR][9];
-#pragma unroll
-    for (int t = 0; t < NGR; ++t)
-#pragma unroll
-        for (int k = 0; k < 9; ++k) g[t][k] = 0.0;
-    const int64_t r1 = (int64_t)sl.z * 3;
-    // two register sets: the next GU rows load into one while the products of the
-    // other run; full steps (all GU rows in the slice) load without guards
-    TA av[2][GU][3];
-    TB bv[2][NGR][GU][3];
-    auto load = [&](int set, int64_t row0) {
-#pragma unroll
-        for (int u = 0; u < GU; ++u) {
-            const int64_t row = row0 + 4 * u;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                av[set][u][i] = A[row * R + ci + i];
-                bv[set][0][u][i] = B[row * R + cj + i];
-                if (NGR == 2) bv[set][NGR - 1][u][i] = C[row * R + cj + i];
-            }
-        }
-    };
-    auto product = [&](const TA (&a)[3], const TB (&b)[3], double (&gg)[9]) {
-        double ad[3], bd[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            ad[i] = (double)a[i];
-            bd[i] = (double)b[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) gg[3 * i + j] = fma(ad[i], bd[j], gg[3 * i + j]);
-    };
-    auto products = [&](int set) {
-#pragma unroll
-        for (int u = 0; u < GU; ++u)
-#pragma unroll
-            for (int t = 0; t < NGR; ++t) product(av[set][u], bv[set][t][u], g[t]);
-    };
-    int64_t row0 = (int64_t)sl.y * 3 + wave;
-    const int64_t full_end = r1 - 4 * (GU - 1);   // row0 < full_end: rows row0 + 4u < r1
-    if (row0 < full_end) load(0, row0);
-    while (row0 < full_end) {
-        if (row0 + 4 * GU < full_end) load(1, row0 + 4 * GU);
-        products(0);
-        row0 += 4 * GU;
-        if (row0 >= full_end) break;
-        if (row0 + 4 * GU < full_end) load(0, row0 + 4 * GU);
-        products(1);
-        row0 += 4 * GU;
-    }
-    for (; row0 < r1; row0 += 4) {      // the last rows of the wave (fewer than GU)
-        TA a[3];
-        TB b[NGR][3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            a[i] = A[row0 * R + ci + i];
-            b[0][i] = B[row0 * R + cj + i];
-            if (NGR == 2) b[NGR - 1][i] = C[row0 * R + cj + i];
-        }
-#pragma unroll
-        for (int t = 0; t < NGR; ++t) product(a, b[t], g[t]);
-    }
-    for (int w = 0; w < 4; ++w) {
-        if (wave == w)
-#pragma unroll
-            for (int t = 0; t < NGR; ++t)
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        const int e = t * RR + (ci + i) * R + cj + j;
-                        s_g[e] = w == 0 ? g[t][3 * i + j] : s_g[e] + g[t][3 * i + j];
-                    }
-        __syncthreads();
-    }
-    double* out = gpart + (int64_t)blockIdx.x * 2 * RR;
-    for (int e = tid; e < 2 * RR; e += GR_NT) out[e] = e < NGR * RR ? s_g[e] : 0.0;
-}
-
-// The same Gram partials with the rows staged through LDS: the workgroup loads
-// blocks of GB_ROWS vector rows of A, B (and C) with coalesced 16-byte loads (the
-// next block's loads issued before the current block's products), and lane (i, j)
-// reads its 3 + 3 (+ 3) values of a row from LDS, where the 8 lanes sharing an
-// address are served by one broadcast.  (Loading them from global memory sends
-// each value through the vector memory path 8 times.)  Wave w takes rows w, w + 4,
-// ... of each block in order, so every wave sums the same rows in the same order
-// as k_gram and the results are identical.
+// products of FP32 (or FP64) operands.  Lane (i, j) of a wave keeps rows 3i..3i+2 x
+// columns 3j..3j+2.  The workgroup loads blocks of GB_ROWS vector rows of A, B (and C)
+// with coalesced 16-byte loads (the next block's loads issued before the current
+// block's products) into LDS, where the 8 lanes sharing an address are served by one
+// broadcast; wave w takes rows w, w + 4, ... of each block in order, and the waves' sums
+// are added in wave order.
 constexpr int GB_ROWS = 32;
 template <int NGR, typename TA = float, typename TB = float>
-__global__ __launch_bounds__(GR_NT) void k_gram_lds(const int4* __restrict__ slices, const int* __restrict__ done,
+__global__ __launch_bounds__(GR_NT) void k_gram(const int4* __restrict__ slices, const int* __restrict__ done,
                                                    const TA* __restrict__ A, const TB* __restrict__ B,
                                                    const TB* __restrict__ C, double* __restrict__ gpart) {
     constexpr int EA = 16 / sizeof(TA), EB = 16 / sizeof(TB);      // elements per 16-byte vector
@@ -1501,7 +819,7 @@ __global__ __launch_bounds__(NT_UPD) void k_bupdate64(const int4* __restrict__ s
 // GRAM: also the per-slice Gram partials pnᵀpn of the rows written (for the
 // orthonormalisation that follows): the block's new rows are staged in LDS and wave w
 // sums rows w, w + 3, ... of each block, lane (i, j) its 3 x 3 entries, in FP64 (the
-// layout of k_gram_lds's partials, another summation order)
+// layout of k_gram's partials, another summation order)
 template <bool GRAM>
 __global__ __launch_bounds__(NT_UPD) void k_bdir(const int4* __restrict__ slices, const int* __restrict__ done,
                                                 const float* __restrict__ coef, const float* __restrict__ p,
@@ -1749,79 +1067,6 @@ __global__ void k_dinv(const BrickInfo* __restrict__ bricks, const DomInfo* __re
     for (int d = 0; d < 3; ++d) {              // one value per DOF (isotropic for the HEX08 voxel)
         d64[3 * q + d] = inv;
         d32[3 * q + d] = (float)inv;
-    }
-}
-
-// ---------------------------------------------------------------- matvec tables
-// solid elements of the element tile of each brick (blockDim >= NET)
-__global__ void k_brick_ecount(const BrickInfo* __restrict__ bricks, const DomInfo* __restrict__ doms,
-                               const double* __restrict__ emod, int* __restrict__ cnt) {
-    __shared__ int s;
-    const BrickInfo B = bricks[blockIdx.x];
-    const DomInfo D = doms[B.dom];
-    const int i = threadIdx.x;
-    if (i == 0) s = 0;
-    __syncthreads();
-    if (i < NET) {
-        const int vx = B.x0 - 1 + i % EX, vy = B.y0 - 1 + (i / EX) % EY, vz = B.z0 - 1 + i / (EX * EY);
-        if (vx >= 0 && vy >= 0 && vz >= 0 && vx < D.nx && vy < D.ny && vz < D.nz &&
-            emod[D.vox_off + vx + (int64_t)D.nx * (vy + (int64_t)D.ny * vz)] != 0.0)
-            atomicAdd(&s, 1);
-    }
-    __syncthreads();
-    if (i == 0) cnt[blockIdx.x] = s;
-}
-
-// halo node table (solver node | BC_BIT) and the packed tile element list of
-// each brick, elements in lexicographic tile order (blockDim >= NET)
-__global__ void k_brick_tables(const BrickInfo* __restrict__ bricks, const DomInfo* __restrict__ doms,
-                               const int* __restrict__ lat2node, const double* __restrict__ emod,
-                               int* __restrict__ halo, unsigned char* __restrict__ nmask, int* __restrict__ einfo,
-                               double* __restrict__ eE64, float* __restrict__ eE32) {
-    __shared__ int s_flag[NET];
-    const BrickInfo B = bricks[blockIdx.x];
-    const DomInfo D = doms[B.dom];
-    const int tid = threadIdx.x;
-    const int Lx = D.nx + 1, Ly = D.ny + 1, Lz = D.nz + 1;
-    for (int i = tid; i < NH; i += blockDim.x) {
-        const int gx = B.x0 - 1 + i % HX, gy = B.y0 - 1 + (i / HX) % HY, gz = B.z0 - 1 + i / (HX * HY);
-        int q = -1;
-        if (gx >= 0 && gy >= 0 && gz >= 0 && gx < Lx && gy < Ly && gz < Lz) {
-            q = lat2node[D.lat_off + gx + (int64_t)Lx * (gy + (int64_t)Ly * gz)];
-            if (q >= 0 && is_bc(D, gx, gy, gz)) q |= BC_BIT;
-        }
-        halo[(int64_t)blockIdx.x * NH + i] = q;
-    }
-    double e = 0.0;
-    const int ex = tid % EX, ey = (tid / EX) % EY, ez = tid / (EX * EY);
-    if (tid < NET) {
-        const int vx = B.x0 - 1 + ex, vy = B.y0 - 1 + ey, vz = B.z0 - 1 + ez;
-        if (vx >= 0 && vy >= 0 && vz >= 0 && vx < D.nx && vy < D.ny && vz < D.nz)
-            e = emod[D.vox_off + vx + (int64_t)D.nx * (vy + (int64_t)D.ny * vz)];
-        s_flag[tid] = e != 0.0 ? 1 : 0;
-    }
-    __syncthreads();
-    if (tid < NO) {   // solid tile elements around owned node tid, bit b = element at corner offset -b
-        const int hx = tid % BX + 1, hy = (tid / BX) % BY + 1, hz = tid / (BX * BY) + 1;
-        unsigned m = 0;
-        for (int b = 0; b < 8; ++b)
-            if (s_flag[(hx - (b & 1)) + EX * ((hy - ((b >> 1) & 1)) + EY * (hz - (b >> 2)))]) m |= 1u << b;
-        nmask[(int64_t)blockIdx.x * NO + tid] = (unsigned char)m;
-    }
-    if (tid < NET && e != 0.0) {
-        int rank = 0;
-        for (int k = 0; k < tid; ++k) rank += s_flag[k];
-        unsigned mask = 0;
-        for (int b = 0; b < 8; ++b) {
-            const int hx = ex + (b & 1), hy = ey + ((b >> 1) & 1), hz = ez + (b >> 2);
-            if (hx >= 1 && hx <= BX && hy >= 1 && hy <= BY && hz >= 1 && hz <= BZ) mask |= 1u << b;
-        }
-        const int hb = ex + HX * (ey + HY * ez);
-        const int ob = (ex - 1) + BX * ((ey - 1) + BY * (ez - 1)) + OB_BIAS;
-        const int64_t o = (int64_t)B.e_off + rank;
-        einfo[o] = (int)((unsigned)hb | ((unsigned)ob << 9) | (mask << 24));
-        eE64[o] = e;
-        eE32[o] = (float)e;
     }
 }
 
@@ -2365,38 +1610,54 @@ __global__ __launch_bounds__(NT_UPD) void k_sub(const BrickInfo* __restrict__ br
     for (int64_t i = threadIdx.x; i < cnt; i += NT_UPD) res[base + i] = b[base + i] - t[base + i];
 }
 
+// per-brick sums of a . b per load case
+template <typename T>
+__global__ __launch_bounds__(NT_UPD) void k_dot(const BrickInfo* __restrict__ bricks, const int* __restrict__ done,
+                                                const T* __restrict__ a, const T* __restrict__ b,
+                                                double* __restrict__ part) {
+    __shared__ double s1[NT_UPD];
+    const BrickInfo B = bricks[blockIdx.x];
+    if (done && done[B.dom]) return;
+    const int tid = threadIdx.x;
+    double s = 0.0;
+    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
+    for (int64_t i = tid; i < cnt; i += NT_UPD) s += (double)a[base + i] * (double)b[base + i];
+    s1[tid] = s;
+    __syncthreads();
+    if (tid < R) {
+        double u = 0.0;
+        for (int k = tid; k < NT_UPD; k += R) u += s1[k];
+        part[(int64_t)blockIdx.x * R + tid] = u;
+    }
+}
+
+// x = Dirichlet values on the box-face nodes of each brick, unchanged elsewhere;
+// blockIdx.y takes a share of the brick's positions
+__global__ __launch_bounds__(NT_UPD) void k_set_bc(const BrickInfo* __restrict__ bricks, const DomInfo* __restrict__ doms,
+                                                   const int* __restrict__ lat2node, double* __restrict__ x) {
+    const BrickInfo B = bricks[blockIdx.x];
+    const DomInfo D = doms[B.dom];
+    if (B.x0 != 0 && B.y0 != 0 && B.z0 != 0 && B.x0 + BX <= D.nx && B.y0 + BY <= D.ny && B.z0 + BZ <= D.nz) return;
+    const int Lx = D.nx + 1, Ly = D.ny + 1;
+    const int lc = threadIdx.x % R;
+    for (int o = threadIdx.x / R + NT_UPD / R * (int)blockIdx.y; o < BX * BY * BZ; o += NT_UPD / R * (int)gridDim.y) {
+        const int gx = B.x0 + o % BX, gy = B.y0 + (o / BX) % BY, gz = B.z0 + o / (BX * BY);
+        if (gx > D.nx || gy > D.ny || gz > D.nz || !is_bc(D, gx, gy, gz)) continue;
+        const int q = lat2node[D.lat_off + gx + (int64_t)Lx * (gy + (int64_t)Ly * gz)];
+        if (q < 0) continue;
+        double c[3], N[20];
+        node_coord(D, gx, gy, gz, c);
+        macro_shape(D.macro_order, c, D.min_c, D.max_c, N);
+        for (int d = 0; d < 3; ++d)
+            x[((int64_t)q * 3 + d) * R + lc] = bc_value_m(D.macro_order, N, d, D.lc_base + lc);
+    }
+}
+
 inline unsigned nb(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// Grids of fewer than FILL_BLOCKS workgroups leave CUs idle: the matvec then
-// splits each brick's load-case chunks over blockIdx.y (a divisor of nch), the
-// transfer kernels split each brick's nodes.
+// Grids of fewer than FILL_BLOCKS workgroups leave CUs idle: the transfer kernels then
+// split each brick's nodes over blockIdx.y
 constexpr int FILL_BLOCKS = 2048;
-inline int chunk_split(int n_bricks, int nch) {
-    int want = n_bricks > 0 ? (FILL_BLOCKS + n_bricks - 1) / n_bricks : 1;
-    if (want >= nch) return nch;
-    int best = 1;
-    for (int s = 1; s <= want; ++s)
-        if (nch % s == 0) best = s;
-    return best;
-}
-// Launch-shape autotuner.  The split of a brick's load-case chunks over
-// gridDim.y workgroups (1, 2, 3 or 6) changes how the chip is filled, not the
-// arithmetic (every chunk is computed whole by one workgroup), so it can be
-// picked by timing without changing any result.  autotune_splits() times the
-// candidates of each FP32 matvec kernel on each multigrid level of a batch
-// before its first solve and caches the fastest per (kernel, variant, bricks);
-// the launches look the choice up (chunk_split's rule when absent, or with
-// DTC_TUNE=0).  DTC_TUNE_LOG=1 prints each decision.
-enum TuneKind { TK_MV = 0, TK_CHEB = 1, TK_BRES = 2 };
-std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int>, int> g_tune;
-
-int tuned_split(int kind, int variant, int n_bricks, int nch) {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tune.find(std::make_tuple(kind, variant, n_bricks));
-    return it != g_tune.end() ? it->second : chunk_split(n_bricks, nch);
-}
-
 inline int node_split(int n_bricks) {
     const int want = n_bricks > 0 ? (FILL_BLOCKS + n_bricks - 1) / n_bricks : 1;
     return want < 1 ? 1 : want > 8 ? 8 : want;
@@ -2530,6 +1791,28 @@ int batch_add_empty(SolverBatch& b, const dtc_domain_desc& d, int status, int lc
     return DTC_OK;
 }
 
+// Order of a domain's bricks: a Z-curve over the brick grid (y, z, x from the lowest bit
+// up, which makes runs of the 8x4x4 bricks compact), so that consecutive nodes, and with
+// them the clusters, are close together.
+static std::vector<int> brick_order(int bnx, int bny, int bnz) {
+    auto spread = [](int v) {   // bit i -> bit 3 i
+        int64_t r = 0;
+        for (int i = 0; (v >> i) != 0; ++i) r |= (int64_t)((v >> i) & 1) << (3 * i);
+        return r;
+    };
+    std::vector<std::pair<int64_t, int>> key;
+    key.reserve((size_t)bnx * bny * bnz);
+    for (int z = 0; z < bnz; ++z)
+        for (int y = 0; y < bny; ++y)
+            for (int x = 0; x < bnx; ++x)
+                key.emplace_back(spread(y) | spread(z) << 1 | spread(x) << 2, x + bnx * (y + bny * z));
+    std::sort(key.begin(), key.end());
+    std::vector<int> o;
+    o.reserve(key.size());
+    for (const auto& k : key) o.push_back(k.second);
+    return o;
+}
+
 int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d, const double* modulus_dev,
                      double escale, int lc_base, hipStream_t s) {
     if (m.nen != 8) return set_error(DTC_ERR_UNSUPPORTED, "the solver implements HEX08 micro elements");
@@ -2576,7 +1859,7 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
     D.node_begin = b.n_nodes;
     int64_t node = b.n_nodes;
     std::vector<BrickInfo> mine;
-    for (int i = 0; i < nbr; ++i) {
+    for (int i : brick_order(D.bnx, D.bny, D.bnz)) {
         if (!hc[i]) continue;
         BrickInfo B{};
         B.dom = b.n_dom;
@@ -2641,83 +1924,88 @@ double sym_lmax(const double* A, int n) {
     return lam;
 }
 
-// matvec tables of a brick list: tile element counts -> offsets -> halo table,
-// owned-node element masks and packed element lists (bricks re-uploaded with offsets)
-// (owned node, element corner) pairs of each brick: the population count of its
-// owned-node element masks
-__global__ __launch_bounds__(256) void k_brick_slots(const unsigned char* __restrict__ nmask, int nbr,
-                                                    int* __restrict__ out) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbr) return;
-    const unsigned* w = reinterpret_cast<const unsigned*>(nmask + (int64_t)b * NO);
-    int c = 0;
-#pragma unroll 8
-    for (int k = 0; k < NO / 4; ++k) c += __popc(w[k]);
-    out[b] = c;
+// Most nodes of a level's clusters.  The matvec sums a node in the same order whatever
+// its cluster is, so with the block PCG, which takes no other sums from it, the cap
+// follows the grid: nodes / CL_GRID, so that small levels still make enough workgroups,
+// each with a short walk over its elements (single 64^3 domain, 146 iterations: 148 ms with
+// 128 everywhere, 132 ms so; 16 of them 517 and 509 ms).  The one-column PCGs also sum p.q per cluster;
+// theirs is fixed, so that a domain's sums do not depend on the batch it is in.
+constexpr int CL_GRID = 1024, CL_MIN = 8;
+int cluster_cap(int64_t nodes, bool block, int precision) {
+    if (!block) return precision == DTC_FP64 ? CL_CAP64 : CL_CAP;
+    return (int)std::min<int64_t>(CL_CAP, std::max<int64_t>(CL_MIN, nodes / CL_GRID));
 }
 
-// bricks of a level for the FP32 matvecs: those with at most MV_SLOTS corner
-// slots first (the sparse kernel), then the rest (the dense kernel)
-int brick_lists(hipStream_t s, int nbr, const DevMem& nmask, DevMem& blist, int* n_sparse) {
-    // DTC_SPARSE=1: bricks with few corner slots run the 256-thread variant (measured
-    // 10% slower over the whole mixed solve on trabecular batches, so not the default);
-    // otherwise no list is kept (brick = workgroup)
-    *n_sparse = 0;
-    const char* se = std::getenv("DTC_SPARSE");
-    if (nbr == 0 || !(se && se[0] == '1')) {
-        blist.release();
-        return DTC_OK;
+// Clusters of a level: consecutive nodes of each domain in brick order, whole bricks
+// while they fit the cap, a brick of more nodes alone in equal pieces.
+void make_clusters(std::vector<DomInfo>& hd, const std::vector<BrickInfo>& hb, int cap, Clusters& c) {
+    c.h.clear();
+    c.cap = cap;
+    for (size_t d = 0; d < hd.size(); ++d) {
+        DomInfo& D = hd[d];
+        D.cl_begin = (int)c.h.size();
+        ClusterInfo cur{};
+        auto close = [&]() {
+            if (cur.node_end > cur.node_begin) c.h.push_back(cur);
+            cur = ClusterInfo{};
+        };
+        for (int i = D.brick_begin; i < D.brick_end; ++i) {
+            const BrickInfo& B = hb[i];
+            const int n = B.node_end - B.node_begin;
+            if (cur.node_end - cur.node_begin + n > cap) close();
+            if (n > cap) {
+                const int pieces = (n + cap - 1) / cap;
+                for (int k = 0; k < pieces; ++k)
+                    c.h.push_back(ClusterInfo{(int)d, B.node_begin + n * k / pieces, B.node_begin + n * (k + 1) / pieces,
+                                              i, i + 1, 0, 0});
+                continue;
+            }
+            if (cur.node_end == cur.node_begin) {
+                cur.dom = (int)d;
+                cur.node_begin = B.node_begin;
+                cur.brick_begin = i;
+            }
+            cur.node_end = B.node_end;
+            cur.brick_end = i + 1;
+        }
+        close();
+        D.cl_end = (int)c.h.size();
     }
-    DevMem cnt;
-    DTC_TRY(cnt.alloc((size_t)nbr * 4));
-    k_brick_slots<<<(nbr + 255) / 256, 256, 0, s>>>(nmask.as<unsigned char>(), nbr, cnt.as<int>());
-    DTC_HIP(hipGetLastError());
-    std::vector<int> hc(nbr), order;
-    DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)nbr * 4, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
-    order.reserve(nbr);
-    for (int i = 0; i < nbr; ++i)
-        if (hc[i] <= MV_SLOTS) order.push_back(i);
-    *n_sparse = (int)order.size();
-    for (int i = 0; i < nbr; ++i)
-        if (hc[i] > MV_SLOTS) order.push_back(i);
-    DTC_TRY(blist.ensure((size_t)nbr * 4));
-    DTC_HIP(hipMemcpyAsync(blist.p, order.data(), (size_t)nbr * 4, hipMemcpyHostToDevice, s));
-    DTC_HIP(hipStreamSynchronize(s));
-    return DTC_OK;
+    c.n = (int)c.h.size();
 }
 
-int build_tables(hipStream_t s, std::vector<BrickInfo>& hb, DevMem& brick, const DevMem& dom, const DevMem& lat2node,
-                 const DevMem& emod, DevMem& halo, DevMem& nmask, DevMem& einfo, DevMem& eE64, DevMem& eE32,
-                 int64_t* n_tile) {
-    const int nbr = (int)hb.size();
-    *n_tile = 0;
-    if (nbr == 0) return DTC_OK;
+// element tables of a level's clusters (fine: FP64 moduli too)
+int build_clusters(hipStream_t s, Clusters& c, const DevMem& brick, const DevMem& dom, const DevMem& lat2node,
+                   const DevMem& emod, bool fine) {
+    if (c.n == 0) return DTC_OK;
     DevMem cnt;
-    DTC_TRY(cnt.alloc((size_t)nbr * 4));
-    k_brick_ecount<<<nbr, 256, 0, s>>>(brick.as<BrickInfo>(), dom.as<DomInfo>(), emod.as<double>(), cnt.as<int>());
+    DTC_TRY(cnt.alloc((size_t)c.n * 4));
+    DTC_TRY(c.info.ensure(c.h.size() * sizeof(ClusterInfo)));
+    DTC_HIP(hipMemcpyAsync(c.info.p, c.h.data(), c.h.size() * sizeof(ClusterInfo), hipMemcpyHostToDevice, s));
+    k_cluster_elems<false><<<c.n, 256, 0, s>>>(c.info.as<ClusterInfo>(), brick.as<BrickInfo>(), dom.as<DomInfo>(),
+                                               lat2node.as<int>(), emod.as<double>(), cnt.as<int>(), nullptr, nullptr,
+                                               nullptr, nullptr, c.cap);
     DTC_HIP(hipGetLastError());
-    std::vector<int> hc(nbr);
-    DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)nbr * 4, hipMemcpyDeviceToHost, s));
+    std::vector<int> hc(c.n);
+    DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)c.n * 4, hipMemcpyDeviceToHost, s));
     DTC_HIP(hipStreamSynchronize(s));
     int64_t off = 0;
-    for (int i = 0; i < nbr; ++i) {
-        hb[i].e_off = (int)off;
-        hb[i].e_cnt = hc[i];
+    for (int i = 0; i < c.n; ++i) {
+        c.h[i].e_off = (int)off;
+        c.h[i].e_cnt = hc[i];
         off += hc[i];
     }
-    if (off >= INT32_MAX) return set_error(DTC_ERR_BAD_ARGUMENT, "batch exceeds %d tile elements", INT32_MAX);
-    *n_tile = off;
-    DTC_HIP(hipMemcpyAsync(brick.p, hb.data(), hb.size() * sizeof(BrickInfo), hipMemcpyHostToDevice, s));
+    if (off >= INT32_MAX) return set_error(DTC_ERR_BAD_ARGUMENT, "batch exceeds %d cluster elements", INT32_MAX);
+    DTC_HIP(hipMemcpyAsync(c.info.p, c.h.data(), c.h.size() * sizeof(ClusterInfo), hipMemcpyHostToDevice, s));
     const size_t ne = (size_t)(off > 0 ? off : 1);
-    DTC_TRY(halo.ensure((size_t)nbr * NH * 4));
-    DTC_TRY(nmask.ensure((size_t)nbr * NO));
-    DTC_TRY(einfo.ensure(ne * 4));
-    DTC_TRY(eE64.ensure(ne * 8));
-    DTC_TRY(eE32.ensure(ne * 4));
-    k_brick_tables<<<nbr, 256, 0, s>>>(brick.as<BrickInfo>(), dom.as<DomInfo>(), lat2node.as<int>(), emod.as<double>(),
-                                       halo.as<int>(), nmask.as<unsigned char>(), einfo.as<int>(), eE64.as<double>(),
-                                       eE32.as<float>());
+    DTC_TRY(c.enode.ensure(ne * 32));
+    DTC_TRY(c.eown.ensure(ne * 8));
+    if (fine) DTC_TRY(c.eE64.ensure(ne * 8));
+    DTC_TRY(c.eE32.ensure(ne * 4));
+    k_cluster_elems<true><<<c.n, 256, 0, s>>>(c.info.as<ClusterInfo>(), brick.as<BrickInfo>(), dom.as<DomInfo>(),
+                                              lat2node.as<int>(), emod.as<double>(), nullptr, c.enode.as<int4>(),
+                                              c.eown.as<uint2>(), fine ? c.eE64.as<double>() : nullptr,
+                                              c.eE32.as<float>(), c.cap);
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipStreamSynchronize(s));   // cnt goes out of scope
     return DTC_OK;
@@ -2725,47 +2013,19 @@ int build_tables(hipStream_t s, std::vector<BrickInfo>& hb, DevMem& brick, const
 
 }  // namespace
 
-// B operands of k_matvec_mf: B[4 b' + d'][4 b + d] = Khat(3 b + d, 3 b' + d') / kmax in
-// corner-bit order (b = ox + 2 oy + 4 oz), direction 3 a zero pad, as FP16 pairs
-// hi + lo; lane l of column tile t holds column j = l % 16 (n = 16 t + j) and
-// rows 8 (l / 16) .. 8 (l / 16) + 7.  Also which FP32 matvecs use it: none unless
-// DTC_MFMA=1 (then Q = K P with 3 FP16 terms and the smoothing steps with
-// DTC_MG_TERMS = 1 or 3, default 3).
-int mf_table(const double* Khat, SolverBatch& b) {
-    int l_of_b[8];
-    for (int l = 0; l < 8; ++l) l_of_b[h08_off(l, 0) + 2 * h08_off(l, 1) + 4 * h08_off(l, 2)] = l;
-    double kmax = 0.0;
-    for (int i = 0; i < 576; ++i) kmax = std::fmax(kmax, std::fabs(Khat[i]));
-    if (!(kmax > 0.0)) return set_error(DTC_ERR_DEVICE, "element stiffness is zero");
-    std::vector<_Float16> tab((size_t)2 * 2 * 64 * 8);
-    for (int t = 0; t < 2; ++t)
-        for (int q = 0; q < 2; ++q)
-            for (int l = 0; l < 64; ++l)
-                for (int e = 0; e < 8; ++e) {
-                    const int k = 8 * (l / 16) + e, n = 16 * t + (l % 16);
-                    const int bo = n / 4, dd = n % 4, bi = k / 4, di = k % 4;
-                    const double v = (dd < 3 && di < 3)
-                                         ? Khat[(3 * l_of_b[bo] + dd) + 24 * (3 * l_of_b[bi] + di)] / kmax
-                                         : 0.0;
-                    const _Float16 hi = (_Float16)v;
-                    tab[(((size_t)t * 2 + q) * 64 + l) * 8 + e] = q == 0 ? hi : (_Float16)(v - (double)hi);
-                }
-    DTC_TRY(b.kmf.ensure(tab.size() * sizeof(_Float16)));
-    DTC_HIP(hipMemcpyAsync(b.kmf.p, tab.data(), tab.size() * sizeof(_Float16), hipMemcpyHostToDevice, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
-    b.kmf_max = (float)kmax;
-    const char* e = std::getenv("DTC_MFMA");
-    const bool on = e && e[0] == '1';   // opt-in: slower than the Walsh kernel on the bench batch (measured)
-    b.mf_cg = on ? 1 : 0;
-    int terms = 3;
-    if (const char* t = std::getenv("DTC_MG_TERMS")) terms = std::atoi(t) == 1 ? 1 : 3;
-    b.mf_smooth = on ? terms : 0;
-    return DTC_OK;
+// the mixed multigrid solve iterates the load cases as one block (DTC_BLOCK_PCG=0: one
+// PCG per load case)
+static bool block_pcg(const SolverBatch& b) {
+    const char* e = std::getenv("DTC_BLOCK_PCG");
+    return b.precond == DTC_PC_MG && !(e && e[0] == '0');
 }
 
 int batch_finalize(SolverBatch& b, int precision) {
     b.n_bricks = (int)b.h_brick.size();
     hipStream_t s = b.stream;
+    b.cl.n = 0;
+    const bool block = precision == DTC_FP32_REFINE && block_pcg(b);
+    if (!b.micro20) make_clusters(b.h_dom, b.h_brick, cluster_cap(b.n_nodes, block, precision), b.cl);
     DTC_TRY(b.dom.ensure(b.h_dom.size() * sizeof(DomInfo)));
     DTC_HIP(hipMemcpyAsync(b.dom.p, b.h_dom.data(), b.h_dom.size() * sizeof(DomInfo), hipMemcpyHostToDevice, s));
     DTC_TRY(b.brick.ensure((b.h_brick.size() + 1) * sizeof(BrickInfo)));
@@ -2786,7 +2046,8 @@ int batch_finalize(SolverBatch& b, int precision) {
         DTC_TRY(b.p32.ensure(v32));
         DTC_TRY(b.q32.ensure(v32));
     }
-    const size_t nbk = (size_t)(b.n_bricks > 0 ? b.n_bricks : 1);
+    // partial sums per brick, or per cluster (matvec)
+    const size_t nbk = (size_t)std::max({b.n_bricks, b.cl.n, 1});
     DTC_TRY(b.part_a.ensure(nbk * R * 8));
     DTC_TRY(b.part_b.ensure(nbk * R * 8));
     DTC_TRY(b.part_c.ensure(nbk * R * 8));
@@ -2805,7 +2066,6 @@ int batch_finalize(SolverBatch& b, int precision) {
     DTC_TRY(element_stiffness(8, 1.0, b.nu, b.a, Khat));
     DTC_TRY(walsh_blocks(Khat, &b.wk64));
     b.kdiag = Khat[0];
-    DTC_TRY(mf_table(Khat, b));
     // element-by-element bound lambda_max(D^-1 K) <= lambda_max(diag(Khat)^-1/2 Khat diag(Khat)^-1/2);
     // the diagonal of the cube element is constant
     b.cheb_lmax = sym_lmax(Khat, 24) / b.kdiag;
@@ -2815,9 +2075,7 @@ int batch_finalize(SolverBatch& b, int precision) {
         k_dinv<<<b.n_bricks, BX * BY * BZ, 0, s>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(), b.lat2node.as<int>(),
                                                    b.emod.as<double>(), b.kdiag, b.dinv64.as<double>(), b.dinv32.as<float>());
         DTC_HIP(hipGetLastError());
-        DTC_TRY(build_tables(s, b.h_brick, b.brick, b.dom, b.lat2node, b.emod, b.halo, b.nmask, b.einfo, b.eE64,
-                             b.eE32, &b.n_tile_elems));
-        DTC_TRY(brick_lists(s, b.n_bricks, b.nmask, b.blist, &b.n_sparse));
+        DTC_TRY(build_clusters(s, b.cl, b.brick, b.dom, b.lat2node, b.emod, true));
     }
     DTC_HIP(hipStreamSynchronize(s));
     b.precision = precision;
@@ -2884,8 +2142,7 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
             DomInfo& D = C.h_dom[d];
             D.brick_begin = (int)C.h_brick.size();
             D.node_begin = node;
-            const int nbr = D.bnx * D.bny * D.bnz;
-            for (int i = 0; i < nbr; ++i) {
+            for (int i : brick_order(D.bnx, D.bny, D.bnz)) {
                 const int c = hc[boff[d] + i];
                 if (!c) continue;
                 BrickInfo B{};
@@ -2901,6 +2158,7 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
         }
         C.n_bricks = (int)C.h_brick.size();
         C.n_nodes = node;
+        make_clusters(C.h_dom, C.h_brick, cluster_cap(node, true, DTC_FP32_REFINE), C.cl);
         DTC_TRY(C.dom.ensure(C.h_dom.size() * sizeof(DomInfo)));
         DTC_HIP(hipMemcpyAsync(C.dom.p, C.h_dom.data(), C.h_dom.size() * sizeof(DomInfo), hipMemcpyHostToDevice, s));
         DTC_TRY(C.brick.ensure((C.h_brick.size() + 1) * sizeof(BrickInfo)));
@@ -2923,9 +2181,7 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
             k_dinv<<<C.n_bricks, NO, 0, s>>>(C.brick.as<BrickInfo>(), C.dom.as<DomInfo>(), C.lat2node.as<int>(),
                                             C.emod.as<double>(), b.kdiag, C.dinv64.as<double>(), C.dinv32.as<float>());
             DTC_HIP(hipGetLastError());
-            DTC_TRY(build_tables(s, C.h_brick, C.brick, C.dom, C.lat2node, C.emod, C.halo, C.nmask, C.einfo, C.eE64,
-                                 C.eE32, &C.n_tile_elems));
-            DTC_TRY(brick_lists(s, C.n_bricks, C.nmask, C.blist, &C.n_sparse));
+            DTC_TRY(build_clusters(s, C.cl, C.brick, C.dom, C.lat2node, C.emod, false));
         }
         DTC_HIP(hipStreamSynchronize(s));   // ex, cnt go out of scope
     }
@@ -2993,12 +2249,39 @@ int harvest_events(SolverBatch& b) {
     return DTC_OK;
 }
 
-// split > 0: that gridDim.y (the autotuner's candidates), else the tuned one
+// Load cases per wave of k_ebe (LCW): eight from EBE_FILL clusters on, where the vector
+// cache's lookups bound the kernel (one per 32-byte run of x); on smaller grids (coarse
+// levels, single domains) four, which halves the elements that each wave walks through.
+// The sums do not depend on it.
+constexpr int EBE_FILL = 1024;
+template <int LCW, int CAP, typename T, typename TI, typename TO, int IN, int OUT>
+void ebe_grid(int n, hipStream_t s, const EbeArgs& a, const WK<T>& wk, const TI* x, TO* y) {
+    k_ebe<T, TI, TO, IN, OUT, LCW, CAP><<<n, 64 * R / LCW, 0, s>>>(a, wk, x, y);
+}
+template <typename T, typename TI, typename TO, int IN, int OUT>
+int ebe_launch(const Clusters& c, hipStream_t s, EbeArgs a, const WK<T>& wk, const TI* x, TO* y) {
+    if (c.n == 0) return DTC_OK;
+    a.cl = c.info.as<ClusterInfo>();
+    a.enode = c.enode.as<int4>();
+    a.eown = c.eown.as<uint2>();
+    a.eE = sizeof(T) == 4 ? c.eE32.p : c.eE64.p;
+    const bool wide = c.n >= EBE_FILL;
+    if (c.cap != CL_CAP64 || sizeof(T) == 4) {
+        if (wide) ebe_grid<8, CL_CAP, T, TI, TO, IN, OUT>(c.n, s, a, wk, x, y);
+        else ebe_grid<4, CL_CAP, T, TI, TO, IN, OUT>(c.n, s, a, wk, x, y);
+    } else if constexpr (sizeof(T) == 8) {
+        if (wide) ebe_grid<8, CL_CAP64, T, TI, TO, IN, OUT>(c.n, s, a, wk, x, y);
+        else ebe_grid<4, CL_CAP64, T, TI, TO, IN, OUT>(c.n, s, a, wk, x, y);
+    }
+    DTC_HIP(hipGetLastError());
+    return DTC_OK;
+}
+
+// HEX08: x of the IN_U modes holds the Dirichlet values itself (k_set_bc), so they gather
+// it like any vector; HEX20 adds them on the fly (null x: zero)
 template <typename T, int IN, int OUT>
-int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* part, const int* done, int split = 0) {
+int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* part, const int* done) {
     if (b.n_bricks == 0) return DTC_OK;
-    MvArgs a{b.brick.as<BrickInfo>(), nullptr, 0, b.dom.as<DomInfo>(), b.halo.as<int>(), b.nmask.as<unsigned char>(),
-             b.einfo.as<int>(), sizeof(T) == 4 ? b.eE32.p : b.eE64.p, done, part};
     // timed: the CG matvec (OUT_MASKED: of the block PCG) and the FP64 true residual
     constexpr int kind = (IN == IN_V && (OUT == OUT_MASKED_DOT || OUT == OUT_MASKED)) ? DTC_KSTAT_MV
                        : (IN == IN_U && OUT == OUT_RESID)                              ? DTC_KSTAT_RESID
@@ -3007,38 +2290,12 @@ int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* pa
     if (kind >= 0) DTC_TRY(timed_begin(b, kind, &slot));
     if (b.micro20) {
         DTC_TRY(mv20(b, sizeof(T) == 8, IN, OUT, xin, yout, part, done));
-    } else if constexpr (sizeof(T) == 4 && IN == IN_V && (OUT == OUT_MASKED || OUT == OUT_MASKED_DOT)) {
-        if (b.mf_cg) {
-            const dim3 grid(b.n_bricks, split > 0 ? split : tuned_split(TK_MV, 3, b.n_bricks, R / MF_RC));
-            k_matvec_mf<OUT, 3><<<grid, MV_NT, 0, b.stream>>>(a, b.kmf.as<uint4>(), b.kmf_max,
-                                                             reinterpret_cast<const float*>(xin),
-                                                             reinterpret_cast<float*>(yout));
-        } else {
-            const int gy = split > 0 ? split : tuned_split(TK_MV, 0, b.n_bricks, R / MvCfg<T>::RC);
-            if (b.blist.p) {
-                // sparse bricks (256-thread kernel), then the dense ones
-                a.blist = b.blist.as<int>();
-                a.boff = 0;
-                if (b.n_sparse > 0)
-                    k_matvec<T, IN, OUT, false, true><<<dim3(b.n_sparse, gy), MV_NT_SP, 0, b.stream>>>(a, wk, xin, yout);
-                a.boff = b.n_sparse;
-                if (b.n_bricks > b.n_sparse) {
-                    const dim3 gd(b.n_bricks - b.n_sparse, gy);
-                    if (mv_defer()) k_matvec<T, IN, OUT, false, false><<<gd, MV_NT, 0, b.stream>>>(a, wk, xin, yout);
-                    else k_matvec<T, IN, OUT, false, false, false, false><<<gd, MV_NT, 0, b.stream>>>(a, wk, xin, yout);
-                }
-            } else if (mv_defer()) {
-                k_matvec<T, IN, OUT><<<dim3(b.n_bricks, gy), MV_NT, 0, b.stream>>>(a, wk, xin, yout);
-            } else {
-                k_matvec<T, IN, OUT, false, false, false, false><<<dim3(b.n_bricks, gy), MV_NT, 0, b.stream>>>(a, wk, xin,
-                                                                                                         yout);
-            }
-        }
-        DTC_HIP(hipGetLastError());
     } else {
-        const dim3 grid(b.n_bricks, chunk_split(b.n_bricks, R / MvCfg<T>::RC));
-        k_matvec<T, IN, OUT><<<grid, MV_NT, 0, b.stream>>>(a, wk, xin, yout);
-        DTC_HIP(hipGetLastError());
+        EbeArgs a{};
+        a.done = done;
+        a.dinv = sizeof(T) == 4 ? b.dinv32.p : b.dinv64.p;
+        a.partial = part;
+        DTC_TRY((ebe_launch<T, T, T, IN_V, OUT>(b.cl, b.stream, a, wk, xin, yout)));
     }
     // IN_U without x (x = 0) reads no vector
     DTC_TRY(timed_end(b, slot, (IN == IN_U && !xin) ? 1 : 2, sizeof(T) == 8, false, done));
@@ -3047,94 +2304,40 @@ int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* pa
 
 // topology of one level for the FP32 matvec
 struct MvTopo {
+    const Clusters* cl;
     int n_bricks;
     const BrickInfo* bricks;
-    const int* blist;              // sparse bricks first (n_sparse of them), then the dense ones; null: all dense
-    int n_sparse;
     const DomInfo* doms;
-    const int* halo;
-    const unsigned char* nmask;
-    const int* einfo;
-    const void* eE32;
 };
-
-// element products of the smoothing matvecs: 0 Walsh VALU kernel, else MFMA with
-// `terms` FP16 terms (table and normalisation of the batch)
-struct MfUse {
-    int terms;
-    const uint4* tab;
-    float kmax;
-};
-
-// the dense FP32 Chebyshev step without a brick list: whole-segment stores unless
-// DTC_MV_DEFER=0 (df false)
-template <int IN, int OUT, bool PART>
-void mv32_dense(bool df, dim3 grid, hipStream_t s, const MvArgs& a, const WK<float>& wk, const float* x, float* y) {
-    if (df) k_matvec<float, IN, OUT, 0, false, PART, true><<<grid, MV_NT, 0, s>>>(a, wk, x, y);
-    else k_matvec<float, IN, OUT, 0, false, PART, false><<<grid, MV_NT, 0, s>>>(a, wk, x, y);
-}
 
 // tb: the batch whose fine level this is (its launches are timed), else null
-template <int OUT>
-// cin != 0 (OUT_CHEB, dense bricks, VALU element products only): x is cin D^-1 x
+// cin != 0 (OUT_CHEB only): x is cin D^-1 x
 // (the zero-start step formed on the fly, IN_JS)
+template <int OUT>
 int launch_mv32(const MvTopo& T, hipStream_t s, const WK<float>& wk, const float* x, float* y, const int* done,
-                const float* bv = nullptr, const float* dinv = nullptr, float* dv = nullptr, float c1 = 0.f,
-                float c2 = 0.f, double* partial = nullptr, int cflags = CH_READ_D | CH_WRITE_D,
-                SolverBatch* tb = nullptr, MfUse mf = MfUse{0, nullptr, 0.f}, int split = 0, float cin = 0.f) {
+                const float* bv, const float* dinv, float* dv, float c1, float c2, int cflags, SolverBatch* tb,
+                float cin) {
+    static_assert(OUT == OUT_CHEB || OUT == OUT_BRES, "smoothing step or restriction residual");
     if (T.n_bricks == 0) return DTC_OK;
-    if (cin != 0.f && (OUT != OUT_CHEB || mf.terms != 0 || T.n_sparse > 0))
-        return set_error(DTC_ERR_BAD_ARGUMENT, "zero-start input needs the dense FP32 Chebyshev step");
-    MvArgs a{T.bricks, nullptr, 0, T.doms, T.halo, T.nmask, T.einfo, T.eE32, done, partial, bv, dinv, dv, c1, c2, cflags};
-    a.cin = cin;
-    const int tk = OUT == OUT_CHEB ? TK_CHEB : TK_BRES;
-    const dim3 grid(T.n_bricks, split > 0 ? split : tuned_split(tk, mf.terms, T.n_bricks, R / MvCfg<float>::RC));
-    constexpr int kind = OUT == OUT_CHEB ? DTC_KSTAT_CHEB : OUT == OUT_BRES ? DTC_KSTAT_BRES : -1;
+    if (cin != 0.f && OUT != OUT_CHEB) return set_error(DTC_ERR_BAD_ARGUMENT, "zero-start input needs the Chebyshev step");
+    constexpr int kind = OUT == OUT_CHEB ? DTC_KSTAT_CHEB : DTC_KSTAT_BRES;
     int slot = -1;
-    if (tb && kind >= 0) DTC_TRY(timed_begin(*tb, kind, &slot));
-    if (mf.terms == 3 && partial) k_matvec_mf<OUT, 3, true><<<grid, MV_NT, 0, s>>>(a, mf.tab, mf.kmax, x, y);
-    else if (mf.terms == 3) k_matvec_mf<OUT, 3><<<grid, MV_NT, 0, s>>>(a, mf.tab, mf.kmax, x, y);
-    else if (mf.terms == 1 && partial) k_matvec_mf<OUT, 1, true><<<grid, MV_NT, 0, s>>>(a, mf.tab, mf.kmax, x, y);
-    else if (mf.terms == 1) k_matvec_mf<OUT, 1><<<grid, MV_NT, 0, s>>>(a, mf.tab, mf.kmax, x, y);
-    else if (T.blist) {
-        // sparse bricks (256-thread kernel), then the dense ones
-        constexpr bool CP = OUT == OUT_CHEB;
-        MvArgs as = a;
-        as.blist = T.blist;
-        as.boff = 0;
-        if (T.n_sparse > 0) {
-            const dim3 gs(T.n_sparse, grid.y);
-            if (CP && partial) k_matvec<float, IN_V, OUT, false, true, CP><<<gs, MV_NT_SP, 0, s>>>(as, wk, x, y);
-            else k_matvec<float, IN_V, OUT, false, true, false><<<gs, MV_NT_SP, 0, s>>>(as, wk, x, y);
-        }
-        as.boff = T.n_sparse;
-        if (T.n_bricks > T.n_sparse) {
-            const dim3 gd(T.n_bricks - T.n_sparse, grid.y);
-            const bool df = mv_defer();
-            bool js = false;
-            if constexpr (OUT == OUT_CHEB) {
-                js = cin != 0.f;
-                if (js && CP && partial && df) k_matvec<float, IN_JS, OUT, false, false, CP><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-                else if (js && CP && partial) k_matvec<float, IN_JS, OUT, false, false, CP, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-                else if (js && df) k_matvec<float, IN_JS, OUT, false, false, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-                else if (js) k_matvec<float, IN_JS, OUT, false, false, false, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-            }
-            if (js) {
-            } else if (CP && partial && df) k_matvec<float, IN_V, OUT, false, false, CP><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-            else if (CP && partial) k_matvec<float, IN_V, OUT, false, false, CP, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-            else if (df) k_matvec<float, IN_V, OUT, false, false, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-            else k_matvec<float, IN_V, OUT, false, false, false, false><<<gd, MV_NT, 0, s>>>(as, wk, x, y);
-        }
-    } else if constexpr (OUT == OUT_CHEB) {
-        const bool df = mv_defer();
-        if (cin != 0.f && partial) mv32_dense<IN_JS, OUT, true>(df, grid, s, a, wk, x, y);
-        else if (cin != 0.f) mv32_dense<IN_JS, OUT, false>(df, grid, s, a, wk, x, y);
-        else if (partial) mv32_dense<IN_V, OUT, true>(df, grid, s, a, wk, x, y);
-        else mv32_dense<IN_V, OUT, false>(df, grid, s, a, wk, x, y);
-    } else {
-        k_matvec<float, IN_V, OUT><<<grid, MV_NT, 0, s>>>(a, wk, x, y);
+    if (tb) DTC_TRY(timed_begin(*tb, kind, &slot));
+    EbeArgs a{};
+    a.done = done;
+    a.dinv = dinv;
+    a.bvec = bv;
+    a.dvec = dv;
+    a.c1 = c1;
+    a.c2 = c2;
+    a.cflags = cflags;
+    a.cin = cin;
+    bool js = false;
+    if constexpr (OUT == OUT_CHEB) {
+        js = cin != 0.f;
+        if (js) DTC_TRY((ebe_launch<float, float, float, IN_JS, OUT>(*T.cl, s, a, wk, x, y)));
     }
-    DTC_HIP(hipGetLastError());
+    if (!js) DTC_TRY((ebe_launch<float, float, float, IN_V, OUT>(*T.cl, s, a, wk, x, y)));
     if (tb) {
         // x, y, b (with the zero-start input x is b itself: 2 vectors); Chebyshev: the
         // direction read and written as the flags say
@@ -3187,12 +2390,10 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     const int* done = b.done_ext ? b.done_ext : b.done.as<int>();
     static const MgParams P = mg_params();
     const int deg = b.mg_degree > 0 ? b.mg_degree : 2;
-    const MfUse mfu{b.mf_smooth, b.kmf.as<uint4>(), b.kmf_max};
     auto view = [&](int l) {
         LvView v;
         if (l == 0) {
-            v.T = {b.n_bricks, b.brick.as<BrickInfo>(), b.blist.as<int>(), b.n_sparse, b.dom.as<DomInfo>(), b.halo.as<int>(),
-                   b.nmask.as<unsigned char>(), b.einfo.as<int>(), b.eE32.p};
+            v.T = {&b.cl, b.n_bricks, b.brick.as<BrickInfo>(), b.dom.as<DomInfo>()};
             v.l2n = b.lat2node.as<int>();
             v.dinv = b.dinv32.as<float>();
             v.b = const_cast<float*>(r);
@@ -3201,8 +2402,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
             v.d = b.d32.as<float>();
         } else {
             Level& C = b.mg[l - 1];
-            v.T = {C.n_bricks, C.brick.as<BrickInfo>(), C.blist.as<int>(), C.n_sparse, C.dom.as<DomInfo>(), C.halo.as<int>(),
-                   C.nmask.as<unsigned char>(), C.einfo.as<int>(), C.eE32.p};
+            v.T = {&C.cl, C.n_bricks, C.brick.as<BrickInfo>(), C.dom.as<DomInfo>()};
             v.l2n = C.lat2node.as<int>();
             v.dinv = C.dinv32.as<float>();
             v.b = C.b.as<float>();
@@ -3213,7 +2413,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
         return v;
     };
     std::vector<int> cur(L + 1, 0);
-    auto smooth = [&](int l, int m, bool zero, double ratio, double* dot) -> int {
+    auto smooth = [&](int l, int m, bool zero, double ratio) -> int {
         const LvView v = view(l);
         if (v.T.n_bricks == 0) return DTC_OK;
         const double hi = b.cheb_lmax * P.lscale, lo = hi / ratio;
@@ -3228,23 +2428,21 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
                 c2 = (float)(2.0 * rn / delta);
                 rho = rn;
             }
-            double* dk = k == m - 1 ? dot : nullptr;
             // the zero-start step x_1 = c2 D^-1 b is formed inside the next step's
             // staging (IN_JS) instead of being stored, where that kernel form runs
-            const bool fuse = zero && m >= 2 && mfu.terms == 0 && v.T.n_sparse == 0 && cheb_fuse();
+            const bool fuse = zero && m >= 2 && cheb_fuse();
             if (zero && k == 0 && fuse) {
                 c0 = c2;
             } else if (zero && k == 0) {
                 // x_1 = d_0: the next step takes its previous direction from x
                 k_cheb<<<v.T.n_bricks, NT_UPD, 0, s>>>(v.T.bricks, done, v.b, nullptr, v.dinv, nullptr, v.buf[cur[l]],
-                                                       c1, c2, 1, dk);
+                                                       c1, c2, 1, nullptr);
                 DTC_HIP(hipGetLastError());
             } else {
                 const int fl = (k == 0 ? 0 : (zero && k == 1) ? CH_D_FROM_X : CH_READ_D) | (k < m - 1 ? CH_WRITE_D : 0);
                 const bool js = fuse && k == 1;
                 DTC_TRY(launch_mv32<OUT_CHEB>(v.T, s, wk, js ? v.b : v.buf[cur[l]], v.buf[1 - cur[l]], done, v.b,
-                                              v.dinv, v.d, c1, c2, dk, fl, l == 0 ? &b : nullptr, mfu, 0,
-                                              js ? c0 : 0.f));
+                                              v.dinv, v.d, c1, c2, fl, l == 0 ? &b : nullptr, js ? c0 : 0.f));
                 cur[l] = 1 - cur[l];
             }
         }
@@ -3254,17 +2452,17 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     // coarse levels): start in the buffer that makes it end in z
     cur[0] = (L > 0 ? 2 * deg - 1 : P.coarse_degree - 1) % 2;
     for (int l = 0; l < L; ++l) {
-        DTC_TRY(smooth(l, deg, true, P.ratio, nullptr));
+        DTC_TRY(smooth(l, deg, true, P.ratio));
         const LvView f = view(l), c = view(l + 1);
         cur[l + 1] = 0;
         if (c.T.n_bricks == 0 || f.T.n_bricks == 0) continue;
         float* res = f.buf[1 - cur[l]];
-        DTC_TRY(launch_mv32<OUT_BRES>(f.T, s, wk, f.buf[cur[l]], res, done, f.b, nullptr, nullptr, 0.f, 0.f, nullptr,
-                                      0, l == 0 ? &b : nullptr, mfu));
+        DTC_TRY(launch_mv32<OUT_BRES>(f.T, s, wk, f.buf[cur[l]], res, done, f.b, f.dinv, nullptr, 0.f, 0.f, 0,
+                                      l == 0 ? &b : nullptr, 0.f));
         k_restrict<<<dim3(c.T.n_bricks, node_split(c.T.n_bricks)), 256, 0, s>>>(c.T.bricks, c.T.doms, c.l2n, f.T.doms, f.l2n, res, done, c.b);
         DTC_HIP(hipGetLastError());
     }
-    DTC_TRY(smooth(L, P.coarse_degree, true, P.coarse_ratio, L == 0 ? prz : nullptr));
+    DTC_TRY(smooth(L, P.coarse_degree, true, P.coarse_ratio));
     for (int l = L - 1; l >= 0; --l) {
         const LvView f = view(l), c = view(l + 1);
         if (f.T.n_bricks > 0 && c.T.n_bricks > 0) {
@@ -3272,7 +2470,11 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
                                                    f.buf[cur[l]]);
             DTC_HIP(hipGetLastError());
         }
-        DTC_TRY(smooth(l, deg, false, P.ratio, l == 0 ? prz : nullptr));
+        DTC_TRY(smooth(l, deg, false, P.ratio));
+    }
+    if (prz && b.n_bricks > 0) {
+        k_dot<<<b.n_bricks, NT_UPD, 0, s>>>(b.brick.as<BrickInfo>(), done, r, z, prz);
+        DTC_HIP(hipGetLastError());
     }
     return DTC_OK;
 }
@@ -3372,7 +2574,8 @@ int pcg_iteration(SolverBatch& b, const WK<T>& wk, T* x, T* r, T* p, T* q, const
     const int D = b.n_dom, NBk = b.n_bricks;
     int* done = b.done.as<int>();
     DTC_TRY((launch_mv<T, IN_V, OUT_MASKED_DOT>(b, wk, p, q, b.part_a.as<double>(), done)));
-    k_red_alpha<<<D, RED_NT, 0, b.stream>>>(b.dom.as<DomInfo>(), done, b.part_a.as<double>(), b.active.as<int>(),
+    k_red_alpha<<<D, RED_NT, 0, b.stream>>>(b.dom.as<DomInfo>(), done, b.part_a.as<double>(),
+                                            !b.micro20, b.active.as<int>(),
                                         b.rz.as<double>(), b.alpha.as<double>());
     k_cg_update<T><<<NBk, NT_UPD, 0, b.stream>>>(b.brick.as<BrickInfo>(), done, b.alpha.as<double>(), x, r, p, q, dinv,
                                                  zmg ? nullptr : b.part_a.as<double>(), b.part_b.as<double>());
@@ -3417,18 +2620,14 @@ int pcg_run(SolverBatch& b, const WK<T>& wk, T* x, T* r, T* p, T* q, const T* di
 // W's small eigenvalues (the ones that steer the block) drown in that error.
 // q64 set: Q is written as an FP64 vector (the block PCG on FP64 vectors)
 int launch_mv_q64(SolverBatch& b, const float* p, float* q, const int* done, double* q64 = nullptr) {
-    MvArgs a{b.brick.as<BrickInfo>(), nullptr, 0, b.dom.as<DomInfo>(), b.halo.as<int>(), b.nmask.as<unsigned char>(),
-             b.einfo.as<int>(), b.eE64.p, done, nullptr};
+    EbeArgs a{};
+    a.done = done;
+    a.dinv = b.dinv64.p;
     int slot = -1;
     DTC_TRY(timed_begin(b, DTC_KSTAT_MV, &slot));
-    const dim3 grid(b.n_bricks, chunk_split(b.n_bricks, R / MvCfg<double>::RC));
-    if (q64)
-        k_matvec<double, IN_V, OUT_MASKED, 2><<<grid, MV_NT, 0, b.stream>>>(
-            a, cast_wk<double>(b.wk64), reinterpret_cast<const double*>(p), q64);
-    else
-        k_matvec<double, IN_V, OUT_MASKED, 1><<<grid, MV_NT, 0, b.stream>>>(
-            a, cast_wk<double>(b.wk64), reinterpret_cast<const double*>(p), reinterpret_cast<double*>(q));
-    DTC_HIP(hipGetLastError());
+    const WK<double> wk = cast_wk<double>(b.wk64);
+    if (q64) DTC_TRY((ebe_launch<double, float, double, IN_V, OUT_MASKED>(b.cl, b.stream, a, wk, p, q64)));
+    else DTC_TRY((ebe_launch<double, float, float, IN_V, OUT_MASKED>(b.cl, b.stream, a, wk, p, q)));
     DTC_TRY(timed_end(b, slot, 2, false, false, done));
     return DTC_OK;
 }
@@ -3467,19 +2666,6 @@ int block_setup(SolverBatch& b) {
 
 // per-domain Grams a^T b and a^T c (c may be null) into gsum
 template <typename T> struct NoDeduce { using type = T; };
-// the Gram partials of the orthonormalisation formed in the direction kernel that
-// writes the new block (DTC_ORTH_FUSE=0: a separate Gram kernel reads it back)
-inline bool orth_fuse() {
-    const char* e = std::getenv("DTC_ORTH_FUSE");
-    return !(e && e[0] == '0');
-}
-
-// Gram form: rows staged through LDS (default) or read by every lane from global
-// memory (DTC_GRAM_LDS=0; the same sums, for measurements)
-inline bool gram_lds() {
-    const char* e = std::getenv("DTC_GRAM_LDS");
-    return !(e && e[0] == '0');
-}
 template <typename TA = float, typename TB = float>
 int block_gram(SolverBatch& b, const TA* a, const TB* bb, const typename NoDeduce<TB>::type* c) {
     hipStream_t s = b.stream;
@@ -3487,13 +2673,8 @@ int block_gram(SolverBatch& b, const TA* a, const TB* bb, const typename NoDeduc
     if (b.n_slices > 0) {
         const int4* sl = b.slices.as<int4>();
         double* gp = b.gpart.as<double>();
-        if (gram_lds()) {
-            if (c) k_gram_lds<2, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, c, gp);
-            else k_gram_lds<1, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, nullptr, gp);
-        } else {
-            if (c) k_gram<2, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, c, gp);
-            else k_gram<1, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, nullptr, gp);
-        }
+        if (c) k_gram<2, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, c, gp);
+        else k_gram<1, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, nullptr, gp);
     }
     k_gram_sum<<<dim3(b.n_dom, 2 * RR / 64), 256, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
                                                          b.gsum.as<double>());
@@ -3521,19 +2702,15 @@ int block_orth(SolverBatch& b, const float* src, float* dst, bool partials_done 
     return DTC_OK;
 }
 
-// the new direction block Z + P beta and, with orth_fuse(), its Gram partials in the
-// same kernel; then the orthonormalisation into p
+// the new direction block Z + P beta and its Gram partials in one kernel, then the
+// orthonormalisation into p
 int block_dir_orth(SolverBatch& b, float* p, const float* z, float* q) {
     hipStream_t s = b.stream;
     int* done = b.done.as<int>();
-    const int4* sl = b.slices.as<int4>();
-    const bool fuse = orth_fuse() && b.n_slices > 0;
-    if (fuse)
-        k_bdir<true><<<b.n_slices, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), p, z, q, b.gpart.as<double>());
-    else
-        k_bdir<false><<<b.n_slices, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), p, z, q, nullptr);
+    k_bdir<true><<<b.n_slices, NT_UPD, 0, s>>>(b.slices.as<int4>(), done, b.bcoef.as<float>(), p, z, q,
+                                               b.gpart.as<double>());
     DTC_HIP(hipGetLastError());
-    return block_orth(b, q, p, fuse);
+    return block_orth(b, q, p, true);
 }
 
 // one block PCG iteration on FP64 vectors (x64, r64) with the FP32 multigrid as
@@ -3704,10 +2881,14 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
     return DTC_OK;
 }
 
-// FP64 true residual r64 = -(K u)_free, u = x64 + x_bc (x64 == null: u = x_bc),
+// FP64 true residual r64 = -(K u)_free, u = x64 + x_bc (x64 == null: u = x_bc; HEX08: x64
+// holds the Dirichlet values),
 // then per load case activity and targets (k_red_outer)
 int residual64(SolverBatch& b, const WK<double>& wk, const double* x64, int first, const dtc_solve_opts& o) {
-    DTC_TRY((launch_mv<double, IN_U, OUT_RESID>(b, wk, x64, b.r64.as<double>(), b.part_c.as<double>(), nullptr)));
+    double* r64 = b.r64.as<double>();
+    DTC_TRY((launch_mv<double, IN_U, OUT_RESID>(b, wk, x64, r64, b.part_c.as<double>(), nullptr)));
+    if (!b.micro20)   // (the HEX20 operator forms the sums itself)
+        k_dot<double><<<b.n_bricks, NT_UPD, 0, b.stream>>>(b.brick.as<BrickInfo>(), nullptr, r64, r64, b.part_c.as<double>());
     const double* itol2 = b.precision == DTC_FP32_REFINE && !b.block64 ? b.itol2.as<double>() : nullptr;
     k_red_outer<<<b.n_dom, RED_NT, 0, b.stream>>>(b.dom.as<DomInfo>(), b.part_c.as<double>(), first,
                                                   o.rel_tol * o.rel_tol, itol2, b.rr0.as<double>(), b.rr.as<double>(),
@@ -3793,110 +2974,14 @@ int apply_cap(SolverBatch& b, int64_t cap, std::vector<int64_t>& nouter, bool* a
 
 }  // namespace
 
-// Times every candidate split of the FP32 matvec kernels the mixed multigrid solve
-// launches (Q = K P on the fine level; the Chebyshev step and the restriction
-// residual on every level) on this batch's own tables, and caches the fastest
-// (see tuned_split).  The timed launches read the level's work vectors and write
-// its scratch vector, before the solve starts, with no done flags.
-int autotune_splits(SolverBatch& b, const WK<float>& wk) {
-    const char* te = std::getenv("DTC_TUNE");
-    if ((te && te[0] == '0') || b.n_bricks == 0 || b.micro20) return DTC_OK;
-    const char* le = std::getenv("DTC_TUNE_LOG");
-    const bool log = le && le[0] == '1';
-    hipStream_t s = b.stream;
-    hipEvent_t e0, e1;
-    DTC_HIP(hipEventCreate(&e0));
-    DTC_HIP(hipEventCreate(&e1));
-    int rc = DTC_OK;
-    auto measure = [&](int kind, int variant, int nbr, const char* what, int level,
-                       const std::function<int(int)>& launch) {
-        if (rc != DTC_OK || nbr == 0) return;
-        {
-            std::lock_guard<std::mutex> lk(g_tune_mu);
-            if (g_tune.count(std::make_tuple(kind, variant, nbr))) return;
-        }
-        const int cand[4] = {1, 2, 3, 6};
-        int best = chunk_split(nbr, R / MF_RC);
-        float best_ms = 1e30f;
-        for (int c : cand) {
-            if ((rc = launch(c)) != DTC_OK) return;   // warm-up
-            if (hipEventRecord(e0, s) != hipSuccess) { rc = set_error(DTC_ERR_DEVICE, "hipEventRecord"); return; }
-            for (int k = 0; k < 3 && rc == DTC_OK; ++k) rc = launch(c);
-            if (rc != DTC_OK) return;
-            float ms = 0.f;
-            if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = set_error(DTC_ERR_DEVICE, "autotune timing");
-                return;
-            }
-            if (log)
-                std::fprintf(stderr, "dtc autotune:   %s level %d candidate gridDim.y %d: %.1f us\n", what, level, c,
-                             1e3f * ms / 3.f);
-            if (ms < best_ms) { best_ms = ms; best = c; }
-        }
-        if (log)
-            std::fprintf(stderr, "dtc autotune: %s level %d, %d bricks: gridDim.y %d (%.1f us)\n", what, level, nbr,
-                         best, 1e3f * best_ms / 3.f);
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tune[std::make_tuple(kind, variant, nbr)] = best;
-    };
-    float* p = b.p32.as<float>();
-    float* q = b.q32.as<float>();
-    measure(TK_MV, b.mf_cg ? 3 : 0, b.n_bricks, "Q = K P", 0, [&](int c) {
-        return launch_mv<float, IN_V, OUT_MASKED>(b, wk, p, q, nullptr, nullptr, c);
-    });
-    const MfUse mfu{b.mf_smooth, b.kmf.as<uint4>(), b.kmf_max};
-    for (int l = 0; l <= (int)b.mg.size() && rc == DTC_OK; ++l) {
-        MvTopo T;
-        float *x, *bb, *y, *d;
-        const float* dinv;
-        if (l == 0) {
-            T = {b.n_bricks, b.brick.as<BrickInfo>(), b.blist.as<int>(), b.n_sparse, b.dom.as<DomInfo>(), b.halo.as<int>(),
-                 b.nmask.as<unsigned char>(),
-                 b.einfo.as<int>(), b.eE32.p};
-            x = b.z32.as<float>(); bb = b.r32.as<float>(); y = b.t32.as<float>(); d = b.d32.as<float>();
-            dinv = b.dinv32.as<float>();
-        } else {
-            Level& C = b.mg[l - 1];
-            T = {C.n_bricks, C.brick.as<BrickInfo>(), C.blist.as<int>(), C.n_sparse, C.dom.as<DomInfo>(), C.halo.as<int>(),
-                 C.nmask.as<unsigned char>(),
-                 C.einfo.as<int>(), C.eE32.p};
-            x = C.x.as<float>(); bb = C.b.as<float>(); y = C.t.as<float>(); d = C.d.as<float>();
-            dinv = C.dinv32.as<float>();
-        }
-        if (!x || !bb || !y) continue;
-        measure(TK_CHEB, mfu.terms, T.n_bricks, "Chebyshev step", l, [&](int c) {
-            return launch_mv32<OUT_CHEB>(T, s, wk, x, y, nullptr, bb, dinv, d, 0.f, 1.f, nullptr, 0, nullptr, mfu, c);
-        });
-        measure(TK_BRES, mfu.terms, T.n_bricks, "restriction residual", l, [&](int c) {
-            return launch_mv32<OUT_BRES>(T, s, wk, x, y, nullptr, bb, nullptr, nullptr, 0.f, 0.f, nullptr, 0, nullptr,
-                                         mfu, c);
-        });
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    return rc;
-}
-
 int batch_build_pmg(SolverBatch& b, SolverBatch& c) { return build_pmg(b, c); }
-
-// the launch-shape tuning of a mixed multigrid solve, ahead of it (after the
-// multigrid hierarchy is built): sub-batches solved at the same time are tuned one
-// after another before their solves start, so that no tuning launch overlaps
-// another sub-batch's kernels (batch_solve then finds the choices cached)
-int batch_autotune(SolverBatch& b) {
-    if (b.precision != DTC_FP32_REFINE || b.precond != DTC_PC_MG || (b.micro20 && !b.p08)) return DTC_OK;
-    return autotune_splits(b, cast_wk<float>(b.wk64));
-}
 
 int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>& iters,
                 std::vector<int64_t>& outer, std::vector<double>& relres) {
     const int D = b.n_dom;
     // with the multigrid, the 24 load cases of a domain iterate as one block
     // (DTC_BLOCK_PCG=0: one PCG per load case)
-    const char* be = std::getenv("DTC_BLOCK_PCG");
-    const bool block = b.precision == DTC_FP32_REFINE && b.precond == DTC_PC_MG && (!b.micro20 || b.p08) &&
-                       !(be && be[0] == '0');
+    const bool block = b.precision == DTC_FP32_REFINE && block_pcg(b) && (!b.micro20 || b.p08);
     // inner_tol outside (0, 1): automatic, per domain.  The block restarts at every
     // FP64 residual replacement, so it takes its FP32 phases as deep as FP32
     // allows: 1e-6 (two phases to 1e-8 instead of three) where the moduli of the
@@ -3972,7 +3057,13 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         b.block64 = block && (e64 ? e64[0] == '1' : cmax > 100.0);
         if (b.block64) DTC_TRY(b.q64.ensure((size_t)nv * 8));
     }
-    DTC_TRY(residual64(b, wk64, nullptr, 1, o));          // r64 = f (lifted right-hand side)
+    // r64 = f (lifted right-hand side).  HEX08: the Dirichlet values are written into x64
+    // once; every update of x64 adds zero there, and its other readers form them again
+    if (!b.micro20) {
+        k_set_bc<<<dim3(b.n_bricks, 8), NT_UPD, 0, s>>>(bl, dl, b.lat2node.as<int>(), b.x64.as<double>());
+        DTC_HIP(hipGetLastError());
+    }
+    DTC_TRY(residual64(b, wk64, b.micro20 ? nullptr : b.x64.as<double>(), 1, o));
 
     if (b.precision == DTC_FP64) {
         // PCG in FP64 on (x64, r64); a true-residual check restarts it if the
@@ -4027,7 +3118,6 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         float* bq = b.q32.as<float>();
         float* bz = z32;
         if (block) DTC_TRY(block_setup(b));
-        if (mg) DTC_TRY(autotune_splits(b, wk32));
         bool first = true;
         for (int it = 0; it < 100000; ++it) {
             bool left = false;

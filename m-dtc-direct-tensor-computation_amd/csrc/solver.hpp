@@ -10,16 +10,26 @@ struct KernelStat {
     int64_t count = 0;
 };
 
+// Clusters of one level (device) and their element tables.
+struct Clusters {
+    int n = 0;
+    int cap = CL_CAP;              // most nodes of one
+    std::vector<ClusterInfo> h;
+    DevMem info;                   // ClusterInfo[]
+    DevMem enode;                  // int4 [element][2]: solver nodes of the 8 corners
+    DevMem eown;                   // uint2 per element: the corners' node indices in the cluster, cap = not owned
+    DevMem eE64, eE32;             // element modulus (eE64: the fine level only)
+};
+
 // One coarse level of the multigrid preconditioner: voxels of 2^l fine voxels,
 // same brick layout and matvec tables as the fine level, FP32 vectors.
 struct Level {
     int n_bricks = 0;
-    int64_t n_nodes = 0, n_lat = 0, n_vox = 0, n_tile_elems = 0;
+    int64_t n_nodes = 0, n_lat = 0, n_vox = 0;
     std::vector<DomInfo> h_dom;
     std::vector<BrickInfo> h_brick;
-    DevMem dom, brick, lat2node, emod, halo, nmask, einfo, eE64, eE32, dinv64, dinv32;
-    DevMem blist;                  // bricks for the FP32 matvecs: n_sparse sparse ones first, then the dense ones
-    int n_sparse = 0;
+    DevMem dom, brick, lat2node, emod, dinv64, dinv32;
+    Clusters cl;
     DevMem b, x, t, d;             // right-hand side, iterate, matvec output, Chebyshev direction
 };
 
@@ -93,14 +103,7 @@ struct SolverBatch {
     DevMem lat2node;               // int32 per lattice node (-1 = no solver node)
     DevMem sol2ref;                // int32 per solver node: mesh node id (1-based)
     DevMem emod;                   // double per voxel (0 = no element)
-    // per-brick matvec tables, built once per solve
-    DevMem halo;                   // int [brick][HX*HY*HZ]: solver node | BC_BIT, -1 = none
-    DevMem nmask;                  // uint8 [brick][BX*BY*BZ]: solid tile elements around each owned node
-    DevMem einfo;                  // int per tile element: halo base | (owned base + 41) << 9 | owned corners << 24
-    DevMem eE64, eE32;             // element modulus per tile element
-    int64_t n_tile_elems = 0;
-    DevMem blist;                  // bricks for the FP32 matvecs: n_sparse sparse ones first, then the dense ones
-    int n_sparse = 0;
+    Clusters cl;                   // HEX08 matvec clusters, built once per solve
     DevMem dinv64, dinv32;         // Jacobi: 1 / diag(K) per DOF [node][3] (0 on Dirichlet DOFs)
     // vectors, layout [node][3][24]
     DevMem x64, r64, p64, q64;
@@ -150,12 +153,6 @@ struct SolverBatch {
     std::vector<double> khat20;    // E = 1 element stiffness, 60 x 60
     DevMem k20_64, k20_32;
     WalshK wk64{};
-    // element products on the matrix cores (FP32 matvecs): B operands of the
-    // normalised element stiffness, its normalisation, and which kernels use them
-    DevMem kmf;                    // uint4 [tile 2][term 2][lane 64]
-    float kmf_max = 0.f;
-    int mf_cg = 0;                 // Q = K P (and q = K p): 0 Walsh VALU kernel, 1 MFMA (3 FP16 terms)
-    int mf_smooth = 0;             // smoothing and restriction residual: 0 Walsh, 1 or 3 MFMA terms
     double kdiag = 0.0;            // diagonal entry of the E = 1 element stiffness
     double nu = 0.3, a = 1.0;
     std::vector<double> h_contrast;   // per domain group: modulus contrast (max / min) over its solid voxels
@@ -211,7 +208,6 @@ int batch_build_mg(SolverBatch& b, int max_levels);
 // p-multigrid of a HEX20 micro batch b over c, the HEX08 discretisation of the same
 // voxels and domain groups (both finalised): builds c's levels and links c to b.
 int batch_build_pmg(SolverBatch& b, SolverBatch& c);
-int batch_autotune(SolverBatch& b);
 // DTC_HEX20_GATHER=1: the HEX20 operator as the node-gather kernel (the reference form;
 // no Chebyshev epilogue), else element pass + node sums
 inline bool hex20_gather_form() {
