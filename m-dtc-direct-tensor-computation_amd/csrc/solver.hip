@@ -442,14 +442,20 @@ __global__ __launch_bounds__(NT_UPD) void k_acc64(const BrickInfo* __restrict__ 
 //   Z = M R,  beta = -W^+ (Q^T Z),  P = Z + P beta.
 // A vector row is one (node, direction) pair holding the 24 load cases.
 constexpr int GR_NT = 256;          // 4 waves
-constexpr int SLICE_NODES = 512;    // nodes per Gram workgroup (at least)
-constexpr int MAX_SLICES = 1024;    // Gram workgroups per domain (at most)
+// Slices of a domain's nodes, one workgroup each in the block's vector kernels: a slice is a
+// serial walk over its rows, so a domain is cut into as many as pay (domains alone, 22 / 56 /
+// 146 iterations: 512 nodes a slice 12.0 ms at 12^3, 39 at 33^3, 131 at 64^3; 32 nodes, at most
+// 512 slices 6.5, 26 and 104; 1024 slices 106).  In a batch that fills the chip the
+// longer partial-sum lists cost what the shorter walks give (16 x 64^3: 512 against 508 ms).
+// The cut follows from the domain alone, so its sums do not depend on the batch.
+constexpr int SLICE_NODES = 32;     // nodes per slice (at least)
+constexpr int MAX_SLICES = 512;     // slices per domain (at most)
 constexpr int RR = R * R;           // entries of a 24 x 24 coefficient matrix
 constexpr double PIVOT_DROP = 1e-9;   // of P^T A P
 constexpr double ORTH_DROP = 1e-10;   // of P^T P
 
 // Gram partial sums over the rows of one slice of a domain's nodes:
-//   g[0] = A^T B, g[1] = A^T C (NGR = 2; zero for NGR = 1), FP64 sums of the
+//   g[0] = A^T B, g[1] = A^T C (NGR = 2; not written for NGR = 1), FP64 sums of the
 // products of FP32 (or FP64) operands.  Lane (i, j) of a wave keeps rows 3i..3i+2 x
 // columns 3j..3j+2.  The workgroup loads blocks of GB_ROWS vector rows of A, B (and C)
 // with coalesced 16-byte loads (the next block's loads issued before the current
@@ -546,28 +552,39 @@ __global__ __launch_bounds__(GR_NT) void k_gram(const int4* __restrict__ slices,
         __syncthreads();
     }
     double* out = gpart + (int64_t)blockIdx.x * 2 * RR;
-    for (int e = tid; e < 2 * RR; e += GR_NT) out[e] = e < NGR * RR ? s_g[e] : 0.0;
+    for (int e = tid; e < NGR * RR; e += GR_NT) out[e] = s_g[e];
 }
 
 // gsum[d] = sum over the domain's slices of the Gram partials, in a fixed order:
-// workgroup (d, c) sums entries 64c..64c+63 of the 2 x 576; wave w takes the
-// slices w, w + 4, ... and the four waves are added in order
-__global__ __launch_bounds__(256) void k_gram_sum(const int* __restrict__ dslice, const int* __restrict__ done,
-                                                 const double* __restrict__ gpart, double* __restrict__ gsum) {
-    __shared__ double s_w[4][64];
+// workgroup (d, c) sums entries 64c..64c+63; wave w takes the slices w, w + 16, ... four
+// at a time and the waves are added in order
+constexpr int GS_W = 16;
+__global__ __launch_bounds__(64 * GS_W) void k_gram_sum(const int* __restrict__ dslice, const int* __restrict__ done,
+                                                       const double* __restrict__ gpart, double* __restrict__ gsum) {
+    __shared__ double s_w[GS_W][64];
     const int d = blockIdx.x;
     if (done[d]) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, e = (int)blockIdx.y * 64 + lane;
     const int s0 = dslice[d], s1 = dslice[d + 1];
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
-    int s = s0 + wave;
-    for (; s + 12 < s1; s += 16)
+    constexpr int U = 8;
+    double a[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] += gpart[(int64_t)(s + 4 * u) * 2 * RR + e];
-    for (int u = 0; s < s1; s += 4, ++u) a[u & 3] += gpart[(int64_t)s * 2 * RR + e];
-    s_w[wave][lane] = ((a[0] + a[1]) + a[2]) + a[3];
+    for (int u = 0; u < U; ++u) a[u] = 0.0;
+    for (int s = s0 + wave; s < s1; s += U * GS_W)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u * GS_W < s1) a[u] += gpart[(int64_t)(s + u * GS_W) * 2 * RR + e];
+    double t = a[0];
+#pragma unroll
+    for (int u = 1; u < U; ++u) t += a[u];
+    s_w[wave][lane] = t;
     __syncthreads();
-    if (wave == 0) gsum[(int64_t)d * 2 * RR + e] = ((s_w[0][lane] + s_w[1][lane]) + s_w[2][lane]) + s_w[3][lane];
+    if (wave == 0) {
+        t = s_w[0][lane];
+#pragma unroll
+        for (int w = 1; w < GS_W; ++w) t += s_w[w][lane];
+        gsum[(int64_t)d * 2 * RR + e] = t;
+    }
 }
 
 // Per domain: takes the Gram sums of k_gram_sum, then
@@ -899,7 +916,7 @@ __global__ __launch_bounds__(NT_UPD) void k_bdir(const int4* __restrict__ slices
             __syncthreads();
         }
         double* out = gpart + (int64_t)blockIdx.x * 2 * RR;
-        for (int e = tid; e < 2 * RR; e += NT_UPD) out[e] = e < RR ? s_g[e] : 0.0;
+        for (int e = tid; e < RR; e += NT_UPD) out[e] = s_g[e];
     }
 }
 
@@ -2633,8 +2650,8 @@ int launch_mv_q64(SolverBatch& b, const float* p, float* q, const int* done, dou
 }
 
 // block PCG set-up: slices of SLICE_NODES nodes (more for domains of over
-// MAX_SLICES * SLICE_NODES nodes) within each domain for the Gram sums, and the
-// per-domain factor and coefficient storage
+// MAX_SLICES * SLICE_NODES nodes) within each domain for the block's vector kernels, and
+// the per-domain factor and coefficient storage
 int block_setup(SolverBatch& b) {
     if (b.n_slices > 0) return DTC_OK;
     std::vector<int4> sl;
@@ -2676,8 +2693,8 @@ int block_gram(SolverBatch& b, const TA* a, const TB* bb, const typename NoDeduc
         if (c) k_gram<2, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, c, gp);
         else k_gram<1, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, nullptr, gp);
     }
-    k_gram_sum<<<dim3(b.n_dom, 2 * RR / 64), 256, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
-                                                         b.gsum.as<double>());
+    k_gram_sum<<<dim3(b.n_dom, (c ? 2 : 1) * RR / 64), 64 * GS_W, 0, s>>>(b.dslice.as<int>(), done,
+                                                                        b.gpart.as<double>(), b.gsum.as<double>());
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
@@ -2690,8 +2707,8 @@ int block_orth(SolverBatch& b, const float* src, float* dst, bool partials_done 
     hipStream_t s = b.stream;
     int* done = b.done.as<int>();
     if (partials_done) {   // the direction kernel wrote src's Gram partials
-        k_gram_sum<<<dim3(b.n_dom, 2 * RR / 64), 256, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
-                                                             b.gsum.as<double>());
+        k_gram_sum<<<dim3(b.n_dom, RR / 64), 64 * GS_W, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
+                                                               b.gsum.as<double>());
     } else {
         DTC_TRY(block_gram(b, src, src, nullptr));
     }
