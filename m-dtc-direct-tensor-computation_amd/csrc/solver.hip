@@ -257,75 +257,71 @@ __global__ __launch_bounds__(NT_UPD) void k_cg_dir(const BrickInfo* __restrict__
 }
 
 // ---------------------------------------------------------------- per-domain reductions (one block per domain)
-constexpr int RED_NT = 256;
-
-// sum over the bricks of a domain of part[b][lc] for the 24 load cases:
-// strided per thread, then a fixed shuffle/LDS tree (deterministic)
-__device__ inline void dom_sum24(const double* __restrict__ part, int b0, int b1, double* s_out /* [4][24] */,
-                                 double out[R]) {
-    const int tid = threadIdx.x;
-    double acc[R];
+// sum over the bricks (clusters, slices) b0..b1-1 of a domain of part[b][lc] for the 24 load
+// cases, in a fixed order: thread row g takes b0 + g, b0 + g + 32, ..., eight loads at a
+// time (the sum takes as long as its chain of loads), and the rows are added in a tree of
+// fixed shape; thread lc < 24 receives the sum of load case lc
+constexpr int RED_G = 32, RED_NT = RED_G * R;
+__device__ inline double dom_sum24(const double* __restrict__ part, int b0, int b1, double* s_w /* [RED_G][R] */) {
+    const int tid = threadIdx.x, g = tid / R, lc = tid % R;
+    constexpr int U = 8;
+    double t = 0.0;
+    for (int b = b0 + g; b < b1; b += U * RED_G) {
+        double a[U];
 #pragma unroll
-    for (int lc = 0; lc < R; ++lc) acc[lc] = 0.0;
-    for (int b = b0 + tid; b < b1; b += RED_NT)
+        for (int u = 0; u < U; ++u) a[u] = b + u * RED_G < b1 ? part[(int64_t)(b + u * RED_G) * R + lc] : 0.0;
 #pragma unroll
-        for (int lc = 0; lc < R; ++lc) acc[lc] += part[(int64_t)b * R + lc];
-#pragma unroll
-    for (int lc = 0; lc < R; ++lc) {
-        double v = acc[lc];
-        for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-        acc[lc] = v;
+        for (int u = 0; u < U; ++u) t += a[u];
     }
-    const int wave = tid / 64, lane = tid % 64;
-    if (lane == 0)
-        for (int lc = 0; lc < R; ++lc) s_out[wave * R + lc] = acc[lc];
+    s_w[tid] = t;
     __syncthreads();
-    for (int lc = 0; lc < R; ++lc) out[lc] = ((s_out[lc] + s_out[R + lc]) + s_out[2 * R + lc]) + s_out[3 * R + lc];
+    for (int w = RED_G / 2; w > 0; w >>= 1) {
+        if (g < w) s_w[tid] += s_w[tid + w * R];
+        __syncthreads();
+    }
+    t = tid < R ? s_w[tid] : 0.0;
     __syncthreads();
+    return t;
 }
 
 __global__ __launch_bounds__(RED_NT) void k_red_init(const DomInfo* __restrict__ doms, const int* __restrict__ skip,
                                                      const double* __restrict__ prz, const double* __restrict__ prr,
                                                      const double* __restrict__ thr2, int* __restrict__ active,
                                                      double* __restrict__ rz, int* __restrict__ done) {
-    __shared__ double s_out[4 * R];
-    const int d = blockIdx.x, tid = threadIdx.x;
+    __shared__ double s_out[RED_NT];
+    const int d = blockIdx.x, tid = threadIdx.x, i = d * R + tid;
     const DomInfo D = doms[d];
-    double z[R], rr[R];
-    dom_sum24(prz, D.brick_begin, D.brick_end, s_out, z);
-    dom_sum24(prr, D.brick_begin, D.brick_end, s_out, rr);
-    if (tid == 0) {
-        int any = 0;
-        for (int lc = 0; lc < R; ++lc) {
-            int a = (skip && skip[d]) ? 0 : active[d * R + lc];
-            if (a && !(rr[lc] > thr2[d * R + lc])) a = 0;
-            active[d * R + lc] = a;
-            rz[d * R + lc] = z[lc];
-            any |= a;
-        }
-        done[d] = any ? 0 : 1;
+    const double z = dom_sum24(prz, D.brick_begin, D.brick_end, s_out);
+    const double rr = dom_sum24(prr, D.brick_begin, D.brick_end, s_out);
+    if (tid >= 64) return;
+    int a = 0;
+    if (tid < R) {
+        a = (skip && skip[d]) ? 0 : active[i];
+        if (a && !(rr > thr2[i])) a = 0;
+        active[i] = a;
+        rz[i] = z;
     }
+    const bool any = __ballot(a != 0) != 0;
+    if (tid == 0) done[d] = any ? 0 : 1;
 }
 
 __global__ __launch_bounds__(RED_NT) void k_red_alpha(const DomInfo* __restrict__ doms, const int* __restrict__ done,
                                                       const double* __restrict__ ppq, int clus,
                                                       int* __restrict__ active, const double* __restrict__ rz,
                                                       double* __restrict__ alpha) {
-    __shared__ double s_out[4 * R];
+    __shared__ double s_out[RED_NT];
     const int d = blockIdx.x, tid = threadIdx.x;
     if (done[d]) return;
     const DomInfo D = doms[d];
-    double pq[R];
-    dom_sum24(ppq, clus ? D.cl_begin : D.brick_begin, clus ? D.cl_end : D.brick_end, s_out, pq);
+    const double pq = dom_sum24(ppq, clus ? D.cl_begin : D.brick_begin, clus ? D.cl_end : D.brick_end, s_out);
     if (tid < R) {
-        const int lc = tid;
-        int a = active[d * R + lc];
+        const int i = d * R + tid;
         double al = 0.0;
-        if (a) {
-            if (pq[lc] > 0.0) al = rz[d * R + lc] / pq[lc];
-            else active[d * R + lc] = 0;      // breakdown: freeze this load case
+        if (active[i]) {
+            if (pq > 0.0) al = rz[i] / pq;
+            else active[i] = 0;      // breakdown: freeze this load case
         }
-        alpha[d * R + lc] = al;
+        alpha[i] = al;
     }
 }
 
@@ -334,30 +330,31 @@ __global__ __launch_bounds__(RED_NT) void k_red_beta(const DomInfo* __restrict__
                                                      const double* __restrict__ thr2, int* __restrict__ active,
                                                      double* __restrict__ rz, double* __restrict__ beta,
                                                      int64_t* __restrict__ iters, int64_t max_iters) {
-    __shared__ double s_out[4 * R];
+    __shared__ double s_out[RED_NT];
     const int d = blockIdx.x, tid = threadIdx.x;
     if (done[d]) return;
     const DomInfo D = doms[d];
-    double z[R], rr[R];
-    dom_sum24(prz, D.brick_begin, D.brick_end, s_out, z);
-    dom_sum24(prr, D.brick_begin, D.brick_end, s_out, rr);
-    if (tid == 0) {
-        int any = 0;
-        for (int lc = 0; lc < R; ++lc) {
-            int a = active[d * R + lc];
-            double bt = 0.0;
-            if (a) {
-                if (!(rr[lc] > thr2[d * R + lc])) a = 0;
-                else {
-                    const double old = rz[d * R + lc];
-                    bt = old != 0.0 ? z[lc] / old : 0.0;
-                }
+    const double z = dom_sum24(prz, D.brick_begin, D.brick_end, s_out);
+    const double rr = dom_sum24(prr, D.brick_begin, D.brick_end, s_out);
+    if (tid >= 64) return;
+    const int i = d * R + tid;
+    int a = 0;
+    if (tid < R) {
+        a = active[i];
+        double bt = 0.0;
+        if (a) {
+            if (!(rr > thr2[i])) a = 0;
+            else {
+                const double old = rz[i];
+                bt = old != 0.0 ? z / old : 0.0;
             }
-            active[d * R + lc] = a;
-            rz[d * R + lc] = z[lc];
-            beta[d * R + lc] = bt;
-            any |= a;
         }
+        active[i] = a;
+        rz[i] = z;
+        beta[i] = bt;
+    }
+    const bool any = __ballot(a != 0) != 0;
+    if (tid == 0) {
         const int64_t it = iters[d] + 1;
         iters[d] = it;
         if (!any || it >= max_iters) done[d] = 1;
@@ -375,24 +372,25 @@ __global__ __launch_bounds__(RED_NT) void k_red_outer(const DomInfo* __restrict_
                                                       double* __restrict__ rrcur, int* __restrict__ active64,
                                                       int* __restrict__ active, double* __restrict__ thr2,
                                                       int* __restrict__ done64, int* __restrict__ done) {
-    __shared__ double s_out[4 * R];
+    __shared__ double s_out[RED_NT];
     const int d = blockIdx.x, tid = threadIdx.x;
     const DomInfo D = doms[d];
-    double rr[R];
-    dom_sum24(prr, D.brick_begin, D.brick_end, s_out, rr);
-    if (tid == 0) {
-        int any = 0;
+    const double rr = dom_sum24(prr, D.brick_begin, D.brick_end, s_out);
+    if (tid >= 64) return;
+    const int i = d * R + tid;
+    int a = 0;
+    if (tid < R) {
         const double itol2 = itol2v ? itol2v[d] : 0.0;
-        for (int lc = 0; lc < R; ++lc) {
-            if (first) rr0[d * R + lc] = rr[lc];
-            const double r0 = rr0[d * R + lc];
-            rrcur[d * R + lc] = rr[lc];
-            const int a = (r0 > 0.0) && (rr[lc] > tol2 * r0);
-            active64[d * R + lc] = a;
-            active[d * R + lc] = a;
-            thr2[d * R + lc] = fmax(0.25 * tol2 * r0, itol2 * rr[lc]);
-            any |= a;
-        }
+        if (first) rr0[i] = rr;
+        const double r0 = rr0[i];
+        rrcur[i] = rr;
+        a = (r0 > 0.0) && (rr > tol2 * r0);
+        active64[i] = a;
+        active[i] = a;
+        thr2[i] = fmax(0.25 * tol2 * r0, itol2 * rr);
+    }
+    const bool any = __ballot(a != 0) != 0;
+    if (tid == 0) {
         done64[d] = any ? 0 : 1;
         done[d] = any ? 0 : 1;
     }
@@ -555,36 +553,36 @@ __global__ __launch_bounds__(GR_NT) void k_gram(const int4* __restrict__ slices,
     for (int e = tid; e < NGR * RR; e += GR_NT) out[e] = s_g[e];
 }
 
-// gsum[d] = sum over the domain's slices of the Gram partials, in a fixed order:
-// workgroup (d, c) sums entries 64c..64c+63; wave w takes the slices w, w + 16, ... four
-// at a time and the waves are added in order
-constexpr int GS_W = 16;
-__global__ __launch_bounds__(64 * GS_W) void k_gram_sum(const int* __restrict__ dslice, const int* __restrict__ done,
-                                                       const double* __restrict__ gpart, double* __restrict__ gsum) {
-    __shared__ double s_w[GS_W][64];
+// gsum[d] = sum over the domain's slices of the Gram partials, in a fixed order: workgroup
+// (d, c) sums entries 16c..16c+15; thread row g takes the slices g, g + 64, ..., eight loads
+// at a time, and the rows are added in a tree of fixed shape.  (A chain of loads: it takes
+// as long as its longest row; 512 slices of a 64^3 domain 12 us with 64 entries a
+// workgroup, 4.6 us so.)
+constexpr int GS_E = 16, GS_G = 64;
+__global__ __launch_bounds__(GS_E * GS_G) void k_gram_sum(const int* __restrict__ dslice, const int* __restrict__ done,
+                                                         const double* __restrict__ gpart, double* __restrict__ gsum) {
+    __shared__ double s_w[GS_G][GS_E];
     const int d = blockIdx.x;
     if (done[d]) return;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, e = (int)blockIdx.y * 64 + lane;
+    const int tid = threadIdx.x, g = tid / GS_E, e = (int)blockIdx.y * GS_E + tid % GS_E;
     const int s0 = dslice[d], s1 = dslice[d + 1];
     constexpr int U = 8;
-    double a[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) a[u] = 0.0;
-    for (int s = s0 + wave; s < s1; s += U * GS_W)
+    double t = 0.0;
+    for (int s = s0 + g; s < s1; s += U * GS_G) {
+        double a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (s + u * GS_W < s1) a[u] += gpart[(int64_t)(s + u * GS_W) * 2 * RR + e];
-    double t = a[0];
+            a[u] = s + u * GS_G < s1 ? gpart[(int64_t)(s + u * GS_G) * 2 * RR + e] : 0.0;
 #pragma unroll
-    for (int u = 1; u < U; ++u) t += a[u];
-    s_w[wave][lane] = t;
-    __syncthreads();
-    if (wave == 0) {
-        t = s_w[0][lane];
-#pragma unroll
-        for (int w = 1; w < GS_W; ++w) t += s_w[w][lane];
-        gsum[(int64_t)d * 2 * RR + e] = t;
+        for (int u = 0; u < U; ++u) t += a[u];
     }
+    s_w[g][tid % GS_E] = t;
+    __syncthreads();
+    for (int w = GS_G / 2; w > 0; w >>= 1) {
+        if (g < w) s_w[g][tid % GS_E] += s_w[g + w][tid % GS_E];
+        __syncthreads();
+    }
+    if (g == 0) gsum[(int64_t)d * 2 * RR + e] = s_w[0][tid];
 }
 
 // Per domain: takes the Gram sums of k_gram_sum, then
@@ -598,81 +596,86 @@ __global__ __launch_bounds__(64 * GS_W) void k_gram_sum(const int* __restrict__ 
 //           1e-10 dropped, L not kept) and coef = L^-T, so that P coef has
 //           orthonormal columns (zero columns for the dropped directions).
 // coef[k * 24 + j] multiplies vector column k in the update of column j.
-constexpr int BS_NT = 256;
+//
+// A chain of 24 pivots: latency is all there is.  One wave per domain, no LDS and no barrier
+// inside the chain: lane i holds row i of the matrix in registers, and the entries that
+// all lanes need are read from the row's lane into scalar registers (v_readlane); for the
+// solves lane j holds column j of the right-hand sides.  The three modes take 13, 9 and
+// 10 us; 256 threads with the matrix in LDS and three barriers a pivot took 25 each.
+__device__ inline double lane_f64(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
 
-__global__ __launch_bounds__(BS_NT) void k_bsolve(const int* __restrict__ done, const double* __restrict__ gsum,
-                                                 int mode, double* __restrict__ lfac, float* __restrict__ coef) {
-    __shared__ double s_l[RR], s_b[RR], s_d[R];
+template <int MODE>
+__global__ __launch_bounds__(64) void k_bsolve(const int* __restrict__ done, const double* __restrict__ gsum,
+                                              double* __restrict__ lfac, float* __restrict__ coef) {
     const int d = blockIdx.x, lane = threadIdx.x;
     if (done[d]) return;
+    const int row = lane < R ? lane : R - 1;      // (the lanes past 23 repeat the last row)
     double* L = lfac + (int64_t)d * RR;
-    for (int e = lane; e < RR; e += BS_NT) {
-        const double w = gsum[(int64_t)d * 2 * RR + e];
-        const double g = mode == 0 ? gsum[(int64_t)d * 2 * RR + RR + e] : 0.0;
-        if (mode == 0) {
-            s_l[e] = w;
-            s_b[e] = g;
-        } else if (mode == 1) {
-            s_b[e] = w;
-            s_l[e] = L[e];
-        } else {
-            s_l[e] = w;
-            s_b[e] = (e / R == e % R) ? 1.0 : 0.0;
-        }
-    }
-    __syncthreads();
-    if (mode != 1) {
-        const double drop = mode == 0 ? PIVOT_DROP : ORTH_DROP;
-        constexpr int NV = (RR + BS_NT - 1) / BS_NT;
-        double v[NV];
+    const double* G = gsum + (int64_t)d * 2 * RR;
+    double a[R], b[R];                            // row `row` of the matrix, column `row` of the right-hand sides
+    if (MODE == 1) {
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            const int e = lane + BS_NT * n, i = e / R, j = e % R;
-            if (e < RR) v[n] = 0.5 * (s_l[i * R + j] + s_l[j * R + i]);
-        }
-        __syncthreads();
+        for (int k = 0; k < R; ++k) a[k] = L[row * R + k];
+    } else {
 #pragma unroll
-        for (int n = 0; n < NV; ++n)
-            if (lane + BS_NT * n < RR) s_l[lane + BS_NT * n] = v[n];
-        __syncthreads();
-        if (lane < R) s_d[lane] = s_l[lane * (R + 1)];
-        __syncthreads();
-        for (int k = 0; k < R; ++k) {
-            const double dk = s_l[k * R + k];
-            const bool keep = dk > drop * s_d[k] && dk < INFINITY;
-            const double lk = keep ? sqrt(dk) : 0.0;
-            __syncthreads();
-            if (lane >= k && lane < R) s_l[lane * R + k] = keep ? (lane == k ? lk : s_l[lane * R + k] / lk) : 0.0;
-            __syncthreads();
-            for (int e = lane; e < RR; e += BS_NT) {
-                const int i = e / R, j = e % R;
-                if (j > k && i >= j) s_l[e] -= s_l[i * R + k] * s_l[j * R + k];
-            }
-            __syncthreads();
-        }
-        if (mode == 0)
-            for (int e = lane; e < RR; e += BS_NT) L[e] = s_l[e];
+        for (int k = 0; k < R; ++k) a[k] = 0.5 * (G[row * R + k] + G[k * R + row]);
     }
-    __syncthreads();
-    // L L^T y = b (modes 0, 1) or L^T y = I (mode 2) for column j of b, in place
-    // (lane j owns column j of s_b)
-    if (lane < R) {
-        const int j = lane;
-        for (int k = 0; k < R && mode != 2; ++k) {
-            double t = s_b[k * R + j];
-            for (int m = 0; m < k; ++m) t -= s_l[k * R + m] * s_b[m * R + j];
-            const double lkk = s_l[k * R + k];
-            s_b[k * R + j] = lkk > 0.0 ? t / lkk : 0.0;
-        }
-        for (int k = R - 1; k >= 0; --k) {
-            double t = s_b[k * R + j];
-            for (int m = k + 1; m < R; ++m) t -= s_l[m * R + k] * s_b[m * R + j];
-            const double lkk = s_l[k * R + k];
-            s_b[k * R + j] = lkk > 0.0 ? t / lkk : 0.0;
-        }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+        b[k] = MODE == 2 ? (k == row ? 1.0 : 0.0) : G[(MODE == 0 ? RR : 0) + k * R + row];
+    double rd = 0.0;                              // 1 / L_kk of this row, 0 for a dropped direction
+    if (MODE != 1) {
+        constexpr double DROP = MODE == 0 ? PIVOT_DROP : ORTH_DROP;
+        double diag = 0.0;                        // this row's diagonal entry before elimination
+#pragma unroll
         for (int k = 0; k < R; ++k)
-            coef[(int64_t)d * RR + k * R + j] = (float)(mode == 1 ? -s_b[k * R + j] : s_b[k * R + j]);
+            if (k == row) diag = a[k];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const double dk = lane_f64(a[k], k);
+            const bool keep = dk > DROP * lane_f64(diag, k) && dk < INFINITY;
+            const double lk = keep ? sqrt(dk) : 0.0, rk = keep ? 1.0 / lk : 0.0;
+            if (row == k) rd = rk;
+            a[k] = row == k ? lk : row > k ? a[k] * rk : 0.0;
+#pragma unroll
+            for (int m = k + 1; m < R; ++m) a[m] -= a[k] * lane_f64(a[k], m);
+        }
+        if (MODE == 0 && lane < R)
+#pragma unroll
+            for (int k = 0; k < R; ++k) L[row * R + k] = k <= row ? a[k] : 0.0;
     }
+    if (MODE == 1)
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (k == row) rd = a[k] > 0.0 ? 1.0 / a[k] : 0.0;
+    // L L^T y = b (modes 0, 1) or L^T y = I (mode 2), each lane its column.  The empty
+    // statements hold each entry's lane reads at their step: moved to the front, as the
+    // compiler would have them, the 276 values overflow the scalar registers
+    if (MODE != 2)
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            b[k] *= lane_f64(rd, k);
+            asm volatile("" : "+v"(a[k]), "+v"(b[k]));
+#pragma unroll
+            for (int m = k + 1; m < R; ++m) b[m] -= lane_f64(a[k], m) * b[k];
+        }
+#pragma unroll
+    for (int k = R - 1; k >= 0; --k) {
+        b[k] *= lane_f64(rd, k);
+#pragma unroll
+        for (int m = 0; m < k; ++m) {
+            asm volatile("" : "+v"(a[m]), "+v"(b[m]));
+            b[m] -= lane_f64(a[m], k) * b[k];
+        }
+    }
+    if (lane < R)
+#pragma unroll
+        for (int k = 0; k < R; ++k) coef[(int64_t)d * RR + k * R + row] = (float)(MODE == 1 ? -b[k] : b[k]);
 }
 
 // X += P alpha, R -= Q alpha on the rows of each node slice of a domain (the Gram
@@ -927,17 +930,18 @@ __global__ __launch_bounds__(RED_NT) void k_bcheck(const int* __restrict__ dslic
                                                   const double* __restrict__ prr, const double* __restrict__ thr2,
                                                   const double* __restrict__ rrcur, int64_t* __restrict__ iters,
                                                   int64_t max_iters) {
-    __shared__ double s_out[4 * R];
+    __shared__ double s_out[RED_NT];
     const int d = blockIdx.x, tid = threadIdx.x;
     if (done[d]) return;
-    double rr[R];
-    dom_sum24(prr, dslice[d], dslice[d + 1], s_out, rr);   // per-slice partials of k_bupdate
+    const double rr = dom_sum24(prr, dslice[d], dslice[d + 1], s_out);   // per-slice partials of k_bupdate
+    if (tid >= 64) return;
+    bool left = false;
+    if (tid < R) {
+        const double sc = col_scale(rrcur, d, tid);
+        left = !(rr <= thr2[d * R + tid] * sc * sc);
+    }
+    const bool any = __ballot(left) != 0;
     if (tid == 0) {
-        int any = 0;
-        for (int lc = 0; lc < R; ++lc) {
-            const double sc = col_scale(rrcur, d, lc);
-            any |= !(rr[lc] <= thr2[d * R + lc] * sc * sc);
-        }
         const int64_t it = iters[d] + 1;
         iters[d] = it;
         if (!any || it >= max_iters) done[d] = 1;
@@ -2693,8 +2697,8 @@ int block_gram(SolverBatch& b, const TA* a, const TB* bb, const typename NoDeduc
         if (c) k_gram<2, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, c, gp);
         else k_gram<1, TA, TB><<<b.n_slices, GR_NT, 0, s>>>(sl, done, a, bb, nullptr, gp);
     }
-    k_gram_sum<<<dim3(b.n_dom, (c ? 2 : 1) * RR / 64), 64 * GS_W, 0, s>>>(b.dslice.as<int>(), done,
-                                                                        b.gpart.as<double>(), b.gsum.as<double>());
+    k_gram_sum<<<dim3(b.n_dom, (c ? 2 : 1) * RR / GS_E), GS_E * GS_G, 0, s>>>(b.dslice.as<int>(), done,
+                                                                            b.gpart.as<double>(), b.gsum.as<double>());
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
@@ -2707,12 +2711,12 @@ int block_orth(SolverBatch& b, const float* src, float* dst, bool partials_done 
     hipStream_t s = b.stream;
     int* done = b.done.as<int>();
     if (partials_done) {   // the direction kernel wrote src's Gram partials
-        k_gram_sum<<<dim3(b.n_dom, RR / 64), 64 * GS_W, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
-                                                               b.gsum.as<double>());
+        k_gram_sum<<<dim3(b.n_dom, RR / GS_E), GS_E * GS_G, 0, s>>>(b.dslice.as<int>(), done, b.gpart.as<double>(),
+                                                                   b.gsum.as<double>());
     } else {
         DTC_TRY(block_gram(b, src, src, nullptr));
     }
-    k_bsolve<<<b.n_dom, BS_NT, 0, s>>>(done, b.gsum.as<double>(), 2, b.lfac.as<double>(), b.bcoef.as<float>());
+    k_bsolve<2><<<b.n_dom, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     k_bdir<false><<<b.n_slices, NT_UPD, 0, s>>>(b.slices.as<int4>(), done, b.bcoef.as<float>(), src, nullptr, dst,
                                                 nullptr);
     DTC_HIP(hipGetLastError());
@@ -2748,7 +2752,7 @@ int block_iteration64(SolverBatch& b, const WK<float>& wk, float* p, float* q, f
     if (b.micro20) DTC_TRY(mv20_q64(b, p, nullptr, done, q64));
     else DTC_TRY(launch_mv_q64(b, p, nullptr, done, q64));
     DTC_TRY((block_gram<float, double>(b, p, q64, r)));
-    k_bsolve<<<D, BS_NT, 0, s>>>(done, b.gsum.as<double>(), 0, b.lfac.as<double>(), b.bcoef.as<float>());
+    k_bsolve<0><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     k_bupdate64<<<NSl, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), x, r, p, q64, b.part_b.as<double>());
     k_bcheck<<<D, RED_NT, 0, s>>>(b.dslice.as<int>(), done, b.part_b.as<double>(), b.thr2.as<double>(), nullptr,
                                   b.iters.as<int64_t>(), max_iters);
@@ -2756,7 +2760,7 @@ int block_iteration64(SolverBatch& b, const WK<float>& wk, float* p, float* q, f
     DTC_HIP(hipGetLastError());
     DTC_TRY(mg_vcycle(b, wk, b.r32.as<float>(), z, nullptr));
     DTC_TRY((block_gram<double, float>(b, q64, z, nullptr)));
-    k_bsolve<<<D, BS_NT, 0, s>>>(done, b.gsum.as<double>(), 1, b.lfac.as<double>(), b.bcoef.as<float>());
+    k_bsolve<1><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     return block_dir_orth(b, p, z, q);
 }
 
@@ -2773,14 +2777,14 @@ int block_iteration(SolverBatch& b, const WK<float>& wk, float* x, float* r, flo
     else if (b.block_q64) DTC_TRY(launch_mv_q64(b, p, q, done));
     else DTC_TRY((launch_mv<float, IN_V, OUT_MASKED>(b, wk, p, q, nullptr, done)));
     DTC_TRY(block_gram(b, p, q, r));
-    k_bsolve<<<D, BS_NT, 0, s>>>(done, b.gsum.as<double>(), 0, b.lfac.as<double>(), b.bcoef.as<float>());
+    k_bsolve<0><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     k_bupdate<<<NSl, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), x, r, p, q, b.part_b.as<double>());
     k_bcheck<<<D, RED_NT, 0, s>>>(b.dslice.as<int>(), done, b.part_b.as<double>(), b.thr2.as<double>(),
                                   b.rr.as<double>(), b.iters.as<int64_t>(), max_iters);
     DTC_HIP(hipGetLastError());
     DTC_TRY(mg_vcycle(b, wk, r, z, nullptr));
     DTC_TRY(block_gram(b, q, z, nullptr));
-    k_bsolve<<<D, BS_NT, 0, s>>>(done, b.gsum.as<double>(), 1, b.lfac.as<double>(), b.bcoef.as<float>());
+    k_bsolve<1><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     return block_dir_orth(b, p, z, q);
 }
 
