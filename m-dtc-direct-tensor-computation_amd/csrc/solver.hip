@@ -1355,8 +1355,21 @@ __global__ void k_brick_assign_ex(const BrickInfo* __restrict__ bl, const int* _
     }
 }
 
-// Transfer kernels: 18 lanes per node, each lane one float4 = 4 load cases of one
-// direction of the node's [3][24] segment.
+// ---- transfers between levels
+// Every transfer is, per node of its output, a weighted sum over a few nodes of its
+// input; which ones is written once per set-up into a table row per node (T_ROW ints).
+// 18 lanes per node, each lane one float4 = 4 load cases of one direction.
+//   T_RESTRICT   b_c = P^T r_f, trilinear weights over the 3^3 fine nodes around (free ones)
+//   T_PROLONG    x_f += P x_c, the mean of 1, 2, 4 or 8 coarse nodes
+//   T_PRESTRICT  HEX20 -> HEX08: the corner node and half of its (up to 6) mid-edge ones
+//   T_PPROLONG   HEX08 -> HEX20: the corner node, or the mean of an edge's two ends
+// Rows: input nodes; -1: none, -2 (prolongations): counted in the mean, but without a
+// node.  A Dirichlet node's row is all -1.
+enum TransferKind { T_RESTRICT = 0, T_PROLONG = 1, T_PRESTRICT = 2, T_PPROLONG = 3 };
+__host__ __device__ constexpr int t_row(int kind) { return kind == T_RESTRICT ? 28 : kind == T_PPROLONG ? 2 : 8; }
+__host__ __device__ constexpr int t_terms(int kind) {
+    return kind == T_RESTRICT ? 27 : kind == T_PROLONG ? 8 : kind == T_PRESTRICT ? 7 : 2;
+}
 constexpr int T_LPN = 3 * R / 4;           // float4 per node
 constexpr int T_NPP = 256 / T_LPN;         // nodes per pass of a 256-thread workgroup
 
@@ -1364,126 +1377,115 @@ __device__ inline void f4_axpy(float4& s, float w, const float4& a) {
     s.x += w * a.x; s.y += w * a.y; s.z += w * a.z; s.w += w * a.w;
 }
 
-// s_pos[k] = position (0..NO-1) of the brick's k-th solver node (owned nodes are
-// numbered in position order), so the transfer loops visit occupied positions only
-__device__ inline int brick_positions(const BrickInfo& B, const DomInfo& D, const int* __restrict__ l2n,
-                                      unsigned char* s_pos) {
-    const int t = threadIdx.x;
-    if (t < NO) {
-        const int gx = B.x0 + t % BX, gy = B.y0 + (t / BX) % BY, gz = B.z0 + t / (BX * BY);
-        const int Lx = D.nx + 1, Ly = D.ny + 1;
-        if (gx <= D.nx && gy <= D.ny && gz <= D.nz) {
-            const int q = l2n[D.lat_off + gx + (int64_t)Lx * (gy + (int64_t)Ly * gz)];
-            if (q >= 0) s_pos[q - B.node_begin] = (unsigned char)t;
+// One workgroup per (brick of the output, blockIdx.y-th share of its nodes).  All loads of a
+// node are issued together: a missing node's lane loads node 0 and selects zero (it takes
+// no part in any product).  Memory latency bounds the small levels, HBM the large ones.
+// Sixteen 64^3 trabecular domains (1.05 M fine nodes), us per launch against lattice look-ups
+// staged in LDS per brick: restriction 221 -> 152 and 64 -> 37 (second level), prolongation
+// 240 -> 219 and 60 -> 57 (600 MB of the 700 MB it moves are x_f, read and written: 3 TB/s);
+// a 48^3 greyscale domain 22.6 -> 11 and 13.5 -> 11.6; HEX20 prolongation (27^3) 43 -> 5.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_transfer(const BrickInfo* __restrict__ bricks, const int* __restrict__ tab,
+                                                  const int* __restrict__ done, const float* __restrict__ x,
+                                                  float* __restrict__ y) {
+    constexpr int K = t_terms(KIND), ROW = t_row(KIND);
+    constexpr bool ADD = KIND == T_PROLONG || KIND == T_PPROLONG;
+    const BrickInfo B = bricks[blockIdx.x];
+    if (done && done[B.dom]) return;
+    const int tid = threadIdx.x;
+    if (tid >= T_NPP * T_LPN) return;
+    const int slot = tid / T_LPN, j = tid % T_LPN;
+    const float4* x4 = reinterpret_cast<const float4*>(x);
+    float4* y4 = reinterpret_cast<float4*>(y);
+    for (int q = B.node_begin + slot + (int)blockIdx.y * T_NPP; q < B.node_end; q += T_NPP * (int)gridDim.y) {
+        int id[ROW];
+        if constexpr (ROW % 4 == 0) {
+#pragma unroll
+            for (int k = 0; k < ROW; k += 4) {
+                const int4 v = reinterpret_cast<const int4*>(tab)[(int64_t)q * (ROW / 4) + k / 4];
+                id[k] = v.x; id[k + 1] = v.y; id[k + 2] = v.z; id[k + 3] = v.w;
+            }
+        } else {
+            const int2 v = reinterpret_cast<const int2*>(tab)[q];
+            id[0] = v.x;
+            id[1] = v.y;
         }
+        float4 old;
+        if (ADD) old = y4[(int64_t)q * T_LPN + j];
+        float4 v[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[k] = x4[(int64_t)max(id[k], 0) * T_LPN + j];
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        int cnt = 0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const bool on = id[k] >= 0;
+            const float4 a = make_float4(on ? v[k].x : 0.f, on ? v[k].y : 0.f, on ? v[k].z : 0.f, on ? v[k].w : 0.f);
+            if constexpr (KIND == T_RESTRICT) {
+                constexpr float W[3] = {0.5f, 1.f, 0.5f};
+                f4_axpy(sum, W[k % 3] * W[(k / 3) % 3] * W[k / 9], a);
+            } else {
+                f4_axpy(sum, KIND == T_PRESTRICT && k > 0 ? 0.5f : 1.f, a);
+                cnt += id[k] != -1;
+            }
+        }
+        if constexpr (ADD) {
+            if (cnt == 0) continue;   // Dirichlet
+            f4_axpy(old, cnt == 1 ? 1.f : cnt == 2 ? 0.5f : cnt == 4 ? 0.25f : 0.125f, sum);
+            sum = old;
+        }
+        y4[(int64_t)q * T_LPN + j] = sum;
     }
-    __syncthreads();
-    return B.node_end - B.node_begin;
 }
 
-// b_c = P^T r_f: trilinear weights over the free (interior) fine nodes; one
-// workgroup per (coarse brick, blockIdx.y-th share of its nodes)
-__global__ __launch_bounds__(256) void k_restrict(const BrickInfo* __restrict__ cbr, const DomInfo* __restrict__ cdom,
-                                                  const int* __restrict__ cl2n, const DomInfo* __restrict__ fdom,
-                                                  const int* __restrict__ fl2n, const float* __restrict__ rf,
-                                                  const int* __restrict__ done, float* __restrict__ bc) {
-    // fine lattice nodes of the brick's restriction stencils, staged once: positions
-    // 2 x0 - 1 .. 2 (x0 + BX - 1) + 1 (and likewise in y, z); -1 = no node
-    constexpr int FX = 2 * BX + 1, FY = 2 * BY + 1, FZ = 2 * BZ + 1;
-    __shared__ unsigned char s_pos[NO];
-    __shared__ int s_f2n[FX * FY * FZ];
+// lattice position of a brick's thread t (t < NO) and its node, -1 outside
+__device__ inline int brick_node(const BrickInfo& B, const DomInfo& D, const int* __restrict__ l2n, int t, int g[3]) {
+    g[0] = B.x0 + t % BX;
+    g[1] = B.y0 + (t / BX) % BY;
+    g[2] = B.z0 + t / (BX * BY);
+    if (g[0] > D.nx || g[1] > D.ny || g[2] > D.nz) return -1;
+    return l2n[D.lat_off + g[0] + (int64_t)(D.nx + 1) * (g[1] + (int64_t)(D.ny + 1) * g[2])];
+}
+
+// T_RESTRICT rows of the coarse nodes (one workgroup of NO threads per coarse brick)
+__global__ void k_rtab(const BrickInfo* __restrict__ cbr, const DomInfo* __restrict__ cdom, const int* __restrict__ cl2n,
+                       const DomInfo* __restrict__ fdom, const int* __restrict__ fl2n, int* __restrict__ tab) {
     const BrickInfo B = cbr[blockIdx.x];
-    if (done && done[B.dom]) return;
-    const int tid = threadIdx.x;
     const DomInfo C = cdom[B.dom], F = fdom[B.dom];
-    const int fLx = F.nx + 1, fLy = F.ny + 1;
-    const int fx0 = 2 * B.x0 - 1, fy0 = 2 * B.y0 - 1, fz0 = 2 * B.z0 - 1;
-    for (int i = tid; i < FX * FY * FZ; i += 256) {
-        const int X = fx0 + i % FX, Y = fy0 + (i / FX) % FY, Z = fz0 + i / (FX * FY);
-        s_f2n[i] = (X >= 0 && Y >= 0 && Z >= 0 && X <= F.nx && Y <= F.ny && Z <= F.nz)
-                       ? fl2n[F.lat_off + X + (int64_t)fLx * (Y + (int64_t)fLy * Z)]
-                       : -1;
-    }
-    const int n = brick_positions(B, C, cl2n, s_pos);   // (its barrier also publishes s_f2n)
-    if (tid >= T_NPP * T_LPN) return;
-    const int slot = tid / T_LPN, j = tid % T_LPN;
-    const float4* rf4 = reinterpret_cast<const float4*>(rf);
-    float4* bc4 = reinterpret_cast<float4*>(bc);
-    for (int k = slot + (int)blockIdx.y * T_NPP; k < n; k += T_NPP * (int)gridDim.y) {
-        const int o = s_pos[k], qc = B.node_begin + k;
-        const int gx = B.x0 + o % BX, gy = B.y0 + (o / BX) % BY, gz = B.z0 + o / (BX * BY);
-        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!is_bc(C, gx, gy, gz)) {
-#pragma unroll
-            for (int k = -1; k <= 1; ++k)
-#pragma unroll
-                for (int jj = -1; jj <= 1; ++jj)
-#pragma unroll
-                    for (int i = -1; i <= 1; ++i) {
-                        const int X = 2 * gx + i, Y = 2 * gy + jj, Z = 2 * gz + k;
-                        if (X > 0 && Y > 0 && Z > 0 && X < F.nx && Y < F.ny && Z < F.nz) {   // free fine node
-                            const int qf = s_f2n[(X - fx0) + FX * ((Y - fy0) + FY * (Z - fz0))];
-                            if (qf >= 0) {
-                                constexpr float W[3] = {0.5f, 1.f, 0.5f};
-                                const float w = W[i + 1] * W[jj + 1] * W[k + 1];
-                                f4_axpy(sum, w, rf4[(int64_t)qf * T_LPN + j]);
-                            }
-                        }
-                    }
-        }
-        bc4[(int64_t)qc * T_LPN + j] = sum;
+    int g[3];
+    const int q = brick_node(B, C, cl2n, threadIdx.x, g);
+    if (q < 0) return;
+    int* row = tab + (int64_t)q * t_row(T_RESTRICT);
+    const bool bc = is_bc(C, g[0], g[1], g[2]);
+    for (int k = 0; k < t_row(T_RESTRICT); ++k) {
+        const int X = 2 * g[0] + k % 3 - 1, Y = 2 * g[1] + (k / 3) % 3 - 1, Z = 2 * g[2] + k / 9 - 1;
+        int f = -1;
+        if (!bc && k < 27 && X > 0 && Y > 0 && Z > 0 && X < F.nx && Y < F.ny && Z < F.nz)   // free fine node
+            f = fl2n[F.lat_off + X + (int64_t)(F.nx + 1) * (Y + (int64_t)(F.ny + 1) * Z)];
+        row[k] = f;
     }
 }
 
-// x_f += P x_c on the free nodes of each fine brick (trilinear interpolation);
-// blockIdx.y selects a share of the brick's nodes
-__global__ __launch_bounds__(256) void k_prolong(const BrickInfo* __restrict__ fbr, const DomInfo* __restrict__ fdom,
-                                                 const int* __restrict__ fl2n, const DomInfo* __restrict__ cdom,
-                                                 const int* __restrict__ cl2n, const float* __restrict__ xc,
-                                                 const int* __restrict__ done, float* __restrict__ xf) {
-    // coarse lattice nodes the brick's fine nodes interpolate from, staged once:
-    // positions x0 / 2 .. (x0 + BX - 1) / 2 + 1 (and likewise in y, z); -1 = no node
-    constexpr int CXM = BX / 2 + 2, CYM = BY / 2 + 2, CZM = BZ / 2 + 2;   // room for odd origins
-    __shared__ unsigned char s_pos[NO];
-    __shared__ int s_c2n[CXM * CYM * CZM];
+// T_PROLONG rows of the fine nodes (one workgroup of NO threads per fine brick)
+__global__ void k_ptab(const BrickInfo* __restrict__ fbr, const DomInfo* __restrict__ fdom, const int* __restrict__ fl2n,
+                       const DomInfo* __restrict__ cdom, const int* __restrict__ cl2n, int* __restrict__ tab) {
     const BrickInfo B = fbr[blockIdx.x];
-    if (done && done[B.dom]) return;
-    const int tid = threadIdx.x;
     const DomInfo F = fdom[B.dom], C = cdom[B.dom];
-    const int cLx = C.nx + 1, cLy = C.ny + 1;
-    const int cx0 = B.x0 >> 1, cy0 = B.y0 >> 1, cz0 = B.z0 >> 1;
-    for (int i = tid; i < CXM * CYM * CZM; i += 256) {
-        const int X = cx0 + i % CXM, Y = cy0 + (i / CXM) % CYM, Z = cz0 + i / (CXM * CYM);
-        s_c2n[i] = (X <= C.nx && Y <= C.ny && Z <= C.nz)
-                       ? cl2n[C.lat_off + X + (int64_t)cLx * (Y + (int64_t)cLy * Z)]
-                       : -1;
-    }
-    const int n = brick_positions(B, F, fl2n, s_pos);   // (its barrier also publishes s_c2n)
-    if (tid >= T_NPP * T_LPN) return;
-    const int slot = tid / T_LPN, j = tid % T_LPN;
-    const float4* xc4 = reinterpret_cast<const float4*>(xc);
-    float4* xf4 = reinterpret_cast<float4*>(xf);
-    for (int k = slot + (int)blockIdx.y * T_NPP; k < n; k += T_NPP * (int)gridDim.y) {
-        const int o = s_pos[k], qf = B.node_begin + k;
-        const int gx = B.x0 + o % BX, gy = B.y0 + (o / BX) % BY, gz = B.z0 + o / (BX * BY);
-        if (!(gx > 0 && gy > 0 && gz > 0 && gx < F.nx && gy < F.ny && gz < F.nz)) continue;   // free nodes only
-        const int X0 = gx >> 1, Y0 = gy >> 1, Z0 = gz >> 1;
-        const int ox = gx & 1, oy = gy & 1, oz = gz & 1;
-        const float w = (ox ? 0.5f : 1.f) * (oy ? 0.5f : 1.f) * (oz ? 0.5f : 1.f);
-        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    if ((i && !ox) || (jj && !oy) || (k && !oz)) continue;
-                    const int qc = s_c2n[(X0 + i - cx0) + CXM * ((Y0 + jj - cy0) + CYM * (Z0 + k - cz0))];
-                    if (qc >= 0) f4_axpy(sum, 1.f, xc4[(int64_t)qc * T_LPN + j]);
-                }
-        float4 v = xf4[(int64_t)qf * T_LPN + j];
-        f4_axpy(v, w, sum);
-        xf4[(int64_t)qf * T_LPN + j] = v;
+    int g[3];
+    const int q = brick_node(B, F, fl2n, threadIdx.x, g);
+    if (q < 0) return;
+    int* row = tab + (int64_t)q * t_row(T_PROLONG);
+    const bool bc = is_bc(F, g[0], g[1], g[2]);
+    for (int k = 0; k < 8; ++k) {
+        const int i = k & 1, j = (k >> 1) & 1, l = k >> 2;
+        int c = -1;
+        if (!bc && !(i && !(g[0] & 1)) && !(j && !(g[1] & 1)) && !(l && !(g[2] & 1))) {
+            const int X = (g[0] >> 1) + i, Y = (g[1] >> 1) + j, Z = (g[2] >> 1) + l;
+            if (X <= C.nx && Y <= C.ny && Z <= C.nz)
+                c = cl2n[C.lat_off + X + (int64_t)(C.nx + 1) * (Y + (int64_t)(C.ny + 1) * Z)];
+            if (c < 0) c = -2;
+        }
+        row[k] = c;
     }
 }
 
@@ -1537,98 +1539,58 @@ __global__ __launch_bounds__(NT_UPD) void k_cheb(const BrickInfo* __restrict__ b
 // element: identity at corners, the mean of the edge's two ends at a mid-edge
 // node.  Restriction is P^T in gather form, in a fixed order per coarse node.
 
-// r08 = P^T res for one domain group: coarse lattice node (i, j, k) takes the fine
-// node at (2i, 2j, 2k) and half of each mid-edge node at (2i +- 1, 2j, 2k),
-// (2i, 2j +- 1, 2k), (2i, 2j, 2k +- 1); 0 on box-face (Dirichlet) nodes.
-__global__ __launch_bounds__(256) void k_pmg_restrict(Dom20Dev G, DomInfo D08, const int* __restrict__ lat2node08,
-                                                     const int* __restrict__ done, int dom,
-                                                     const float* __restrict__ res, float* __restrict__ r08) {
-    if (done && done[dom]) return;
+// T_PRESTRICT rows of the HEX08 twin's nodes of one domain group (one thread per lattice
+// point): its corner node and the mid-edge nodes around it on the half-voxel lattice
+__global__ void k_pmg_rtab(Dom20Dev G, DomInfo D08, const int* __restrict__ lat2node08, int* __restrict__ tab) {
     const int Lx = D08.nx + 1, Ly = D08.ny + 1, Lz = D08.nz + 1;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)Lx * Ly * Lz * R) return;
-    const int lc = (int)(i % R);
-    const int64_t p = i / R;
-    const int cx = (int)(p % Lx), cy = (int)((p / Lx) % Ly), cz = (int)(p / ((int64_t)Lx * Ly));
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= (int64_t)Lx * Ly * Lz) return;
     const int c = lat2node08[D08.lat_off + p];
     if (c < 0) return;
-    const int fx = 2 * cx, fy = 2 * cy, fz = 2 * cz;
+    const int f[3] = {2 * (int)(p % Lx), 2 * (int)((p / Lx) % Ly), 2 * (int)(p / ((int64_t)Lx * Ly))};
     auto fine = [&](int x, int y, int z) -> int {
         if (x < 0 || y < 0 || z < 0 || x >= G.Lx || y >= G.Ly || z >= G.Lz) return -1;
-        return G.lat20[x + (int64_t)G.Lx * (y + (int64_t)G.Ly * z)];
+        const int q = G.lat20[x + (int64_t)G.Lx * (y + (int64_t)G.Ly * z)];
+        return q < 0 ? -1 : (int)(G.node_begin + q);
     };
-    const int q0 = fine(fx, fy, fz);
-    const bool bc = q0 >= 0 && G.bcf[q0];
-    const int nb6[6] = {fine(fx - 1, fy, fz), fine(fx + 1, fy, fz), fine(fx, fy - 1, fz),
-                        fine(fx, fy + 1, fz), fine(fx, fy, fz - 1), fine(fx, fy, fz + 1)};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        float v = 0.f;
-        if (!bc) {
-            if (q0 >= 0) v = res[((G.node_begin + q0) * 3 + d) * R + lc];
-#pragma unroll
-            for (int k = 0; k < 6; ++k)
-                if (nb6[k] >= 0) v += 0.5f * res[((G.node_begin + nb6[k]) * 3 + d) * R + lc];
-        }
-        r08[((int64_t)c * 3 + d) * R + lc] = v;
+    int* row = tab + (int64_t)c * t_row(T_PRESTRICT);
+    const int q0 = fine(f[0], f[1], f[2]);
+    const bool bc = q0 >= 0 && G.bcf[q0 - G.node_begin];
+    row[0] = bc ? -1 : q0;
+    for (int k = 0; k < 6; ++k) {
+        const int dx = k == 0 ? -1 : k == 1 ? 1 : 0, dy = k == 2 ? -1 : k == 3 ? 1 : 0, dz = k == 4 ? -1 : k == 5 ? 1 : 0;
+        row[1 + k] = bc ? -1 : fine(f[0] + dx, f[1] + dy, f[2] + dz);
     }
+    row[7] = -1;
 }
 
-// z += P z08 on the free HEX20 nodes of the pseudo-bricks
-__global__ __launch_bounds__(NT_UPD) void k_pmg_prolong(const BrickInfo* __restrict__ bricks,
-                                                       const DomInfo* __restrict__ doms,
-                                                       const Dom20Dev* __restrict__ d20,
-                                                       const DomInfo* __restrict__ doms08,
-                                                       const int* __restrict__ lat2node08,
-                                                       const int* __restrict__ done, const float* __restrict__ z08,
-                                                       float* __restrict__ z) {
+// T_PPROLONG rows of the HEX20 nodes: the HEX08 node at a corner, an edge's two ends
+__global__ void k_pmg_ptab(const BrickInfo* __restrict__ bricks, const DomInfo* __restrict__ doms,
+                           const Dom20Dev* __restrict__ d20, const DomInfo* __restrict__ doms08,
+                           const int* __restrict__ lat2node08, int* __restrict__ tab) {
     const BrickInfo B = bricks[blockIdx.x];
-    if (done && done[B.dom]) return;
-    const DomInfo D = doms[B.dom];
-    const DomInfo C = doms08[B.dom];
+    const DomInfo D = doms[B.dom], C = doms08[B.dom];
     const Dom20Dev G = d20[B.dom];
     const int Lx = C.nx + 1, Ly = C.ny + 1;
-    for (int i = threadIdx.x; i < (B.node_end - B.node_begin) * R; i += NT_UPD) {
-        const int64_t q = B.node_begin + i / R;
-        const int lc = i % R;
+    for (int q = B.node_begin + (int)threadIdx.x; q < B.node_end; q += blockDim.x) {
         const int ql = (int)(q - G.node_begin);
-        if (G.bcf[ql]) continue;
-        int l[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) l[k] = (int)lrint(2.0 * (G.coords[3 * ql + k] / D.delta[k] - D.xa1[k]));
-        int odd = -1;
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (l[k] & 1) odd = k;
-        int lo[3] = {l[0] >> 1, l[1] >> 1, l[2] >> 1};
-        const int c0 = lat2node08[C.lat_off + lo[0] + (int64_t)Lx * (lo[1] + (int64_t)Ly * lo[2])];
-        int c1 = -1;
-        if (odd >= 0) {
-            lo[odd] += 1;
-            c1 = lat2node08[C.lat_off + lo[0] + (int64_t)Lx * (lo[1] + (int64_t)Ly * lo[2])];
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            float v = 0.f;
-            if (odd < 0) {
-                if (c0 >= 0) v = z08[((int64_t)c0 * 3 + d) * R + lc];
-            } else {
-                if (c0 >= 0) v += 0.5f * z08[((int64_t)c0 * 3 + d) * R + lc];
-                if (c1 >= 0) v += 0.5f * z08[((int64_t)c1 * 3 + d) * R + lc];
+        int c[2] = {-1, -1};
+        if (!G.bcf[ql]) {
+            int lo[3], odd = -1;
+            for (int k = 0; k < 3; ++k) {
+                const int l = (int)lrint(2.0 * (G.coords[3 * ql + k] / D.delta[k] - D.xa1[k]));
+                if (l & 1) odd = k;
+                lo[k] = l >> 1;
             }
-            z[(q * 3 + d) * R + lc] += v;
+            for (int k = 0; k < (odd >= 0 ? 2 : 1); ++k) {
+                if (k) lo[odd] += 1;
+                c[k] = lat2node08[C.lat_off + lo[0] + (int64_t)Lx * (lo[1] + (int64_t)Ly * lo[2])];
+                if (c[k] < 0) c[k] = -2;
+            }
         }
+        tab[2 * (int64_t)q] = c[0];
+        tab[2 * (int64_t)q + 1] = c[1];
     }
-}
-
-// res = b - t on the rows of the pseudo-bricks (t = K x, masked on Dirichlet rows)
-__global__ __launch_bounds__(NT_UPD) void k_sub(const BrickInfo* __restrict__ bricks, const int* __restrict__ done,
-                                               const float* __restrict__ b, const float* __restrict__ t,
-                                               float* __restrict__ res) {
-    const BrickInfo B = bricks[blockIdx.x];
-    if (done && done[B.dom]) return;
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = threadIdx.x; i < cnt; i += NT_UPD) res[base + i] = b[base + i] - t[base + i];
 }
 
 // per-brick sums of a . b per load case
@@ -2203,6 +2165,19 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
                                             C.emod.as<double>(), b.kdiag, C.dinv64.as<double>(), C.dinv32.as<float>());
             DTC_HIP(hipGetLastError());
             DTC_TRY(build_clusters(s, C.cl, C.brick, C.dom, C.lat2node, C.emod, false));
+            // transfer tables between this level and the finer one
+            const int fbn = l == 0 ? b.n_bricks : b.mg[l - 1].n_bricks;
+            const int64_t fnn = l == 0 ? b.n_nodes : b.mg[l - 1].n_nodes;
+            const DevMem &fbr = l == 0 ? b.brick : b.mg[l - 1].brick, &fdm = l == 0 ? b.dom : b.mg[l - 1].dom,
+                         &fln = l == 0 ? b.lat2node : b.mg[l - 1].lat2node;
+            DTC_TRY(C.rtab.ensure(nn * t_row(T_RESTRICT) * 4));
+            DTC_TRY(C.ptab.ensure((size_t)std::max<int64_t>(fnn, 1) * t_row(T_PROLONG) * 4));
+            k_rtab<<<C.n_bricks, NO, 0, s>>>(C.brick.as<BrickInfo>(), C.dom.as<DomInfo>(), C.lat2node.as<int>(),
+                                             fdm.as<DomInfo>(), fln.as<int>(), C.rtab.as<int>());
+            if (fbn > 0)
+                k_ptab<<<fbn, NO, 0, s>>>(fbr.as<BrickInfo>(), fdm.as<DomInfo>(), fln.as<int>(), C.dom.as<DomInfo>(),
+                                          C.lat2node.as<int>(), C.ptab.as<int>());
+            DTC_HIP(hipGetLastError());
         }
         DTC_HIP(hipStreamSynchronize(s));   // ex, cnt go out of scope
     }
@@ -2298,8 +2273,7 @@ int ebe_launch(const Clusters& c, hipStream_t s, EbeArgs a, const WK<T>& wk, con
     return DTC_OK;
 }
 
-// HEX08: x of the IN_U modes holds the Dirichlet values itself (k_set_bc), so they gather
-// it like any vector; HEX20 adds them on the fly (null x: zero)
+// x of the IN_U modes holds the Dirichlet values itself (set_bc in batch_solve)
 template <typename T, int IN, int OUT>
 int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* part, const int* done) {
     if (b.n_bricks == 0) return DTC_OK;
@@ -2310,7 +2284,7 @@ int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* pa
     int slot = -1;
     if (kind >= 0) DTC_TRY(timed_begin(b, kind, &slot));
     if (b.micro20) {
-        DTC_TRY(mv20(b, sizeof(T) == 8, IN, OUT, xin, yout, part, done));
+        DTC_TRY(mv20(b, sizeof(T) == 8, OUT, xin, yout, part, done));
     } else {
         EbeArgs a{};
         a.done = done;
@@ -2318,8 +2292,7 @@ int launch_mv(SolverBatch& b, const WK<T>& wk, const T* xin, T* yout, double* pa
         a.partial = part;
         DTC_TRY((ebe_launch<T, T, T, IN_V, OUT>(b.cl, b.stream, a, wk, xin, yout)));
     }
-    // IN_U without x (x = 0) reads no vector
-    DTC_TRY(timed_end(b, slot, (IN == IN_U && !xin) ? 1 : 2, sizeof(T) == 8, false, done));
+    DTC_TRY(timed_end(b, slot, 2, sizeof(T) == 8, false, done));
     return DTC_OK;
 }
 
@@ -2328,7 +2301,6 @@ struct MvTopo {
     const Clusters* cl;
     int n_bricks;
     const BrickInfo* bricks;
-    const DomInfo* doms;
 };
 
 // tb: the batch whose fine level this is (its launches are timed), else null
@@ -2373,7 +2345,6 @@ int launch_mv32(const MvTopo& T, hipStream_t s, const WK<float>& wk, const float
 // side is the PCG residual); the iterate alternates between buf[0] and buf[1]
 struct LvView {
     MvTopo T;
-    const int* l2n;
     const float* dinv;
     float* b;
     float* buf[2];
@@ -2414,8 +2385,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     auto view = [&](int l) {
         LvView v;
         if (l == 0) {
-            v.T = {&b.cl, b.n_bricks, b.brick.as<BrickInfo>(), b.dom.as<DomInfo>()};
-            v.l2n = b.lat2node.as<int>();
+            v.T = {&b.cl, b.n_bricks, b.brick.as<BrickInfo>()};
             v.dinv = b.dinv32.as<float>();
             v.b = const_cast<float*>(r);
             v.buf[0] = z;
@@ -2423,8 +2393,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
             v.d = b.d32.as<float>();
         } else {
             Level& C = b.mg[l - 1];
-            v.T = {&C.cl, C.n_bricks, C.brick.as<BrickInfo>(), C.dom.as<DomInfo>()};
-            v.l2n = C.lat2node.as<int>();
+            v.T = {&C.cl, C.n_bricks, C.brick.as<BrickInfo>()};
             v.dinv = C.dinv32.as<float>();
             v.b = C.b.as<float>();
             v.buf[0] = C.x.as<float>();
@@ -2480,15 +2449,16 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
         float* res = f.buf[1 - cur[l]];
         DTC_TRY(launch_mv32<OUT_BRES>(f.T, s, wk, f.buf[cur[l]], res, done, f.b, f.dinv, nullptr, 0.f, 0.f, 0,
                                       l == 0 ? &b : nullptr, 0.f));
-        k_restrict<<<dim3(c.T.n_bricks, node_split(c.T.n_bricks)), 256, 0, s>>>(c.T.bricks, c.T.doms, c.l2n, f.T.doms, f.l2n, res, done, c.b);
+        k_transfer<T_RESTRICT><<<dim3(c.T.n_bricks, node_split(c.T.n_bricks)), 256, 0, s>>>(
+            c.T.bricks, b.mg[l].rtab.as<int>(), done, res, c.b);
         DTC_HIP(hipGetLastError());
     }
     DTC_TRY(smooth(L, P.coarse_degree, true, P.coarse_ratio));
     for (int l = L - 1; l >= 0; --l) {
         const LvView f = view(l), c = view(l + 1);
         if (f.T.n_bricks > 0 && c.T.n_bricks > 0) {
-            k_prolong<<<dim3(f.T.n_bricks, node_split(f.T.n_bricks)), 256, 0, s>>>(f.T.bricks, f.T.doms, f.l2n, c.T.doms, c.l2n, c.buf[cur[l + 1]], done,
-                                                   f.buf[cur[l]]);
+            k_transfer<T_PROLONG><<<dim3(f.T.n_bricks, node_split(f.T.n_bricks)), 256, 0, s>>>(
+                f.T.bricks, b.mg[l].ptab.as<int>(), done, c.buf[cur[l + 1]], f.buf[cur[l]]);
             DTC_HIP(hipGetLastError());
         }
         DTC_TRY(smooth(l, deg, false, P.ratio));
@@ -2530,11 +2500,11 @@ int pmg_vcycle(SolverBatch& b, const float* r, float* z, double* prz) {
             double* dk = k == deg - 1 ? dot : nullptr;
             if (zero && k == 0) {
                 k_cheb<<<b.n_bricks, NT_UPD, 0, s>>>(bl, done, r, nullptr, b.dinv32.as<float>(), d, z, c1, c2, 1, dk);
-            } else if (!dk && cheb_fuse() && !hex20_gather_form()) {
+            } else if (!dk && cheb_fuse()) {
                 // the step in the epilogue of the operator's node gather (no t vector)
                 DTC_TRY(mv20_cheb(b, z, done, r, b.dinv32.as<float>(), d, c1, c2));
             } else {
-                DTC_TRY(mv20(b, false, IN_V, OUT_MASKED, z, t, nullptr, done));
+                DTC_TRY(mv20(b, false, OUT_MASKED, z, t, nullptr, done));
                 k_cheb<<<b.n_bricks, NT_UPD, 0, s>>>(bl, done, r, t, b.dinv32.as<float>(), d, z, c1, c2, 0, dk);
             }
             DTC_HIP(hipGetLastError());
@@ -2542,23 +2512,18 @@ int pmg_vcycle(SolverBatch& b, const float* r, float* z, double* prz) {
         return DTC_OK;
     };
     DTC_TRY(smooth(true, nullptr));
-    // residual, restricted to the HEX08 nodes of each domain group
-    DTC_TRY(mv20(b, false, IN_V, OUT_MASKED, z, t, nullptr, done));
-    k_sub<<<b.n_bricks, NT_UPD, 0, s>>>(bl, done, r, t, t);
-    DTC_HIP(hipGetLastError());
+    // residual, restricted to the HEX08 nodes
+    DTC_TRY(mv20_bres(b, z, t, done, r));
     float* r08 = c.r32.as<float>();
     float* z08 = c.z32.as<float>();
-    for (int g = 0; g < b.n_dom && g < c.n_dom; ++g) {
-        const DomInfo& D08 = c.h_dom[g];
-        if (b.h_status[g] != DTC_OK || c.h_status[g] != DTC_OK) continue;
-        const int64_t n = (int64_t)(D08.nx + 1) * (D08.ny + 1) * (D08.nz + 1) * R;
-        k_pmg_restrict<<<nb(n, 256), 256, 0, s>>>(b.h_d20dev[g], D08, c.lat2node.as<int>(), done, g, t, r08);
-    }
+    if (c.n_bricks > 0)
+        k_transfer<T_PRESTRICT><<<dim3(c.n_bricks, node_split(c.n_bricks)), 256, 0, s>>>(
+            c.brick.as<BrickInfo>(), b.pmg_rtab.as<int>(), done, t, r08);
     DTC_HIP(hipGetLastError());
     c.done_ext = done;
     DTC_TRY(mg_vcycle(c, cast_wk<float>(c.wk64), r08, z08, nullptr));
-    k_pmg_prolong<<<b.n_bricks, NT_UPD, 0, s>>>(bl, b.dom.as<DomInfo>(), b.d20dev.as<Dom20Dev>(), c.dom.as<DomInfo>(),
-                                                c.lat2node.as<int>(), done, z08, z);
+    k_transfer<T_PPROLONG><<<dim3(b.n_bricks, node_split(b.n_bricks)), 256, 0, s>>>(bl, b.pmg_ptab.as<int>(), done,
+                                                                                    z08, z);
     DTC_HIP(hipGetLastError());
     return smooth(false, prz);
 }
@@ -2584,6 +2549,21 @@ int build_pmg(SolverBatch& b, SolverBatch& c) {
     DTC_TRY(b.z32.ensure(v0));
     DTC_TRY(b.t32.ensure(v0));
     DTC_TRY(b.d32.ensure(v0));
+    DTC_TRY(b.pmg_rtab.ensure((size_t)std::max<int64_t>(c.n_nodes, 1) * t_row(T_PRESTRICT) * 4));
+    DTC_TRY(b.pmg_ptab.ensure((size_t)std::max<int64_t>(b.n_nodes, 1) * t_row(T_PPROLONG) * 4));
+    // rows without a HEX20 domain of their own stay empty
+    if (c.n_nodes > 0)
+        k_fill_i32b<<<nb(c.n_nodes * t_row(T_PRESTRICT), 256), 256, 0, b.stream>>>(b.pmg_rtab.as<int>(), c.n_nodes * t_row(T_PRESTRICT), -1);
+    for (int g = 0; g < b.n_dom && g < c.n_dom; ++g) {
+        const DomInfo& D08 = c.h_dom[g];
+        if (b.h_status[g] != DTC_OK || c.h_status[g] != DTC_OK) continue;
+        const int64_t n = (int64_t)(D08.nx + 1) * (D08.ny + 1) * (D08.nz + 1);
+        k_pmg_rtab<<<nb(n, 256), 256, 0, b.stream>>>(b.h_d20dev[g], D08, c.lat2node.as<int>(), b.pmg_rtab.as<int>());
+    }
+    if (b.n_bricks > 0)
+        k_pmg_ptab<<<b.n_bricks, 64, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(), b.d20dev.as<Dom20Dev>(),
+                                                    c.dom.as<DomInfo>(), c.lat2node.as<int>(), b.pmg_ptab.as<int>());
+    DTC_HIP(hipGetLastError());
     b.p08 = &c;
     return DTC_OK;
 }
@@ -2902,8 +2882,7 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
     return DTC_OK;
 }
 
-// FP64 true residual r64 = -(K u)_free, u = x64 + x_bc (x64 == null: u = x_bc; HEX08: x64
-// holds the Dirichlet values),
+// FP64 true residual r64 = -(K u)_free, u = x64, which holds the Dirichlet values,
 // then per load case activity and targets (k_red_outer)
 int residual64(SolverBatch& b, const WK<double>& wk, const double* x64, int first, const dtc_solve_opts& o) {
     double* r64 = b.r64.as<double>();
@@ -3078,13 +3057,12 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         b.block64 = block && (e64 ? e64[0] == '1' : cmax > 100.0);
         if (b.block64) DTC_TRY(b.q64.ensure((size_t)nv * 8));
     }
-    // r64 = f (lifted right-hand side).  HEX08: the Dirichlet values are written into x64
-    // once; every update of x64 adds zero there, and its other readers form them again
-    if (!b.micro20) {
-        k_set_bc<<<dim3(b.n_bricks, 8), NT_UPD, 0, s>>>(bl, dl, b.lat2node.as<int>(), b.x64.as<double>());
-        DTC_HIP(hipGetLastError());
-    }
-    DTC_TRY(residual64(b, wk64, b.micro20 ? nullptr : b.x64.as<double>(), 1, o));
+    // r64 = f (lifted right-hand side).  The Dirichlet values are written into x64 once;
+    // every update of x64 adds zero there, and its other readers form them again
+    if (b.micro20) DTC_TRY(set_bc20(b, b.x64.as<double>()));
+    else k_set_bc<<<dim3(b.n_bricks, 8), NT_UPD, 0, s>>>(bl, dl, b.lat2node.as<int>(), b.x64.as<double>());
+    DTC_HIP(hipGetLastError());
+    DTC_TRY(residual64(b, wk64, b.x64.as<double>(), 1, o));
 
     if (b.precision == DTC_FP64) {
         // PCG in FP64 on (x64, r64); a true-residual check restarts it if the

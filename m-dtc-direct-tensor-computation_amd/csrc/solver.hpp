@@ -30,6 +30,7 @@ struct Level {
     std::vector<BrickInfo> h_brick;
     DevMem dom, brick, lat2node, emod, dinv64, dinv32;
     Clusters cl;
+    DevMem rtab, ptab;             // transfer tables: restriction to this level, prolongation from it
     DevMem b, x, t, d;             // right-hand side, iterate, matvec output, Chebyshev direction
 };
 
@@ -143,6 +144,7 @@ struct SolverBatch {
     // the coarse space; the fine level is smoothed with Chebyshev-Jacobi on the
     // interval [cheb_lmax / ratio, cheb_lmax] of D^-1 K (HEX20 element bound)
     SolverBatch* p08 = nullptr;
+    DevMem pmg_rtab, pmg_ptab;     // its transfer tables
     const int* done_ext = nullptr;  // done flags to use instead of `done` (the coarse batch of a p-multigrid)
     std::vector<Dom20> d20;        // per domain group (empty entries for failed groups)
     DevMem d20dev;                 // Dom20Dev[]
@@ -208,12 +210,6 @@ int batch_build_mg(SolverBatch& b, int max_levels);
 // p-multigrid of a HEX20 micro batch b over c, the HEX08 discretisation of the same
 // voxels and domain groups (both finalised): builds c's levels and links c to b.
 int batch_build_pmg(SolverBatch& b, SolverBatch& c);
-// DTC_HEX20_GATHER=1: the HEX20 operator as the node-gather kernel (the reference form;
-// no Chebyshev epilogue), else element pass + node sums
-inline bool hex20_gather_form() {
-    const char* e = std::getenv("DTC_HEX20_GATHER");
-    return e && e[0] == '1';
-}
 // HEX20 FP32 operator with one Chebyshev-Jacobi step in its epilogue: on free rows
 // d = c1 d + c2 dinv (bv - K x), x += d (x updated in place; Dirichlet rows: K x = 0)
 int mv20_cheb(SolverBatch& b, float* x, const int* done, const float* bv, const float* dinv, float* d, float c1,
@@ -232,7 +228,11 @@ int batch_fields(SolverBatch& b, int i, int ncol, double* u_out, double* r_out);
 int batch_add_domain20(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d, const double* modulus_dev,
                        double escale, int lc_base, hipStream_t s);
 int finalize20(SolverBatch& b);
-int mv20(SolverBatch& b, bool fp64, int in, int out, const void* xin, void* yout, double* part, const int* done);
+int mv20(SolverBatch& b, bool fp64, int out, const void* xin, void* yout, double* part, const int* done);
+// y = bv - K x on free rows, 0 on Dirichlet rows (FP32)
+int mv20_bres(SolverBatch& b, const float* x, float* y, const int* done, const float* bv);
+// Dirichlet values into x
+int set_bc20(SolverBatch& b, double* x);
 // Q = K P of the block PCG on a HEX20 batch: FP32 directions, FP64 arithmetic
 // (masked rows); Q is written to q (FP32), or to q64 (FP64) when that is set
 int mv20_q64(SolverBatch& b, const float* p, float* q, const int* done, double* q64 = nullptr);

@@ -5,12 +5,11 @@
 // reductions and FP64 refinement as the HEX08 voxel lattice; only the operator
 // and the node-indexed auxiliaries differ:
 //  * solver nodes are the mesh nodes in mesh order (node_begin + mesh id - 1);
-//    consecutive runs of 128 nodes form the pseudo-bricks that the vector
+//    consecutive runs of 32 nodes form the pseudo-bricks that the vector
 //    kernels and the per-brick partial sums work on;
-//  * y = K x is a gather per node: for every (element, local node a) that
-//    touches the node, the three rows 3a..3a+2 of the 60x60 element stiffness
-//    (E = 1, in LDS) times the element's 60 gathered values, scaled by the
-//    element modulus.  Adjacency lists are sorted, so sums are deterministic;
+//  * y = K x in two passes, the element forces as small products with the 60x60
+//    element stiffness on the matrix cores (FP32 or FP64), then their sum per node
+//    over its sorted list of elements (deterministic);
 //  * Dirichlet nodes are the mesh nodes on the domain box faces
 //    (f-src/mod_struct_preprocess.f90:564-592), Jacobi uses diag(K) per DOF.
 #include <algorithm>
@@ -25,7 +24,7 @@ namespace {
 
 constexpr int R = R24;
 constexpr int NT20 = 192;        // 8 nodes x 24 load cases per pass
-constexpr int PB = 128;          // nodes per pseudo-brick
+constexpr int PB = 32;           // nodes per pseudo-brick (128 left a 27^3 domain with 270 workgroups)
 constexpr int FFD = 60;          // macro DOF slots of the force partials
 
 // element -> voxel modulus (kept elements only)
@@ -117,82 +116,19 @@ __device__ inline double bc20(const DomInfo& D, const Dom20Dev& G, int ql, int d
     return bc_value_m(D.macro_order, N, d, D.lc_base + lc);
 }
 
-struct Mv20 {
-    const BrickInfo* bricks;
-    const DomInfo* doms;
-    const Dom20Dev* d20;
-    const int* done;
-    double* partial;
-};
-
-// y = K x on the pseudo-bricks; modes as the HEX08 kernel (IN_V / IN_U input,
-// MASKED_DOT / RESID / PLAIN / MASKED output)
-// VT: the vectors' type (T, or float with T = double: FP32 vectors, FP64 arithmetic)
-template <typename T, int IN, int OUT, typename VT = T>
-__global__ __launch_bounds__(NT20) void k_matvec20(Mv20 A, const T* __restrict__ Kg, const VT* __restrict__ xin,
-                                                   VT* __restrict__ yout) {
-    __shared__ T sK[3600];
-    __shared__ double s_red[NT20];
-    const BrickInfo B = A.bricks[blockIdx.x];
-    if (A.done && A.done[B.dom]) return;
-    for (int i = threadIdx.x; i < 3600; i += NT20) sK[i] = Kg[i];
-    __syncthreads();
-    const DomInfo D = A.doms[B.dom];
-    const Dom20Dev G = A.d20[B.dom];
-    const int tid = threadIdx.x, r = tid % R, g = tid / R;
-    double acc = 0.0;
-    for (int q = B.node_begin + g; q < B.node_end; q += NT20 / R) {
+// x = Dirichlet values on the box-face nodes, unchanged elsewhere
+__global__ __launch_bounds__(NT20) void k20_set_bc(const BrickInfo* __restrict__ bricks, const DomInfo* __restrict__ doms,
+                                                   const Dom20Dev* __restrict__ d20, double* __restrict__ x) {
+    const BrickInfo B = bricks[blockIdx.x];
+    const DomInfo D = doms[B.dom];
+    const Dom20Dev G = d20[B.dom];
+    const int lc = threadIdx.x % R;
+    for (int q = B.node_begin + (int)threadIdx.x / R; q < B.node_end; q += NT20 / R) {
         const int ql = (int)(q - G.node_begin);
-        T y[3] = {T(0), T(0), T(0)};
-        for (int k = G.adj_off[ql]; k < G.adj_off[ql + 1]; ++k) {
-            const int e = G.adj[k] >> 5, a = G.adj[k] & 31;
-            const int* en = G.elems + (int64_t)e * 20;
-            const T* Ka = sK + 3 * a * 60;
-            T s[3] = {T(0), T(0), T(0)};
-            for (int bb = 0; bb < 20; ++bb) {
-                const int qb = en[bb];
-                if (qb < 0) continue;
-                T xv[3];
-#pragma unroll
-                for (int d2 = 0; d2 < 3; ++d2) {
-                    if (IN == 1 && G.bcf[qb]) xv[d2] = (T)bc20(D, G, qb, d2, r);
-                    else if (IN == 1 && !xin) xv[d2] = T(0);
-                    else xv[d2] = (T)xin[((int64_t)(G.node_begin + qb) * 3 + d2) * R + r];
-                }
-#pragma unroll
-                for (int dd = 0; dd < 3; ++dd)
-#pragma unroll
-                    for (int d2 = 0; d2 < 3; ++d2) s[dd] += Ka[dd * 60 + 3 * bb + d2] * xv[d2];
-            }
-            const T E = (T)G.emod[e];
-#pragma unroll
-            for (int dd = 0; dd < 3; ++dd) y[dd] += E * s[dd];
-        }
-        const bool bc = G.bcf[ql] != 0;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const int64_t o = ((int64_t)q * 3 + d) * R + r;
-            T v = y[d];
-            if (OUT == 0) {          // masked, x . y
-                if (bc) v = T(0);
-                acc += (double)xin[o] * (double)v;
-            } else if (OUT == 1) {   // -y on free rows, y . y
-                v = bc ? T(0) : -v;
-                acc += (double)v * (double)v;
-            } else if (OUT == 3) {
-                if (bc) v = T(0);
-            }
-            yout[o] = (VT)v;
-        }
-    }
-    if (OUT == 0 || OUT == 1) {
-        s_red[tid] = acc;
-        __syncthreads();
-        if (tid < R) {
-            double sum = 0.0;
-            for (int gg = 0; gg < NT20 / R; ++gg) sum += s_red[gg * R + tid];
-            A.partial[(int64_t)blockIdx.x * R + tid] = sum;
-        }
+        if (!G.bcf[ql]) continue;
+        double N[20];
+        macro_shape(D.macro_order, G.coords + 3 * ql, D.min_c, D.max_c, N);
+        for (int d = 0; d < 3; ++d) x[((int64_t)q * 3 + d) * R + lc] = bc_value_m(D.macro_order, N, d, D.lc_base + lc);
     }
 }
 
@@ -261,72 +197,23 @@ __global__ __launch_bounds__(NT20) void k_fields20(const BrickInfo* __restrict__
     }
 }
 
-// ---------------------------------------------------------------- element-wise FP32 operator
-// y = K x in two passes (FP32, IN_V): k20_elem forms every element's forces
-// y_e = E_e Khat x_e for the 24 load cases into a per-element buffer (60 rows x
-// 24 load cases), k20_gather sums them per node over the node's sorted
-// (element, local node) list.  The products and sums run in the node-gather
-// kernel's order (k = 3 b + d per row, elements in list order).
-constexpr int E20_EPB = 4;                 // elements per workgroup
-constexpr int E20_NT = 240;                // 24 load cases x 10 row groups of 6 rows
-
-__global__ __launch_bounds__(E20_NT) void k20_elem(Dom20Dev G, int dom, const int* __restrict__ done,
-                                                  const float* __restrict__ Kg, const float* __restrict__ x,
-                                                  float* __restrict__ ye, int64_t ne) {
-    __shared__ float sK[3600];
-    __shared__ float sx[E20_EPB][60][R];
-    if (done && done[dom]) return;
-    const int tid = threadIdx.x;
-    const int64_t e0 = (int64_t)blockIdx.x * E20_EPB;
-    for (int i = tid; i < 3600; i += E20_NT) sK[i] = Kg[i];
-    // x of the block's elements: 20 nodes x 72 contiguous values each
-    for (int i = tid; i < E20_EPB * 20 * 72; i += E20_NT) {
-        const int el = i / (20 * 72), rem = i % (20 * 72), a = rem / 72, v = rem % 72;
-        const int64_t e = e0 + el;
-        float val = 0.f;
-        if (e < ne) {
-            const int q = G.elems[e * 20 + a];
-            if (q >= 0) val = x[(G.node_begin + q) * 72 + v];
-        }
-        sx[el][3 * a + v / R][v % R] = val;
-    }
-    __syncthreads();
-    const int r = tid % R, g = tid / R;
-    float acc[E20_EPB][6];
-#pragma unroll
-    for (int el = 0; el < E20_EPB; ++el)
-#pragma unroll
-        for (int j = 0; j < 6; ++j) acc[el][j] = 0.f;
-    for (int k = 0; k < 60; ++k) {
-        float xk[E20_EPB], kk[6];
-#pragma unroll
-        for (int el = 0; el < E20_EPB; ++el) xk[el] = sx[el][k][r];
-#pragma unroll
-        for (int j = 0; j < 6; ++j) kk[j] = sK[(g * 6 + j) * 60 + k];
-#pragma unroll
-        for (int el = 0; el < E20_EPB; ++el)
-#pragma unroll
-            for (int j = 0; j < 6; ++j) acc[el][j] += kk[j] * xk[el];
-    }
-#pragma unroll
-    for (int el = 0; el < E20_EPB; ++el) {
-        const int64_t e = e0 + el;
-        if (e >= ne) break;
-        const float E = (float)G.emod[e];
-#pragma unroll
-        for (int j = 0; j < 6; ++j) ye[(e * 60 + g * 6 + j) * R + r] = E * acc[el][j];
-    }
-}
-
-// The same element forces on the matrix cores, FP32 (v_mfma_f32_16x16x4_f32) or
+// ---------------------------------------------------------------- operator
+// y = K x in two passes: k20_elem forms every element's forces y_e = E_e Khat x_e for the
+// 24 load cases into a per-element buffer (60 rows x 24 load cases), k20_gather sums them
+// per node over the node's sorted (element, local node) list.
+//
+// Element forces on the matrix cores, FP32 (v_mfma_f32_16x16x4_f32) or
 // FP64 (v_mfma_f64_16x16x4_f64) products and sums: for a group of EM elements,
 // Y (64 x 24 EM) = Khat (60 x 60, rows padded to 64) X (60 x 24 EM), column
 // c = 24 e + load case.  Wave w owns rows 16 w .. 16 w + 15 and keeps its Khat
-// fragments in registers for the whole block; X (FP32 vectors, widened to T) is
+// fragments in registers for the whole block; X (vectors of type TX, widened to T) is
 // staged in LDS with a padded row stride.  Lane layout of the 16x16x4 products
 // (l = lane, measured on gfx950): A[i][k] in lane i + 16 k, B[k][j] in lane
 // j + 16 k; D[i][j] in lane j + 16 (i / 4), component i % 4 (f32), and in lane
-// j + 16 (i % 4), component i / 4 (f64).
+// j + 16 (i % 4), component i / 4 (f64).  blockIdx.y: domain group.  A 27^3 domain
+// (5,800 elements): 22 us in FP32 (the products take 8 at the rate of a large FP32 matrix
+// product, the 33 MB of forces as long), 31 us in FP64; the gather then 13.  The FP64
+// residual in one gather kernel, 60 products per entry on the vector units, took 4,500.
 typedef float em_float4 __attribute__((ext_vector_type(4)));
 typedef double em_double4 __attribute__((ext_vector_type(4)));
 template <typename T> struct EmCfg;
@@ -345,31 +232,36 @@ template <> struct EmCfg<double> {
     __device__ static int drow(int k4, int c) { return k4 + 4 * c; }
 };
 
-template <typename T>
-__global__ __launch_bounds__(256) void k20_elem_mf(Dom20Dev G, int dom, const int* __restrict__ done,
-                                                   const T* __restrict__ Kg, const float* __restrict__ x,
-                                                   T* __restrict__ ye, int64_t ne) {
+template <typename T, typename TX>
+__global__ __launch_bounds__(256) void k20_elem(const Dom20Dev* __restrict__ d20, const int64_t* __restrict__ ebase,
+                                                const int* __restrict__ done, const T* __restrict__ Kg,
+                                                const TX* __restrict__ x, T* __restrict__ yall) {
     constexpr int EM = EmCfg<T>::EM, XS = EmCfg<T>::XS, NCT = 24 * EM / 16;
     using V4 = typename EmCfg<T>::V4;
     __shared__ T sX[60 * XS];
     __shared__ T sE[EM];
+    const int dom = blockIdx.y;
     if (done && done[dom]) return;
+    const int64_t ne = ebase[dom + 1] - ebase[dom], e0 = (int64_t)blockIdx.x * EM;
+    if (e0 >= ne) return;
+    const Dom20Dev G = d20[dom];
+    T* __restrict__ ye = yall + ebase[dom] * 60 * R;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int64_t e0 = (int64_t)blockIdx.x * EM;
-    // X: 20 nodes x 72 contiguous floats per element, read as float4 (18 per node)
-    for (int i = tid; i < EM * 20 * 18; i += 256) {
-        const int el = i / 360, rem = i % 360, a = rem / 18, v = 4 * (rem % 18), d = v / R, r = v % R;
+    // X: 20 nodes x 72 contiguous values per element, read as 16-byte vectors
+    constexpr int VX = 16 / sizeof(TX), NVX = 72 / VX;
+    for (int i = tid; i < EM * 20 * NVX; i += 256) {
+        const int el = i / (20 * NVX), rem = i % (20 * NVX), a = rem / NVX, v = VX * (rem % NVX), d = v / R, r = v % R;
         const int64_t e = e0 + el;
-        float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
+        TX val[VX];
+#pragma unroll
+        for (int k = 0; k < VX; ++k) val[k] = TX(0);
         if (e < ne) {
             const int q = G.elems[e * 20 + a];
-            if (q >= 0) val = *reinterpret_cast<const float4*>(x + (G.node_begin + q) * 72 + v);
+            if (q >= 0) *reinterpret_cast<uint4*>(val) = *reinterpret_cast<const uint4*>(x + (G.node_begin + q) * 72 + v);
         }
         T* dst = sX + (3 * a + d) * XS + el * R + r;
-        dst[0] = (T)val.x;
-        dst[1] = (T)val.y;
-        dst[2] = (T)val.z;
-        dst[3] = (T)val.w;
+#pragma unroll
+        for (int k = 0; k < VX; ++k) dst[k] = (T)val[k];
     }
     if (tid < EM) sE[tid] = e0 + tid < ne ? (T)G.emod[e0 + tid] : T(0);
     // Khat fragments of this wave's row tile: A[i][k] = Khat[16 w + i][4 ks + k]
@@ -403,29 +295,30 @@ __global__ __launch_bounds__(256) void k20_elem_mf(Dom20Dev G, int dom, const in
     }
 }
 
-// Operands of the Chebyshev epilogue of k20_gather (OUT 4)
+// Operands of k20_gather's epilogues that combine y with other vectors
 struct Cheb20 {
-    const float* b;      // right-hand side
-    const float* dinv;   // Jacobi scaling per (node, direction)
+    const float* b;      // right-hand side (G_CHEB, G_BRES)
+    const float* dinv;   // G_CHEB: Jacobi scaling per (node, direction)
     float* d;            // direction, read and written
     float c1, c2;
 };
+// G_DOT masked, and per-brick sums of x . y; G_RESID -y on free rows, and per-brick sums of
+// y . y; G_PLAIN; G_MASKED zero on Dirichlet rows (the HEX08 matvec's modes by number);
+// G_CHEB (FP32): one Chebyshev-Jacobi step on x in place, with t the masked sum
+// d = c1 d + c2 dinv (b - t), x = x + d (yout is x); G_BRES (FP32): b - y on free rows
+enum { G_DOT = 0, G_RESID = 1, G_PLAIN = 2, G_MASKED = 3, G_CHEB = 4, G_BRES = 5 };
 
-// y on the pseudo-bricks: the sum of the adjacent elements' forces; MASKED zeroes
-// Dirichlet rows, MASKED_DOT also writes per-brick sums of x . y; OUT 4 (FP32) applies
-// one Chebyshev-Jacobi step to x in place instead of writing y: with t the masked sum,
-// d = c1 d + c2 dinv (b - t), x = x + d (yout is x)
-// (T: the type of the element forces and of the sums; x is an FP32 vector, y one
-// of type TO)
-template <typename T, int OUT, typename TO = float>
+// y on the pseudo-bricks: the sum of the adjacent elements' forces (type T), written as TO
+template <typename T, int OUT, typename TO>
 __global__ __launch_bounds__(NT20) void k20_gather(const BrickInfo* __restrict__ bricks,
                                                   const Dom20Dev* __restrict__ d20,
                                                   const int64_t* __restrict__ ebase, const int* __restrict__ done,
-                                                  const T* __restrict__ ye, const float* __restrict__ xin,
+                                                  const T* __restrict__ ye, const TO* __restrict__ xin,
                                                   TO* __restrict__ yout, double* __restrict__ partial,
                                                   Cheb20 ch) {
-    static_assert(OUT != 4 || (sizeof(T) == 4 && sizeof(TO) == 4), "Chebyshev epilogue: FP32");
-    __shared__ double s_red[NT20];
+    static_assert((OUT != G_CHEB && OUT != G_BRES) || (sizeof(T) == 4 && sizeof(TO) == 4), "smoothing modes: FP32");
+    constexpr bool SUMS = OUT == G_DOT || OUT == G_RESID;
+    __shared__ double s_red[SUMS ? NT20 : 1];
     const BrickInfo B = bricks[blockIdx.x];
     if (done && done[B.dom]) return;
     const Dom20Dev G = d20[B.dom];
@@ -459,22 +352,25 @@ __global__ __launch_bounds__(NT20) void k20_gather(const BrickInfo* __restrict__
 #pragma unroll
                 for (int d = 0; d < 3; ++d) y[d] += v[u][d];
         }
-        const bool bc = G.bcf[ql] != 0;
+        const bool bc = OUT != G_PLAIN && G.bcf[ql] != 0;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const int64_t o = ((int64_t)q * 3 + d) * R + r;
-            const TO v = bc ? TO(0) : (TO)y[d];
-            if constexpr (OUT == 4) {
-                const float dv = cheb_dir(ch.c1, ch.d[o], ch.c2, ch.dinv[o / R], ch.b[o], (float)v);
+            const TO v = bc ? TO(0) : (TO)(OUT == G_RESID ? -y[d] : y[d]);
+            if constexpr (OUT == G_CHEB) {
+                const float dv = cheb_dir(ch.c1, ch.d[o], ch.c2, ch.dinv[(int64_t)q * 3 + d], ch.b[o], (float)v);
                 ch.d[o] = dv;
                 yout[o] = (TO)(yout[o] + dv);
+            } else if constexpr (OUT == G_BRES) {
+                yout[o] = bc ? TO(0) : (TO)(ch.b[o] - v);
             } else {
-                if (OUT == 0) acc += (double)xin[o] * (double)v;
+                if (OUT == G_DOT) acc += (double)xin[o] * (double)v;
+                if (OUT == G_RESID) acc += (double)v * (double)v;
                 yout[o] = v;
             }
         }
     }
-    if (OUT == 0) {
+    if constexpr (SUMS) {
         s_red[tid] = acc;
         __syncthreads();
         if (tid < R) {
@@ -487,102 +383,71 @@ __global__ __launch_bounds__(NT20) void k20_gather(const BrickInfo* __restrict__
 
 inline unsigned nb(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-template <typename T, int IN, int OUT>
-int mv20_launch(SolverBatch& b, const void* xin, void* yout, double* part, const int* done) {
-    if (b.n_bricks == 0) return DTC_OK;
-    Mv20 a{b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(), b.d20dev.as<Dom20Dev>(), done, part};
+// element forces of every domain group into ye20
+template <typename T, typename TX>
+int elem_pass(SolverBatch& b, const TX* x, const int* done) {
+    int64_t most = 0;
+    for (int g = 0; g < b.n_dom; ++g) most = std::max(most, b.h_ebase20[g + 1] - b.h_ebase20[g]);
+    if (most == 0) return DTC_OK;
     const T* K = sizeof(T) == 8 ? (const T*)b.k20_64.p : (const T*)b.k20_32.p;
-    k_matvec20<T, IN, OUT><<<b.n_bricks, NT20, 0, b.stream>>>(a, K, (const T*)xin, (T*)yout);
+    k20_elem<T, TX><<<dim3(nb(most, EmCfg<T>::EM), b.n_dom), 256, 0, b.stream>>>(
+        b.d20dev.as<Dom20Dev>(), b.ebase20.as<int64_t>(), done, K, x, b.ye20.as<T>());
+    DTC_HIP(hipGetLastError());
+    return DTC_OK;
+}
+
+template <typename T, int OUT, typename TO>
+int gather_pass(SolverBatch& b, const TO* x, TO* y, double* part, const int* done, const Cheb20& ch = Cheb20{}) {
+    k20_gather<T, OUT, TO><<<b.n_bricks, NT20, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
+                                                            b.ebase20.as<int64_t>(), done, b.ye20.as<T>(), x, y, part, ch);
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
 
 }  // namespace
 
-// FP32 element forces of every domain group into ye20 (on the matrix cores;
-// DTC_HEX20_MFMA=0: the VALU form)
-int elem_pass32(SolverBatch& b, const float* xin, const int* done) {
-    const char* me = std::getenv("DTC_HEX20_MFMA");
-    const bool use_mf = !(me && me[0] == '0');
-    hipStream_t s = b.stream;
-    for (int g = 0; g < b.n_dom; ++g) {
-        const Dom20Dev& G = b.h_d20dev[g];
-        const int64_t ne = b.h_elems[g];   // the count ye20 was sized for (0 for a domain that failed set-up)
-        if (ne <= 0 || !G.elems) continue;
-        float* ye = b.ye20.as<float>() + b.h_ebase20[g] * 60 * R;
-        if (use_mf)
-            k20_elem_mf<float><<<nb(ne, EmCfg<float>::EM), 256, 0, s>>>(G, g, done, b.k20_32.as<float>(), xin, ye, ne);
-        else
-            k20_elem<<<nb(ne, E20_EPB), E20_NT, 0, s>>>(G, g, done, b.k20_32.as<float>(), xin, ye, ne);
-    }
-    DTC_HIP(hipGetLastError());
-    return DTC_OK;
-}
-
 int mv20_cheb(SolverBatch& b, float* x, const int* done, const float* bv, const float* dinv, float* d, float c1,
               float c2) {
-    if (hex20_gather_form()) return set_error(DTC_ERR_UNSUPPORTED, "Chebyshev epilogue of the node-gather form");
     if (b.n_bricks == 0) return DTC_OK;
-    DTC_TRY(elem_pass32(b, x, done));
-    k20_gather<float, 4><<<b.n_bricks, NT20, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
-                                                         b.ebase20.as<int64_t>(), done, b.ye20.as<float>(), nullptr, x,
-                                                         nullptr, Cheb20{bv, dinv, d, c1, c2});
-    DTC_HIP(hipGetLastError());
-    return DTC_OK;
+    DTC_TRY((elem_pass<float, float>(b, x, done)));
+    return gather_pass<float, G_CHEB, float>(b, nullptr, x, nullptr, done, Cheb20{bv, dinv, d, c1, c2});
 }
 
-int mv20(SolverBatch& b, bool fp64, int in, int out, const void* xin, void* yout, double* part, const int* done) {
+int mv20_bres(SolverBatch& b, const float* x, float* y, const int* done, const float* bv) {
+    if (b.n_bricks == 0) return DTC_OK;
+    DTC_TRY((elem_pass<float, float>(b, x, done)));
+    return gather_pass<float, G_BRES, float>(b, nullptr, y, nullptr, done, Cheb20{bv, nullptr, nullptr, 0.f, 0.f});
+}
+
+int mv20(SolverBatch& b, bool fp64, int out, const void* xin, void* yout, double* part, const int* done) {
+    if (b.n_bricks == 0) return DTC_OK;
     if (fp64) {
-        if (in == 0 && out == 0) return mv20_launch<double, 0, 0>(b, xin, yout, part, done);
-        if (in == 1 && out == 1) return mv20_launch<double, 1, 1>(b, xin, yout, part, done);
-        if (in == 1 && out == 2) return mv20_launch<double, 1, 2>(b, xin, yout, part, done);
-    } else if (in == 0 && (out == 0 || out == 3)) {
-        if (hex20_gather_form()) {   // the node-gather kernel (reference form of the operator)
-            if (out == 0) return mv20_launch<float, 0, 0>(b, xin, yout, part, done);
-            return mv20_launch<float, 0, 3>(b, xin, yout, part, done);
-        }
-        if (b.n_bricks == 0) return DTC_OK;
-        hipStream_t s = b.stream;
-        DTC_TRY(elem_pass32(b, (const float*)xin, done));
-        if (out == 0)
-            k20_gather<float, 0><<<b.n_bricks, NT20, 0, s>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
-                                                      b.ebase20.as<int64_t>(), done, b.ye20.as<float>(),
-                                                      (const float*)xin, (float*)yout, part, Cheb20{});
-        else
-            k20_gather<float, 3><<<b.n_bricks, NT20, 0, s>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
-                                                      b.ebase20.as<int64_t>(), done, b.ye20.as<float>(),
-                                                      (const float*)xin, (float*)yout, part, Cheb20{});
-        DTC_HIP(hipGetLastError());
-        return DTC_OK;
+        const double* x = (const double*)xin;
+        double* y = (double*)yout;
+        DTC_TRY((elem_pass<double, double>(b, x, done)));
+        if (out == G_DOT) return gather_pass<double, G_DOT, double>(b, x, y, part, done);
+        if (out == G_RESID) return gather_pass<double, G_RESID, double>(b, x, y, part, done);
+        if (out == G_PLAIN) return gather_pass<double, G_PLAIN, double>(b, x, y, part, done);
+    } else {
+        const float* x = (const float*)xin;
+        float* y = (float*)yout;
+        DTC_TRY((elem_pass<float, float>(b, x, done)));
+        if (out == G_DOT) return gather_pass<float, G_DOT, float>(b, x, y, part, done);
+        if (out == G_MASKED) return gather_pass<float, G_MASKED, float>(b, x, y, part, done);
     }
-    return set_error(DTC_ERR_UNSUPPORTED, "HEX20 micro operator: mode (%d, %d)", in, out);
+    return set_error(DTC_ERR_UNSUPPORTED, "HEX20 micro operator: mode %d", out);
 }
 
 int mv20_q64(SolverBatch& b, const float* p, float* q, const int* done, double* q64) {
     if (b.n_bricks == 0) return DTC_OK;
-    hipStream_t s = b.stream;
-    if (hex20_gather_form()) {   // the node-gather form
-        Mv20 a{b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(), b.d20dev.as<Dom20Dev>(), done, nullptr};
-        if (q64) return set_error(DTC_ERR_UNSUPPORTED, "HEX20 node-gather operator with an FP64 output");
-        k_matvec20<double, 0, 3, float><<<b.n_bricks, NT20, 0, s>>>(a, b.k20_64.as<double>(), p, q);
-        DTC_HIP(hipGetLastError());
-        return DTC_OK;
-    }
-    for (int g = 0; g < b.n_dom; ++g) {
-        const Dom20Dev& G = b.h_d20dev[g];
-        const int64_t ne = b.h_elems[g];
-        if (ne <= 0 || !G.elems) continue;
-        k20_elem_mf<double><<<nb(ne, EmCfg<double>::EM), 256, 0, s>>>(G, g, done, b.k20_64.as<double>(), p,
-                                                                      b.ye20.as<double>() + b.h_ebase20[g] * 60 * R, ne);
-    }
-    if (q64)
-        k20_gather<double, 3, double><<<b.n_bricks, NT20, 0, s>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
-                                                                  b.ebase20.as<int64_t>(), done, b.ye20.as<double>(),
-                                                                  p, q64, nullptr, Cheb20{});
-    else
-        k20_gather<double, 3><<<b.n_bricks, NT20, 0, s>>>(b.brick.as<BrickInfo>(), b.d20dev.as<Dom20Dev>(),
-                                                          b.ebase20.as<int64_t>(), done, b.ye20.as<double>(), p, q,
-                                                          nullptr, Cheb20{});
+    DTC_TRY((elem_pass<double, float>(b, p, done)));
+    if (q64) return gather_pass<double, G_MASKED, double>(b, nullptr, q64, nullptr, done);
+    return gather_pass<double, G_MASKED, float>(b, nullptr, q, nullptr, done);
+}
+
+int set_bc20(SolverBatch& b, double* x) {
+    if (b.n_bricks == 0) return DTC_OK;
+    k20_set_bc<<<b.n_bricks, NT20, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(), b.d20dev.as<Dom20Dev>(), x);
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
@@ -697,15 +562,15 @@ int finalize20(SolverBatch& b) {
     }
     b.h_d20dev = h;
     // per-element force buffer of the FP32 operator: element offsets per domain group
-    b.h_ebase20.assign(b.n_dom, 0);
+    b.h_ebase20.assign(b.n_dom + 1, 0);
     int64_t ne_all = 0;
     for (int i = 0; i < b.n_dom; ++i) {
         b.h_ebase20[i] = ne_all;
-        ne_all += b.h_elems[i];
+        if (h[i].elems) ne_all += b.h_elems[i];   // (none for a domain that failed set-up)
     }
-    DTC_TRY(b.ebase20.ensure(std::max<size_t>(b.h_ebase20.size(), 1) * 8));
-    if (!b.h_ebase20.empty())
-        DTC_HIP(hipMemcpyAsync(b.ebase20.p, b.h_ebase20.data(), b.h_ebase20.size() * 8, hipMemcpyHostToDevice, s));
+    b.h_ebase20[b.n_dom] = ne_all;
+    DTC_TRY(b.ebase20.ensure(b.h_ebase20.size() * 8));
+    DTC_HIP(hipMemcpyAsync(b.ebase20.p, b.h_ebase20.data(), b.h_ebase20.size() * 8, hipMemcpyHostToDevice, s));
     // FP64 element forces of the block's Q = K P, FP32 ones of the smoothing steps (one buffer)
     DTC_TRY(b.ye20.ensure((size_t)std::max<int64_t>(ne_all, 1) * 60 * R * 8));
     DTC_TRY(b.d20dev.ensure(std::max<size_t>(h.size(), 1) * sizeof(Dom20Dev)));
