@@ -30,6 +30,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <thread>
 #include <type_traits>
 
 #include "bc.hpp"
@@ -1749,6 +1750,7 @@ int batch_begin(SolverBatch& b, const dtc_domain_desc* d, int64_t n_dom) {
     b.d20.clear();
     b.h_contrast.clear();
     b.n_slices = 0;   // the block PCG slices follow the batch's domains (block_setup)
+    if (b.block_graph.e) DTC_HIP(hipStreamSynchronize(b.stream));
     b.block_graph.reset();   // captured with the previous composition's buffers
     return DTC_OK;
 }
@@ -2602,15 +2604,120 @@ int all_done(SolverBatch& b, const DevMem& flags, bool* out) {
     return DTC_OK;
 }
 
+// ---- convergence words
+// After a run of iterations k_all_set counts the run in a device word and writes
+// 2 * runs + (every domain's done flag is set) to a page-locked host word, one 8-byte
+// store.  The host reads that word while the next run already executes (a copy of the
+// flags between the runs left the GPU idle for 20 us each time).
+__global__ __launch_bounds__(256) void k_all_set(const int* __restrict__ flags, int n, unsigned long long* __restrict__ runs,
+                                                 unsigned long long* __restrict__ host) {
+    __shared__ int s_any[256];
+    int miss = 0;
+    for (int d = threadIdx.x; d < n; d += 256) miss |= flags[d] == 0;
+    s_any[threadIdx.x] = miss;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (threadIdx.x < w) s_any[threadIdx.x] |= s_any[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const unsigned long long k = *runs + 1;
+        *runs = k;
+        __hip_atomic_store(host, 2 * k + (s_any[0] ? 0 : 1), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+__global__ void k_fill_u64(unsigned long long* __restrict__ p, int n, unsigned long long v) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+}
+
+// per domain [done64, iterations, rr (24), rr0 (24)] to page-locked host memory
+constexpr int STAT_N = 2 + 2 * R;
+__global__ __launch_bounds__(64) void k_status(const int* __restrict__ done64, const int64_t* __restrict__ iters,
+                                               const double* __restrict__ rr, const double* __restrict__ rr0,
+                                               double* __restrict__ host) {
+    const int d = blockIdx.x, t = threadIdx.x;
+    if (t >= STAT_N) return;
+    host[(int64_t)d * STAT_N + t] = t == 0   ? (double)done64[d]
+                                    : t == 1 ? (double)iters[d]
+                                    : t < 2 + R ? rr[d * R + t - 2]
+                                                : rr0[d * R + t - 2 - R];
+}
+
+int words_setup(SolverBatch& b) {
+    const size_t need = 64 + (size_t)b.n_dom * STAT_N * 8;
+    if (b.host_words.n < need) {
+        DTC_HIP(hipStreamSynchronize(b.stream));
+        b.host_words.reset();
+        DTC_TRY(b.host_words.alloc(need));
+        *b.host_words.word() = 0;
+        b.runs = 0;
+        DTC_TRY(b.runs_dev.ensure(8));
+        k_fill_u64<<<1, 1, 0, b.stream>>>(b.runs_dev.as<unsigned long long>(), 1, 0);
+        DTC_HIP(hipGetLastError());
+    }
+    return DTC_OK;
+}
+
+int post_done(SolverBatch& b) {
+    k_all_set<<<1, 256, 0, b.stream>>>(b.done.as<int>(), b.n_dom, b.runs_dev.as<unsigned long long>(),
+                                       b.host_words.word());
+    DTC_HIP(hipGetLastError());
+    return DTC_OK;
+}
+
+// waits for the summary of run number `run`
+int wait_done(SolverBatch& b, uint64_t run, bool* fin) {
+    const unsigned long long* w = b.host_words.word();
+    for (uint32_t k = 1;; ++k) {
+        const unsigned long long v = __atomic_load_n(w, __ATOMIC_ACQUIRE);
+        if (v / 2 >= run) {
+            *fin = (v & 1) != 0;
+            return DTC_OK;
+        }
+        if (k % 64 == 0) std::this_thread::yield();
+        if (k % 4096 == 0) {   // a stream that ended without the word has failed
+            const hipError_t e = hipStreamQuery(b.stream);
+            if (e == hipSuccess && __atomic_load_n(w, __ATOMIC_ACQUIRE) / 2 < run)
+                return set_error(DTC_ERR_DEVICE, "the iterations ended without a summary");
+            if (e != hipSuccess && e != hipErrorNotReady)
+                return set_error(DTC_ERR_DEVICE, "hipStreamQuery: %s", hipGetErrorString(e));
+            if (e == hipErrorNotReady) (void)hipGetLastError();
+        }
+    }
+}
+
+// status of every domain on the host (the stream is idle afterwards)
+int read_status(SolverBatch& b, const double** out) {
+    DTC_TRY(words_setup(b));
+    k_status<<<b.n_dom, 64, 0, b.stream>>>(b.done64.as<int>(), b.iters.as<int64_t>(), b.rr.as<double>(),
+                                           b.rr0.as<double>(), b.host_words.status());
+    DTC_HIP(hipGetLastError());
+    DTC_HIP(hipStreamSynchronize(b.stream));
+    *out = b.host_words.status();
+    return DTC_OK;
+}
+
+// iterations until every domain is done or max_steps (rounded up to CHECK) ran.  The host
+// is one run of CHECK iterations ahead of the summary that it decides by: iterations after
+// the last domain finished are early exits, every kernel skips done domains
 template <typename T>
 int pcg_run(SolverBatch& b, const WK<T>& wk, T* x, T* r, T* p, T* q, const T* dinv, int64_t max_iters,
             int64_t max_steps, T* zmg) {
-    const int CHECK = zmg ? 4 : 20;
+    const int CHECK = zmg ? 4 : 8;
+    if (!b.timing) DTC_TRY(words_setup(b));
+    const uint64_t first = b.runs;
     for (int64_t steps = 0; steps < max_steps; steps += CHECK) {
         bool fin = false;
-        DTC_TRY(all_done(b, b.done, &fin));
-        if (fin) return DTC_OK;
+        if (b.timing) DTC_TRY(all_done(b, b.done, &fin));
+        else if (b.runs > first + 1) DTC_TRY(wait_done(b, b.runs - 1, &fin));
+        if (fin) break;
         for (int k = 0; k < CHECK; ++k) DTC_TRY(pcg_iteration<T>(b, wk, x, r, p, q, dinv, max_iters, zmg));
+        if (!b.timing) {
+            DTC_TRY(post_done(b));
+            ++b.runs;
+        }
     }
     return DTC_OK;
 }
@@ -2768,31 +2875,16 @@ int block_iteration(SolverBatch& b, const WK<float>& wk, float* x, float* r, flo
     return block_dir_orth(b, p, z, q);
 }
 
-// *out = 1 when every domain's flag is set (one workgroup, fixed order)
-__global__ __launch_bounds__(256) void k_all_set(const int* __restrict__ flags, int n, int* __restrict__ out) {
-    __shared__ int s_any[256];
-    int miss = 0;
-    for (int d = threadIdx.x; d < n; d += 256) miss |= flags[d] == 0;
-    s_any[threadIdx.x] = miss;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) s_any[threadIdx.x] |= s_any[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = s_any[0] ? 0 : 1;
-}
-
 // block PCG iterations until every domain is done or max_steps iterations ran.
 //
-// Without kernel timing (the default), GROUP iterations are captured once per
-// solve into a HIP graph together with a kernel that writes "every domain done"
-// to a device word; the graph is replayed, and after each replay that word is
-// copied into one of two page-locked host words.  The host decides to stop
-// from the previous replay's word while the current replay already runs, so the
-// GPU never waits for the host; a replay issued after every domain finished is
-// a sequence of early exits (every kernel skips done domains), which leaves the
-// results unchanged.  DTC_GRAPH=0 (or kernel timing) launches the iterations one
-// by one with a synchronous check every GROUP iterations.
+// Without kernel timing (the default), RUN iterations and their summary (k_all_set) are
+// captured once per solve into a HIP graph and replayed; the host stays one replay ahead of
+// the summary that it decides by, so the GPU never waits for it, and at most 2 RUN - 1
+// iterations of early exits follow the last one that counts.  An empty iteration costs its
+// launches, 2-4 us each: a 12^3 domain (22 iterations in two phases) took 5.07 ms with runs of
+// 4 and the flags copied between them, 4.55 with runs of 4, 4.36 with 2, 4.40 with 1.
+// DTC_GRAPH=0 (or kernel timing) launches the iterations one by one with a synchronous
+// check every GROUP iterations.
 inline bool trace_on() {
     static const bool on = std::getenv("DTC_TRACE") && std::getenv("DTC_TRACE")[0] == '1';
     return on;
@@ -2800,13 +2892,14 @@ inline bool trace_on() {
 
 int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p, float* q, float* z,
               int64_t max_iters, int64_t max_steps) {
-    constexpr int GROUP = 4;
+    constexpr int GROUP = 4, RUN = 2;   // max_steps is rounded up to GROUP iterations
+    static_assert(GROUP % RUN == 0, "");
     const char* ge = std::getenv("DTC_GRAPH");
     const bool use_graph = !(ge && ge[0] == '0') && !b.timing;
     bool fin = false;
-    DTC_TRY(all_done(b, b.done, &fin));
-    if (fin) return DTC_OK;
     if (!use_graph) {
+        DTC_TRY(all_done(b, b.done, &fin));
+        if (fin) return DTC_OK;
         for (int64_t steps = 0; steps < max_steps; steps += GROUP) {
             if (steps > 0) {
                 DTC_TRY(all_done(b, b.done, &fin));
@@ -2822,14 +2915,14 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
                 b.graph_mode == (int)b.block64;
     for (int k = 0; k < 6; ++k) same = same && b.graph_key[k] == key[k];
     if (!same) {
+        if (b.block_graph.e) DTC_HIP(hipStreamSynchronize(s));   // no replay of the old one is in flight
         b.block_graph.reset();
-        DTC_TRY(b.all_done_dev.ensure(4));
-        if (!b.all_done_host.p) DTC_HIP(hipHostMalloc((void**)&b.all_done_host.p, 2 * sizeof(int), hipHostMallocDefault));
+        DTC_TRY(words_setup(b));
         hipGraph_t g = nullptr;
         DTC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         int rc = DTC_OK;
-        for (int k = 0; k < GROUP && rc == DTC_OK; ++k) rc = block_iteration(b, wk, x, r, p, q, z, max_iters);
-        if (rc == DTC_OK) k_all_set<<<1, 256, 0, s>>>(b.done.as<int>(), b.n_dom, b.all_done_dev.as<int>());
+        for (int k = 0; k < RUN && rc == DTC_OK; ++k) rc = block_iteration(b, wk, x, r, p, q, z, max_iters);
+        if (rc == DTC_OK) rc = post_done(b);
         const hipError_t ec = hipStreamEndCapture(s, &g);
         if (rc != DTC_OK && g) (void)hipGraphDestroy(g);
         DTC_TRY(rc);
@@ -2846,39 +2939,24 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
         b.graph_bricks = b.n_bricks;
         b.graph_mode = (int)b.block64;
     }
-    // launch n copies the summary to host word n % 2 and records event n % 2
-    hipEvent_t ev[2];
-    for (hipEvent_t& e : ev) DTC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    int rc = DTC_OK;
-    int64_t launched = 0;
-    auto launch = [&](int64_t n) -> int {
+    const int64_t total = (std::min<int64_t>(max_steps, INT64_MAX - GROUP) + GROUP - 1) / GROUP * GROUP;
+    auto run = [&](int64_t steps) -> int {
         DTC_HIP(hipGraphLaunch(b.block_graph.e, s));
-        DTC_HIP(hipMemcpyAsync(b.all_done_host.p + (n & 1), b.all_done_dev.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        DTC_HIP(hipEventRecord(ev[n & 1], s));
+        ++b.runs;
         ++b.graph_launches;
+        if (steps > 0) DTC_TRY(wait_done(b, b.runs - 1, &fin));   // the replay before this one
         return DTC_OK;
     };
-    rc = launch(0);
-    launched = 1;
-    for (int64_t steps = GROUP; rc == DTC_OK && steps < max_steps; steps += GROUP) {
-        rc = launch(launched);
-        if (rc != DTC_OK) break;
-        ++launched;
-        // the replay before this one has finished: its summary decides
-        const hipError_t e = hipEventSynchronize(ev[(launched - 2) & 1]);
-        if (e != hipSuccess) {
-            rc = set_error(DTC_ERR_DEVICE, "hipEventSynchronize: %s", hipGetErrorString(e));
-            break;
+    for (int64_t steps = 0; steps < total && !fin; steps += RUN) {
+        const int rc = run(steps);
+        if (rc != DTC_OK) {
+            (void)hipStreamSynchronize(s);   // nothing is in flight when the caller gives up
+            return rc;
         }
-        if (b.all_done_host.p[(launched - 2) & 1]) break;
         // DTC_TRACE=1: a progress line every 1,000 block iterations of a long phase
-        if (trace_on() && (steps + GROUP) % 1000 < GROUP)
-            std::fprintf(stderr, "[dtc] block phase: %lld iterations\n", (long long)(steps + GROUP));
+        if (trace_on() && (steps + RUN) % 1000 < RUN)
+            std::fprintf(stderr, "[dtc] block phase: %lld iterations\n", (long long)(steps + RUN));
     }
-    const hipError_t es = hipStreamSynchronize(s);
-    for (hipEvent_t& e : ev) (void)hipEventDestroy(e);
-    DTC_TRY(rc);
-    if (es != hipSuccess) return set_error(DTC_ERR_DEVICE, "hipStreamSynchronize: %s", hipGetErrorString(es));
     return DTC_OK;
 }
 
@@ -2912,22 +2990,20 @@ struct Progress {
 // mark them finished
 int apply_cap(SolverBatch& b, int64_t cap, std::vector<int64_t>& nouter, bool* any_left, Progress* pg = nullptr) {
     const int D = b.n_dom;
+    const double* st = nullptr;
+    DTC_TRY(read_status(b, &st));
     std::vector<int> h(D);
     std::vector<int64_t> hi(D);
-    std::vector<double> hrr, hr0;
-    DTC_HIP(hipMemcpyAsync(h.data(), b.done64.p, (size_t)D * 4, hipMemcpyDeviceToHost, b.stream));
-    DTC_HIP(hipMemcpyAsync(hi.data(), b.iters.p, (size_t)D * 8, hipMemcpyDeviceToHost, b.stream));
-    if (pg) {
-        hrr.resize((size_t)D * R);
-        hr0.resize((size_t)D * R);
-        DTC_HIP(hipMemcpyAsync(hrr.data(), b.rr.p, hrr.size() * 8, hipMemcpyDeviceToHost, b.stream));
-        DTC_HIP(hipMemcpyAsync(hr0.data(), b.rr0.p, hr0.size() * 8, hipMemcpyDeviceToHost, b.stream));
-        if ((int)pg->best.size() != D) {
-            pg->best.assign(D, -1.0);
-            pg->at.assign(D, 0);
-        }
+    for (int d = 0; d < D; ++d) {
+        h[d] = st[(size_t)d * STAT_N] != 0.0;
+        hi[d] = (int64_t)st[(size_t)d * STAT_N + 1];
     }
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    auto rr_of = [&](int d, int lc) { return st[(size_t)d * STAT_N + 2 + lc]; };
+    auto rr0_of = [&](int d, int lc) { return st[(size_t)d * STAT_N + 2 + R + lc]; };
+    if (pg && (int)pg->best.size() != D) {
+        pg->best.assign(D, -1.0);
+        pg->at.assign(D, 0);
+    }
     // DTC_TRACE=1: one stderr line per residual replacement of the mixed solve
     // (domain: PCG iterations so far / worst relative FP64 residual)
     static const bool trace = std::getenv("DTC_TRACE") && std::getenv("DTC_TRACE")[0] == '1';
@@ -2936,8 +3012,8 @@ int apply_cap(SolverBatch& b, int64_t cap, std::vector<int64_t>& nouter, bool* a
         for (int d = 0; d < D; ++d) {
             double worst = 0.0;
             for (int lc = 0; lc < R; ++lc) {
-                const double r0 = hr0[(size_t)d * R + lc];
-                if (r0 > 0.0) worst = std::fmax(worst, std::sqrt(hrr[(size_t)d * R + lc] / r0));
+                const double r0 = rr0_of(d, lc);
+                if (r0 > 0.0) worst = std::fmax(worst, std::sqrt(rr_of(d, lc) / r0));
             }
             std::fprintf(stderr, " %d:%lld/%.1e", d, (long long)hi[d], worst);
         }
@@ -2949,7 +3025,7 @@ int apply_cap(SolverBatch& b, int64_t cap, std::vector<int64_t>& nouter, bool* a
         if (pg && !h[d] && !stop) {
             double worst = 0.0;
             for (int lc = 0; lc < R; ++lc) {
-                const double r0 = hr0[(size_t)d * R + lc], rr = hrr[(size_t)d * R + lc];
+                const double r0 = rr0_of(d, lc), rr = rr_of(d, lc);
                 const double v = r0 > 0.0 ? std::sqrt(rr / r0) : 0.0;
                 worst = std::isfinite(v) && std::isfinite(r0) ? std::fmax(worst, v) : INFINITY;
             }
@@ -3170,20 +3246,17 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         }
     }
     // results: iterations, true relative residual, convergence status
-    std::vector<int64_t> hi(D);
-    std::vector<double> hrr(D * R), hr0(D * R);
-    DTC_HIP(hipMemcpyAsync(hi.data(), b.iters.p, (size_t)D * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipMemcpyAsync(hrr.data(), b.rr.p, (size_t)D * R * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipMemcpyAsync(hr0.data(), b.rr0.p, (size_t)D * R * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    const double* st = nullptr;
+    DTC_TRY(read_status(b, &st));
     DTC_TRY(harvest_events(b));
     for (int d = 0; d < D; ++d) {
-        iters[d] = hi[d];
+        const double* sd = st + (size_t)d * STAT_N;
+        iters[d] = (int64_t)sd[1];
         outer[d] = nouter[d];
         double mx = 0.0;
         bool finite = true;
         for (int lc = 0; lc < R; ++lc) {
-            const double r0 = hr0[d * R + lc], rr = hrr[d * R + lc];
+            const double r0 = sd[2 + R + lc], rr = sd[2 + lc];
             if (!std::isfinite(r0) || !std::isfinite(rr)) finite = false;
             else if (r0 > 0.0) mx = std::fmax(mx, std::sqrt(rr / r0));
         }

@@ -79,15 +79,27 @@ struct GraphExec {
     }
 };
 
-// Page-locked host words the device writes (hipHostMalloc, freed with the owner).
-struct HostFlags {
-    int* p = nullptr;
-    HostFlags() = default;
-    HostFlags(const HostFlags&) = delete;
-    HostFlags& operator=(const HostFlags&) = delete;
-    ~HostFlags() {
-        if (p) (void)hipHostFree(p);
+// Page-locked host memory the device writes: a summary word, then each domain's status
+// (hipHostMalloc, freed with the owner).
+struct HostWords {
+    void* p = nullptr;
+    size_t n = 0;
+    HostWords() = default;
+    HostWords(const HostWords&) = delete;
+    HostWords& operator=(const HostWords&) = delete;
+    ~HostWords() { reset(); }
+    int alloc(size_t bytes) {
+        DTC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        n = bytes;
+        return DTC_OK;
     }
+    void reset() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+    }
+    unsigned long long* word() const { return (unsigned long long*)p; }
+    double* status() const { return (double*)p + 8; }
 };
 
 // One batch of domains resident on the device: topology, vectors, scalars.
@@ -183,8 +195,9 @@ struct SolverBatch {
     int64_t graph_iters = -1;
     int graph_bricks = -1;
     int graph_mode = -1;           // block64 of the captured iterations
-    DevMem all_done_dev;           // int: 1 when every domain's done flag is set
-    HostFlags all_done_host;       // int [2]: copies of all_done_dev, one per launch parity
+    DevMem runs_dev;               // uint64: runs of iterations summarised so far
+    HostWords host_words;          // summary word and status of n_dom domains
+    uint64_t runs = 0;             // runs launched (host count)
     int graph_launches = 0;        // graph launches of the last solve (statistics)
 };
 
