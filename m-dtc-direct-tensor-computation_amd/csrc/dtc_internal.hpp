@@ -156,9 +156,10 @@ struct ClusterInfo {
 
 // New Chebyshev-Jacobi direction of one unknown, c1 d + c2 D^-1 (b - t) with t = (K x)
 // of the unknown: one expression for every kernel that forms it, so that a step fused
-// into an operator's epilogue rounds like the separate vector kernel
+// into an operator's epilogue rounds like the separate vector kernel (the fused
+// multiply-add is written out: left to contraction it may take either product)
 __device__ __forceinline__ float cheb_dir(float c1, float d, float c2, float di, float b, float t) {
-    return c1 * d + c2 * di * (b - t);
+    return __builtin_fmaf(c1, d, c2 * di * (b - t));
 }
 
 // 45 coefficients of the HEX08 element stiffness in the signed Walsh basis

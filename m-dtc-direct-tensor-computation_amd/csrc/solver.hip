@@ -169,7 +169,53 @@ inline bool cheb_fuse() {
 #include "ebe.hpp"
 
 // ---------------------------------------------------------------- vector kernels
-// per brick, thread t keeps load case t % 24
+// One workgroup per brick; a vector row is one (node, direction) pair holding the 24 load
+// cases.  Each thread takes 16 bytes of a row (VecN load cases) and keeps its load cases,
+// ROW_U rows at a time with their loads issued together: bounded by HBM, or by the
+// Infinity Cache for small batches.
+template <typename T> constexpr int VecN = 16 / (int)sizeof(T);
+template <typename T, int N> struct alignas(16) Vec {
+    T v[N];
+};
+template <typename T, int N> __device__ inline Vec<T, N> vload(const T* p) { return *reinterpret_cast<const Vec<T, N>*>(p); }
+template <typename T, int N> __device__ inline void vstore(T* p, const Vec<T, N>& a) { *reinterpret_cast<Vec<T, N>*>(p) = a; }
+constexpr int ROW_U = 4;
+
+// rows of the brick taken by this thread: row0, row0 + RPP, ... below row1; load cases lc0 ..
+template <int N> struct BrickRows {
+    static constexpr int LPR = R / N;          // threads per row
+    static constexpr int RPP = NT_UPD / LPR;   // rows per pass
+    int64_t row0, row1;
+    int lc0;
+    __device__ explicit BrickRows(const BrickInfo& B)
+        : row0((int64_t)B.node_begin * 3 + (int)threadIdx.x / LPR), row1((int64_t)B.node_end * 3),
+          lc0((int)threadIdx.x % LPR * N) {}
+    // f(row, u) for the rows of one group; groups of ROW_U rows
+    template <typename L, typename F> __device__ void each(L load, F use) const {
+        for (int64_t row = row0; row < row1; row += ROW_U * RPP) {
+#pragma unroll
+            for (int u = 0; u < ROW_U; ++u) load(min(row + u * RPP, row1 - 1), u);   // (the last row again past the end)
+#pragma unroll
+            for (int u = 0; u < ROW_U; ++u)
+                if (row + u * RPP < row1) use(row + u * RPP, u);
+        }
+    }
+    // out[lc] = sum over the brick's threads of acc, in a fixed order
+    __device__ void sum(const double (&acc)[N], double* s /* [RPP][R] */, double* __restrict__ out) const {
+        const int tid = threadIdx.x;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; ++k) s[tid / LPR * R + lc0 + k] = acc[k];
+        __syncthreads();
+        if (tid < R) {
+            double t = 0.0;
+#pragma unroll
+            for (int g = 0; g < RPP; ++g) t += s[g * R + tid];
+            out[tid] = t;
+        }
+    }
+};
+
 template <typename T>
 __global__ __launch_bounds__(NT_UPD) void k_cg_init(const BrickInfo* __restrict__ bricks, const int* __restrict__ done,
                                                     const int* __restrict__ active, T* __restrict__ x,
@@ -177,68 +223,96 @@ __global__ __launch_bounds__(NT_UPD) void k_cg_init(const BrickInfo* __restrict_
                                                     const T* __restrict__ dinv, double* __restrict__ prz,
                                                     double* __restrict__ prr, int zero_x, int set_p,
                                                     const int* __restrict__ keep_p, const T* __restrict__ zin) {
-    __shared__ double s1[NT_UPD], s2[NT_UPD];
+    constexpr int N = VecN<T>;
+    using V = Vec<T, N>;
+    using Rows = BrickRows<N>;
+    __shared__ double s_sum[Rows::RPP * R];
     const BrickInfo B = bricks[blockIdx.x];
-    const int tid = threadIdx.x, lc = tid % R;
-    double a1 = 0.0, a2 = 0.0;
+    const Rows rows(B);
+    double a1[N] = {}, a2[N] = {};
     if (!(done && done[B.dom])) {
-        const int act = active[B.dom * R + lc];
         // keep the search direction of a load case still iterating when its
         // residual was replaced; restart it otherwise
-        const int sp = set_p || !(keep_p && keep_p[B.dom * R + lc]);
-        const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-        for (int64_t i = tid; i < cnt; i += NT_UPD) {
-            int64_t idx = base + i;
-            T rv = r[idx];
-            T z = act ? (zin ? zin[idx] : rv * dinv[idx / R]) : T(0);
-            if (act && sp) p[idx] = z;
-            if (zero_x) x[idx] = T(0);
-            a1 += (double)rv * (double)z;
-            a2 += (double)rv * (double)rv;
+        bool act[N], sp[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int lc = B.dom * R + rows.lc0 + k;
+            act[k] = active[lc] != 0;
+            sp[k] = act[k] && (set_p || !(keep_p && keep_p[lc]));
         }
+        V rv[ROW_U], zv[ROW_U], pv[ROW_U];
+        T di[ROW_U];
+        rows.each([&](int64_t row, int u) {
+            const int64_t o = row * R + rows.lc0;
+            rv[u] = vload<T, N>(r + o);
+            pv[u] = vload<T, N>(p + o);
+            if (zin) zv[u] = vload<T, N>(zin + o);
+            else di[u] = dinv[row];
+        }, [&](int64_t row, int u) {
+            const int64_t o = row * R + rows.lc0;
+            V xz;
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const T z = act[k] ? (zin ? zv[u].v[k] : rv[u].v[k] * di[u]) : T(0);
+                if (sp[k]) pv[u].v[k] = z;
+                xz.v[k] = T(0);
+                a1[k] += (double)rv[u].v[k] * (double)z;
+                a2[k] += (double)rv[u].v[k] * (double)rv[u].v[k];
+            }
+            vstore(p + o, pv[u]);
+            if (zero_x) vstore(x + o, xz);
+        });
     }
-    s1[tid] = a1; s2[tid] = a2;
-    __syncthreads();
-    if (tid < R) {
-        double u = 0.0, v = 0.0;
-        for (int k = tid; k < NT_UPD; k += R) { u += s1[k]; v += s2[k]; }
-        prz[(int64_t)blockIdx.x * R + tid] = u;
-        prr[(int64_t)blockIdx.x * R + tid] = v;
-    }
+    rows.sum(a1, s_sum, prz + (int64_t)blockIdx.x * R);
+    rows.sum(a2, s_sum, prr + (int64_t)blockIdx.x * R);
 }
 
+// Three 33^3 domains in FP64 (40,000 nodes, 23 MB a vector, six of them moved): 36 -> 23.5 us
+// (5.9 TB/s) against one load case per thread; k_cg_dir, three vectors, 36 -> 12.5
 template <typename T>
 __global__ __launch_bounds__(NT_UPD) void k_cg_update(const BrickInfo* __restrict__ bricks, const int* __restrict__ done,
                                                       const double* __restrict__ alpha, T* __restrict__ x,
                                                       T* __restrict__ r, const T* __restrict__ p,
                                                       const T* __restrict__ q, const T* __restrict__ dinv,
                                                       double* __restrict__ prz, double* __restrict__ prr) {
-    __shared__ double s1[NT_UPD], s2[NT_UPD];
+    constexpr int N = VecN<T>;
+    using V = Vec<T, N>;
+    using Rows = BrickRows<N>;
+    __shared__ double s_sum[Rows::RPP * R];
     const BrickInfo B = bricks[blockIdx.x];
-    const int tid = threadIdx.x, lc = tid % R;
     if (done && done[B.dom]) return;
-    const T a = (T)alpha[B.dom * R + lc];
-    double a1 = 0.0, a2 = 0.0;
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = tid; i < cnt; i += NT_UPD) {
-        int64_t idx = base + i;
-        T rv = r[idx];
-        if (a != T(0)) {      // frozen load cases keep x and r
-            rv -= a * q[idx];
-            x[idx] += a * p[idx];
-            r[idx] = rv;
+    const Rows rows(B);
+    T a[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) a[k] = (T)alpha[B.dom * R + rows.lc0 + k];
+    double a1[N] = {}, a2[N] = {};
+    V xv[ROW_U], rv[ROW_U], pv[ROW_U], qv[ROW_U];
+    T di[ROW_U];
+    rows.each([&](int64_t row, int u) {
+        const int64_t o = row * R + rows.lc0;
+        rv[u] = vload<T, N>(r + o);
+        qv[u] = vload<T, N>(q + o);
+        xv[u] = vload<T, N>(x + o);
+        pv[u] = vload<T, N>(p + o);
+        di[u] = dinv[row];
+    }, [&](int64_t row, int u) {
+        const int64_t o = row * R + rows.lc0;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            T t = rv[u].v[k];
+            if (a[k] != T(0)) {      // frozen load cases keep x and r
+                t -= a[k] * qv[u].v[k];
+                xv[u].v[k] += a[k] * pv[u].v[k];
+                rv[u].v[k] = t;
+            }
+            a1[k] += (double)t * (double)(t * di[u]);
+            a2[k] += (double)t * (double)t;
         }
-        if (prz) a1 += (double)rv * (double)(rv * dinv[idx / R]);
-        a2 += (double)rv * (double)rv;
-    }
-    s1[tid] = a1; s2[tid] = a2;
-    __syncthreads();
-    if (tid < R) {
-        double u = 0.0, v = 0.0;
-        for (int k = tid; k < NT_UPD; k += R) { u += s1[k]; v += s2[k]; }
-        if (prz) prz[(int64_t)blockIdx.x * R + tid] = u;
-        prr[(int64_t)blockIdx.x * R + tid] = v;
-    }
+        vstore(x + o, xv[u]);
+        vstore(r + o, rv[u]);
+    });
+    if (prz) rows.sum(a1, s_sum, prz + (int64_t)blockIdx.x * R);
+    rows.sum(a2, s_sum, prr + (int64_t)blockIdx.x * R);
 }
 
 template <typename T>
@@ -246,15 +320,26 @@ __global__ __launch_bounds__(NT_UPD) void k_cg_dir(const BrickInfo* __restrict__
                                                    const double* __restrict__ beta, const T* __restrict__ r,
                                                    T* __restrict__ p, const T* __restrict__ dinv,
                                                    const T* __restrict__ zin) {
+    constexpr int N = VecN<T>;
+    using V = Vec<T, N>;
     const BrickInfo B = bricks[blockIdx.x];
     if (done && done[B.dom]) return;
-    const int tid = threadIdx.x, lc = tid % R;
-    const T b = (T)beta[B.dom * R + lc];
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = tid; i < cnt; i += NT_UPD) {
-        int64_t idx = base + i;
-        p[idx] = (zin ? zin[idx] : r[idx] * dinv[idx / R]) + b * p[idx];
-    }
+    const BrickRows<N> rows(B);
+    T b[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) b[k] = (T)beta[B.dom * R + rows.lc0 + k];
+    V zv[ROW_U], pv[ROW_U];
+    T di[ROW_U];
+    rows.each([&](int64_t row, int u) {
+        const int64_t o = row * R + rows.lc0;
+        zv[u] = vload<T, N>((zin ? zin : r) + o);
+        pv[u] = vload<T, N>(p + o);
+        di[u] = zin ? T(1) : dinv[row];
+    }, [&](int64_t row, int u) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) pv[u].v[k] = zv[u].v[k] * di[u] + b[k] * pv[u].v[k];
+        vstore(p + row * R + rows.lc0, pv[u]);
+    });
 }
 
 // ---------------------------------------------------------------- per-domain reductions (one block per domain)
@@ -411,12 +496,18 @@ __global__ __launch_bounds__(NT_UPD) void k_to32(const BrickInfo* __restrict__ b
                                                  float* __restrict__ x32, const double* __restrict__ rr) {
     const BrickInfo B = bricks[blockIdx.x];
     if (done[B.dom]) return;
-    const double sc = col_scale(rr, B.dom, threadIdx.x % R);      // NT_UPD is a multiple of 24
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = threadIdx.x; i < cnt; i += NT_UPD) {
-        r32[base + i] = (float)(r64[base + i] * sc);
-        if (x32) x32[base + i] = 0.f;
-    }
+    const BrickRows<4> rows(B);
+    double sc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sc[k] = col_scale(rr, B.dom, rows.lc0 + k);
+    Vec<double, 4> v[ROW_U];
+    rows.each([&](int64_t row, int u) { v[u] = vload<double, 4>(r64 + row * R + rows.lc0); }, [&](int64_t row, int u) {
+        Vec<float, 4> f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f.v[k] = (float)(v[u].v[k] * sc[k]);
+        vstore(r32 + row * R + rows.lc0, f);
+        if (x32) vstore(x32 + row * R + rows.lc0, Vec<float, 4>{});
+    });
 }
 
 // x64 += x32 (divided by its column scale when rr is given), x32 = 0 (group
@@ -426,12 +517,21 @@ __global__ __launch_bounds__(NT_UPD) void k_acc64(const BrickInfo* __restrict__ 
                                                   const double* __restrict__ rr) {
     const BrickInfo B = bricks[blockIdx.x];
     if (skip[B.dom]) return;
-    const double sc = 1.0 / col_scale(rr, B.dom, threadIdx.x % R);
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = threadIdx.x; i < cnt; i += NT_UPD) {
-        x64[base + i] += (double)x32[base + i] * sc;
-        x32[base + i] = 0.f;
-    }
+    const BrickRows<4> rows(B);
+    double sc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sc[k] = 1.0 / col_scale(rr, B.dom, rows.lc0 + k);
+    Vec<double, 4> v[ROW_U];
+    Vec<float, 4> f[ROW_U];
+    rows.each([&](int64_t row, int u) {
+        v[u] = vload<double, 4>(x64 + row * R + rows.lc0);
+        f[u] = vload<float, 4>(x32 + row * R + rows.lc0);
+    }, [&](int64_t row, int u) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[u].v[k] += (double)f[u].v[k] * sc[k];
+        vstore(x64 + row * R + rows.lc0, v[u]);
+        vstore(x32 + row * R + rows.lc0, Vec<float, 4>{});
+    });
 }
 
 // ---------------------------------------------------------------- block PCG
@@ -1500,37 +1600,42 @@ __global__ __launch_bounds__(NT_UPD) void k_cheb(const BrickInfo* __restrict__ b
                                                  const float* __restrict__ dinv, float* __restrict__ d,
                                                  float* __restrict__ x, float c1, float c2, int zero,
                                                  double* __restrict__ prz) {
-    __shared__ double s1[NT_UPD];
+    using V = Vec<float, 4>;
+    using Rows = BrickRows<4>;
+    __shared__ double s_sum[Rows::RPP * R];
     const BrickInfo B = bricks[blockIdx.x];
     if (done && done[B.dom]) return;
-    const int tid = threadIdx.x;
-    double a1 = 0.0;
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = tid; i < cnt; i += NT_UPD) {
-        const int64_t idx = base + i;
-        const float bv = b[idx];
-        const float di = dinv[idx / R];
-        float dv, xv;
-        if (zero) {
-            dv = c2 * di * bv;
-            xv = dv;
-        } else {
-            dv = cheb_dir(c1, d[idx], c2, di, bv, t[idx]);
-            xv = x[idx] + dv;
+    const Rows rows(B);
+    double a1[4] = {};
+    V bv[ROW_U], dv[ROW_U], tv[ROW_U], xv[ROW_U];
+    float di[ROW_U];
+    rows.each([&](int64_t row, int u) {
+        const int64_t o = row * R + rows.lc0;
+        bv[u] = vload<float, 4>(b + o);
+        di[u] = dinv[row];
+        if (!zero) {
+            dv[u] = vload<float, 4>(d + o);
+            tv[u] = vload<float, 4>(t + o);
+            xv[u] = vload<float, 4>(x + o);
         }
-        if (d) d[idx] = dv;
-        x[idx] = xv;
-        a1 += (double)bv * (double)xv;
-    }
-    if (prz) {
-        s1[tid] = a1;
-        __syncthreads();
-        if (tid < R) {
-            double u = 0.0;
-            for (int k = tid; k < NT_UPD; k += R) u += s1[k];
-            prz[(int64_t)blockIdx.x * R + tid] = u;
+    }, [&](int64_t row, int u) {
+        const int64_t o = row * R + rows.lc0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float bk = bv[u].v[k];
+            if (zero) {
+                dv[u].v[k] = c2 * di[u] * bk;
+                xv[u].v[k] = dv[u].v[k];
+            } else {
+                dv[u].v[k] = cheb_dir(c1, dv[u].v[k], c2, di[u], bk, tv[u].v[k]);
+                xv[u].v[k] += dv[u].v[k];
+            }
+            a1[k] += (double)bk * (double)xv[u].v[k];
         }
-    }
+        if (d) vstore(d + o, dv[u]);
+        vstore(x + o, xv[u]);
+    });
+    if (prz) rows.sum(a1, s_sum, prz + (int64_t)blockIdx.x * R);
 }
 
 // ---------------------------------------------------------------- p-multigrid transfers (HEX20 -> HEX08)
@@ -1599,20 +1704,22 @@ template <typename T>
 __global__ __launch_bounds__(NT_UPD) void k_dot(const BrickInfo* __restrict__ bricks, const int* __restrict__ done,
                                                 const T* __restrict__ a, const T* __restrict__ b,
                                                 double* __restrict__ part) {
-    __shared__ double s1[NT_UPD];
+    constexpr int N = VecN<T>;
+    using Rows = BrickRows<N>;
+    __shared__ double s_sum[Rows::RPP * R];
     const BrickInfo B = bricks[blockIdx.x];
     if (done && done[B.dom]) return;
-    const int tid = threadIdx.x;
-    double s = 0.0;
-    const int64_t base = (int64_t)B.node_begin * 3 * R, cnt = (int64_t)(B.node_end - B.node_begin) * 3 * R;
-    for (int64_t i = tid; i < cnt; i += NT_UPD) s += (double)a[base + i] * (double)b[base + i];
-    s1[tid] = s;
-    __syncthreads();
-    if (tid < R) {
-        double u = 0.0;
-        for (int k = tid; k < NT_UPD; k += R) u += s1[k];
-        part[(int64_t)blockIdx.x * R + tid] = u;
-    }
+    const Rows rows(B);
+    double acc[N] = {};
+    Vec<T, N> av[ROW_U], bv[ROW_U];
+    rows.each([&](int64_t row, int u) {
+        av[u] = vload<T, N>(a + row * R + rows.lc0);
+        bv[u] = vload<T, N>(b + row * R + rows.lc0);
+    }, [&](int64_t, int u) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc[k] += (double)av[u].v[k] * (double)bv[u].v[k];
+    });
+    rows.sum(acc, s_sum, part + (int64_t)blockIdx.x * R);
 }
 
 // x = Dirichlet values on the box-face nodes of each brick, unchanged elsewhere;
