@@ -12,7 +12,11 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
+#include <list>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -35,6 +39,119 @@ int set_error(int code, const char* fmt, ...) {
     va_end(ap);
     g_err = buf;
     return code;
+}
+
+// ---- pool of idle device and page-locked memory
+thread_local bool t_recycle = false;
+
+namespace {
+
+struct Pool {
+    using Clock = std::chrono::steady_clock;
+    struct Block {
+        void* p;
+        size_t n;
+        int dev;
+        Clock::time_point since;
+    };
+    std::mutex mu;
+    std::list<Block> idle;                                                         // newest first
+    std::multimap<std::pair<int, size_t>, std::list<Block>::iterator> by_size;
+    size_t bytes = 0;
+    std::vector<std::pair<void*, size_t>> pinned;
+
+    // unlinks the oldest blocks while over the bound or past their time; the caller frees them
+    void expire(std::vector<Block>& out, size_t bound) {
+        const Clock::time_point now = Clock::now();
+        while (!idle.empty() &&
+               (bytes > bound || std::chrono::duration<double>(now - idle.back().since).count() > POOL_SECONDS)) {
+            const auto last = std::prev(idle.end());
+            auto r = by_size.equal_range({last->dev, last->n});
+            while (r.first->second != last) ++r.first;
+            by_size.erase(r.first);
+            bytes -= last->n;
+            out.push_back(*last);
+            idle.erase(last);
+        }
+    }
+};
+
+// never destroyed: the runtime may be gone when static objects are
+Pool& pool() {
+    static Pool& p = *new Pool;
+    return p;
+}
+
+void free_blocks(const std::vector<Pool::Block>& v) {
+    for (const Pool::Block& b : v) (void)hipFree(b.p);
+}
+
+}  // namespace
+
+void* pool_take(size_t n, int dev) {
+    Pool& P = pool();
+    void* p = nullptr;
+    std::vector<Pool::Block> old;
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        const auto it = P.by_size.find({dev, n});
+        if (it != P.by_size.end()) {
+            p = it->second->p;
+            P.bytes -= n;
+            P.idle.erase(it->second);
+            P.by_size.erase(it);
+        }
+        P.expire(old, POOL_BYTES);
+    }
+    free_blocks(old);
+    return p;
+}
+
+void pool_put(void* p, size_t n, int dev) {
+    Pool& P = pool();
+    std::vector<Pool::Block> old;
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        P.idle.push_front({p, n, dev, Pool::Clock::now()});
+        P.by_size.emplace(std::make_pair(dev, n), P.idle.begin());
+        P.bytes += n;
+        P.expire(old, POOL_BYTES);
+    }
+    free_blocks(old);
+}
+
+void pool_trim() {
+    Pool& P = pool();
+    std::vector<Pool::Block> old;
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        P.expire(old, 0);
+    }
+    free_blocks(old);
+}
+
+void* pool_take_pinned(size_t n) {
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    for (size_t i = P.pinned.size(); i-- > 0;)
+        if (P.pinned[i].second == n) {
+            void* p = P.pinned[i].first;
+            P.pinned.erase(P.pinned.begin() + (ptrdiff_t)i);
+            return p;
+        }
+    return nullptr;
+}
+
+void pool_put_pinned(void* p, size_t n) {
+    Pool& P = pool();
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        if (n <= ((size_t)1 << 20) && P.pinned.size() < POOL_PINNED) {
+            P.pinned.emplace_back(p, n);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
 }
 
 namespace {
@@ -270,7 +387,7 @@ struct dtc_batch {
     // nodes stay below NODE_CAP (32-bit vector indexing); each sub-batch keeps
     // its topology and solutions for the sensitivity pass.
     struct Sub {
-        Stream own;                // the sub-batch's stream
+        Stream own;                // the sub-batch's stream (the first one uses the object's)
         SolverBatch sb;
         SolverBatch sb08;          // HEX20 micro elements: the HEX08 twin of the p-multigrid
         std::vector<double> ff;
@@ -343,9 +460,11 @@ int dtc_extract_block(const void* vol, int kind, const int64_t vdim[3], const in
         n[k] = xe_n[k] - xa_n[k] + 1;
         if (n[k] <= 0 || xa_n[k] < 1 || xe_n[k] > vdim[k]) return set_error(DTC_ERR_BAD_ARGUMENT, "block outside the volume");
     }
+    CallEnd end;
     Stream st;
-    DTC_TRY(st.create());
     DevMem dv, dout;
+    IdleOnExit idle{st.s};
+    DTC_TRY(st.create());
     const size_t vb = (size_t)vdim[0] * vdim[1] * vdim[2] * es, ob = (size_t)n[0] * n[1] * n[2] * es;
     DTC_TRY(dv.alloc(vb));
     DTC_TRY(dout.alloc(ob));
@@ -372,9 +491,11 @@ static int mesh_common(const void* phi, int kind, const int64_t n[3], int64_t ll
 int dtc_mesh_count(const void* phi, int kind, const int64_t n[3], int64_t llimit, int nen, int64_t* n_elems,
                    int64_t* n_nodes) {
     if (!n_elems || !n_nodes) return set_error(DTC_ERR_BAD_ARGUMENT, "NULL output");
-    MeshDev m;
+    CallEnd end;
     Stream st;
+    MeshDev m;
     DevMem dphi;
+    IdleOnExit idle{st.s};
     int rc = mesh_common(phi, kind, n, llimit, nen, m, st, dphi);
     if (rc == DTC_ERR_EMPTY_MESH) { *n_elems = 0; *n_nodes = 0; return rc; }
     DTC_TRY(rc);
@@ -387,14 +508,15 @@ int dtc_mesh_build(const void* phi, int kind, const int64_t n[3], int64_t llimit
                    const int64_t xa_n[3], int64_t elems_cap, int64_t nodes_cap, double* nodes, int64_t* elems,
                    int64_t* n_elems, int64_t* n_nodes) {
     if (!delta || !xa_n || !nodes || !elems || !n_elems || !n_nodes) return set_error(DTC_ERR_BAD_ARGUMENT, "NULL argument");
-    MeshDev m;
+    CallEnd end;
     Stream st;
-    DevMem dphi;
+    MeshDev m;
+    DevMem dphi, dn, de;
+    IdleOnExit idle{st.s};
     DTC_TRY(mesh_common(phi, kind, n, llimit, nen, m, st, dphi));
     if (m.n_elems > elems_cap || m.n_nodes > nodes_cap)
         return set_error(DTC_ERR_BAD_ARGUMENT, "mesh has %lld elements / %lld nodes, capacity %lld / %lld",
                          (long long)m.n_elems, (long long)m.n_nodes, (long long)elems_cap, (long long)nodes_cap);
-    DevMem dn, de;
     DTC_TRY(dn.alloc((size_t)m.n_nodes * 3 * 8));
     DTC_TRY(de.alloc((size_t)m.n_elems * nen * 8));
     DTC_TRY(mesh_write_outputs(m, delta, xa_n, dn.as<double>(), de.as<int64_t>(), st.s));
@@ -413,9 +535,11 @@ int dtc_boundaries(const double* nodes, int64_t n_nodes, const double min_c[3], 
     const int RM = macro_lcs(macro_order);
     if ((bnode_ids == nullptr) != (bvals == nullptr)) return set_error(DTC_ERR_BAD_ARGUMENT, "ids and values go together");
     DTC_TRY(check_device());
+    CallEnd end;
     Stream st;
-    DTC_TRY(st.create());
     DevMem dn, flag, pos, tmp, di, dv;
+    IdleOnExit idle{st.s};
+    DTC_TRY(st.create());
     DTC_TRY(dn.alloc((size_t)n_nodes * 3 * 8));
     DTC_HIP(hipMemcpyAsync(dn.p, nodes, (size_t)n_nodes * 3 * 8, hipMemcpyHostToDevice, st.s));
     int64_t nb = 0;
@@ -574,9 +698,12 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
     auto setup_sub = [&](int k, const std::vector<int>& list, int precision) -> int {
         while ((int)b->subs.size() <= k) b->subs.emplace_back(new dtc_batch::Sub);
         dtc_batch::Sub& S = *b->subs[k];
-        if (!S.own.s) DTC_TRY(S.own.create());
+        // the first sub-batch runs on the object's stream: with the three parts of a batch and
+        // the null stream, four streams share the four hardware queues (a fifth can put two
+        // parts on one queue: 40 domains of 21^3 61 or 70 ms, as the queues happened to fall)
+        if (k > 0 && !S.own.s) DTC_TRY(S.own.create());
         SolverBatch& sb = S.sb;
-        const hipStream_t s = S.own.s;
+        const hipStream_t s = k > 0 ? S.own.s : b->st.s;
         sb.stream = s;
         sb.nu = b->nu;
         sb.a = b->a0;
@@ -635,6 +762,7 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
             }
             DTC_TRY(batch_finalize(tw, DTC_FP32_REFINE));
         }
+        DTC_HIP(hipStreamSynchronize(s));   // the next sub-batch meshes into the same work space on its own stream
         return DTC_OK;
     };
     // one sub-batch, solve: multigrid hierarchy (unless built by prep_sub) -> solve -> reactions
@@ -889,9 +1017,13 @@ int dtc_batch_kernel_flops(dtc_batch* b, int kernel, double* avg_flops) {
 
 int dtc_batch_destroy(dtc_batch* b) {
     if (!b) return DTC_OK;
-    if (b->st.s) (void)hipStreamSynchronize(b->st.s);
-    for (const auto& S : b->subs)
+    // every stream of the object is waited for: its memory is idle
+    bool idle = b->st.s && hipStreamSynchronize(b->st.s) == hipSuccess;
+    for (const auto& S : b->subs) {
+        if (S->own.s && hipStreamSynchronize(S->own.s) != hipSuccess) idle = false;
         for (hipEvent_t e : S->sb.ev) (void)hipEventDestroy(e);
+    }
+    Recycle r(idle);
     delete b;
     return DTC_OK;
 }
@@ -925,7 +1057,9 @@ int dtc_rotation_search(const double EE[36], int criterion, double step_deg, dou
     if (!EE || !alpha || !n || !aa || !EE_opt) return set_error(DTC_ERR_BAD_ARGUMENT, "NULL argument");
     if (criterion != 1 && criterion != 2) return set_error(DTC_ERR_BAD_ARGUMENT, "criterion %d", criterion);
     DTC_TRY(check_device());
+    CallEnd end;
     Stream st;
+    IdleOnExit idle{st.s};
     DTC_TRY(st.create());
     std::vector<RotResult> rr;
     DTC_TRY(rotation_search_batch(EE, 1, step_deg, num_zero > 0.0 ? num_zero : 1e-9, st.s, rr));

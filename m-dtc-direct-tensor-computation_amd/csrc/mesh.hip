@@ -409,7 +409,7 @@ int mesh_build_device(const void* phi_dev, int kind, const int64_t n[3], int64_t
     DTC_TRY(m.newE.ensure(nvox * 4));
     DTC_TRY(m.numLat.ensure(nlat * 4));
     DTC_TRY(m.bbox.ensure(6 * 4));
-    DevMem flag;
+    DevMem& flag = m.flag;
     DTC_TRY(flag.ensure(nvox * 4));
 
     switch (kind) {

@@ -348,7 +348,9 @@ int rotation_search_batch(const double* EE_host, int n_dom, double step_deg, dou
     int64_t na, ne;
     int bpd;
     rotation_grid(step_deg, &na, &ne, &bpd);
+    CallEnd end;
     DevMem dEE, pv, pi_, best, besti, jobs;
+    IdleOnExit idle{s};
     DTC_TRY(dEE.alloc((size_t)n_dom * 36 * 8));
     DTC_TRY(pv.alloc((size_t)n_dom * bpd * 2 * 8));
     DTC_TRY(pi_.alloc((size_t)n_dom * bpd * 2 * 8));

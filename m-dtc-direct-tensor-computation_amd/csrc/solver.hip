@@ -1854,11 +1854,12 @@ int batch_begin(SolverBatch& b, const dtc_domain_desc* d, int64_t n_dom) {
     DTC_HIP(hipGetLastError());
     b.n_dom = 0; b.n_nodes = 0; b.n_lat = 0; b.n_vox = 0;
     b.h_dom.clear(); b.h_brick.clear(); b.h_elems.clear(); b.h_nodes.clear(); b.h_bnodes.clear(); b.h_status.clear();
-    b.d20.clear();
     b.h_contrast.clear();
     b.n_slices = 0;   // the block PCG slices follow the batch's domains (block_setup)
-    if (b.block_graph.e) DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(hipStreamSynchronize(b.stream));
     b.block_graph.reset();   // captured with the previous composition's buffers
+    Recycle idle(true);
+    b.d20.clear();
     return DTC_OK;
 }
 
@@ -1931,6 +1932,7 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
         DTC_HIP(hipGetLastError());
         DTC_HIP(hipMemcpyAsync(&hb, nbc.p, 4, hipMemcpyDeviceToHost, s));
         DTC_HIP(hipStreamSynchronize(s));
+        nbc.recycle();
         if (3 * hb < 6) {
             DTC_TRY(batch_add_empty(b, d, DTC_ERR_FEW_CONSTRAINTS, lc_base));
             b.h_elems.back() = m.n_elems;
@@ -1947,6 +1949,7 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
     std::vector<int> hc(nbr);
     DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)nbr * 4, hipMemcpyDeviceToHost, s));
     DTC_HIP(hipStreamSynchronize(s));
+    cnt.recycle();
     D.brick_begin = (int)b.h_brick.size();
     D.node_begin = b.n_nodes;
     int64_t node = b.n_nodes;
@@ -1975,7 +1978,8 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
                                                                    m.cref.as<int>(), Lx, Ly, Lz, D.lat_off, b.lat2node.as<int>(),
                                                                    b.sol2ref.as<int>());
         DTC_HIP(hipGetLastError());
-        DTC_HIP(hipStreamSynchronize(s));   // bl goes out of scope
+        DTC_HIP(hipStreamSynchronize(s));
+        bl.recycle();
     }
     k_emod<<<nb(nvox, 256), 256, 0, s>>>(m.keepE.as<int>(), modulus_dev, d.E, escale, nvox, b.emod.as<double>() + D.vox_off);
     DTC_HIP(hipGetLastError());
@@ -2099,7 +2103,8 @@ int build_clusters(hipStream_t s, Clusters& c, const DevMem& brick, const DevMem
                                               c.eown.as<uint2>(), fine ? c.eE64.as<double>() : nullptr,
                                               c.eE32.as<float>(), c.cap);
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(s));   // cnt goes out of scope
+    DTC_HIP(hipStreamSynchronize(s));
+    cnt.recycle();
     return DTC_OK;
 }
 
@@ -2145,7 +2150,7 @@ int batch_finalize(SolverBatch& b, int precision) {
     DTC_TRY(b.part_c.ensure(nbk * R * 8));
     DTC_TRY(b.part_ff.ensure(nbk * R * FFD * 8));
     const size_t nd = (size_t)(b.n_dom > 0 ? b.n_dom : 1);
-    for (DevMem* m : {&b.alpha, &b.beta, &b.rz, &b.rr, &b.rr0, &b.thr2, &b.scale}) DTC_TRY(m->alloc(nd * R * 8));
+    for (DevMem* m : {&b.alpha, &b.beta, &b.rz, &b.rr, &b.rr0, &b.thr2, &b.scale}) DTC_TRY(m->ensure(nd * R * 8));
     DTC_TRY(b.active.ensure(nd * R * 4));
     DTC_TRY(b.active64.ensure(nd * R * 4));
     DTC_TRY(b.active_prev.ensure(nd * R * 4));
@@ -2288,7 +2293,9 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
                                           C.lat2node.as<int>(), C.ptab.as<int>());
             DTC_HIP(hipGetLastError());
         }
-        DTC_HIP(hipStreamSynchronize(s));   // ex, cnt go out of scope
+        DTC_HIP(hipStreamSynchronize(s));
+        ex.recycle();
+        cnt.recycle();
     }
     return DTC_OK;
 }
@@ -3421,6 +3428,8 @@ int batch_fields(SolverBatch& b, int i, int ncol, double* u_out, double* r_out) 
     if (u_out) DTC_HIP(hipMemcpyAsync(u_out, du.p, bytes, hipMemcpyDeviceToHost, b.stream));
     if (r_out) DTC_HIP(hipMemcpyAsync(r_out, dr.p, bytes, hipMemcpyDeviceToHost, b.stream));
     DTC_HIP(hipStreamSynchronize(b.stream));
+    du.recycle();
+    dr.recycle();
     return DTC_OK;
 }
 
@@ -3447,6 +3456,7 @@ int batch_grad(SolverBatch& b, int i, int ng, const double* M, double* dL_dE_hos
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(dL_dE_host, g.p, (size_t)nvox * 8, hipMemcpyDeviceToHost, b.stream));
     DTC_HIP(hipStreamSynchronize(b.stream));
+    for (DevMem* m : {&h, &Md, &g}) m->recycle();
     return DTC_OK;
 }
 

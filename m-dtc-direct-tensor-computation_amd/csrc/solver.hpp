@@ -80,7 +80,7 @@ struct GraphExec {
 };
 
 // Page-locked host memory the device writes: a summary word, then each domain's status
-// (hipHostMalloc, freed with the owner).
+// (hipHostMalloc, given up with the owner).
 struct HostWords {
     void* p = nullptr;
     size_t n = 0;
@@ -89,12 +89,15 @@ struct HostWords {
     HostWords& operator=(const HostWords&) = delete;
     ~HostWords() { reset(); }
     int alloc(size_t bytes) {
-        DTC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        bytes = pool_size(bytes);
+        p = pool_take_pinned(bytes);
+        if (!p) DTC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
         n = bytes;
         return DTC_OK;
     }
     void reset() {
-        if (p) (void)hipHostFree(p);
+        if (p && t_recycle) pool_put_pinned(p, n);
+        else if (p) (void)hipHostFree(p);
         p = nullptr;
         n = 0;
     }

@@ -536,7 +536,8 @@ int batch_add_domain20(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& 
     D.vox_off = b.n_vox;
     G.node_begin = b.n_nodes;
     G.n_nodes = nn;
-    DTC_HIP(hipStreamSynchronize(s));   // temporaries go out of scope
+    DTC_HIP(hipStreamSynchronize(s));
+    for (DevMem* t : {&e64, &dimd, &cnt, &cursor}) t->recycle();
     b.d20.push_back(std::move(G));
     b.h_dom.push_back(D);
     b.n_nodes += nn;
@@ -688,6 +689,7 @@ int grad20(SolverBatch& b, int i, int ng, const double* M, double* dL_dE_host) {
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(dL_dE_host, g.p, (size_t)nvox * 8, hipMemcpyDeviceToHost, s));
     DTC_HIP(hipStreamSynchronize(s));
+    for (DevMem* m : {&h, &Md, &g}) m->recycle();
     return DTC_OK;
 }
 
