@@ -135,8 +135,7 @@ __global__ __launch_bounds__(NT) void k_sweep(const double* __restrict__ EE, int
 }
 
 __global__ __launch_bounds__(NT) void k_sweep_reduce(const double* __restrict__ pv, const int64_t* __restrict__ pi,
-                                                     int blocks_per_dom, double* __restrict__ best,
-                                                     int64_t* __restrict__ besti) {
+                                                     int blocks_per_dom, int64_t na, RotState* __restrict__ st) {
     __shared__ double sv[NT];
     __shared__ int64_t si[NT];
     const int dom = blockIdx.x >> 1, c = blockIdx.x & 1;
@@ -147,30 +146,77 @@ __global__ __launch_bounds__(NT) void k_sweep_reduce(const double* __restrict__ 
         if (better(pv[k], pi[k], v, i)) { v = pv[k]; i = pi[k]; }
     }
     block_argmin(v, i, sv, si);
-    if (threadIdx.x == 0) { best[blockIdx.x] = v; besti[blockIdx.x] = i; }
+    if (threadIdx.x == 0) {
+        RotState S{};
+        S.ang[0] = i % na;
+        S.ang[1] = (i / na) % na;
+        S.ang[2] = i / (na * na);
+        S.prev = v;
+        S.jj = 1;
+        S.active = 1;
+        st[blockIdx.x] = S;
+    }
 }
 
-// one refinement step for each active (domain, criterion) job: 21^3 points
-// from start s0 with spacing div, criterion 1 normalises n, criterion 2 not
-__global__ __launch_bounds__(NT) void k_refine(const double* __restrict__ EE, const RotJob* __restrict__ jobs,
-                                               double* __restrict__ best, int64_t* __restrict__ besti) {
+// ---- refinements
+// All of them are launched in a row without a host decision between them, REF_B workgroups
+// a job, one point a thread: the workgroups of refinement jj first close refinement jj - 1
+// (the minimum over its workgroups, the stopping rule; every workgroup of a job by itself,
+// the first one stores the new state), so that a refinement is one launch, and one of a
+// job that has stopped an early exit.  Latency bounds the chain: one search on a 1-degree
+// grid took 1.25 ms with one workgroup a job (69 us a refinement) and a host decision after
+// each, 0.32 ms now, 0.1 of it the sweep.
+constexpr int REF_N = 21 * 21 * 21, REF_B = (REF_N + NT - 1) / NT;
+static_assert(REF_B <= 64, "one wave closes a refinement");
+
+// closes refinement jj (>= 1) of a job: minimum over its REF_B workgroup minima
+__device__ inline void refine_close(RotState& S, const double* __restrict__ pv, const int64_t* __restrict__ pi, int64_t jj,
+                                    double num_zero) {
+    const int lane = threadIdx.x & 63;
+    double v = lane < REF_B ? pv[lane] : INFINITY;
+    int64_t i = lane < REF_B ? pi[lane] : INT64_MAX;
+    for (int w = 32; w > 0; w >>= 1) {
+        const double ov = __shfl_xor(v, w);
+        const int64_t oi = __shfl_xor((long long)i, w);
+        if (better(ov, oi, v, i)) { v = ov; i = oi; }
+    }
+    S.ang[0] = S.s0[0] + i % 21;
+    S.ang[1] = S.s0[1] + (i / 21) % 21;
+    S.ang[2] = S.s0[2] + i / 441;
+    S.jj = jj;
+    S.crit = v;
+    if (fabs(S.prev - v) < num_zero || jj >= 16) S.active = 0;
+    S.prev = v;
+}
+
+// Refinement jj of each active (domain, criterion) job: 21^3 points around its best point
+// with spacing div, criterion 1 normalises n, criterion 2 not.  Minima and states are
+// double-buffered.  jj = 17 only closes refinement 16.
+__global__ __launch_bounds__(NT) void k_refine(const double* __restrict__ EE, const RotState* __restrict__ st_in,
+                                               RotState* __restrict__ st_out, const double* __restrict__ pv_in,
+                                               const int64_t* __restrict__ pi_in, double* __restrict__ pv_out,
+                                               int64_t* __restrict__ pi_out, int64_t jj, double div, double num_zero) {
     __shared__ double sv[NT];
     __shared__ int64_t si[NT];
-    const RotJob J = jobs[blockIdx.x];
-    if (!J.active) return;
-    const double* E = EE + 36 * J.dom;
+    const int job = blockIdx.x / REF_B, blk = blockIdx.x % REF_B;
+    RotState S = st_in[job];
+    if (S.active && jj > 1) refine_close(S, pv_in + (int64_t)job * REF_B, pi_in + (int64_t)job * REF_B, jj - 1, num_zero);
+    for (int c = 0; c < 3; ++c) S.s0[c] = (S.ang[c] - 1) * 10;
+    if (blk == 0 && threadIdx.x == 0) st_out[job] = S;
+    if (!S.active) return;
+    const double* E = EE + 36 * (job >> 1);
+    const bool cr1 = (job & 1) == 0;
     double bv = INFINITY;
     int64_t bi = INT64_MAX;
-    for (int idx = threadIdx.x; idx < 21 * 21 * 21; idx += NT) {
+    for (int idx = blk * NT + threadIdx.x; idx < REF_N; idx += REF_B * NT) {
         int ia = idx % 21, ip = (idx / 21) % 21, ie = idx / 441;
         double t[12];
-        rot_point(E, (double)(J.s0[0] + ia) * J.div, (double)(J.s0[1] + ip) * J.div, (double)(J.s0[2] + ie) * J.div,
-                  J.criterion == 1, t);
-        double c = J.criterion == 1 ? crit1(t) : crit2(t);
+        rot_point(E, (double)(S.s0[0] + ia) * div, (double)(S.s0[1] + ip) * div, (double)(S.s0[2] + ie) * div, cr1, t);
+        double c = cr1 ? crit1(t) : crit2(t);
         if (better(c, idx, bv, bi)) { bv = c; bi = idx; }
     }
     block_argmin(bv, bi, sv, si);
-    if (threadIdx.x == 0) { best[blockIdx.x] = bv; besti[blockIdx.x] = bi; }
+    if (threadIdx.x == 0) { pv_out[blockIdx.x] = bv; pi_out[blockIdx.x] = bi; }
 }
 
 // host copies of rot_alg / tra_R6 / congruence for the final outputs
@@ -258,16 +304,17 @@ void rotation_finish(const double EE[36], const int64_t ang[3], int64_t jj, doub
     for (int k = 0; k < 9; ++k) out.aa[k] = aa[k];
 }
 
-// Device buffers of one search: n_dom 6x6 tensors, per-block sweep minima
-// (bpd per domain and criterion), per-job minima and the refinement jobs.
+// Device buffers of one search: n_dom 6x6 tensors, per-block sweep minima (bpd per domain
+// and criterion), per-block refinement minima and job states (both double-buffered).
 struct RotBufs {
     double* EE;
     double* pv;
     int64_t* pi;
-    double* best;
-    int64_t* besti;
-    RotJob* jobs;
+    double* rv;
+    int64_t* ri;
+    RotState* st;
 };
+constexpr size_t rot_ref_count(size_t n_dom) { return 2 * 2 * n_dom * REF_B; }
 
 // Grid sizes of the initial sweep for an initial step of step_deg degrees.
 void rotation_grid(double step_deg, int64_t* na, int64_t* ne, int* bpd) {
@@ -277,65 +324,34 @@ void rotation_grid(double step_deg, int64_t* na, int64_t* ne, int* bpd) {
     *bpd = (int)((npts + (int64_t)NT * PPT - 1) / ((int64_t)NT * PPT));
 }
 
-// The search on caller-provided device buffers and host state (hb, prev: 2 n_dom
-// doubles; hbi, jjv: 2 n_dom int64; ang: 6 n_dom int64; J: 2 n_dom jobs), so that
-// a caller without device or host allocations can run it.
+// The search on caller-provided device buffers and host states (2 n_dom), so that a caller
+// without device or host allocations can run it.
 int rotation_search_core(const double* EE_host, int n_dom, double step_deg, double num_zero, hipStream_t s,
-                         const RotBufs& d, double* hb, int64_t* hbi, double* prev, int64_t* jjv, int64_t* ang,
-                         RotJob* J, RotResult* out) {
+                         const RotBufs& d, RotState* J, RotResult* out) {
     const double pi = std::acos(-1.0), pi_div_180 = pi / 180.0;
     int64_t na, ne;
     int bpd;
     rotation_grid(step_deg, &na, &ne, &bpd);
+    const int jobs = n_dom * 2;
+    const size_t nr = (size_t)jobs * REF_B;
     DTC_HIP(hipMemcpyAsync(d.EE, EE_host, (size_t)n_dom * 36 * 8, hipMemcpyHostToDevice, s));
     k_sweep<<<(unsigned)(n_dom * bpd), NT, 0, s>>>(d.EE, na, ne, step_deg * pi_div_180, bpd, d.pv, d.pi);
-    k_sweep_reduce<<<(unsigned)(n_dom * 2), NT, 0, s>>>(d.pv, d.pi, bpd, d.best, d.besti);
-    DTC_HIP(hipGetLastError());
-    DTC_HIP(hipMemcpyAsync(hb, d.best, (size_t)n_dom * 2 * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipMemcpyAsync(hbi, d.besti, (size_t)n_dom * 2 * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
-    // refinement state per job (dom, criterion)
-    for (int k = 0; k < n_dom * 2; ++k) {
-        const int64_t idx = hbi[k];
-        ang[3 * k] = idx % na; ang[3 * k + 1] = (idx / na) % na; ang[3 * k + 2] = idx / (na * na);
-        prev[k] = hb[k];
-        jjv[k] = 1;
-        out[k] = RotResult{};
-        J[k] = RotJob{};
-        J[k].dom = k / 2; J[k].criterion = 1 + (k & 1); J[k].active = 1;
-    }
+    k_sweep_reduce<<<(unsigned)jobs, NT, 0, s>>>(d.pv, d.pi, bpd, na, d.st);
     double div = pi_div_180 * step_deg;
-    for (int jj = 1; jj <= 16; ++jj) {
+    for (int jj = 1; jj <= 17; ++jj) {
         div = div * 0.1;
-        bool any = false;
-        for (int k = 0; k < n_dom * 2; ++k) {
-            if (!J[k].active) continue;
-            any = true;
-            for (int c = 0; c < 3; ++c) J[k].s0[c] = (ang[3 * k + c] - 1) * 10;
-            J[k].div = div;
-        }
-        if (!any) break;
-        DTC_HIP(hipMemcpyAsync(d.jobs, J, (size_t)n_dom * 2 * sizeof(RotJob), hipMemcpyHostToDevice, s));
-        k_refine<<<(unsigned)(n_dom * 2), NT, 0, s>>>(d.EE, d.jobs, d.best, d.besti);
-        DTC_HIP(hipGetLastError());
-        DTC_HIP(hipMemcpyAsync(hb, d.best, (size_t)n_dom * 2 * 8, hipMemcpyDeviceToHost, s));
-        DTC_HIP(hipMemcpyAsync(hbi, d.besti, (size_t)n_dom * 2 * 8, hipMemcpyDeviceToHost, s));
-        DTC_HIP(hipStreamSynchronize(s));
-        for (int k = 0; k < n_dom * 2; ++k) {
-            if (!J[k].active) continue;
-            const int64_t i = hbi[k];
-            ang[3 * k] = J[k].s0[0] + i % 21;
-            ang[3 * k + 1] = J[k].s0[1] + (i / 21) % 21;
-            ang[3 * k + 2] = J[k].s0[2] + i / 441;
-            jjv[k] = jj;
-            out[k].crit = hb[k];
-            if (std::fabs(prev[k] - hb[k]) < num_zero || jj >= 16) J[k].active = 0;
-            prev[k] = hb[k];
-        }
+        const int in = (jj - 1) & 1, to = jj & 1;
+        k_refine<<<(unsigned)(jobs * REF_B), NT, 0, s>>>(d.EE, d.st + in * jobs, d.st + to * jobs, d.rv + in * nr,
+                                                        d.ri + in * nr, d.rv + to * nr, d.ri + to * nr, jj, div, num_zero);
     }
-    for (int k = 0; k < n_dom * 2; ++k) {
-        out[k].jj = jjv[k];
-        rotation_finish(EE_host + 36 * (k / 2), &ang[3 * k], jjv[k], step_deg, out[k]);
+    DTC_HIP(hipGetLastError());
+    DTC_HIP(hipMemcpyAsync(J, d.st + jobs, (size_t)jobs * sizeof(RotState), hipMemcpyDeviceToHost, s));
+    DTC_HIP(hipStreamSynchronize(s));
+    for (int k = 0; k < jobs; ++k) {
+        out[k] = RotResult{};
+        out[k].crit = J[k].crit;
+        out[k].jj = J[k].jj;
+        rotation_finish(EE_host + 36 * (k / 2), J[k].ang, J[k].jj, step_deg, out[k]);
     }
     return DTC_OK;
 }
@@ -349,21 +365,18 @@ int rotation_search_batch(const double* EE_host, int n_dom, double step_deg, dou
     int bpd;
     rotation_grid(step_deg, &na, &ne, &bpd);
     CallEnd end;
-    DevMem dEE, pv, pi_, best, besti, jobs;
+    DevMem dEE, pv, pi_, rv, ri, st;
     IdleOnExit idle{s};
     DTC_TRY(dEE.alloc((size_t)n_dom * 36 * 8));
     DTC_TRY(pv.alloc((size_t)n_dom * bpd * 2 * 8));
     DTC_TRY(pi_.alloc((size_t)n_dom * bpd * 2 * 8));
-    DTC_TRY(best.alloc((size_t)n_dom * 2 * 8));
-    DTC_TRY(besti.alloc((size_t)n_dom * 2 * 8));
-    DTC_TRY(jobs.alloc((size_t)n_dom * 2 * sizeof(RotJob)));
-    const RotBufs d{dEE.as<double>(), pv.as<double>(), pi_.as<int64_t>(), best.as<double>(), besti.as<int64_t>(),
-                    jobs.as<RotJob>()};
-    std::vector<double> hb(n_dom * 2), prev(n_dom * 2);
-    std::vector<int64_t> hbi(n_dom * 2), jjv(n_dom * 2), ang(n_dom * 2 * 3);
-    std::vector<RotJob> J(n_dom * 2);
-    return rotation_search_core(EE_host, n_dom, step_deg, num_zero, s, d, hb.data(), hbi.data(), prev.data(),
-                                jjv.data(), ang.data(), J.data(), out.data());
+    DTC_TRY(rv.alloc(rot_ref_count(n_dom) * 8));
+    DTC_TRY(ri.alloc(rot_ref_count(n_dom) * 8));
+    DTC_TRY(st.alloc((size_t)n_dom * 4 * sizeof(RotState)));
+    const RotBufs d{dEE.as<double>(), pv.as<double>(), pi_.as<int64_t>(), rv.as<double>(), ri.as<int64_t>(),
+                    st.as<RotState>()};
+    std::vector<RotState> J((size_t)n_dom * 2);
+    return rotation_search_core(EE_host, n_dom, step_deg, num_zero, s, d, J.data(), out.data());
 }
 
 // ---------------------------------------------------------------- no-allocation search
@@ -381,7 +394,8 @@ void* g_scratch_ptr[MAX_DEVICES] = {};
 // byte offsets of the buffers in the work space (one domain, 256-byte aligned)
 constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 size_t rot_scratch_layout(int bpd, size_t off[6]) {
-    const size_t sz[6] = {36 * 8, (size_t)bpd * 2 * 8, (size_t)bpd * 2 * 8, 2 * 8, 2 * 8, 2 * sizeof(RotJob)};
+    const size_t sz[6] = {36 * 8, (size_t)bpd * 2 * 8, (size_t)bpd * 2 * 8, rot_ref_count(1) * 8, rot_ref_count(1) * 8,
+                          4 * sizeof(RotState)};
     size_t o = 0;
     for (int k = 0; k < 6; ++k) {
         off[k] = o;
@@ -435,12 +449,10 @@ int rotation_search_noalloc(const double EE[36], double step_deg, double num_zer
     unsigned char* b = static_cast<unsigned char*>(base);
     const RotBufs d{reinterpret_cast<double*>(b + off[0]), reinterpret_cast<double*>(b + off[1]),
                     reinterpret_cast<int64_t*>(b + off[2]), reinterpret_cast<double*>(b + off[3]),
-                    reinterpret_cast<int64_t*>(b + off[4]), reinterpret_cast<RotJob*>(b + off[5])};
-    double hb[2], prev[2];
-    int64_t hbi[2], jjv[2], ang[6];
-    RotJob J[2];
+                    reinterpret_cast<int64_t*>(b + off[4]), reinterpret_cast<RotState*>(b + off[5])};
+    RotState J[2];
     // the null stream: no stream object is created
-    return rotation_search_core(EE, 1, step_deg, num_zero, nullptr, d, hb, hbi, prev, jjv, ang, J, out);
+    return rotation_search_core(EE, 1, step_deg, num_zero, nullptr, d, J, out);
 }
 
 }  // namespace dtc
