@@ -136,6 +136,37 @@ struct DevMem {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Page-locked host memory that the device writes, given up with the owner.  The solver keeps
+// a summary word and then each domain's status in it.
+struct HostWords {
+    void* p = nullptr;
+    size_t n = 0;
+    HostWords() = default;
+    HostWords(const HostWords&) = delete;
+    HostWords& operator=(const HostWords&) = delete;
+    ~HostWords() { reset(); }
+    int alloc(size_t bytes) {
+        bytes = pool_size(bytes);
+        p = pool_take_pinned(bytes);
+        if (!p) DTC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        n = bytes;
+        return DTC_OK;
+    }
+    void reset() {
+        if (p && t_recycle) pool_put_pinned(p, n);
+        else if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+    }
+    // as DevMem::recycle
+    void recycle() {
+        Recycle r(true);
+        reset();
+    }
+    unsigned long long* word() const { return (unsigned long long*)p; }
+    double* status() const { return (double*)p + 8; }
+};
+
 // ---------------------------------------------------------------- constants
 constexpr int R24 = 24;          // load cases of the HEX08 macro element
 constexpr int BX = 8, BY = 4, BZ = 4;   // owned nodes of one solver brick
@@ -169,6 +200,8 @@ struct MeshDev {
     DevMem keepN;     // int32 per node number
     DevMem cref;      // int32 per node number: kept node number - 1
     DevMem bbox;      // int32[6]
+    DevMem tot;       // int32[4]: counts of the four scans
+    HostWords words;  // the same on the host
     DevMem scratch;   // scan temp storage
 };
 

@@ -73,8 +73,8 @@ int boundaries_device(const double* nodes_dev, int64_t n, const double mn[3], co
                       int order, int64_t* n_b, int64_t* ids_dev, double* vals_dev, DevMem& flag, DevMem& pos,
                       DevMem& tmp, hipStream_t s) {
     if (n <= 0) { *n_b = 0; return DTC_OK; }
-    DTC_TRY(flag.alloc((size_t)n * 4));
-    DTC_TRY(pos.alloc((size_t)n * 4));
+    DTC_TRY(flag.ensure((size_t)n * 4));
+    DTC_TRY(pos.ensure((size_t)n * 4));
     const unsigned g = (unsigned)((n + NT - 1) / NT);
     k_bc_flag<<<g, NT, 0, s>>>(nodes_dev, n, mn[0], mn[1], mn[2], mx[0], mx[1], mx[2], dim[0], dim[1], dim[2], flag.as<int>());
     DTC_HIP(hipGetLastError());

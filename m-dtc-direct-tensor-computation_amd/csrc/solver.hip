@@ -1098,20 +1098,24 @@ __global__ void k_fill_i64(int64_t* __restrict__ a, int64_t n, int64_t v) {
 }
 
 // ---------------------------------------------------------------- topology
+// nodes of every brick of the lattice, and those on the box faces (page-locked host memory)
 __global__ void k_brick_count(const int* __restrict__ numLat, const int* __restrict__ keepN, int Lx, int Ly,
-                              int Lz, int bnx, int bny, int* __restrict__ cnt) {
-    __shared__ int s;
+                              int Lz, int bnx, int bny, int2* __restrict__ cnt) {
+    __shared__ int s[2];
     const int b = blockIdx.x, t = threadIdx.x;     // blockDim = BX*BY*BZ
-    if (t == 0) s = 0;
+    if (t < 2) s[t] = 0;
     __syncthreads();
     const int bx = b % bnx, by = (b / bnx) % bny, bz = b / (bnx * bny);
     const int gx = bx * BX + t % BX, gy = by * BY + (t / BX) % BY, gz = bz * BZ + t / (BX * BY);
     if (gx < Lx && gy < Ly && gz < Lz) {
         int num = numLat[gx + Lx * (gy + Ly * gz)];
-        if (num > 0 && keepN[num - 1]) atomicAdd(&s, 1);
+        if (num > 0 && keepN[num - 1]) {
+            atomicAdd(&s[0], 1);
+            if (gx == 0 || gy == 0 || gz == 0 || gx == Lx - 1 || gy == Ly - 1 || gz == Lz - 1) atomicAdd(&s[1], 1);
+        }
     }
     __syncthreads();
-    if (t == 0) cnt[b] = s;
+    if (t == 0) cnt[b] = make_int2(s[0], s[1]);
 }
 
 __global__ void k_brick_assign(const BrickInfo* __restrict__ bl, int brick0, const int* __restrict__ numLat,
@@ -1136,22 +1140,6 @@ __global__ void k_brick_assign(const BrickInfo* __restrict__ bl, int brick0, con
         lat2node[lat_off + gx + (int64_t)Lx * (gy + (int64_t)Ly * gz)] = s;
         sol2ref[s] = cref[num - 1] + 1;
     }
-}
-
-__global__ void k_count_bc(const int* __restrict__ numLat, const int* __restrict__ keepN, int Lx, int Ly, int Lz,
-                           int* __restrict__ out) {
-    __shared__ int c;
-    if (threadIdx.x == 0) c = 0;
-    __syncthreads();
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < (int64_t)Lx * Ly * Lz) {
-        int x = p % Lx, y = (p / Lx) % Ly, z = p / ((int64_t)Lx * Ly);
-        int num = numLat[p];
-        if (num > 0 && keepN[num - 1] && (x == 0 || y == 0 || z == 0 || x == Lx - 1 || y == Ly - 1 || z == Lz - 1))
-            atomicAdd(&c, 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && c) atomicAdd(out, c);
 }
 
 // element modulus of every voxel; escale folds a domain's edge length a into
@@ -1922,34 +1910,27 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
         D.min_c[k] = (double)(d.xa_n[k] - 1) * d.delta[k];
         D.max_c[k] = (double)(d.xa_n[k] + d.n[k] - 1) * d.delta[k];
     }
-    {   // boundary nodes: fewer than 6 constrained DOFs fails the domain (f-src/mod_struct_preprocess.f90:471-473)
-        DevMem nbc;
-        DTC_TRY(nbc.alloc(4));
-        int zero = 0, hb = 0;
-        DTC_HIP(hipMemcpyAsync(nbc.p, &zero, 4, hipMemcpyHostToDevice, s));
-        const int64_t nl = (int64_t)Lx * Ly * Lz;
-        k_count_bc<<<nb(nl, 256), 256, 0, s>>>(m.numLat.as<int>(), m.keepN.as<int>(), Lx, Ly, Lz, nbc.as<int>());
-        DTC_HIP(hipGetLastError());
-        DTC_HIP(hipMemcpyAsync(&hb, nbc.p, 4, hipMemcpyDeviceToHost, s));
-        DTC_HIP(hipStreamSynchronize(s));
-        nbc.recycle();
-        if (3 * hb < 6) {
-            DTC_TRY(batch_add_empty(b, d, DTC_ERR_FEW_CONSTRAINTS, lc_base));
-            b.h_elems.back() = m.n_elems;
-            b.h_nodes.back() = m.n_nodes;
-            b.h_bnodes.back() = hb;
-            return DTC_OK;
-        }
-        b.h_bnodes.push_back(hb);
-    }
-    DevMem cnt;
-    DTC_TRY(cnt.alloc((size_t)nbr * 4));
-    k_brick_count<<<nbr, BX * BY * BZ, 0, s>>>(m.numLat.as<int>(), m.keepN.as<int>(), Lx, Ly, Lz, D.bnx, D.bny, cnt.as<int>());
+    HostWords cnt;
+    DTC_TRY(cnt.alloc((size_t)nbr * sizeof(int2)));
+    k_brick_count<<<nbr, BX * BY * BZ, 0, s>>>(m.numLat.as<int>(), m.keepN.as<int>(), Lx, Ly, Lz, D.bnx, D.bny, (int2*)cnt.p);
     DTC_HIP(hipGetLastError());
-    std::vector<int> hc(nbr);
-    DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)nbr * 4, hipMemcpyDeviceToHost, s));
     DTC_HIP(hipStreamSynchronize(s));
+    std::vector<int> hc(nbr);
+    int64_t hb = 0;
+    for (int i = 0; i < nbr; ++i) {
+        hc[i] = ((const int2*)cnt.p)[i].x;
+        hb += ((const int2*)cnt.p)[i].y;
+    }
     cnt.recycle();
+    // boundary nodes: fewer than 6 constrained DOFs fails the domain (f-src/mod_struct_preprocess.f90:471-473)
+    if (3 * hb < 6) {
+        DTC_TRY(batch_add_empty(b, d, DTC_ERR_FEW_CONSTRAINTS, lc_base));
+        b.h_elems.back() = m.n_elems;
+        b.h_nodes.back() = m.n_nodes;
+        b.h_bnodes.back() = hb;
+        return DTC_OK;
+    }
+    b.h_bnodes.push_back(hb);
     D.brick_begin = (int)b.h_brick.size();
     D.node_begin = b.n_nodes;
     int64_t node = b.n_nodes;
@@ -1970,20 +1951,19 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
     D.lat_off = b.n_lat;
     D.vox_off = b.n_vox;
     const int64_t nvox = (int64_t)m.nx * m.ny * m.nz;
+    DevMem bl;
     if (!mine.empty()) {
-        DevMem bl;
         DTC_TRY(bl.alloc(mine.size() * sizeof(BrickInfo)));
         DTC_HIP(hipMemcpyAsync(bl.p, mine.data(), mine.size() * sizeof(BrickInfo), hipMemcpyHostToDevice, s));
         k_brick_assign<<<(unsigned)mine.size(), BX * BY * BZ, 0, s>>>(bl.as<BrickInfo>(), 0, m.numLat.as<int>(), m.keepN.as<int>(),
                                                                    m.cref.as<int>(), Lx, Ly, Lz, D.lat_off, b.lat2node.as<int>(),
                                                                    b.sol2ref.as<int>());
         DTC_HIP(hipGetLastError());
-        DTC_HIP(hipStreamSynchronize(s));
-        bl.recycle();
     }
     k_emod<<<nb(nvox, 256), 256, 0, s>>>(m.keepE.as<int>(), modulus_dev, d.E, escale, nvox, b.emod.as<double>() + D.vox_off);
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipStreamSynchronize(s));
+    bl.recycle();
     b.h_brick.insert(b.h_brick.end(), mine.begin(), mine.end());
     b.h_dom.push_back(D);
     b.n_nodes = node;

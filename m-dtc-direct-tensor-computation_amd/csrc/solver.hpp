@@ -79,32 +79,6 @@ struct GraphExec {
     }
 };
 
-// Page-locked host memory the device writes: a summary word, then each domain's status
-// (hipHostMalloc, given up with the owner).
-struct HostWords {
-    void* p = nullptr;
-    size_t n = 0;
-    HostWords() = default;
-    HostWords(const HostWords&) = delete;
-    HostWords& operator=(const HostWords&) = delete;
-    ~HostWords() { reset(); }
-    int alloc(size_t bytes) {
-        bytes = pool_size(bytes);
-        p = pool_take_pinned(bytes);
-        if (!p) DTC_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
-        n = bytes;
-        return DTC_OK;
-    }
-    void reset() {
-        if (p && t_recycle) pool_put_pinned(p, n);
-        else if (p) (void)hipHostFree(p);
-        p = nullptr;
-        n = 0;
-    }
-    unsigned long long* word() const { return (unsigned long long*)p; }
-    double* status() const { return (double*)p + 8; }
-};
-
 // One batch of domains resident on the device: topology, vectors, scalars.
 struct SolverBatch {
     int n_dom = 0;
