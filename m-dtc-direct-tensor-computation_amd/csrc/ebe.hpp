@@ -305,3 +305,103 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
         }
     }
 }
+
+// ---------------------------------------------------------------- coarsest level
+// All m steps of the coarsest level's Chebyshev-Jacobi pass from x = 0 in one launch: one
+// workgroup per (domain, load case), everything in LDS and registers.  A step is two
+// passes: thread v forms the forces of voxel v into s_y, then thread t (a lattice node)
+// sums its up to 8 corners in ascending order of voxel offset and updates its d and x.  At
+// most 8 voxels an edge: 512 voxels, 729 nodes.  One launch per step took 5-7 us each whatever
+// the size, 28 us for degree 6 under a 12^3 domain (343 nodes) and 33 under a 64^3 one (729);
+// this takes 7.8 and 12.3.
+constexpr int COARSE_EDGE = 8, COARSE_STEPS = 16;
+struct CoarseCheb {
+    int m;
+    float c1[COARSE_STEPS], c2[COARSE_STEPS];
+};
+template <int NT>
+__global__ __launch_bounds__(NT) void k_coarse(const DomInfo* __restrict__ doms, const int* __restrict__ lat2node,
+                                               const double* __restrict__ emod, const float* __restrict__ dinv,
+                                               const int* __restrict__ done, WK<float> wk, const float* __restrict__ bvec,
+                                               float* __restrict__ xout, CoarseCheb C) {
+    constexpr int NVX = NT < COARSE_EDGE * COARSE_EDGE * COARSE_EDGE ? NT : COARSE_EDGE * COARSE_EDGE * COARSE_EDGE;
+    __shared__ float s_x[3][NT];
+    __shared__ float s_y[24][NVX];
+    const int dom = blockIdx.x, lc = blockIdx.y, t = threadIdx.x;
+    if (done && done[dom]) return;
+    const DomInfo D = doms[dom];
+    const int Lx = D.nx + 1, Ly = D.ny + 1, NL = Lx * Ly * (D.nz + 1), NV = D.nx * D.ny * D.nz;
+    const int q = t < NL ? lat2node[D.lat_off + t] : -1;
+    const int g[3] = {t % Lx, (t / Lx) % Ly, t / (Lx * Ly)};
+    const float E = t < NV ? (float)emod[D.vox_off + t] : 0.f;
+    const int n0 = t % D.nx + Lx * ((t / D.nx) % D.ny + Ly * (t / (D.nx * D.ny)));   // corner 0 of voxel t
+    float b[3] = {0.f, 0.f, 0.f}, di[3] = {0.f, 0.f, 0.f}, d[3], x[3];
+    if (q >= 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            b[k] = bvec[((int64_t)q * 3 + k) * R + lc];
+            di[k] = dinv[(int64_t)q * 3 + k];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = d[k] = C.c2[0] * di[k] * b[k];
+    for (int st = 1; st < C.m; ++st) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s_x[k][t] = x[k];
+        __syncthreads();
+        if (t < NV) {
+            float w[8][3], y[8][3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                float v[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) v[c] = s_x[k][n0 + (c & 1) + Lx * (((c >> 1) & 1) + Ly * (c >> 2))];
+                fht_fwd(v);
+#pragma unroll
+                for (int c = 0; c < 8; ++c) w[c][k] = v[c];
+            }
+            walsh_apply(wk, w, y);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                float o[8];
+                const float y1 = y[1][k] * E;
+                o[0] = -y1;
+                o[1] = y1;
+#pragma unroll
+                for (int c = 2; c < 8; c += 2) {
+                    const float p = y[c][k] * E, r = y[c + 1][k] * E;
+                    o[c] = p - r;
+                    o[c + 1] = p + r;
+                }
+                fht_inv_tail(o);
+#pragma unroll
+                for (int c = 0; c < 8; ++c) s_y[3 * c + k][t] = o[c];
+            }
+        }
+        __syncthreads();
+        if (t < NL) {
+            float y[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 7; c >= 0; --c) {   // this node is corner c of the voxel
+                const int vx = g[0] - (c & 1), vy = g[1] - ((c >> 1) & 1), vz = g[2] - (c >> 2);
+                const bool in = vx >= 0 && vy >= 0 && vz >= 0 && vx < D.nx && vy < D.ny && vz < D.nz;
+                const int v = in ? vx + D.nx * (vy + D.ny * vz) : 0;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float f = s_y[3 * c + k][v];
+                    y[k] += in ? f : 0.f;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                d[k] = C.c1[st] * d[k] + C.c2[st] * di[k] * (b[k] - y[k]);
+                x[k] += d[k];
+            }
+        }
+    }
+    if (q >= 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) xout[((int64_t)q * 3 + k) * R + lc] = x[k];
+    }
+}
+

@@ -1024,13 +1024,29 @@ __global__ __launch_bounds__(NT_UPD) void k_bdir(const int4* __restrict__ slices
     }
 }
 
+// Where a domain's next phase between residual replacements ends at the latest: the first
+// (and with FP64 vectors every) phase runs to its target or to the cap of all domains; a
+// later one that has not got there after one and a half times the first one's iterations
+// has lost its Krylov space to FP32 rounding (seen with clusters that hang on single
+// voxels) and gains from the restart: a 64^3 domain, 73 iterations in the first phase, took 1004
+// in all with phases of up to 400, 215 with the second one ended after 100.  Ends before the
+// first phase's length cost far more: its directions are not resolved by then (1680 with 60).
+__global__ void k_phase(const int64_t* __restrict__ iters, int n, int phase, int64_t* __restrict__ len0,
+                        int64_t* __restrict__ phase_end) {
+    const int d = blockIdx.x * blockDim.x + threadIdx.x;
+    if (d >= n) return;
+    if (phase == 1) len0[d] = iters[d];
+    phase_end[d] = phase <= 0 ? INT64_MAX : iters[d] + len0[d] + len0[d] / 2 + 16;
+}
+
 // per domain: the inner block iteration has finished when every load case's
 // recursive residual (scaled back by its column scale, see k_to32) is at or
-// below its target (a non-finite one is not), or at the iteration cap
+// below its target (a non-finite one is not), at the end of its phase (k_phase), or at the
+// iteration cap
 __global__ __launch_bounds__(RED_NT) void k_bcheck(const int* __restrict__ dslice, int* __restrict__ done,
                                                   const double* __restrict__ prr, const double* __restrict__ thr2,
                                                   const double* __restrict__ rrcur, int64_t* __restrict__ iters,
-                                                  int64_t max_iters) {
+                                                  const int64_t* __restrict__ phase_end, int64_t max_iters) {
     __shared__ double s_out[RED_NT];
     const int d = blockIdx.x, tid = threadIdx.x;
     if (done[d]) return;
@@ -1045,7 +1061,7 @@ __global__ __launch_bounds__(RED_NT) void k_bcheck(const int* __restrict__ dslic
     if (tid == 0) {
         const int64_t it = iters[d] + 1;
         iters[d] = it;
-        if (!any || it >= max_iters) done[d] = 1;
+        if (!any || it >= max_iters || it >= phase_end[d]) done[d] = 1;
     }
 }
 
@@ -2137,6 +2153,8 @@ int batch_finalize(SolverBatch& b, int precision) {
     DTC_TRY(b.done.ensure(nd * 4));
     DTC_TRY(b.done64.ensure(nd * 4));
     DTC_TRY(b.iters.ensure(nd * 8));
+    DTC_TRY(b.len0.ensure(nd * 8));
+    DTC_TRY(b.phase_end.ensure(nd * 8));
     DTC_TRY(b.ff.ensure(nd * R * FFD * 8));
     // element stiffness (E = 1) and its Walsh blocks
     double Khat[576];
@@ -2447,17 +2465,31 @@ struct LvView {
     float* d;
 };
 
-// Chebyshev smoothing parameters: interval [lmax / ratio, lmax] of D^-1 K
+// Chebyshev smoothing parameters: interval [lmax / ratio, lmax] of D^-1 K.  lmax is the
+// element-by-element bound, about twice the largest eigenvalue of a porous mesh, and what the
+// coarse space misses on thin struts reaches far down, so the intervals are wide.  The levels
+// below the finest are an eighth of its work and less: they smooth with degree 4.  Iterations
+// to 1e-11 and time against degree 2 and ratio 7 on every level: 64^3 trabecular 187 and 146
+// -> 147 and 114, 191 -> 179 ms; 33^3 56 -> 44, 72 -> 67 ms for four; 27^3 HEX20 42 -> 30, 75 -> 65 ms
+// for three; 48^3 greyscale 109 -> 80.  Degree 3 there: 184, 66 and 67 ms; degree 5: 180, 70 and 67;
+// ratio 20: 183, 68 and 66.  (Measured with one launch per step on the coarsest level, degree 4.)
+// The coarsest level takes degree 6: with 4 a domain whose batch has fewer levels (its own
+// coarsest level carries the smooth modes) needed three iterations more than in a deeper one.
 struct MgParams {
-    double ratio = 7.0;        // smoothing passes of the fine and intermediate levels
-    int coarse_degree = 4;     // coarsest level
+    double ratio = 0.0;        // finest level; 0: by its degree (fine_ratio)
+    int level_degree = 4;      // intermediate levels (at least the finest level's degree)
+    double level_ratio = 30.0;
+    int coarse_degree = 6;     // coarsest level
     double coarse_ratio = 50.0;
     double lscale = 1.0;       // multiplies the element-by-element bound of lambda_max
+    double fine_ratio(int deg) const { return ratio > 0.0 ? ratio : deg <= 1 ? 7.0 : deg == 2 ? 12.0 : deg == 3 ? 20.0 : 30.0; }
 };
 
 MgParams mg_params() {
     MgParams p;
     if (const char* e = std::getenv("DTC_MG_RATIO")) p.ratio = std::atof(e);
+    if (const char* e = std::getenv("DTC_MG_LDEG")) p.level_degree = std::max(1, std::atoi(e));
+    if (const char* e = std::getenv("DTC_MG_LRATIO")) p.level_ratio = std::atof(e);
     if (const char* e = std::getenv("DTC_MG_CDEG")) p.coarse_degree = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("DTC_MG_CRATIO")) p.coarse_ratio = std::atof(e);
     if (const char* e = std::getenv("DTC_MG_LSCALE")) p.lscale = std::atof(e);
@@ -2477,7 +2509,10 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     const int L = (int)b.mg.size();
     const int* done = b.done_ext ? b.done_ext : b.done.as<int>();
     static const MgParams P = mg_params();
-    const int deg = b.mg_degree > 0 ? b.mg_degree : 2;
+    // (the twin's finest level is an intermediate level of the p-multigrid)
+    const int deg0 = b.mg_degree > 0 ? b.mg_degree : 2, ldeg = std::max(P.level_degree, deg0);
+    const int deg = b.done_ext ? ldeg : deg0;
+    const double ratio0 = b.done_ext ? P.level_ratio : P.fine_ratio(deg0);
     auto view = [&](int l) {
         LvView v;
         if (l == 0) {
@@ -2534,11 +2569,51 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
         }
         return DTC_OK;
     };
-    // the fine iterate makes (deg - 1) + deg swaps (or coarse_degree - 1 without
-    // coarse levels): start in the buffer that makes it end in z
-    cur[0] = (L > 0 ? 2 * deg - 1 : P.coarse_degree - 1) % 2;
+    // the coarsest level in one launch where it fits k_coarse: always, but for domains of more
+    // than 2048 voxels an edge
+    const std::vector<DomInfo>& cdom = L > 0 ? b.mg[L - 1].h_dom : b.h_dom;
+    int edge = 0, nodes = 0;
+    for (const DomInfo& D : cdom) {
+        edge = std::max({edge, D.nx, D.ny, D.nz});
+        nodes = std::max<int64_t>(nodes, (int64_t)(D.nx + 1) * (D.ny + 1) * (D.nz + 1));
+    }
+    const bool one_launch = edge <= COARSE_EDGE && P.coarse_degree <= COARSE_STEPS;
+    auto coarsest = [&]() -> int {
+        const LvView v = view(L);
+        if (!one_launch) return smooth(L, P.coarse_degree, true, P.coarse_ratio);
+        if (v.T.n_bricks == 0) return DTC_OK;
+        const double hi = b.cheb_lmax * P.lscale, lo = hi / P.coarse_ratio;
+        const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+        double rho = 1.0 / sigma;
+        CoarseCheb cc{};
+        cc.m = P.coarse_degree;
+        cc.c2[0] = (float)(1.0 / theta);
+        for (int k = 1; k < cc.m; ++k) {
+            const double rn = 1.0 / (2.0 * sigma - rho);
+            cc.c1[k] = (float)(rn * rho);
+            cc.c2[k] = (float)(2.0 * rn / delta);
+            rho = rn;
+        }
+        const DevMem& dom = L > 0 ? b.mg[L - 1].dom : b.dom;
+        const DevMem& l2n = L > 0 ? b.mg[L - 1].lat2node : b.lat2node;
+        const DevMem& emod = L > 0 ? b.mg[L - 1].emod : b.emod;
+        const dim3 grid((unsigned)cdom.size(), R);
+        auto run = [&](auto kernel, int nt) {
+            kernel<<<grid, nt, 0, s>>>(dom.as<DomInfo>(), l2n.as<int>(), emod.as<double>(), v.dinv, done, wk, v.b, v.buf[0],
+                                       cc);
+        };
+        if (nodes <= 256) run(k_coarse<256>, 256);
+        else if (nodes <= 384) run(k_coarse<384>, 384);
+        else if (nodes <= 512) run(k_coarse<512>, 512);
+        else run(k_coarse<768>, 768);
+        DTC_HIP(hipGetLastError());
+        return DTC_OK;
+    };
+    // the fine iterate makes (deg - 1) + deg swaps (without coarse levels none, or
+    // coarse_degree - 1): start in the buffer that makes it end in z
+    cur[0] = (L > 0 ? 2 * deg - 1 : one_launch ? 0 : P.coarse_degree - 1) % 2;
     for (int l = 0; l < L; ++l) {
-        DTC_TRY(smooth(l, deg, true, P.ratio));
+        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, true, l == 0 ? ratio0 : P.level_ratio));
         const LvView f = view(l), c = view(l + 1);
         cur[l + 1] = 0;
         if (c.T.n_bricks == 0 || f.T.n_bricks == 0) continue;
@@ -2549,7 +2624,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
             c.T.bricks, b.mg[l].rtab.as<int>(), done, res, c.b);
         DTC_HIP(hipGetLastError());
     }
-    DTC_TRY(smooth(L, P.coarse_degree, true, P.coarse_ratio));
+    DTC_TRY(coarsest());
     for (int l = L - 1; l >= 0; --l) {
         const LvView f = view(l), c = view(l + 1);
         if (f.T.n_bricks > 0 && c.T.n_bricks > 0) {
@@ -2557,7 +2632,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
                 f.T.bricks, b.mg[l].ptab.as<int>(), done, c.buf[cur[l + 1]], f.buf[cur[l]]);
             DTC_HIP(hipGetLastError());
         }
-        DTC_TRY(smooth(l, deg, false, P.ratio));
+        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, false, l == 0 ? ratio0 : P.level_ratio));
     }
     if (prz && b.n_bricks > 0) {
         k_dot<<<b.n_bricks, NT_UPD, 0, s>>>(b.brick.as<BrickInfo>(), done, r, z, prz);
@@ -2581,7 +2656,7 @@ int pmg_vcycle(SolverBatch& b, const float* r, float* z, double* prz) {
     const BrickInfo* bl = b.brick.as<BrickInfo>();
     float* t = b.t32.as<float>();
     float* d = b.d32.as<float>();
-    const double hi = b.cheb_lmax * P.lscale, lo = hi / P.ratio;
+    const double hi = b.cheb_lmax * P.lscale, lo = hi / P.fine_ratio(deg);
     const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
     auto smooth = [&](bool zero, double* dot) -> int {
         double rho = 1.0 / sigma;
@@ -2936,7 +3011,7 @@ int block_iteration64(SolverBatch& b, const WK<float>& wk, float* p, float* q, f
     k_bsolve<0><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     k_bupdate64<<<NSl, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), x, r, p, q64, b.part_b.as<double>());
     k_bcheck<<<D, RED_NT, 0, s>>>(b.dslice.as<int>(), done, b.part_b.as<double>(), b.thr2.as<double>(), nullptr,
-                                  b.iters.as<int64_t>(), max_iters);
+                                  b.iters.as<int64_t>(), b.phase_end.as<int64_t>(), max_iters);
     k_to32<<<NBk, NT_UPD, 0, s>>>(bl, done, r, b.r32.as<float>(), nullptr, nullptr);
     DTC_HIP(hipGetLastError());
     DTC_TRY(mg_vcycle(b, wk, b.r32.as<float>(), z, nullptr));
@@ -2961,7 +3036,7 @@ int block_iteration(SolverBatch& b, const WK<float>& wk, float* x, float* r, flo
     k_bsolve<0><<<D, 64, 0, s>>>(done, b.gsum.as<double>(), b.lfac.as<double>(), b.bcoef.as<float>());
     k_bupdate<<<NSl, NT_UPD, 0, s>>>(sl, done, b.bcoef.as<float>(), x, r, p, q, b.part_b.as<double>());
     k_bcheck<<<D, RED_NT, 0, s>>>(b.dslice.as<int>(), done, b.part_b.as<double>(), b.thr2.as<double>(),
-                                  b.rr.as<double>(), b.iters.as<int64_t>(), max_iters);
+                                  b.rr.as<double>(), b.iters.as<int64_t>(), b.phase_end.as<int64_t>(), max_iters);
     DTC_HIP(hipGetLastError());
     DTC_TRY(mg_vcycle(b, wk, r, z, nullptr));
     DTC_TRY(block_gram(b, q, z, nullptr));
@@ -3280,9 +3355,11 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         const char* brp = std::getenv("DTC_BLOCK_REPLACE");
         const int64_t block_replace = brp ? std::max(1, std::atoi(brp)) : 400;
         // FP64 vectors: the recursion drifts far less, and a restart discards the
-        // block's Krylov space, so a phase runs to its target (the true residual
-        // is checked then)
-        const int64_t block_replace64 = brp ? block_replace : 20000;
+        // block's Krylov space, so a phase runs to its target, or until it clearly got stuck
+        // (sixteen 48^3 greyscale domains, 70 to 870 iterations but for one: 10,031 in all
+        // without this cap, 4,846 of them in one domain; 6,693 and 1,501 with 500, 7,116 with
+        // 300, 9,376 with 200)
+        const int64_t block_replace64 = brp ? block_replace : 500;
         float* bp = p32;
         float* bq = b.q32.as<float>();
         float* bz = z32;
@@ -3292,6 +3369,9 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
             bool left = false;
             DTC_TRY(apply_cap(b, cap, nouter, &left, &progress));
             if (!left) break;
+            if (block)
+                k_phase<<<nb(D, 64), 64, 0, s>>>(b.iters.as<int64_t>(), D, b.block64 ? 0 : it, b.len0.as<int64_t>(),
+                                                 b.phase_end.as<int64_t>());
             // the block solves the correction problem with unit-norm columns: FP32
             // directions mix all 24 load cases, whose residuals drift apart in size
             k_to32<<<b.n_bricks, NT_UPD, 0, s>>>(bl, b.done64.as<int>(), b.r64.as<double>(), r32, x32,

@@ -108,6 +108,7 @@ struct SolverBatch {
     DevMem done;                   // int [dom]: inner iteration finished
     DevMem done64;                 // int [dom]: outer (FP64 residual) converged
     DevMem iters;                  // int64 [dom]
+    DevMem len0, phase_end;        // int64 per domain: iterations of the first phase, end of the running one
     DevMem ff;                     // double [dom][24 lc][60 macro DOF slots]
     DevMem gtmp;                   // gradient work
     // multigrid preconditioner of the FP32 PCG (empty when Jacobi is used)
