@@ -3355,11 +3355,11 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         const char* brp = std::getenv("DTC_BLOCK_REPLACE");
         const int64_t block_replace = brp ? std::max(1, std::atoi(brp)) : 400;
         // FP64 vectors: the recursion drifts far less, and a restart discards the
-        // block's Krylov space, so a phase runs to its target, or until it clearly got stuck
-        // (sixteen 48^3 greyscale domains, 70 to 870 iterations but for one: 10,031 in all
-        // without this cap, 4,846 of them in one domain; 6,693 and 1,501 with 500, 7,116 with
-        // 300, 9,376 with 200)
-        const int64_t block_replace64 = brp ? block_replace : 500;
+        // block's Krylov space, so a phase runs to its target (the true residual
+        // is checked then).  A cap of 500 took the worst of sixteen 48^3 greyscale domains
+        // from 4,846 to 1,501 iterations, but a 128^3 one from 708 to 1,316 (3.6 -> 6.7 s) and
+        // a 96^3 HEX20/HEX20 one, which needs over a thousand in one phase, past 5,500
+        const int64_t block_replace64 = brp ? block_replace : 20000;
         float* bp = p32;
         float* bq = b.q32.as<float>();
         float* bz = z32;
