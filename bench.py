@@ -36,10 +36,10 @@ for p in (ROOT, PKG):
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 MFMA_PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6}   # MI355X dense matrix-core peaks
 # the timed kernels (fine-level launches): kernel_stats name -> kernel
-KERNEL_NAMES = {"mv": "k_matvec<float, IN_V, OUT_MASKED> (Q = K P of the block PCG)",
-                "cheb": "k_matvec<float, IN_V|IN_JS, OUT_CHEB> (Chebyshev-Jacobi smoothing step)",
-                "bres": "k_matvec<float, IN_V, OUT_BRES> (b - K x before restriction)",
-                "resid": "k_matvec<double, IN_U, OUT_RESID> (FP64 true residual)"}
+KERNEL_NAMES = {"mv": "k_ebe<float, IN_V, OUT_MASKED> (Q = K P of the block PCG)",
+                "cheb": "k_ebe<float, IN_V|IN_JS, OUT_CHEB> (Chebyshev-Jacobi smoothing step)",
+                "bres": "k_ebe<float, IN_V, OUT_BRES> (b - K x before restriction)",
+                "resid": "k_ebe<double, IN_V, OUT_RESID> (FP64 true residual)"}
 
 
 def hbm_copy_probe(gib=1.0, iters=10):

@@ -7,9 +7,8 @@ Runs one rocprofv3 --pmc pass (the counters of one pass must fit the hardware's
 per-block limits: at most 8 SQ counters) over one bench.py step of the workload
 (as a child process, the program directly after `--`; the step runs as one part,
 DTC_CONCURRENT=1, the form of bench.py's kernel timing run), and averages every counter
-over the fine-level dispatches (the most dispatched grid, the larger on a tie: the
-coarse levels run smaller grids, the launch-shape autotuner a few split ones) of
-each timed kernel: the CG matvec
+over the fine-level dispatches (the largest grid: the coarse levels run smaller
+ones, more often) of each timed kernel: the CG matvec
 Q = K P (mv), the fused Chebyshev smoothing step (cheb), the restriction
 residual (bres) and the FP64 residual (resid).  Prints one JSON object.
 """
@@ -42,7 +41,7 @@ def main() -> None:
              str(args.batch), "--n", str(args.n), "--fp64-domains", "0", "--no-cpu"]
     res = {}
     with tempfile.TemporaryDirectory(dir="/tmp") as tmp:
-        cmd = ["rocprofv3", "--pmc"] + counters + ["--kernel-include-regex", "k_matvec", "-d", tmp, "-o", "run",
+        cmd = ["rocprofv3", "--pmc"] + counters + ["--kernel-include-regex", "k_ebe", "-d", tmp, "-o", "run",
                                                    "--"] + bench
         print(" ".join(cmd), file=sys.stderr, flush=True)
         subprocess.run(cmd, check=True, timeout=900, stdout=subprocess.DEVNULL, env=dict(os.environ, TMPDIR="/tmp", DTC_CONCURRENT="1"))
@@ -66,12 +65,7 @@ def main() -> None:
         entry = {"kernel": label, "variants": {}}
         for name, rs in variants.items():
             if all(r[1] is not None for r in rs):
-                # the solve's fine-level grid: the most dispatched grid, the larger on a tie
-                # (the launch-shape autotuner runs a few launches on split grids first)
-                cnt = {}
-                for r in rs:
-                    cnt.setdefault(r[1], set()).add(r[2])
-                g = max(cnt, key=lambda k: (len(cnt[k]), k))
+                g = max(r[1] for r in rs)   # the fine level
                 rs = [r for r in rs if r[1] == g]
             per = {}
             for _, _, disp, cn, v in rs:

@@ -11,9 +11,8 @@ Runs (as child processes, the program directly after `--`):
 FETCH_SIZE / WRITE_SIZE are reported in KiB per dispatch.  The copy reads and
 writes exactly 1 GiB, so `factor = 1 GiB / counter(copy)` converts each counter
 into bytes; traffic = FETCH * f_fetch + WRITE * f_write per dispatch, averaged
-over the fine-level dispatches of the kernel (the most dispatched grid, the
-larger on a tie: the coarse multigrid levels launch the same kernel on smaller
-grids, the launch-shape autotuner a few launches on split grids), the launches
+over the fine-level dispatches of the kernel (the largest grid: the coarse
+multigrid levels launch the same kernel on smaller grids, more often), the launches
 whose HIP-event average and algorithmic bytes bench.py reports.
 Writes profiles/traffic_<kernel>.json, which bench.py reports as the kernel's
 traffic (and as roofline.traffic for the dominant kernel) when its batch and
@@ -33,16 +32,14 @@ import tempfile
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # bench kernel key -> (kernel name prefix as rocprofv3 writes it, the name bench.py reports).
-# A fine-level FP32 matvec is one launch of the sparse-brick variant and one of the
-# dense variant (template flags after the prefix): their per-dispatch averages add.
 # name pattern (regular expression) of each timed kernel, and its label; the
 # Chebyshev step runs with a vector input (IN_V = 0) or, after a zero start, with
 # the scaled right-hand side (IN_JS = 2): both are that kernel's launches
 KERNELS = {
-    "mv": (r"k_matvec<float, 0, 3,", "k_matvec<float, IN_V, OUT_MASKED>"),
-    "cheb": (r"k_matvec<float, [02], 4,", "k_matvec<float, IN_V|IN_JS, OUT_CHEB>"),
-    "bres": (r"k_matvec<float, 0, 5,", "k_matvec<float, IN_V, OUT_BRES>"),
-    "resid": (r"k_matvec<double, 1, 1,", "k_matvec<double, IN_U, OUT_RESID>"),
+    "mv": (r"k_ebe<float, float, float, 0, 3,", "k_ebe<float, IN_V, OUT_MASKED>"),
+    "cheb": (r"k_ebe<float, float, float, [02], 4,", "k_ebe<float, IN_V|IN_JS, OUT_CHEB>"),
+    "bres": (r"k_ebe<float, float, float, 0, 5,", "k_ebe<float, IN_V, OUT_BRES>"),
+    "resid": (r"k_ebe<double, double, double, 0, 1,", "k_ebe<double, IN_V, OUT_RESID>"),
 }
 COPY = ("import torch; a = torch.ones(2**28, device='cuda'); b = torch.empty_like(a); torch.cuda.synchronize(); "
         "b.copy_(a); torch.cuda.synchronize(); print(float(b[-1]))")
@@ -76,17 +73,14 @@ def _counter(dbdir: str, counter: str, kname: str) -> tuple[float, int]:
     vals = []
     for name, rs in by.items():
         if all(r[1] is not None for r in rs):
-            cnt = {}
-            for r in rs:
-                cnt[r[1]] = cnt.get(r[1], 0) + 1
-            g = max(cnt, key=lambda k: (cnt[k], k))   # most dispatched grid, the larger on a tie
+            g = max(r[1] for r in rs)   # the fine level
             rs = [r for r in rs if r[1] == g]
         vals += [r[2] for r in rs]
     return sum(vals) / len(vals), len(vals)
 
 
 def _pmc(counter: str, out: str, cmd: list[str]) -> str:
-    full = ["rocprofv3", "--pmc", counter, "--kernel-include-regex", "k_matvec|copyBuffer", "-d", out, "-o", "run",
+    full = ["rocprofv3", "--pmc", counter, "--kernel-include-regex", "k_ebe|copyBuffer", "-d", out, "-o", "run",
             "--"] + cmd
     print(" ".join(full), flush=True)
     p = subprocess.run(full, check=True, timeout=600, stdout=subprocess.PIPE, text=True,
