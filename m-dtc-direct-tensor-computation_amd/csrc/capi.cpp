@@ -61,7 +61,7 @@ struct Pool {
     std::vector<std::pair<void*, size_t>> pinned;
 
     // unlinks the oldest blocks while over the bound or past their time; the caller frees them
-    void expire(std::vector<Block>& out, size_t bound) {
+    void expire(std::list<Block>& out, size_t bound) {
         const Clock::time_point now = Clock::now();
         while (!idle.empty() &&
                (bytes > bound || std::chrono::duration<double>(now - idle.back().since).count() > POOL_SECONDS)) {
@@ -70,8 +70,7 @@ struct Pool {
             while (r.first->second != last) ++r.first;
             by_size.erase(r.first);
             bytes -= last->n;
-            out.push_back(*last);
-            idle.erase(last);
+            out.splice(out.begin(), idle, last);
         }
     }
 };
@@ -82,7 +81,7 @@ Pool& pool() {
     return p;
 }
 
-void free_blocks(const std::vector<Pool::Block>& v) {
+void free_blocks(const std::list<Pool::Block>& v) {
     for (const Pool::Block& b : v) (void)hipFree(b.p);
 }
 
@@ -91,7 +90,7 @@ void free_blocks(const std::vector<Pool::Block>& v) {
 void* pool_take(size_t n, int dev) {
     Pool& P = pool();
     void* p = nullptr;
-    std::vector<Pool::Block> old;
+    std::list<Pool::Block> old;
     {
         std::lock_guard<std::mutex> lk(P.mu);
         const auto it = P.by_size.find({dev, n});
@@ -109,20 +108,29 @@ void* pool_take(size_t n, int dev) {
 
 void pool_put(void* p, size_t n, int dev) {
     Pool& P = pool();
-    std::vector<Pool::Block> old;
+    std::list<Pool::Block> old;
     {
         std::lock_guard<std::mutex> lk(P.mu);
-        P.idle.push_front({p, n, dev, Pool::Clock::now()});
-        P.by_size.emplace(std::make_pair(dev, n), P.idle.begin());
-        P.bytes += n;
+        // (called from destructors: without host memory for the entry the block is freed; so is
+        // one that would push most of the others out)
+        std::list<Pool::Block> one;
+        if (n <= POOL_BYTES / 4) try {
+            one.push_front({p, n, dev, Pool::Clock::now()});
+            P.by_size.emplace(std::make_pair(dev, n), one.begin());
+            P.idle.splice(P.idle.begin(), one);
+            P.bytes += n;
+            p = nullptr;
+        } catch (...) {
+        }
         P.expire(old, POOL_BYTES);
     }
+    if (p) (void)hipFree(p);
     free_blocks(old);
 }
 
 void pool_trim() {
     Pool& P = pool();
-    std::vector<Pool::Block> old;
+    std::list<Pool::Block> old;
     {
         std::lock_guard<std::mutex> lk(P.mu);
         P.expire(old, 0);
@@ -147,8 +155,11 @@ void pool_put_pinned(void* p, size_t n) {
     {
         std::lock_guard<std::mutex> lk(P.mu);
         if (n <= ((size_t)1 << 20) && P.pinned.size() < POOL_PINNED) {
-            P.pinned.emplace_back(p, n);
-            return;
+            try {
+                P.pinned.emplace_back(p, n);
+                return;
+            } catch (...) {
+            }
         }
     }
     (void)hipHostFree(p);
@@ -762,7 +773,9 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
             }
             DTC_TRY(batch_finalize(tw, DTC_FP32_REFINE));
         }
-        DTC_HIP(hipStreamSynchronize(s));   // the next sub-batch meshes into the same work space on its own stream
+        // the next sub-batch meshes into the same work space on its own stream.  (Not the whole
+        // device: that is an error while another thread's call captures its iterations.)
+        DTC_HIP(hipStreamSynchronize(s));
         return DTC_OK;
     };
     // one sub-batch, solve: multigrid hierarchy (unless built by prep_sub) -> solve -> reactions
@@ -792,7 +805,6 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
         for (int i = first[k]; i < first[k + 1]; ++i) list.push_back(i);
         DTC_TRY(setup_sub(k, list, b->o.precision));
     }
-    DTC_HIP(hipDeviceSynchronize());
     const auto t_setup = std::chrono::steady_clock::now();
     if (!concurrent) {
         for (int k = 0; k < NS; ++k) DTC_TRY(solve_sub(k, false));
