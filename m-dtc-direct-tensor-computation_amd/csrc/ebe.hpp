@@ -143,6 +143,8 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
     const uint2* __restrict__ eo = A.eown + C.e_off;
     const T* __restrict__ eE = static_cast<const T*>(A.eE) + C.e_off;
     const T* __restrict__ dinv = static_cast<const T*>(A.dinv);
+    // A cluster has no element where every voxel around its nodes is solid with modulus 0:
+    // then no record is read (there is none to repeat) and the rows leave as sums of nothing.
     // Software pipeline: the records of the group after next and x of the next group are
     // loaded while the current group is computed.  Lanes past the last element repeat it
     // into the row that is not read; nothing is selected from a loaded record before it
@@ -170,13 +172,17 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
             if constexpr (IN == IN_JS) sc[b] = dinv[(int64_t)nd[b] * 3];
         }
     };
-    fetch(le);
+    if (ne > 0) fetch(le);
     if (A.done && A.done[C.dom]) return;
     for (int i = tid; i < nv; i += NT) vzero(s_yv[i]);
-    gather();
-    uint2 oc = ow;
-    T Ec = E;
-    fetch(EPW + le);
+    uint2 oc;
+    T Ec;
+    if (ne > 0) {
+        gather();
+        oc = ow;
+        Ec = E;
+        fetch(EPW + le);
+    }
     __syncthreads();
     for (int e0 = 0; e0 < ne; e0 += EPW) {
         T y[8][3];
