@@ -222,6 +222,15 @@ int dtc_rotation_search_noalloc(const double EE[36], int criterion, double step_
                                 int64_t* jj, double* crit);
 int64_t dtc_rotation_noalloc_max_points(void);
 
+/* ---- memory ---------------------------------------------------------------
+ * The library keeps device memory of finished calls and destroyed batches for the next
+ * ones: at most 4 GiB, and a block not taken for 20 s goes at the next call that
+ * allocates or frees.  It is emptied when an allocation of the library fails; a program that
+ * wants the memory for others (another library, another process) frees it here.  Memory
+ * that a batch or a running call uses is not touched.  Any thread, any time; no
+ * counterpart in the reference (host allocations only). */
+int dtc_release_memory(void);
+
 #ifdef __cplusplus
 }
 #endif

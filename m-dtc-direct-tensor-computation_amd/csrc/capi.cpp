@@ -12,11 +12,7 @@
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
-#include <iterator>
-#include <list>
-#include <map>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -39,130 +35,6 @@ int set_error(int code, const char* fmt, ...) {
     va_end(ap);
     g_err = buf;
     return code;
-}
-
-// ---- pool of idle device and page-locked memory
-thread_local bool t_recycle = false;
-
-namespace {
-
-struct Pool {
-    using Clock = std::chrono::steady_clock;
-    struct Block {
-        void* p;
-        size_t n;
-        int dev;
-        Clock::time_point since;
-    };
-    std::mutex mu;
-    std::list<Block> idle;                                                         // newest first
-    std::multimap<std::pair<int, size_t>, std::list<Block>::iterator> by_size;
-    size_t bytes = 0;
-    std::vector<std::pair<void*, size_t>> pinned;
-
-    // unlinks the oldest blocks while over the bound or past their time; the caller frees them
-    void expire(std::list<Block>& out, size_t bound) {
-        const Clock::time_point now = Clock::now();
-        while (!idle.empty() &&
-               (bytes > bound || std::chrono::duration<double>(now - idle.back().since).count() > POOL_SECONDS)) {
-            const auto last = std::prev(idle.end());
-            auto r = by_size.equal_range({last->dev, last->n});
-            while (r.first->second != last) ++r.first;
-            by_size.erase(r.first);
-            bytes -= last->n;
-            out.splice(out.begin(), idle, last);
-        }
-    }
-};
-
-// never destroyed: the runtime may be gone when static objects are
-Pool& pool() {
-    static Pool& p = *new Pool;
-    return p;
-}
-
-void free_blocks(const std::list<Pool::Block>& v) {
-    for (const Pool::Block& b : v) (void)hipFree(b.p);
-}
-
-}  // namespace
-
-void* pool_take(size_t n, int dev) {
-    Pool& P = pool();
-    void* p = nullptr;
-    std::list<Pool::Block> old;
-    {
-        std::lock_guard<std::mutex> lk(P.mu);
-        const auto it = P.by_size.find({dev, n});
-        if (it != P.by_size.end()) {
-            p = it->second->p;
-            P.bytes -= n;
-            P.idle.erase(it->second);
-            P.by_size.erase(it);
-        }
-        P.expire(old, POOL_BYTES);
-    }
-    free_blocks(old);
-    return p;
-}
-
-void pool_put(void* p, size_t n, int dev) {
-    Pool& P = pool();
-    std::list<Pool::Block> old;
-    {
-        std::lock_guard<std::mutex> lk(P.mu);
-        // (called from destructors: without host memory for the entry the block is freed; so is
-        // one that would push most of the others out)
-        std::list<Pool::Block> one;
-        if (n <= POOL_BYTES / 4) try {
-            one.push_front({p, n, dev, Pool::Clock::now()});
-            P.by_size.emplace(std::make_pair(dev, n), one.begin());
-            P.idle.splice(P.idle.begin(), one);
-            P.bytes += n;
-            p = nullptr;
-        } catch (...) {
-        }
-        P.expire(old, POOL_BYTES);
-    }
-    if (p) (void)hipFree(p);
-    free_blocks(old);
-}
-
-void pool_trim() {
-    Pool& P = pool();
-    std::list<Pool::Block> old;
-    {
-        std::lock_guard<std::mutex> lk(P.mu);
-        P.expire(old, 0);
-    }
-    free_blocks(old);
-}
-
-void* pool_take_pinned(size_t n) {
-    Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
-    for (size_t i = P.pinned.size(); i-- > 0;)
-        if (P.pinned[i].second == n) {
-            void* p = P.pinned[i].first;
-            P.pinned.erase(P.pinned.begin() + (ptrdiff_t)i);
-            return p;
-        }
-    return nullptr;
-}
-
-void pool_put_pinned(void* p, size_t n) {
-    Pool& P = pool();
-    {
-        std::lock_guard<std::mutex> lk(P.mu);
-        if (n <= ((size_t)1 << 20) && P.pinned.size() < POOL_PINNED) {
-            try {
-                P.pinned.emplace_back(p, n);
-                return;
-            } catch (...) {
-            }
-        }
-    }
-    (void)hipHostFree(p);
 }
 
 namespace {

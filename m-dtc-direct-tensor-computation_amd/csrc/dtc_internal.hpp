@@ -39,7 +39,7 @@ int set_error(int code, const char* fmt, ...);
 // and Recycle below; anything else is freed), so that any thread may take it out for any
 // stream.  What is kept is bounded (POOL_BYTES, POOL_PINNED), the oldest goes first, what
 // was not used for POOL_SECONDS is freed at the next call that uses the pool, and all of it
-// when an allocation fails.  Streams are not kept: kept ones end up on one hardware queue,
+// when an allocation fails or the program asks (dtc_release_memory).  Streams are not kept: kept ones end up on one hardware queue,
 // and the parts of a batch no longer overlap (40 domains of 21^3 61 -> 70 ms).
 constexpr size_t POOL_BYTES = (size_t)4 << 30;
 constexpr size_t POOL_PINNED = 8;
@@ -53,7 +53,7 @@ inline size_t pool_size(size_t n) {
 }
 void* pool_take(size_t n, int dev);               // an idle allocation of n = pool_size(n) bytes, or null
 void pool_put(void* p, size_t n, int dev);        // takes ownership
-void pool_trim();                                 // frees all idle memory
+void pool_trim();                                 // frees all idle memory, device and page-locked
 void* pool_take_pinned(size_t n);
 void pool_put_pinned(void* p, size_t n);
 

@@ -31,7 +31,7 @@ from ._lib import (DTC_ERR_EMPTY_MESH, DTC_ERR_FEW_CONSTRAINTS, DTC_ERR_NO_CONVE
 KIND = {np.dtype(np.int8): 1, np.dtype(np.int16): 2, np.dtype(np.int32): 4}
 
 __all__ = ["Domain", "Batch", "mesh", "mesh_count", "boundaries", "element_stiffness", "solve_domain", "solve_batch",
-           "rotation_search", "ddc_params", "domain_bounds", "extract_block", "DTCError", "DTC_FP64",
+           "rotation_search", "release_memory", "ddc_params", "domain_bounds", "extract_block", "DTCError", "DTC_FP64",
            "DTC_FP32_REFINE", "load"]
 
 
@@ -313,3 +313,8 @@ def rotation_search(EE, criterion, step_deg=1.0, num_zero=1e-9, noalloc=False):
                                   C.byref(alpha), _p(n), _p(aa), _p(EEo), C.byref(jj), C.byref(crit)))
     return dict(alpha=alpha.value, n=n, aa=aa.reshape(3, 3).T.copy(), EE_opt=EEo.reshape(6, 6).T.copy(),
                 jj=jj.value, crit=crit.value)
+
+
+def release_memory():
+    """Frees the idle device memory that the library keeps for its next calls (at most 4 GiB)."""
+    check("dtc_release_memory", load().dtc_release_memory())

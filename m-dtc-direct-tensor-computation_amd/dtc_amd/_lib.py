@@ -86,6 +86,7 @@ SIGNATURES = {
     "dtc_rotation_search": (C.c_int, [P, C.c_int, C.c_double, C.c_double, P, P, P, P, P, P]),
     "dtc_rotation_search_noalloc": (C.c_int, [P, C.c_int, C.c_double, C.c_double, P, P, P, P, P, P]),
     "dtc_rotation_noalloc_max_points": (I64, []),
+    "dtc_release_memory": (C.c_int, []),
 }
 
 _lib = None

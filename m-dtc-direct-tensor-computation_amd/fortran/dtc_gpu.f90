@@ -76,6 +76,10 @@ module dtc_gpu
        import :: c_int
      end function dtc_version
 
+     integer(c_int) function dtc_release_memory() bind(c, name="dtc_release_memory")
+       import :: c_int
+     end function dtc_release_memory
+
      integer(c_int) function dtc_ddc_params(size_domain, delta, vdim, x_D, nn_D, x_D_phy) &
           bind(c, name="dtc_ddc_params")
        import :: c_int, c_int64_t, c_double
