@@ -15,7 +15,6 @@ constexpr double ORTH_DROP = 1e-10;   // of P^T P
 //           1e-10 dropped, L not kept) and coef = L^-T, so that P coef has
 //           orthonormal columns (zero columns for the dropped directions).
 // coef[k * 24 + j] multiplies vector column k in the update of column j.
-// (A dropped direction's zeros are selected, not multiplied: its entries may not be finite.)
 //
 // A chain of 24 pivots: latency is all there is.  One wave per domain, no LDS and no barrier
 // inside the chain: lane i holds row i of the matrix in registers, and the entries that
@@ -41,6 +40,17 @@ __global__ __launch_bounds__(64) void k_bsolve(const int* __restrict__ done, con
 #pragma unroll
     for (int k = 0; k < R; ++k)
         b[k] = MODE == 2 ? (k == row ? 1.0 : 0.0) : G[(MODE == 0 ? RR : 0) + k * R + row];
+    // Entries that are not finite become 0 before the chain: a direction that brings them in
+    // has such a diagonal entry too and is dropped, and the products with its 0 stay 0
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) sum += a[k] + b[k];
+    if (!(fabs(sum) < INFINITY))
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            if (!(fabs(a[k]) < INFINITY)) a[k] = 0.0;
+            if (!(fabs(b[k]) < INFINITY)) b[k] = 0.0;
+        }
     double rd = 0.0;                              // 1 / L_kk of this row, 0 for a dropped direction
     if (MODE != 1) {
         constexpr double DROP = MODE == 0 ? PIVOT_DROP : ORTH_DROP;
@@ -54,7 +64,7 @@ __global__ __launch_bounds__(64) void k_bsolve(const int* __restrict__ done, con
             const bool keep = dk > DROP * lane_f64(diag, k) && dk < INFINITY;
             const double lk = keep ? sqrt(dk) : 0.0, rk = keep ? 1.0 / lk : 0.0;
             if (row == k) rd = rk;
-            a[k] = row == k ? lk : row > k && keep ? a[k] * rk : 0.0;
+            a[k] = row == k ? lk : row > k ? a[k] * rk : 0.0;
 #pragma unroll
             for (int m = k + 1; m < R; ++m) a[m] -= a[k] * lane_f64(a[k], m);
         }
@@ -72,16 +82,14 @@ __global__ __launch_bounds__(64) void k_bsolve(const int* __restrict__ done, con
     if (MODE != 2)
 #pragma unroll
         for (int k = 0; k < R; ++k) {
-            const double rk = lane_f64(rd, k);
-            b[k] = rk != 0.0 ? b[k] * rk : 0.0;
+            b[k] *= lane_f64(rd, k);
             asm volatile("" : "+v"(a[k]), "+v"(b[k]));
 #pragma unroll
             for (int m = k + 1; m < R; ++m) b[m] -= lane_f64(a[k], m) * b[k];
         }
 #pragma unroll
     for (int k = R - 1; k >= 0; --k) {
-        const double rk = lane_f64(rd, k);
-        b[k] = rk != 0.0 ? b[k] * rk : 0.0;
+        b[k] *= lane_f64(rd, k);
 #pragma unroll
         for (int m = 0; m < k; ++m) {
             asm volatile("" : "+v"(a[m]), "+v"(b[m]));
