@@ -31,6 +31,24 @@ int set_error(int code, const char* fmt, ...);
         if (rc_ != DTC_OK) return rc_; \
     } while (0)
 
+// Host waits.  hipStreamSynchronize and hipStreamQuery are not used for them: where several
+// threads launch on streams of their own, both have returned success at once with 0.2 to
+// 0.9 ms of work in flight, about once in ten million waits; an event recorded at that
+// moment was waited for every time.
+// Waits for everything enqueued on s so far.
+inline hipError_t stream_wait(hipStream_t s) {
+    hipEvent_t e;
+    hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+    if (rc != hipSuccess) return rc;
+    rc = hipEventRecord(e, s);
+    if (rc == hipSuccess) rc = hipEventSynchronize(e);
+    (void)hipEventDestroy(e);
+    return rc;
+}
+// Waits until *w, a page-locked word that work on s stores, is at least v: where more work is
+// enqueued behind it, or a copy of the results is saved.
+int wait_word(hipStream_t s, const unsigned long long* w, unsigned long long v);
+
 // ---------------------------------------------------------------- device buffers
 // Idle device memory and page-locked host words, kept from one call or object for the next.
 // hipFree waits for the device and unmaps: 40 us each, 5 ms after one 64^3 solve, 19 ms
@@ -75,7 +93,8 @@ struct CallEnd {
 };
 struct IdleOnExit {
     const hipStream_t& s;
-    ~IdleOnExit() { t_recycle = s && hipStreamSynchronize(s) == hipSuccess; }
+    bool waited = false;   // set by the function: nothing was enqueued after its last wait
+    ~IdleOnExit() { t_recycle = s && (waited || stream_wait(s) == hipSuccess); }
 };
 
 // Owning device allocation; allocation failure is reported as DTC_ERR_OOM.

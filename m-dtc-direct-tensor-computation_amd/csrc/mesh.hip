@@ -439,9 +439,11 @@ __global__ __launch_bounds__(SCAN_NT) void k_scan_apply(const int* __restrict__ 
     }
 }
 
+size_t scan_bytes(int64_t n) { return (size_t)((n + SCAN_TILE - 1) / SCAN_TILE) * sizeof(int); }
+
+// tmp: scan_bytes(n) at least, allocated before anything that uses it is in flight
 int scan_launch(const int* in, int* out, int64_t n, int* tot_dev, int* tot_host, DevMem& tmp, hipStream_t s) {
     const int64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-    DTC_TRY(tmp.ensure((size_t)tiles * sizeof(int)));
     k_scan_tiles<<<(unsigned)tiles, SCAN_NT, 0, s>>>(in, n, tmp.as<int>());
     if (tiles <= SCAN_LOOK) {
         k_scan_apply<true><<<(unsigned)tiles, SCAN_NT, 0, s>>>(in, n, tmp.as<int>(), out, tot_dev, tot_host);
@@ -459,8 +461,9 @@ int scan_exclusive_i32(const int* in, int* out, int64_t n, int64_t* total, DevMe
     if (n <= 0) { *total = 0; return DTC_OK; }
     HostWords w;
     DTC_TRY(w.alloc(sizeof(int)));
+    DTC_TRY(tmp.ensure(scan_bytes(n)));
     DTC_TRY(scan_launch(in, out, n, nullptr, (int*)w.p, tmp, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     *total = *(const volatile int*)w.p;
     w.recycle();
     return DTC_OK;
@@ -501,6 +504,7 @@ int mesh_build_device(const void* phi_dev, int kind, const int64_t n[3], int64_t
     DTC_TRY(m.bbox.ensure(6 * 4));
     DTC_TRY(m.tot.ensure(4 * 4));
     DTC_TRY(m.flag.ensure(nvox * 4));
+    DTC_TRY(m.scratch.ensure(scan_bytes(std::max(nvox, nmax))));
     if (!m.words.p) DTC_TRY(m.words.alloc(4 * 4));
     int* flag = m.flag.as<int>();
     int* tot = m.tot.as<int>();          // elements, nodes before filtering; elements, nodes kept
@@ -541,7 +545,7 @@ int mesh_build_device(const void* phi_dev, int kind, const int64_t n[3], int64_t
                                          m.keepN.as<int>());
     DTC_HIP(hipGetLastError());
     DTC_TRY(scan_launch(m.keepN.as<int>(), m.cref.as<int>(), nmax, tot + 3, hw + 3, m.scratch, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     const volatile int* h = hw;
     m.n_elems0 = h[0];
     m.n_nodes0 = h[1];

@@ -13,6 +13,7 @@
 // the same in one loop); ~3M points per domain are spread over the GPU and
 // reduced per block, then per domain.
 #include <cmath>
+#include <cstring>
 #include <mutex>
 
 #include "dtc_internal.hpp"
@@ -313,7 +314,20 @@ struct RotBufs {
     double* rv;
     int64_t* ri;
     RotState* st;
+    unsigned long long* host = nullptr;   // page-locked, zero: a word, then (from 8) the final states; null: copied
 };
+// The final states and then, when every wave's stores have arrived, the word to page-locked
+// memory (a search 0.29 -> 0.26 ms against a copy and an event)
+__global__ __launch_bounds__(NT) void k_post_states(const RotState* __restrict__ st, int jobs,
+                                                    unsigned long long* __restrict__ host) {
+    static_assert(sizeof(RotState) % 8 == 0, "whole words");
+    const unsigned long long* s = reinterpret_cast<const unsigned long long*>(st);
+    for (int i = threadIdx.x; i < jobs * (int)(sizeof(RotState) / 8); i += NT)
+        __hip_atomic_store(host + 8 + i, s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(host, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 constexpr size_t rot_ref_count(size_t n_dom) { return 2 * 2 * n_dom * REF_B; }
 
 // Grid sizes of the initial sweep for an initial step of step_deg degrees.
@@ -345,8 +359,15 @@ int rotation_search_core(const double* EE_host, int n_dom, double step_deg, doub
                                                         d.ri + in * nr, d.rv + to * nr, d.ri + to * nr, jj, div, num_zero);
     }
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipMemcpyAsync(J, d.st + jobs, (size_t)jobs * sizeof(RotState), hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    if (d.host) {
+        k_post_states<<<1, NT, 0, s>>>(d.st + jobs, jobs, d.host);
+        DTC_HIP(hipGetLastError());
+        DTC_TRY(wait_word(s, d.host, 1));
+        std::memcpy(J, d.host + 8, (size_t)jobs * sizeof(RotState));
+    } else {
+        DTC_HIP(hipMemcpyAsync(J, d.st + jobs, (size_t)jobs * sizeof(RotState), hipMemcpyDeviceToHost, s));
+        DTC_HIP(stream_wait(s));
+    }
     for (int k = 0; k < jobs; ++k) {
         out[k] = RotResult{};
         out[k].crit = J[k].crit;
@@ -366,6 +387,7 @@ int rotation_search_batch(const double* EE_host, int n_dom, double step_deg, dou
     rotation_grid(step_deg, &na, &ne, &bpd);
     CallEnd end;
     DevMem dEE, pv, pi_, rv, ri, st;
+    HostWords host;
     IdleOnExit idle{s};
     DTC_TRY(dEE.alloc((size_t)n_dom * 36 * 8));
     DTC_TRY(pv.alloc((size_t)n_dom * bpd * 2 * 8));
@@ -373,10 +395,14 @@ int rotation_search_batch(const double* EE_host, int n_dom, double step_deg, dou
     DTC_TRY(rv.alloc(rot_ref_count(n_dom) * 8));
     DTC_TRY(ri.alloc(rot_ref_count(n_dom) * 8));
     DTC_TRY(st.alloc((size_t)n_dom * 4 * sizeof(RotState)));
+    DTC_TRY(host.alloc(64 + (size_t)n_dom * 2 * sizeof(RotState)));
+    *host.word() = 0;
     const RotBufs d{dEE.as<double>(), pv.as<double>(), pi_.as<int64_t>(), rv.as<double>(), ri.as<int64_t>(),
-                    st.as<RotState>()};
+                    st.as<RotState>(), host.word()};
     std::vector<RotState> J((size_t)n_dom * 2);
-    return rotation_search_core(EE_host, n_dom, step_deg, num_zero, s, d, J.data(), out.data());
+    DTC_TRY(rotation_search_core(EE_host, n_dom, step_deg, num_zero, s, d, J.data(), out.data()));
+    idle.waited = true;
+    return DTC_OK;
 }
 
 // ---------------------------------------------------------------- no-allocation search

@@ -1775,10 +1775,13 @@ int batch_begin(SolverBatch& b, const dtc_domain_desc* d, int64_t n_dom) {
     b.h_dom.clear(); b.h_brick.clear(); b.h_elems.clear(); b.h_nodes.clear(); b.h_bnodes.clear(); b.h_status.clear();
     b.h_contrast.clear();
     b.n_slices = 0;   // the block PCG slices follow the batch's domains (block_setup)
-    DTC_HIP(hipStreamSynchronize(b.stream));
-    b.block_graph.reset();   // captured with the previous composition's buffers
-    Recycle idle(true);
-    b.d20.clear();
+    // captured with the previous composition's buffers, and filled by them
+    if (b.block_graph.e || !b.d20.empty()) {
+        DTC_HIP(stream_wait(b.stream));
+        b.block_graph.reset();
+        Recycle idle(true);
+        b.d20.clear();
+    }
     return DTC_OK;
 }
 
@@ -1845,7 +1848,7 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
     DTC_TRY(cnt.alloc((size_t)nbr * sizeof(int2)));
     k_brick_count<<<nbr, BX * BY * BZ, 0, s>>>(m.numLat.as<int>(), m.keepN.as<int>(), Lx, Ly, Lz, D.bnx, D.bny, (int2*)cnt.p);
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     std::vector<int> hc(nbr);
     int64_t hb = 0;
     for (int i = 0; i < nbr; ++i) {
@@ -1893,7 +1896,7 @@ int batch_add_domain(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& d,
     }
     k_emod<<<nb(nvox, 256), 256, 0, s>>>(m.keepE.as<int>(), modulus_dev, d.E, escale, nvox, b.emod.as<double>() + D.vox_off);
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     bl.recycle();
     b.h_brick.insert(b.h_brick.end(), mine.begin(), mine.end());
     b.h_dom.push_back(D);
@@ -1985,17 +1988,16 @@ void make_clusters(std::vector<DomInfo>& hd, const std::vector<BrickInfo>& hb, i
 int build_clusters(hipStream_t s, Clusters& c, const DevMem& brick, const DevMem& dom, const DevMem& lat2node,
                    const DevMem& emod, bool fine) {
     if (c.n == 0) return DTC_OK;
-    DevMem cnt;
+    HostWords cnt;
     DTC_TRY(cnt.alloc((size_t)c.n * 4));
     DTC_TRY(c.info.ensure(c.h.size() * sizeof(ClusterInfo)));
     DTC_HIP(hipMemcpyAsync(c.info.p, c.h.data(), c.h.size() * sizeof(ClusterInfo), hipMemcpyHostToDevice, s));
     k_cluster_elems<false><<<c.n, 256, 0, s>>>(c.info.as<ClusterInfo>(), brick.as<BrickInfo>(), dom.as<DomInfo>(),
-                                               lat2node.as<int>(), emod.as<double>(), cnt.as<int>(), nullptr, nullptr,
+                                               lat2node.as<int>(), emod.as<double>(), (int*)cnt.p, nullptr, nullptr,
                                                nullptr, nullptr, c.cap);
     DTC_HIP(hipGetLastError());
-    std::vector<int> hc(c.n);
-    DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)c.n * 4, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
+    const int* hc = (const int*)cnt.p;
     int64_t off = 0;
     for (int i = 0; i < c.n; ++i) {
         c.h[i].e_off = (int)off;
@@ -2014,7 +2016,6 @@ int build_clusters(hipStream_t s, Clusters& c, const DevMem& brick, const DevMem
                                               c.eown.as<uint2>(), fine ? c.eE64.as<double>() : nullptr,
                                               c.eE32.as<float>(), c.cap);
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(s));
     cnt.recycle();
     return DTC_OK;
 }
@@ -2087,7 +2088,7 @@ int batch_finalize(SolverBatch& b, int precision) {
         DTC_HIP(hipGetLastError());
         DTC_TRY(build_clusters(s, b.cl, b.brick, b.dom, b.lat2node, b.emod, true));
     }
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     b.precision = precision;
     return DTC_OK;
 }
@@ -2105,6 +2106,7 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
     DTC_TRY(b.z32.ensure(v0));
     DTC_TRY(b.t32.ensure(v0));
     DTC_TRY(b.d32.ensure(v0));
+    std::vector<DevMem> exist((size_t)L);   // of each level: lattice nodes of its voxels
     for (int l = 0; l < L; ++l) {
         Level& C = b.mg[l];
         const std::vector<DomInfo>& FD = l == 0 ? b.h_dom : b.mg[l - 1].h_dom;
@@ -2128,7 +2130,8 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
         C.n_vox = nvox;
         DTC_TRY(C.emod.ensure((size_t)std::max<int64_t>(nvox, 1) * 8));
         DTC_TRY(C.lat2node.ensure((size_t)std::max<int64_t>(nlat, 1) * 4));
-        DevMem ex, cnt;
+        DevMem& ex = exist[l];
+        HostWords cnt;
         DTC_TRY(ex.alloc((size_t)std::max<int64_t>(nlat, 1) * 4));
         DTC_TRY(cnt.alloc((size_t)std::max<int64_t>(nbt, 1) * 4));
         k_fill_i32b<<<nb(nlat, 256), 256, 0, s>>>(C.lat2node.as<int>(), nlat, -1);
@@ -2140,12 +2143,11 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
             k_exist<<<nb(cl, 256), 256, 0, s>>>(C.emod.as<double>() + D.vox_off, D.nx, D.ny, D.nz,
                                                ex.as<int>() + D.lat_off);
             k_brick_count_ex<<<D.bnx * D.bny * D.bnz, NO, 0, s>>>(ex.as<int>() + D.lat_off, D.nx + 1, D.ny + 1,
-                                                                   D.nz + 1, D.bnx, D.bny, cnt.as<int>() + boff[d]);
+                                                                   D.nz + 1, D.bnx, D.bny, (int*)cnt.p + boff[d]);
         }
         DTC_HIP(hipGetLastError());
-        std::vector<int> hc((size_t)std::max<int64_t>(nbt, 1));
-        DTC_HIP(hipMemcpyAsync(hc.data(), cnt.p, (size_t)nbt * 4, hipMemcpyDeviceToHost, s));
-        DTC_HIP(hipStreamSynchronize(s));
+        DTC_HIP(stream_wait(s));
+        const int* hc = (const int*)cnt.p;
         C.h_brick.clear();
         int64_t node = 0;
         for (size_t d = 0; d < C.h_dom.size(); ++d) {
@@ -2166,6 +2168,7 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
             D.brick_end = (int)C.h_brick.size();
             D.node_end = node;
         }
+        cnt.recycle();
         C.n_bricks = (int)C.h_brick.size();
         C.n_nodes = node;
         make_clusters(C.h_dom, C.h_brick, cluster_cap(node, true, DTC_FP32_REFINE), C.cl);
@@ -2206,9 +2209,10 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
                                           C.lat2node.as<int>(), C.ptab.as<int>());
             DTC_HIP(hipGetLastError());
         }
-        DTC_HIP(hipStreamSynchronize(s));
-        ex.recycle();
-        cnt.recycle();
+    }
+    if (L > 0) {
+        DTC_HIP(stream_wait(s));
+        for (DevMem& ex : exist) ex.recycle();
     }
     return DTC_OK;
 }
@@ -2680,7 +2684,7 @@ int pcg_iteration(SolverBatch& b, const WK<T>& wk, T* x, T* r, T* p, T* q, const
 int all_done(SolverBatch& b, const DevMem& flags, bool* out) {
     std::vector<int> h(b.n_dom);
     DTC_HIP(hipMemcpyAsync(h.data(), flags.p, (size_t)b.n_dom * 4, hipMemcpyDeviceToHost, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(stream_wait(b.stream));
     DTC_TRY(harvest_events(b));
     bool all = true;
     for (int v : h) all = all && (v != 0);
@@ -2732,7 +2736,7 @@ __global__ __launch_bounds__(64) void k_status(const int* __restrict__ done64, c
 int words_setup(SolverBatch& b) {
     const size_t need = 64 + (size_t)b.n_dom * STAT_N * 8;
     if (b.host_words.n < need) {
-        DTC_HIP(hipStreamSynchronize(b.stream));
+        if (b.host_words.p) DTC_HIP(stream_wait(b.stream));
         b.host_words.reset();
         DTC_TRY(b.host_words.alloc(need));
         *b.host_words.word() = 0;
@@ -2754,22 +2758,9 @@ int post_done(SolverBatch& b) {
 // waits for the summary of run number `run`
 int wait_done(SolverBatch& b, uint64_t run, bool* fin) {
     const unsigned long long* w = b.host_words.word();
-    for (uint32_t k = 1;; ++k) {
-        const unsigned long long v = __atomic_load_n(w, __ATOMIC_ACQUIRE);
-        if (v / 2 >= run) {
-            *fin = (v & 1) != 0;
-            return DTC_OK;
-        }
-        if (k % 64 == 0) std::this_thread::yield();
-        if (k % 4096 == 0) {   // a stream that ended without the word has failed
-            const hipError_t e = hipStreamQuery(b.stream);
-            if (e == hipSuccess && __atomic_load_n(w, __ATOMIC_ACQUIRE) / 2 < run)
-                return set_error(DTC_ERR_DEVICE, "the iterations ended without a summary");
-            if (e != hipSuccess && e != hipErrorNotReady)
-                return set_error(DTC_ERR_DEVICE, "hipStreamQuery: %s", hipGetErrorString(e));
-            if (e == hipErrorNotReady) (void)hipGetLastError();
-        }
-    }
+    DTC_TRY(wait_word(b.stream, w, 2 * run));
+    *fin = (__atomic_load_n(w, __ATOMIC_ACQUIRE) & 1) != 0;
+    return DTC_OK;
 }
 
 // status of every domain on the host (the stream is idle afterwards)
@@ -2778,7 +2769,7 @@ int read_status(SolverBatch& b, const double** out) {
     k_status<<<b.n_dom, 64, 0, b.stream>>>(b.done64.as<int>(), b.iters.as<int64_t>(), b.rr.as<double>(),
                                            b.rr0.as<double>(), b.host_words.status());
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(stream_wait(b.stream));
     *out = b.host_words.status();
     return DTC_OK;
 }
@@ -2829,8 +2820,10 @@ int launch_mv_q64(SolverBatch& b, const float* p, float* q, const int* done, dou
 // the per-domain factor and coefficient storage
 int block_setup(SolverBatch& b) {
     if (b.n_slices > 0) return DTC_OK;
-    std::vector<int4> sl;
-    std::vector<int> ds((size_t)b.n_dom + 1);
+    std::vector<int4>& sl = b.h_slices;
+    std::vector<int>& ds = b.h_dslice;
+    sl.clear();
+    ds.assign((size_t)b.n_dom + 1, 0);
     for (int d = 0; d < b.n_dom; ++d) {
         ds[d] = (int)sl.size();
         const DomInfo& D = b.h_dom[d];
@@ -2851,7 +2844,6 @@ int block_setup(SolverBatch& b) {
     if (!sl.empty())
         DTC_HIP(hipMemcpyAsync(b.slices.p, sl.data(), sl.size() * sizeof(int4), hipMemcpyHostToDevice, b.stream));
     DTC_HIP(hipMemcpyAsync(b.dslice.p, ds.data(), ds.size() * 4, hipMemcpyHostToDevice, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
     b.n_slices = (int)sl.size();
     return DTC_OK;
 }
@@ -2999,7 +2991,7 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
                 b.graph_mode == (int)b.block64;
     for (int k = 0; k < 6; ++k) same = same && b.graph_key[k] == key[k];
     if (!same) {
-        if (b.block_graph.e) DTC_HIP(hipStreamSynchronize(s));   // no replay of the old one is in flight
+        if (b.block_graph.e) DTC_HIP(stream_wait(s));   // no replay of the old one is in flight
         b.block_graph.reset();
         DTC_TRY(words_setup(b));
         hipGraph_t g = nullptr;
@@ -3034,7 +3026,7 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
     for (int64_t steps = 0; steps < total && !fin; steps += RUN) {
         const int rc = run(steps);
         if (rc != DTC_OK) {
-            (void)hipStreamSynchronize(s);   // nothing is in flight when the caller gives up
+            (void)stream_wait(s);   // nothing is in flight when the caller gives up
             return rc;
         }
         // DTC_TRACE=1: a progress line every 1,000 block iterations of a long phase
@@ -3150,7 +3142,8 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
     // case (it keeps its direction over a replacement)
     const dtc_solve_opts& o = opts;
     if (D > 0) {
-        std::vector<double> it2(D);
+        std::vector<double>& it2 = b.h_itol2;
+        it2.resize(D);
         for (int d = 0; d < D; ++d) {
             double t = o.inner_tol;
             if (!(t > 0.0 && t < 1.0)) {
@@ -3161,7 +3154,6 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         }
         DTC_TRY(b.itol2.ensure((size_t)D * 8));
         DTC_HIP(hipMemcpyAsync(b.itol2.p, it2.data(), (size_t)D * 8, hipMemcpyHostToDevice, b.stream));
-        DTC_HIP(hipStreamSynchronize(b.stream));
     }
     iters.assign(D, 0);
     outer.assign(D, 0);
@@ -3204,7 +3196,7 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
         DTC_TRY(b.dom_bytes.ensure(db.size() * 8));
         DTC_TRY(b.launch_bytes.ensure((size_t)MAX_SLOTS * 2 * 8));
         DTC_HIP(hipMemcpyAsync(b.dom_bytes.p, db.data(), db.size() * 8, hipMemcpyHostToDevice, s));
-        DTC_HIP(hipStreamSynchronize(s));
+        DTC_HIP(stream_wait(s));
         b.n_slots = 0;
     }
     std::vector<int64_t> nouter(D, 0);
@@ -3358,7 +3350,10 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
 int batch_forces(SolverBatch& b, std::vector<double>& ff) {
     const int D = b.n_dom;
     ff.assign((size_t)D * R * FFD, 0.0);
-    if (D == 0 || b.n_bricks == 0) return DTC_OK;
+    if (D == 0 || b.n_bricks == 0) {
+        DTC_HIP(stream_wait(b.stream));
+        return DTC_OK;
+    }
     const WK<double> wk64 = cast_wk<double>(b.wk64);
     // reactions on the unmodified operator: rf = K (x + x_bc), stored in r64
     DTC_TRY((launch_mv<double, IN_U, OUT_PLAIN>(b, wk64, b.x64.as<double>(), b.r64.as<double>(), nullptr, nullptr)));
@@ -3376,7 +3371,7 @@ int batch_forces(SolverBatch& b, std::vector<double>& ff) {
                                                                                 b.part_ff.as<double>(), b.ff.as<double>());
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(ff.data(), b.ff.p, ff.size() * 8, hipMemcpyDeviceToHost, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(stream_wait(b.stream));
     b.reactions_valid = true;
     return DTC_OK;
 }
@@ -3402,7 +3397,7 @@ int batch_fields(SolverBatch& b, int i, int ncol, double* u_out, double* r_out) 
     }
     if (u_out) DTC_HIP(hipMemcpyAsync(u_out, du.p, bytes, hipMemcpyDeviceToHost, b.stream));
     if (r_out) DTC_HIP(hipMemcpyAsync(r_out, dr.p, bytes, hipMemcpyDeviceToHost, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(stream_wait(b.stream));
     du.recycle();
     dr.recycle();
     return DTC_OK;
@@ -3430,7 +3425,7 @@ int batch_grad(SolverBatch& b, int i, int ng, const double* M, double* dL_dE_hos
                                                      g.as<double>());
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(dL_dE_host, g.p, (size_t)nvox * 8, hipMemcpyDeviceToHost, b.stream));
-    DTC_HIP(hipStreamSynchronize(b.stream));
+    DTC_HIP(stream_wait(b.stream));
     for (DevMem* m : {&h, &Md, &g}) m->recycle();
     return DTC_OK;
 }

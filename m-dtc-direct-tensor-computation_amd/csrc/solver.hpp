@@ -117,6 +117,9 @@ struct SolverBatch {
     // block PCG of the mixed multigrid solve (the 24 load cases of a domain share one Krylov block)
     int n_slices = 0;
     DevMem slices;                 // int4 [slice]: domain, first node, end node
+    std::vector<int4> h_slices;    // (the sources of uploads stay: nothing waits for them)
+    std::vector<int> h_dslice;
+    std::vector<double> h_itol2;
     DevMem dslice;                 // int [dom + 1]: first slice of each domain
     DevMem gpart;                  // double [slice][2][24 x 24]: Gram partial sums
     DevMem gsum;                   // double [dom][2][24 x 24]: Gram sums

@@ -495,7 +495,7 @@ int batch_add_domain20(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& 
                                        cnt.as<int>() + nn);
     int hb = 0;
     DTC_HIP(hipMemcpyAsync(&hb, cnt.as<int>() + nn, 4, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     if (3 * hb < 6) {
         DTC_TRY(batch_add_empty(b, d, DTC_ERR_FEW_CONSTRAINTS, lc_base));
         b.h_elems.back() = ne;
@@ -536,7 +536,7 @@ int batch_add_domain20(SolverBatch& b, const MeshDev& m, const dtc_domain_desc& 
     D.vox_off = b.n_vox;
     G.node_begin = b.n_nodes;
     G.n_nodes = nn;
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     for (DevMem* t : {&e64, &dimd, &cnt, &cursor}) t->recycle();
     b.d20.push_back(std::move(G));
     b.h_dom.push_back(D);
@@ -587,7 +587,7 @@ int finalize20(SolverBatch& b) {
             k20_dinv<<<nb(h[i].n_nodes, 256), 256, 0, s>>>(h[i], b.k20_64.as<double>(), h[i].node_begin,
                                                            b.dinv64.as<double>(), b.dinv32.as<float>());
     DTC_HIP(hipGetLastError());
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     return DTC_OK;
 }
 
@@ -688,7 +688,7 @@ int grad20(SolverBatch& b, int i, int ng, const double* M, double* dL_dE_host) {
     }
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(dL_dE_host, g.p, (size_t)nvox * 8, hipMemcpyDeviceToHost, s));
-    DTC_HIP(hipStreamSynchronize(s));
+    DTC_HIP(stream_wait(s));
     for (DevMem* m : {&h, &Md, &g}) m->recycle();
     return DTC_OK;
 }
