@@ -60,7 +60,8 @@ int wait_word(hipStream_t s, const unsigned long long* w, unsigned long long v);
 // when an allocation fails or the program asks (dtc_release_memory).  Streams are not kept: kept ones end up on one hardware queue,
 // and the parts of a batch no longer overlap (40 domains of 21^3 61 -> 70 ms).
 constexpr size_t POOL_BYTES = (size_t)4 << 30;
-constexpr size_t POOL_PINNED = 8;
+// (page-locked: blocks kept, and the largest; a multigrid solve takes up to a dozen sizes)
+constexpr size_t POOL_PINNED = 32, POOL_PINNED_BYTES = (size_t)1 << 20;
 constexpr double POOL_SECONDS = 20.0;
 // allocation size of an n-byte request: up to 1/8 more, so that requests of nearby sizes
 // meet; 2 MiB steps from 16 MiB on

@@ -5,7 +5,6 @@
 #include <list>
 #include <map>
 #include <mutex>
-#include <vector>
 
 #include "dtc_internal.hpp"
 
@@ -27,7 +26,7 @@ struct Pool {
     std::list<Block> idle;                                                         // newest first
     std::multimap<std::pair<int, size_t>, std::list<Block>::iterator> by_size;
     size_t bytes = 0;
-    std::vector<std::pair<void*, size_t>> pinned;
+    std::list<Block> pinned;                                                       // page-locked words, newest first
 
     // unlinks the oldest blocks while over the bound or past their time; the caller frees them
     void expire(std::list<Block>& out, size_t bound) {
@@ -42,6 +41,14 @@ struct Pool {
             out.splice(out.begin(), idle, last);
         }
     }
+
+    // the same for the page-locked words
+    void expire_pinned(std::list<Block>& out, size_t bound) {
+        const Clock::time_point now = Clock::now();
+        while (!pinned.empty() && (pinned.size() > bound ||
+                                   std::chrono::duration<double>(now - pinned.back().since).count() > POOL_SECONDS))
+            out.splice(out.begin(), pinned, std::prev(pinned.end()));
+    }
 };
 
 // never destroyed: the runtime may be gone when static objects are
@@ -52,6 +59,10 @@ Pool& pool() {
 
 void free_blocks(const std::list<Pool::Block>& v) {
     for (const Pool::Block& b : v) (void)hipFree(b.p);
+}
+
+void free_words(const std::list<Pool::Block>& v) {
+    for (const Pool::Block& b : v) (void)hipHostFree(b.p);
 }
 
 }  // namespace
@@ -99,42 +110,50 @@ void pool_put(void* p, size_t n, int dev) {
 
 void pool_trim() {
     Pool& P = pool();
-    std::list<Pool::Block> old;
-    std::vector<std::pair<void*, size_t>> words;
+    std::list<Pool::Block> old, words;
     {
         std::lock_guard<std::mutex> lk(P.mu);
         P.expire(old, 0);
         words.swap(P.pinned);
     }
     free_blocks(old);
-    for (const auto& w : words) (void)hipHostFree(w.first);
+    free_words(words);
 }
 
 void* pool_take_pinned(size_t n) {
     Pool& P = pool();
-    std::lock_guard<std::mutex> lk(P.mu);
-    for (size_t i = P.pinned.size(); i-- > 0;)
-        if (P.pinned[i].second == n) {
-            void* p = P.pinned[i].first;
-            P.pinned.erase(P.pinned.begin() + (ptrdiff_t)i);
-            return p;
-        }
-    return nullptr;
+    void* p = nullptr;
+    std::list<Pool::Block> old;
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        for (auto it = P.pinned.begin(); it != P.pinned.end(); ++it)
+            if (it->n == n) {
+                p = it->p;
+                P.pinned.erase(it);
+                break;
+            }
+        P.expire_pinned(old, POOL_PINNED);
+    }
+    free_words(old);
+    return p;
 }
 
 void pool_put_pinned(void* p, size_t n) {
     Pool& P = pool();
+    std::list<Pool::Block> old;
     {
         std::lock_guard<std::mutex> lk(P.mu);
-        if (n <= ((size_t)1 << 20) && P.pinned.size() < POOL_PINNED) {
-            try {
-                P.pinned.emplace_back(p, n);
-                return;
-            } catch (...) {
-            }
+        std::list<Pool::Block> one;
+        if (n <= POOL_PINNED_BYTES) try {
+            one.push_front({p, n, 0, Pool::Clock::now()});
+            P.pinned.splice(P.pinned.begin(), one);
+            p = nullptr;
+        } catch (...) {
         }
+        P.expire_pinned(old, POOL_PINNED);
     }
-    (void)hipHostFree(p);
+    if (p) (void)hipHostFree(p);
+    free_words(old);
 }
 
 }  // namespace dtc

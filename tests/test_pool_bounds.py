@@ -81,10 +81,31 @@ static int release() {                     // everything idle, device and page-l
     CHECK(pool_take(5 * MB, 1) == at(5));
     return 0;
 }
+static int words() {                       // page-locked words: a fixed number stays whatever their sizes, the oldest go first
+    const size_t N = POOL_PINNED;
+    for (size_t k = 1; k <= N; ++k) pool_put_pinned(at(k), 4096 * (k + 1));       // sizes that never come back
+    CHECK(freed_host.empty());
+    pool_put_pinned(at(N + 1), 4096);
+    CHECK(freed_host.size() == 1 && freed_host[0] == 1);
+    CHECK(pool_take_pinned(4096) == at(N + 1) && !pool_take_pinned(4096));        // the next call of that size finds it
+    pool_put_pinned(at(N + 2), 4096);
+    pool_put_pinned(at(N + 3), ((size_t)1 << 20) + 4096);                         // larger than 1 MiB: not kept
+    CHECK(freed_host.size() == 2 && freed_host[1] == N + 3);
+    return 0;
+}
+static int words_age() {
+    pool_put_pinned(at(1), 4096);
+    now_s = POOL_SECONDS - 1.0;
+    pool_put_pinned(at(2), 8192);
+    CHECK(freed_host.empty());
+    now_s = POOL_SECONDS + 1.0;
+    CHECK(pool_take_pinned(8192) == at(2) && freed_host.size() == 1 && freed_host[0] == 1);
+    return 0;
+}
 int main(int, char** argv) {
     const std::string t = argv[1];
     return t == "bound" ? bound() : t == "large" ? large() : t == "age" ? age() : t == "device" ? device()
-         : t == "release" ? release() : 2;
+         : t == "release" ? release() : t == "words" ? words() : t == "words_age" ? words_age() : 2;
 }
 """
 
@@ -99,7 +120,7 @@ def program(tmp_path_factory):
     return str(d / "m")
 
 
-@pytest.mark.parametrize("what", ["bound", "large", "age", "device", "release"])
+@pytest.mark.parametrize("what", ["bound", "large", "age", "device", "release", "words", "words_age"])
 def test_pool(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
