@@ -7,7 +7,9 @@
 // several of those bricks is taken in the brick that holds its lowest node of the
 // cluster.  FILL = false counts them; FILL = true writes them in descending
 // lexicographic order of their voxels (rank by counting, in LDS), so that the matvec
-// adds a node's contributions in corner order 0..7 whatever the clusters are.
+// adds a node's contributions in corner order 0..7 whatever the clusters are.  Behind the
+// last cluster's elements FILL writes a spare record (nodes 0, modulus 0): a last cluster
+// without an element reads it.
 template <bool FILL>
 __global__ __launch_bounds__(256) void k_cluster_elems(const ClusterInfo* __restrict__ cl, const BrickInfo* __restrict__ bricks,
                                                        const DomInfo* __restrict__ doms, const int* __restrict__ lat2node,
@@ -68,6 +70,13 @@ __global__ __launch_bounds__(256) void k_cluster_elems(const ClusterInfo* __rest
             const double e = emod[D.vox_off + v];
             if (eE64) eE64[o] = e;
             eE32[o] = (float)e;
+        }
+        if (blockIdx.x == gridDim.x - 1 && tid == 0) {
+            const int64_t o = (int64_t)C.e_off + n;
+            enode[2 * o] = enode[2 * o + 1] = make_int4(0, 0, 0, 0);
+            eown[o] = make_uint2(cap * 0x01010101u, cap * 0x01010101u);
+            if (eE64) eE64[o] = 0.0;
+            eE32[o] = 0.f;
         }
     }
 }
@@ -143,8 +152,8 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
     const uint2* __restrict__ eo = A.eown + C.e_off;
     const T* __restrict__ eE = static_cast<const T*>(A.eE) + C.e_off;
     const T* __restrict__ dinv = static_cast<const T*>(A.dinv);
-    // A cluster has no element where every voxel around its nodes is solid with modulus 0:
-    // then no record is read (there is none to repeat) and the rows leave as sums of nothing.
+    // (A cluster has no element where every voxel around its nodes is solid with modulus 0: it
+    // reads the record at its offset, the next cluster's or the spare one at the end.)
     // Software pipeline: the records of the group after next and x of the next group are
     // loaded while the current group is computed.  Lanes past the last element repeat it
     // into the row that is not read; nothing is selected from a loaded record before it
@@ -153,8 +162,9 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
     int4 n0, n1;
     uint2 ow;
     T E;
+    const int last = max(ne - 1, 0);
     auto fetch = [&](int e) {
-        const int i = min(e, ne - 1);
+        const int i = min(e, last);
         n0 = en[2 * i];
         n1 = en[2 * i + 1];
         ow = eo[i];
@@ -172,17 +182,13 @@ __global__ __launch_bounds__(64 * R / LCW) void k_ebe(EbeArgs A, WK<T> wk, const
             if constexpr (IN == IN_JS) sc[b] = dinv[(int64_t)nd[b] * 3];
         }
     };
-    if (ne > 0) fetch(le);
+    fetch(le);
     if (A.done && A.done[C.dom]) return;
     for (int i = tid; i < nv; i += NT) vzero(s_yv[i]);
-    uint2 oc;
-    T Ec;
-    if (ne > 0) {
-        gather();
-        oc = ow;
-        Ec = E;
-        fetch(EPW + le);
-    }
+    gather();
+    uint2 oc = ow;
+    T Ec = E;
+    fetch(EPW + le);
     __syncthreads();
     for (int e0 = 0; e0 < ne; e0 += EPW) {
         T y[8][3];

@@ -2006,7 +2006,7 @@ int build_clusters(hipStream_t s, Clusters& c, const DevMem& brick, const DevMem
     }
     if (off >= INT32_MAX) return set_error(DTC_ERR_BAD_ARGUMENT, "batch exceeds %d cluster elements", INT32_MAX);
     DTC_HIP(hipMemcpyAsync(c.info.p, c.h.data(), c.h.size() * sizeof(ClusterInfo), hipMemcpyHostToDevice, s));
-    const size_t ne = (size_t)(off > 0 ? off : 1);
+    const size_t ne = (size_t)off + 1;   // and the spare record
     DTC_TRY(c.enode.ensure(ne * 32));
     DTC_TRY(c.eown.ensure(ne * 8));
     if (fine) DTC_TRY(c.eE64.ensure(ne * 8));
