@@ -145,6 +145,8 @@ struct SolverBatch {
     DevMem ye20;                   // [element][60][24] element forces (FP32 or FP64) of the two-pass operator
     DevMem ebase20;                // int64 [group]: first element of each domain group in ye20
     std::vector<int64_t> h_ebase20;
+    DevMem wgs20;                  // int4 [workgroup] of the element pass, FP32 and then FP64 (elem_groups)
+    unsigned n_wgs20[2] = {0, 0};
     std::vector<double> khat20;    // E = 1 element stiffness, 60 x 60
     DevMem k20_64, k20_32;
     WalshK wk64{};

@@ -16,6 +16,7 @@
 #include <cmath>
 
 #include "bc.hpp"
+#include "elem_groups.hpp"
 #include "solver.hpp"
 
 namespace dtc {
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(NT20) void k_fields20(const BrickInfo* __restrict__
 // staged in LDS with a padded row stride.  Lane layout of the 16x16x4 products
 // (l = lane, measured on gfx950): A[i][k] in lane i + 16 k, B[k][j] in lane
 // j + 16 k; D[i][j] in lane j + 16 (i / 4), component i % 4 (f32), and in lane
-// j + 16 (i % 4), component i / 4 (f64).  blockIdx.y: domain group.  A 27^3 domain
+// j + 16 (i % 4), component i / 4 (f64).  A 27^3 domain
 // (5,800 elements): 22 us in FP32 (the products take 8 at the rate of a large FP32 matrix
 // product, the 33 MB of forces as long), 31 us in FP64; the gather then 13.  The FP64
 // residual in one gather kernel, 60 products per entry on the vector units, took 4,500.
@@ -233,19 +234,19 @@ template <> struct EmCfg<double> {
 };
 
 template <typename T, typename TX>
-__global__ __launch_bounds__(256) void k20_elem(const Dom20Dev* __restrict__ d20, const int64_t* __restrict__ ebase,
+__global__ __launch_bounds__(256) void k20_elem(const Dom20Dev* __restrict__ d20, const int4* __restrict__ wgs,
                                                 const int* __restrict__ done, const T* __restrict__ Kg,
                                                 const TX* __restrict__ x, T* __restrict__ yall) {
     constexpr int EM = EmCfg<T>::EM, XS = EmCfg<T>::XS, NCT = 24 * EM / 16;
     using V4 = typename EmCfg<T>::V4;
     __shared__ T sX[60 * XS];
     __shared__ T sE[EM];
-    const int dom = blockIdx.y;
+    const int4 W = wgs[blockIdx.x];
+    const int dom = W.x;
     if (done && done[dom]) return;
-    const int64_t ne = ebase[dom + 1] - ebase[dom], e0 = (int64_t)blockIdx.x * EM;
-    if (e0 >= ne) return;
+    const int64_t ne = W.z, e0 = W.y;
     const Dom20Dev G = d20[dom];
-    T* __restrict__ ye = yall + ebase[dom] * 60 * R;
+    T* __restrict__ ye = yall + (int64_t)W.w * 60 * R;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // X: 20 nodes x 72 contiguous values per element, read as 16-byte vectors
     constexpr int VX = 16 / sizeof(TX), NVX = 72 / VX;
@@ -386,12 +387,11 @@ inline unsigned nb(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 // element forces of every domain group into ye20
 template <typename T, typename TX>
 int elem_pass(SolverBatch& b, const TX* x, const int* done) {
-    int64_t most = 0;
-    for (int g = 0; g < b.n_dom; ++g) most = std::max(most, b.h_ebase20[g + 1] - b.h_ebase20[g]);
-    if (most == 0) return DTC_OK;
+    constexpr int V = sizeof(T) == 8;
+    if (b.n_wgs20[V] == 0) return DTC_OK;
     const T* K = sizeof(T) == 8 ? (const T*)b.k20_64.p : (const T*)b.k20_32.p;
-    k20_elem<T, TX><<<dim3(nb(most, EmCfg<T>::EM), b.n_dom), 256, 0, b.stream>>>(
-        b.d20dev.as<Dom20Dev>(), b.ebase20.as<int64_t>(), done, K, x, b.ye20.as<T>());
+    k20_elem<T, TX><<<b.n_wgs20[V], 256, 0, b.stream>>>(b.d20dev.as<Dom20Dev>(), b.wgs20.as<int4>() + V * b.n_wgs20[0],
+                                                      done, K, x, b.ye20.as<T>());
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
@@ -572,6 +572,13 @@ int finalize20(SolverBatch& b) {
     b.h_ebase20[b.n_dom] = ne_all;
     DTC_TRY(b.ebase20.ensure(b.h_ebase20.size() * 8));
     DTC_HIP(hipMemcpyAsync(b.ebase20.p, b.h_ebase20.data(), b.h_ebase20.size() * 8, hipMemcpyHostToDevice, s));
+    if (ne_all >= INT32_MAX) return set_error(DTC_ERR_BAD_ARGUMENT, "batch exceeds %d elements", INT32_MAX);
+    std::vector<int4> wgs = elem_groups(b.h_ebase20, EmCfg<float>::EM);
+    b.n_wgs20[0] = (unsigned)wgs.size();
+    for (const int4& w : elem_groups(b.h_ebase20, EmCfg<double>::EM)) wgs.push_back(w);
+    b.n_wgs20[1] = (unsigned)wgs.size() - b.n_wgs20[0];
+    DTC_TRY(b.wgs20.ensure(std::max<size_t>(wgs.size(), 1) * sizeof(int4)));
+    if (!wgs.empty()) DTC_HIP(hipMemcpyAsync(b.wgs20.p, wgs.data(), wgs.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     // FP64 element forces of the block's Q = K P, FP32 ones of the smoothing steps (one buffer)
     DTC_TRY(b.ye20.ensure((size_t)std::max<int64_t>(ne_all, 1) * 60 * R * 8));
     DTC_TRY(b.d20dev.ensure(std::max<size_t>(h.size(), 1) * sizeof(Dom20Dev)));
