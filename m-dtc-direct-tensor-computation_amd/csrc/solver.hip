@@ -2060,7 +2060,7 @@ int batch_finalize(SolverBatch& b, int precision) {
     DTC_TRY(b.part_a.ensure(nbk * R * 8));
     DTC_TRY(b.part_b.ensure(nbk * R * 8));
     DTC_TRY(b.part_c.ensure(nbk * R * 8));
-    DTC_TRY(b.part_ff.ensure(nbk * R * FFD * 8));
+    if (!b.micro20) DTC_TRY(b.part_ff.ensure((size_t)std::max(b.n_bricks, 1) * R * FFD * 8));
     const size_t nd = (size_t)(b.n_dom > 0 ? b.n_dom : 1);
     for (DevMem* m : {&b.alpha, &b.beta, &b.rz, &b.rr, &b.rr0, &b.thr2, &b.scale}) DTC_TRY(m->ensure(nd * R * 8));
     DTC_TRY(b.active.ensure(nd * R * 4));
@@ -3362,13 +3362,13 @@ int batch_forces(SolverBatch& b, std::vector<double>& ff) {
     } else {
         k_project<8><<<b.n_bricks, NT_UPD, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(),
                                                           b.lat2node.as<int>(), b.r64.as<double>(),
-                                                          b.part_ff.as<double>());
+                                                          b.force_partials());
         k_project<20><<<b.n_bricks, NT_UPD, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(),
                                                            b.lat2node.as<int>(), b.r64.as<double>(),
-                                                           b.part_ff.as<double>());
+                                                           b.force_partials());
     }
     k_red_ff<<<dim3(D, (R * FFD + RFF_E - 1) / RFF_E), RFF_E * RFF_P, 0, b.stream>>>(b.dom.as<DomInfo>(),
-                                                                                b.part_ff.as<double>(), b.ff.as<double>());
+                                                                                b.force_partials(), b.ff.as<double>());
     DTC_HIP(hipGetLastError());
     DTC_HIP(hipMemcpyAsync(ff.data(), b.ff.p, ff.size() * 8, hipMemcpyDeviceToHost, b.stream));
     DTC_HIP(stream_wait(b.stream));

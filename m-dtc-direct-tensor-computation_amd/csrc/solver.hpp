@@ -100,7 +100,7 @@ struct SolverBatch {
     DevMem x32, r32, p32, q32;
     // per-brick partial sums
     DevMem part_a, part_b, part_c; // [brick][24]
-    DevMem part_ff;                // [brick][24 lc][60 macro DOF slots]
+    DevMem part_ff;                // [brick][24 lc][60 macro DOF slots] (HEX20: in ye20, idle then)
     // per-domain scalars [dom][24]
     DevMem alpha, beta, rz, rr, rr0, thr2, scale;
     DevMem active, active64;       // int [dom][24]
@@ -143,6 +143,7 @@ struct SolverBatch {
     DevMem d20dev;                 // Dom20Dev[]
     std::vector<Dom20Dev> h_d20dev;   // host copy
     DevMem ye20;                   // [element][60][24] element forces (FP32 or FP64) of the two-pass operator
+    double* force_partials() const { return (micro20 ? ye20 : part_ff).as<double>(); }
     DevMem ebase20;                // int64 [group]: first element of each domain group in ye20
     std::vector<int64_t> h_ebase20;
     DevMem wgs20;                  // int4 [workgroup] of the element pass, FP32 and then FP64 (elem_groups)

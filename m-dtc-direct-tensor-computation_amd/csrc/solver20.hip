@@ -580,7 +580,10 @@ int finalize20(SolverBatch& b) {
     DTC_TRY(b.wgs20.ensure(std::max<size_t>(wgs.size(), 1) * sizeof(int4)));
     if (!wgs.empty()) DTC_HIP(hipMemcpyAsync(b.wgs20.p, wgs.data(), wgs.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     // FP64 element forces of the block's Q = K P, FP32 ones of the smoothing steps (one buffer)
-    DTC_TRY(b.ye20.ensure((size_t)std::max<int64_t>(ne_all, 1) * 60 * R * 8));
+    // (also the force partials, which take as much a pseudo-brick as it takes an element: never
+    // more of them, 20 ne nodes in bricks of 32)
+    static_assert(FFD == 60, "element forces and force partials: 60 rows of 24 load cases");
+    DTC_TRY(b.ye20.ensure((size_t)std::max<int64_t>({ne_all, b.n_bricks, 1}) * 60 * R * 8));
     DTC_TRY(b.d20dev.ensure(std::max<size_t>(h.size(), 1) * sizeof(Dom20Dev)));
     if (!h.empty()) DTC_HIP(hipMemcpyAsync(b.d20dev.p, h.data(), h.size() * sizeof(Dom20Dev), hipMemcpyHostToDevice, s));
     std::vector<float> k32(3600);
@@ -601,10 +604,10 @@ int finalize20(SolverBatch& b) {
 int project20(SolverBatch& b) {
     if (b.n_bricks == 0) return DTC_OK;
     k_project20<8><<<b.n_bricks, NT20, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(),
-                                                      b.d20dev.as<Dom20Dev>(), b.r64.as<double>(), b.part_ff.as<double>());
+                                                      b.d20dev.as<Dom20Dev>(), b.r64.as<double>(), b.force_partials());
     k_project20<20><<<b.n_bricks, NT20, 0, b.stream>>>(b.brick.as<BrickInfo>(), b.dom.as<DomInfo>(),
                                                        b.d20dev.as<Dom20Dev>(), b.r64.as<double>(),
-                                                       b.part_ff.as<double>());
+                                                       b.force_partials());
     DTC_HIP(hipGetLastError());
     return DTC_OK;
 }
