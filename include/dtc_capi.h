@@ -117,7 +117,8 @@ typedef struct {
     double rot_step_deg;    /* initial grid step of the rotation search (1 = reference) */
     double num_zero;        /* refinement stop |dmin| < num_zero (1e-9 in mod_tensor_opt.f90:61) */
     int precond;            /* DTC_PC_JACOBI or DTC_PC_MG (FP32_REFINE only) */
-    int mg_degree;          /* Chebyshev degree per smoothing pass of the finest level (0 = default 2) */
+    int mg_degree;          /* Chebyshev degree per smoothing pass of the finest and intermediate
+                               levels (0 = default: 2 on the finest, 4 on the others) */
 } dtc_solve_opts;
 
 typedef struct {

@@ -663,7 +663,7 @@ int dtc_batch_run(dtc_batch* b, dtc_domain_result* res) {
         // whose coarse space is the HEX08 twin of the same voxels and domain groups
         sb.precond = (precision == DTC_FP32_REFINE && b->o.precond == DTC_PC_MG) ? DTC_PC_MG : DTC_PC_JACOBI;
         DTC_TRY(batch_finalize(sb, precision));
-        sb.mg_degree = b->o.mg_degree > 0 ? b->o.mg_degree : 2;
+        sb.mg_degree = std::max(b->o.mg_degree, 0);
         sb.p08 = nullptr;
         if (sb.micro20 && sb.precond == DTC_PC_MG) {
             SolverBatch& tw = S.sb08;

@@ -2429,9 +2429,11 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     const int* done = b.done_ext ? b.done_ext : b.done.as<int>();
     static const MgParams P = mg_params();
     // (the twin's finest level is an intermediate level of the p-multigrid)
-    const int deg0 = b.mg_degree > 0 ? b.mg_degree : 2, ldeg = std::max(P.level_degree, deg0);
+    const bool given = b.mg_degree > 0;   // by the caller: the intermediate levels take it too
+    const int deg0 = given ? b.mg_degree : 2, ldeg = given ? deg0 : std::max(P.level_degree, deg0);
+    const double lratio = given ? P.fine_ratio(deg0) : P.level_ratio;
     const int deg = b.done_ext ? ldeg : deg0;
-    const double ratio0 = b.done_ext ? P.level_ratio : P.fine_ratio(deg0);
+    const double ratio0 = b.done_ext ? lratio : P.fine_ratio(deg0);
     auto view = [&](int l) {
         LvView v;
         if (l == 0) {
@@ -2532,7 +2534,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
     // coarse_degree - 1): start in the buffer that makes it end in z
     cur[0] = (L > 0 ? 2 * deg - 1 : one_launch ? 0 : P.coarse_degree - 1) % 2;
     for (int l = 0; l < L; ++l) {
-        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, true, l == 0 ? ratio0 : P.level_ratio));
+        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, true, l == 0 ? ratio0 : lratio));
         const LvView f = view(l), c = view(l + 1);
         cur[l + 1] = 0;
         if (c.T.n_bricks == 0 || f.T.n_bricks == 0) continue;
@@ -2551,7 +2553,7 @@ int mg_vcycle(SolverBatch& b, const WK<float>& wk, const float* r, float* z, dou
                 f.T.bricks, b.mg[l].ptab.as<int>(), done, c.buf[cur[l + 1]], f.buf[cur[l]]);
             DTC_HIP(hipGetLastError());
         }
-        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, false, l == 0 ? ratio0 : P.level_ratio));
+        DTC_TRY(smooth(l, l == 0 ? deg : ldeg, false, l == 0 ? ratio0 : lratio));
     }
     if (prz && b.n_bricks > 0) {
         k_dot<<<b.n_bricks, NT_UPD, 0, s>>>(b.brick.as<BrickInfo>(), done, r, z, prz);

@@ -128,7 +128,7 @@ struct SolverBatch {
     bool block_q64 = false;        // Q = A P in FP64 arithmetic
     bool block64 = false;          // block PCG on FP64 vectors (x, r, Q) with the FP32 V-cycle
     int precond = 0;               // DTC_PC_JACOBI / DTC_PC_MG
-    int mg_degree = 2;             // Chebyshev degree of the fine and intermediate levels
+    int mg_degree = 0;             // Chebyshev degree of the finest and intermediate levels, 0: 2 and 4
     double cheb_lmax = 0.0;        // element-by-element bound of lambda_max(D^-1 K)
     // HEX20 micro elements: node-gather operator over pseudo-bricks of mesh nodes
     bool micro20 = false;
