@@ -61,12 +61,15 @@ constexpr int R = R24;
 
 struct Stream {
     hipStream_t s = nullptr;
-    // (without the call before it, whose early returns do no harm here, the destruction of a
-    // stream that was waited for by an event takes 90 us instead of 40)
+    // What the runtime still keeps of finished work goes: no wait that anything depends on (its
+    // early returns do no harm).  Without it the destruction of a stream that was waited for
+    // by an event takes 90 us instead of 40; ahead of a batch's graph it saves 40 us as well.
+    void settle() const {
+        if (s) (void)hipStreamSynchronize(s);
+    }
     ~Stream() {
-        if (!s) return;
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
+        settle();
+        if (s) (void)hipStreamDestroy(s);
     }
     int create() {
         hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
@@ -941,8 +944,11 @@ int dtc_batch_kernel_flops(dtc_batch* b, int kernel, double* avg_flops) {
 int dtc_batch_destroy(dtc_batch* b) {
     if (!b) return DTC_OK;
     const bool idle = b->wait_idle() == hipSuccess;   // then its memory is too
-    for (const auto& S : b->subs)
+    b->st.settle();
+    for (const auto& S : b->subs) {
+        S->own.settle();
         for (hipEvent_t e : S->sb.ev) (void)hipEventDestroy(e);
+    }
     Recycle r(idle);
     delete b;
     return DTC_OK;

@@ -19,5 +19,5 @@ def test_no_result_hangs_on_a_wait_by_stream_or_device():
     for f in glob.glob(os.path.join(PKG, "csrc", "*")):
         src = re.sub(r"//.*", "", open(f).read())
         calls += [os.path.basename(f)] * len(re.findall(r"\bhip(?:Stream|Device)Synchronize\s*\(", src))
-    # the one before a stream's destruction: its work has been waited for, or is given up
+    # the one before the destruction of a stream or its graph: their work has been waited for, or is given up
     assert calls == ["capi.cpp"]
