@@ -3121,6 +3121,7 @@ int apply_cap(SolverBatch& b, int64_t cap, std::vector<int64_t>& nouter, bool* a
     if (changed) {
         DTC_HIP(hipMemcpyAsync(b.done64.p, h.data(), (size_t)D * 4, hipMemcpyHostToDevice, b.stream));
         DTC_HIP(hipMemcpyAsync(b.done.p, h.data(), (size_t)D * 4, hipMemcpyHostToDevice, b.stream));
+        DTC_HIP(stream_wait(b.stream));   // h goes
     }
     *any_left = any;
     return DTC_OK;
