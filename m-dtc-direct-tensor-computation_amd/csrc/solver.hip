@@ -767,7 +767,7 @@ __global__ __launch_bounds__(NT_UPD) void k_bupdate(const int4* __restrict__ sli
 }
 
 // The FP64 form of k_bupdate (block PCG on FP64 vectors): x += P alpha,
-// r -= Q alpha with x, r, Q in FP64 and the directions P in FP32, per-brick r.r.
+// r -= Q alpha with x, r, Q in FP64 and the directions P in FP32, per-slice r.r.
 // Of the 6 threads of a row, thread q keeps load cases 4q..4q+3 (as k_bupdate).
 __global__ __launch_bounds__(NT_UPD) void k_bupdate64(const int4* __restrict__ slices, const int* __restrict__ done,
                                                      const float* __restrict__ coef, double* __restrict__ x,
@@ -1106,7 +1106,7 @@ __global__ void k_dinv(const BrickInfo* __restrict__ bricks, const DomInfo* __re
     double inv = dg != 0.0 ? 1.0 / dg : 1.0;   // PCJACOBI uses 1 for a zero diagonal
     if (is_bc(D, gx, gy, gz)) inv = 0.0;        // constrained DOFs stay zero
     for (int d = 0; d < 3; ++d) {              // one value per DOF (isotropic for the HEX08 voxel)
-        d64[3 * q + d] = inv;
+        if (d64) d64[3 * q + d] = inv;   // (the finest level only)
         d32[3 * q + d] = (float)inv;
     }
 }
@@ -2062,7 +2062,7 @@ int batch_finalize(SolverBatch& b, int precision) {
     DTC_TRY(b.part_c.ensure(nbk * R * 8));
     if (!b.micro20) DTC_TRY(b.part_ff.ensure((size_t)std::max(b.n_bricks, 1) * R * FFD * 8));
     const size_t nd = (size_t)(b.n_dom > 0 ? b.n_dom : 1);
-    for (DevMem* m : {&b.alpha, &b.beta, &b.rz, &b.rr, &b.rr0, &b.thr2, &b.scale}) DTC_TRY(m->ensure(nd * R * 8));
+    for (DevMem* m : {&b.alpha, &b.beta, &b.rz, &b.rr, &b.rr0, &b.thr2}) DTC_TRY(m->ensure(nd * R * 8));
     DTC_TRY(b.active.ensure(nd * R * 4));
     DTC_TRY(b.active64.ensure(nd * R * 4));
     DTC_TRY(b.active_prev.ensure(nd * R * 4));
@@ -2187,12 +2187,11 @@ int batch_build_mg(SolverBatch& b, int max_levels) {
         }
         DTC_HIP(hipGetLastError());
         const size_t nn = (size_t)(C.n_nodes > 0 ? C.n_nodes : 1);
-        DTC_TRY(C.dinv64.ensure(nn * 3 * 8));
         DTC_TRY(C.dinv32.ensure(nn * 3 * 4));
         for (DevMem* m : {&C.b, &C.x, &C.t, &C.d}) DTC_TRY(m->ensure(nn * 3 * R * 4));
         if (C.n_bricks > 0) {
             k_dinv<<<C.n_bricks, NO, 0, s>>>(C.brick.as<BrickInfo>(), C.dom.as<DomInfo>(), C.lat2node.as<int>(),
-                                            C.emod.as<double>(), b.kdiag, C.dinv64.as<double>(), C.dinv32.as<float>());
+                                            C.emod.as<double>(), b.kdiag, nullptr, C.dinv32.as<float>());
             DTC_HIP(hipGetLastError());
             DTC_TRY(build_clusters(s, C.cl, C.brick, C.dom, C.lat2node, C.emod, false));
             // transfer tables between this level and the finer one
@@ -2841,7 +2840,7 @@ int block_setup(SolverBatch& b) {
     DTC_TRY(b.gsum.ensure((size_t)std::max(b.n_dom, 1) * 2 * RR * 8));
     DTC_TRY(b.lfac.ensure((size_t)std::max(b.n_dom, 1) * RR * 8));
     DTC_TRY(b.bcoef.ensure((size_t)std::max(b.n_dom, 1) * RR * 4));
-    // per-slice r.r partials of the block update (fewer slices than bricks, but no assumption)
+    // per-slice r.r partials of the block update (slices of at least 32 nodes, bricks of up to 128)
     DTC_TRY(b.part_b.ensure(std::max<size_t>({sl.size(), (size_t)b.n_bricks, 1}) * R * 8));
     if (!sl.empty())
         DTC_HIP(hipMemcpyAsync(b.slices.p, sl.data(), sl.size() * sizeof(int4), hipMemcpyHostToDevice, b.stream));
@@ -3021,7 +3020,6 @@ int block_run(SolverBatch& b, const WK<float>& wk, float* x, float* r, float* p,
     auto run = [&](int64_t steps) -> int {
         DTC_HIP(hipGraphLaunch(b.block_graph.e, s));
         ++b.runs;
-        ++b.graph_launches;
         if (steps > 0) DTC_TRY(wait_done(b, b.runs - 1, &fin));   // the replay before this one
         return DTC_OK;
     };
@@ -3181,7 +3179,6 @@ int batch_solve(SolverBatch& b, const dtc_solve_opts& opts, std::vector<int64_t>
     DTC_HIP(hipGetLastError());
     for (KernelStat& k : b.kstat) k = KernelStat{};
     b.reactions_valid = false;
-    b.graph_launches = 0;
     if (b.timing) {
         // per domain group: vector bytes (FP32), moduli (FP32), Jacobi scaling (FP32), vector
         // bytes (FP64), dense element-product flops 2 (3 nen)^2 R N_e

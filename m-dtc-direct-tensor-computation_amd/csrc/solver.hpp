@@ -28,7 +28,7 @@ struct Level {
     int64_t n_nodes = 0, n_lat = 0, n_vox = 0;
     std::vector<DomInfo> h_dom;
     std::vector<BrickInfo> h_brick;
-    DevMem dom, brick, lat2node, emod, dinv64, dinv32;
+    DevMem dom, brick, lat2node, emod, dinv32;
     Clusters cl;
     DevMem rtab, ptab;             // transfer tables: restriction to this level, prolongation from it
     DevMem b, x, t, d;             // right-hand side, iterate, matvec output, Chebyshev direction
@@ -102,7 +102,7 @@ struct SolverBatch {
     DevMem part_a, part_b, part_c; // [brick][24]
     DevMem part_ff;                // [brick][24 lc][60 macro DOF slots] (HEX20: in ye20, idle then)
     // per-domain scalars [dom][24]
-    DevMem alpha, beta, rz, rr, rr0, thr2, scale;
+    DevMem alpha, beta, rz, rr, rr0, thr2;
     DevMem active, active64;       // int [dom][24]
     DevMem active_prev;            // inner activity when the residual was last replaced
     DevMem done;                   // int [dom]: inner iteration finished
@@ -130,7 +130,7 @@ struct SolverBatch {
     int precond = 0;               // DTC_PC_JACOBI / DTC_PC_MG
     int mg_degree = 0;             // Chebyshev degree of the finest and intermediate levels, 0: 2 and 4
     double cheb_lmax = 0.0;        // element-by-element bound of lambda_max(D^-1 K)
-    // HEX20 micro elements: node-gather operator over pseudo-bricks of mesh nodes
+    // HEX20 micro elements: two-pass operator (element forces, node sums) over pseudo-bricks of mesh nodes
     bool micro20 = false;
     // p-multigrid of HEX20 micro domains: the HEX08 discretisation of the same
     // voxels (a batch of its own, same domain groups, its geometric V-cycle) as
@@ -157,7 +157,6 @@ struct SolverBatch {
     DevMem itol2;                  // double [dom]: squared inner (FP32 phase) reduction of each domain group
     int precision = DTC_FP64;
     bool reactions_valid = false;
-    bool capturing = false;
     hipStream_t stream = nullptr;
     // kernel timing (off unless enabled): HIP events around the fine-level
     // launches of each timed kernel, and the algorithmic bytes of each launch
@@ -182,7 +181,6 @@ struct SolverBatch {
     DevMem runs_dev;               // uint64: runs of iterations summarised so far
     HostWords host_words;          // summary word and status of n_dom domains
     uint64_t runs = 0;             // runs launched (host count)
-    int graph_launches = 0;        // graph launches of the last solve (statistics)
 };
 
 // Walsh-basis block coefficients of the E = 1 HEX08 element stiffness.
