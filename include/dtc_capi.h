@@ -212,10 +212,10 @@ int dtc_rotation_search(const double EE[36], int criterion, double step_deg, dou
  * creation): no counterpart in the reference.  For callers that cannot
  * allocate device memory (tight serving loops, harnesses that forbid it).
  * Same arguments, results and errors as dtc_rotation_search; it runs on the
- * null stream with its buffers in a fixed per-GPU work space of 256 KB, held
+ * null stream with its buffers in a fixed per-GPU work space of 258 KB, held
  * until the process ends, which bounds the initial sweep to
  * dtc_rotation_noalloc_max_points() grid points (about 33 M: an initial step
- * of 0.45 degrees or more; 1 degree needs 25 KB).  A larger sweep is
+ * of 0.45 degrees or more; 1 degree needs 27 KB).  A larger sweep is
  * rejected with DTC_ERR_BAD_ARGUMENT.  Calls that overlap on one GPU share the
  * work space and race: serialise them per GPU. */
 int dtc_rotation_search_noalloc(const double EE[36], int criterion, double step_deg, double num_zero,
@@ -224,12 +224,13 @@ int dtc_rotation_search_noalloc(const double EE[36], int criterion, double step_
 int64_t dtc_rotation_noalloc_max_points(void);
 
 /* ---- memory ---------------------------------------------------------------
- * The library keeps device memory of finished calls and destroyed batches for the next
- * ones: at most 4 GiB, and a block not taken for 20 s goes at the next call that
- * allocates or frees.  It is emptied when an allocation of the library fails; a program that
- * wants the memory for others (another library, another process) frees it here.  Memory
- * that a batch or a running call uses is not touched.  Any thread, any time; no
- * counterpart in the reference (host allocations only). */
+ * The library keeps memory of finished calls and destroyed batches for the next
+ * ones: at most 4 GiB of device memory and 32 MiB of page-locked memory; a
+ * block not taken for 20 s goes at the next call that allocates or frees, all
+ * of it when an allocation of the library fails.  A program that wants the
+ * memory for others (another library, another process) frees it here.  Memory
+ * that a batch or a running call uses is not touched.  Any thread, any time;
+ * no counterpart in the reference (host allocations only). */
 int dtc_release_memory(void);
 
 #ifdef __cplusplus

@@ -57,8 +57,9 @@ int wait_word(hipStream_t s, const unsigned long long* w, unsigned long long v);
 // and Recycle below; anything else is freed), so that any thread may take it out for any
 // stream.  What is kept is bounded (POOL_BYTES, POOL_PINNED), the oldest goes first, what
 // was not used for POOL_SECONDS is freed at the next call that uses the pool, and all of it
-// when an allocation fails or the program asks (dtc_release_memory).  Streams are not kept: kept ones end up on one hardware queue,
-// and the parts of a batch no longer overlap (40 domains of 21^3 61 -> 70 ms).
+// when an allocation fails or the program asks (dtc_release_memory).  Streams are not kept:
+// kept ones end up on one hardware queue, and the parts of a batch no longer overlap (40
+// domains of 21^3 61 -> 70 ms).
 constexpr size_t POOL_BYTES = (size_t)4 << 30;
 // (page-locked: blocks kept, and the largest; a multigrid solve takes up to a dozen sizes)
 constexpr size_t POOL_PINNED = 32, POOL_PINNED_BYTES = (size_t)1 << 20;

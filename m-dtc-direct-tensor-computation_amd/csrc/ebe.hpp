@@ -119,7 +119,7 @@ struct EbeArgs {
 // What bounds it (16 trabecular 64^3 domains, 1.25 M nodes, one launch over all of them):
 // the vector cache's lookups (65-80 % busy: a load of x takes one per 32-byte run) and the
 // VALU (55 %) together, with 12 waves a CU, as many as the LDS accumulators allow; the
-// Chebyshev step also moves 1.8 GB (4.4 TB/s, a copy reaches 4.9).  Against bricks staged in LDS
+// Chebyshev step also moves 1.66 GB (4.2 TB/s, a copy reaches 5.1).  Against bricks staged in LDS
 // in six load-case chunks with corner buffers and two barriers a chunk (16 waves, most
 // lanes idle on sparse bricks): Q = K P 678 -> 340 us, Chebyshev step 762 -> 411, residual
 // before restriction 693 -> 354, FP64 residual 4114 -> 960.  Measured beside it: clusters of
