@@ -16,8 +16,10 @@ def test_no_result_hangs_on_a_wait_by_stream_or_device():
     names = {line.split()[-1].split("@")[0] for line in out.splitlines()}
     assert "hipEventSynchronize" in names and "hipDeviceSynchronize" not in names
     calls = []
-    for f in glob.glob(os.path.join(PKG, "csrc", "*")):
+    for f in sorted(glob.glob(os.path.join(PKG, "csrc", "*"))):
         src = re.sub(r"//.*", "", open(f).read())
-        calls += [os.path.basename(f)] * len(re.findall(r"\bhip(?:Stream|Device)Synchronize\s*\(", src))
-    # the one before the destruction of a stream or its graph: their work has been waited for, or is given up
-    assert calls == ["capi.cpp"]
+        calls += [(os.path.basename(f), src[m.end():m.end() + 80])
+                  for m in re.finditer(r"\bhip(?:Stream|Device)Synchronize\s*\(", src)]
+    # one ahead of the event's wait, one before the destruction of a stream or its graph
+    assert [c[0] for c in calls] == ["capi.cpp", "dtc_internal.hpp"]
+    assert "hipEventSynchronize" in calls[1][1]
